@@ -75,6 +75,10 @@ static const uint32_t kPairVecBT = 16;
 //! koff[k] = (k / kd) ks0 + (k % kd) ks1 and noff[n] likewise, computed in
 //! the kernel instead of read.
 static const uint32_t kPairOffArith = 32;
+//! B whose consecutive columns are adjacent in memory.
+static const uint32_t kPairBNFast = 64;
+//! Every A row of the pair has coefficient 1.
+static const uint32_t kPairUnit = 128;
 
 //! Work item of a grouped GEMM launch: one output tile of one C block.
 struct gemm_tile {
@@ -87,37 +91,42 @@ struct gemm_tile {
 //! k chunks dealt to the waves, operands loaded straight into MFMA
 //! fragments, partial tiles summed in LDS in a fixed order.
 //! STACK_*: the split-K kernels over stacks (C blocks sharing their B
-//! operands, rows concatenated; _On: compiled for n waves per SIMD; LDS: A
-//! chunks staged in LDS for two column halves, two k groups; _P1:
-//! the two-stage pipeline that loads a pair's row table when it starts
-//! the pair's first chunk); used by grouped launches, per-block launches
-//! run the SPLITK configuration of the same shape.
+//! operands, rows concatenated; _On: compiled for n waves per SIMD); used by
+//! grouped launches, per-block launches run the SPLITK configuration of the
+//! same shape.  WG_*_Gn: workgroup tiles over stacks with both operands
+//! staged in LDS, the k chunks dealt to n groups of four waves (grouped and
+//! per-block launches).
 enum { TILE_64x64 = 0, TILE_32x64 = 1, TILE_64x32 = 2, TILE_32x32 = 3,
        SPLITK_16x64_W4 = 4, SPLITK_32x32_W4 = 5, SPLITK_32x64_W4 = 6,
        SPLITK_64x32_W4 = 7, SPLITK_16x64_W2 = 8, SPLITK_32x32_W2 = 9,
        SPLITK_16x32_W4 = 10, SPLITK_32x16_W4 = 11,
-       STACK_16x64_W4 = 12, STACK_32x32_W4 = 13, STACK_32x64_W4 = 14,
-       STACK_64x32_W4 = 15, STACK_48x64_W4 = 16, STACK_64x48_W4 = 17,
-       STACK_48x32_W4 = 18, STACK_64x32_W4_P1 = 19, STACK_64x48_W2 = 20,
-       STACK_48x64_W2 = 21, STACK_48x32_W4_O2 = 22, STACK_32x32_W4_O3 = 23,
-       STACK_16x64_W4_O3 = 24, STACK_VAR_64x32_W4 = 25, STACK_VAR_64x48_W4 = 26,
-       STACK_LDS_64x64 = 27, TILE_COUNT = 28 };
+       STACK_16x64_W4 = 12, STACK_32x32_W4 = 13, WG_32x64_G4 = 14,
+       WG_80x64_G2 = 15, WG_48x64_G4 = 16, WG_64x64_G4 = 17,
+       STACK_48x32_W4 = 18, WG_64x64_G1 = 19, WG_96x64_G1 = 20,
+       WG_112x64_G1 = 21, STACK_48x32_W4_O2 = 22, STACK_32x32_W4_O3 = 23,
+       STACK_16x64_W4_O3 = 24, STACK_VAR_64x32_W4 = 25, WG_32x64_G2 = 26,
+       WG_16x64_G4 = 27, TILE_COUNT = 28 };
 void tile_shape(int cfg, uint32_t &bm, uint32_t &bn);
-inline bool is_stacked(int cfg) { return cfg >= STACK_16x64_W4 && cfg <= STACK_LDS_64x64; }
+inline bool is_stacked(int cfg) { return cfg >= STACK_16x64_W4 && cfg < TILE_COUNT; }
+//! Workgroup-tiled stacked configurations (launch_gemm_tile, also per C block).
+inline bool is_tile(int cfg) {
+    switch(cfg) {
+    case WG_32x64_G4: case WG_80x64_G2: case WG_48x64_G4: case WG_64x64_G4: case WG_64x64_G1:
+    case WG_96x64_G1: case WG_112x64_G1: case WG_32x64_G2: case WG_16x64_G4: return true;
+    default: return false;
+    }
+}
 //! Stacked configurations over tiles of varying shape (var_tile lists).
-inline bool is_var(int cfg) { return cfg == STACK_VAR_64x32_W4 || cfg == STACK_VAR_64x48_W4; }
+inline bool is_var(int cfg) { return cfg == STACK_VAR_64x32_W4; }
 //! The per-C-block configuration with the same summation order (same
 //! split-K width; the tile shape only partitions the output).
 inline int unstacked(int cfg) {
     switch(cfg) {
     case STACK_16x64_W4: return SPLITK_16x64_W4;
     case STACK_32x32_W4: return SPLITK_32x32_W4;
-    case STACK_32x64_W4: case STACK_48x64_W4: return SPLITK_32x64_W4;
-    case STACK_64x32_W4: case STACK_64x48_W4: case STACK_48x32_W4: case STACK_64x32_W4_P1:
-    case STACK_48x32_W4_O2: case STACK_32x32_W4_O3: case STACK_16x64_W4_O3:
-    case STACK_VAR_64x32_W4: case STACK_VAR_64x48_W4:
+    case STACK_48x32_W4: case STACK_48x32_W4_O2: case STACK_32x32_W4_O3: case STACK_16x64_W4_O3:
+    case STACK_VAR_64x32_W4:
         return SPLITK_64x32_W4;
-    case STACK_64x48_W2: case STACK_48x64_W2: case STACK_LDS_64x64: return SPLITK_32x32_W2;
     default: return cfg;
     }
 }
@@ -144,13 +153,15 @@ struct stack_pair {
     //! noff[n] = (n / nd) ns0 + (n % nd) ns1
     fastdiv kd, nd;
     int32_t ks0, ks1, ns0, ns1;
+    const double *a;                  //!< lowest address of the pair's A rows (workgroup-tiled kernels)
 };
 //! A operand of one row for one pair: row r of A at p[k] (or p[k * lda]
 //! with kPairAKMajor), coefficient d.
 struct stack_arow {
     const double *p;
     double d;
-    uint32_t lda, pad;
+    uint32_t lda;
+    uint32_t off;                     //!< bytes of p from the pair's a
 };
 struct stack_crow {
     double *c;                        //!< start of the row in its C block
@@ -166,6 +177,18 @@ struct var_tile {
 hipError_t launch_gemm_stacked_var(int cfg, const stack_desc *st, const stack_pair *sp,
     const stack_arow *ar, const stack_crow *cr, const var_tile *tiles, uint32_t ntiles,
     hipStream_t s);
+//! A stack as the workgroup-tiled kernels read it: its lists by address, so
+//! stacks of several plans share a launch; row r of pair j reads A through
+//! arow[j * astride + r].
+struct tile_stack {
+    const stack_pair *pairs;
+    const stack_arow *arow;
+    const stack_crow *crow;
+    uint32_t rows, astride, n, npairs;
+    uint32_t nchunk, pad;
+};
+hipError_t launch_gemm_tile(int cfg, const tile_stack *st, const gemm_tile *tiles,
+    uint32_t ntiles, hipStream_t s);
 hipError_t launch_gemm_stacked(int cfg, const stack_desc *st, const stack_pair *sp,
     const stack_arow *ar, const stack_crow *cr, const gemm_tile *tiles, uint32_t ntiles,
     hipStream_t s);

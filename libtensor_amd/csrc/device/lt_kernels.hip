@@ -40,19 +40,17 @@ void tile_shape(int cfg, uint32_t &bm, uint32_t &bn) {
     case TILE_32x64: bm = 32; bn = 64; break;
     case TILE_64x32: bm = 64; bn = 32; break;
     case TILE_32x32: bm = 32; bn = 32; break;
-    case SPLITK_16x64_W4: case SPLITK_16x64_W2: case STACK_16x64_W4: bm = 16; bn = 64; break;
-    case SPLITK_32x32_W4: case SPLITK_32x32_W2: case STACK_32x32_W4: bm = 32; bn = 32; break;
-    case SPLITK_32x64_W4: case STACK_32x64_W4: bm = 32; bn = 64; break;
-    case SPLITK_64x32_W4: case STACK_64x32_W4: case STACK_64x32_W4_P1: bm = 64; bn = 32; break;
-    case STACK_LDS_64x64: bm = 64; bn = 64; break;
-    case STACK_48x64_W4: bm = 48; bn = 64; break;
-    case STACK_64x48_W4: bm = 64; bn = 48; break;
-    case STACK_48x32_W4: bm = 48; bn = 32; break;
-    case STACK_64x48_W2: bm = 64; bn = 48; break;
-    case STACK_48x64_W2: bm = 48; bn = 64; break;
-    case STACK_48x32_W4_O2: bm = 48; bn = 32; break;
-    case STACK_32x32_W4_O3: bm = 32; bn = 32; break;
-    case STACK_16x64_W4_O3: bm = 16; bn = 64; break;
+    case SPLITK_16x64_W4: case SPLITK_16x64_W2: case STACK_16x64_W4: case STACK_16x64_W4_O3:
+    case WG_16x64_G4: bm = 16; bn = 64; break;
+    case SPLITK_32x32_W4: case SPLITK_32x32_W2: case STACK_32x32_W4: case STACK_32x32_W4_O3:
+        bm = 32; bn = 32; break;
+    case SPLITK_32x64_W4: case WG_32x64_G4: case WG_32x64_G2: bm = 32; bn = 64; break;
+    case SPLITK_64x32_W4: bm = 64; bn = 32; break;
+    case WG_48x64_G4: bm = 48; bn = 64; break;
+    case WG_80x64_G2: bm = 80; bn = 64; break;
+    case WG_96x64_G1: bm = 96; bn = 64; break;
+    case WG_112x64_G1: bm = 112; bn = 64; break;
+    case STACK_48x32_W4: case STACK_48x32_W4_O2: bm = 48; bn = 32; break;
     case SPLITK_16x32_W4: bm = 16; bn = 32; break;
     case SPLITK_32x16_W4: bm = 32; bn = 16; break;
     default: bm = 64; bn = 64; break;
@@ -789,126 +787,6 @@ __device__ __forceinline__ void seek_chunk_st(const stack_pair *__restrict__ sp,
     }
 }
 
-//! Operand forms of a stacked pair with a branch-free load path: A in
-//! 16-byte row loads and B k-contiguous (VA_VB), row-major (VA_ROW), through
-//! computed offsets element by element (VA_AR) or in 16-byte pairs
-//! (VA_VTAR); everything else takes the general path (ANY).
-enum { ST_FORM_ANY = 0, ST_FORM_VA_VB = 1, ST_FORM_VA_ROW = 2, ST_FORM_VA_AR = 3,
-       ST_FORM_VA_VTAR = 4 };
-
-__device__ __forceinline__ int st_form(const stack_pair &sp) {
-    const uint32_t f = sp.flags;
-    if(!(f & kPairVecA)) return ST_FORM_ANY;
-    if(f & kPairVecB) return ST_FORM_VA_VB;
-    if(f & kPairVecBT) return (f & kPairOffArith) ? ST_FORM_VA_VTAR : ST_FORM_ANY;
-    if(f & kPairOffArith) return ST_FORM_VA_AR;
-    if(!sp.koff && !(f & kPairBNMajor)) return ST_FORM_VA_ROW;
-    return ST_FORM_ANY;
-}
-
-//! Row sources of one pair without the B column offsets (computed or read
-//! when the operands are loaded, so the row table loads do not wait for the
-//! pair's descriptor).
-template<int FM, int FN>
-__device__ __forceinline__ void st_rows_a(st_rowsrc<FM, FN> &r, const stack_arow *__restrict__ arow,
-    uint32_t base, const int (&srow)[FM]) {
-#pragma unroll
-    for(int i = 0; i < FM; i++) {
-        const stack_arow e = arow[base + srow[i]];
-        r.p[i] = e.p;
-        r.d[i] = e.d;
-        r.lda[i] = e.lda;
-    }
-}
-
-template<int FM, int FN>
-__device__ __forceinline__ void st_cols(st_rowsrc<FM, FN> &r, const stack_pair &sp,
-    const int (&bcol)[FN]) {
-    if(sp.flags & kPairOffArith) {
-#pragma unroll
-        for(int f = 0; f < FN; f++) r.no[f] = off_arith(uint32_t(bcol[f]), sp.nd, sp.ns0, sp.ns1);
-    } else {
-#pragma unroll
-        for(int f = 0; f < FN; f++) r.no[f] = sp.noff ? sp.noff[bcol[f]] : 0;
-    }
-}
-
-//! B operand forms without a condition on A (for kernels that stage A
-//! separately): the same forms as st_form.
-__device__ __forceinline__ int st_bform(const stack_pair &sp) {
-    const uint32_t f = sp.flags;
-    if(f & kPairVecB) return ST_FORM_VA_VB;
-    if(f & kPairVecBT) return (f & kPairOffArith) ? ST_FORM_VA_VTAR : ST_FORM_ANY;
-    if(f & kPairOffArith) return ST_FORM_VA_AR;
-    if(!sp.koff && !(f & kPairBNMajor)) return ST_FORM_VA_ROW;
-    return ST_FORM_ANY;
-}
-
-//! B operand of one chunk in the pair's B form (FORM != ANY: no branches).
-template<int FM, int FN, int FORM>
-__device__ __forceinline__ void load_b_form(double (&bf)[FN][4], st_rowsrc<FM, FN> &ar,
-    const stack_pair &sp, int c, const int (&bcol)[FN], int lg) {
-    if(FORM == ST_FORM_ANY) {
-        st_cols<FM, FN>(ar, sp, bcol);
-        load_b_st<FM, FN>(bf, ar, sp, c, bcol, lg);
-        return;
-    }
-    const uint32_t K = sp.k;
-    const uint32_t kk = 16 * c + 4 * lg;
-    const uint32_t k0 = min(kk, K - 2), k2 = min(kk + 2, K - 2);
-    if(FORM == ST_FORM_VA_VB) {
-#pragma unroll
-        for(int f = 0; f < FN; f++) {
-            gdouble *pb = (gdouble *)sp.b + size_t(uint32_t(bcol[f]) * sp.ldb);
-            const double2_t v0 = *(gdouble2 *)(pb + k0);
-            const double2_t v1 = *(gdouble2 *)(pb + k2);
-            bf[f][0] = v0.x; bf[f][1] = v0.y; bf[f][2] = v1.x; bf[f][3] = v1.y;
-        }
-        return;
-    }
-    int32_t no[FN];
-#pragma unroll
-    for(int f = 0; f < FN; f++)
-        no[f] = FORM == ST_FORM_VA_ROW ? bcol[f] : off_arith(uint32_t(bcol[f]), sp.nd, sp.ns0, sp.ns1);
-    if(FORM == ST_FORM_VA_VTAR) {
-        load_b_vt<FN, 2>(bf, no, sp, k0, k2);
-        return;
-    }
-    uint32_t kc[4];
-#pragma unroll
-    for(int j = 0; j < 4; j++) kc[j] = min(kk + j, K - 1);
-    int32_t ko[4];
-#pragma unroll
-    for(int j = 0; j < 4; j++)
-        ko[j] = FORM == ST_FORM_VA_ROW ? int32_t(kc[j] * sp.ldb) : off_arith(kc[j], sp.kd, sp.ks0, sp.ks1);
-#pragma unroll
-    for(int f = 0; f < FN; f++)
-#pragma unroll
-        for(int j = 0; j < 4; j++) bf[f][j] = ldg(sp.b, 8u * uint32_t(ko[j] + no[f]));
-}
-
-//! Operands of one chunk in the pair's form (FORM != ANY: no branches).
-template<int FM, int FN, int FORM>
-__device__ __forceinline__ void load_form(double (&af)[FM][4], double (&bf)[FN][4],
-    st_rowsrc<FM, FN> &ar, const stack_pair &sp, int c, const int (&bcol)[FN], int lg) {
-    if(FORM == ST_FORM_ANY) {
-        st_cols<FM, FN>(ar, sp, bcol);
-        load_chunk_st_any<FM, FN>(af, bf, ar, sp, c, bcol, lg);
-        return;
-    }
-    const uint32_t K = sp.k;
-    const uint32_t kk = 16 * c + 4 * lg;
-    const uint32_t k0 = min(kk, K - 2), k2 = min(kk + 2, K - 2);
-#pragma unroll
-    for(int i = 0; i < FM; i++) {
-        gdouble *pa = (gdouble *)ar.p[i];
-        const double2_t v0 = *(gdouble2 *)(pa + k0);
-        const double2_t v1 = *(gdouble2 *)(pa + k2);
-        af[i][0] = v0.x; af[i][1] = v0.y; af[i][2] = v1.x; af[i][3] = v1.y;
-    }
-    load_b_form<FM, FN, FORM>(bf, ar, sp, c, bcol, lg);
-}
-
 //! Cursor of a wave over its chunks of a stack's pair list (pair p, chunk
 //! c of that pair) with the pair's descriptor and the lane's row sources.
 //! After the last chunk it stays on it with valid = false, so a load issued
@@ -943,75 +821,20 @@ __device__ __forceinline__ void st_advance(st_cursor<FM, FN> &u,
     u.c = c;
 }
 
-//! As st_advance, loading only the new pair's row sources (st_rows_a).
 template<int FM, int FN, int W>
-__device__ __forceinline__ void st_advance_a(st_cursor<FM, FN> &u,
-    const stack_pair *__restrict__ spairs, const stack_arow *__restrict__ arow,
-    const stack_desc &st, const int (&srow)[FM]) {
-    if(!u.valid) return;
-    int c = u.c + W;
-    const int nch = (int(u.sp.k) + 15) >> 4;
-    if(c < nch) { u.c = c; return; }
-    uint32_t p = u.p + 1;
-    const uint32_t pend = st.pair_begin + st.npairs;
-    c -= nch;
-    seek_chunk_st(spairs, pend, p, c);
-    if(p >= pend) { u.valid = false; return; }
-    u.sp = spairs[p];
-    st_rows_a<FM, FN>(u.r, arow, st.arow_begin + (p - st.pair_begin) * st.rows, srow);
-    u.p = p;
-    u.c = c;
-}
-
-//! Loads chunk u (in its pair's form) and multiplies the chunk held in
-//! (ac, bc): one basic block per form, so the scheduler can interleave the
-//! loads with the products.
-template<int FM, int FN>
-__device__ __forceinline__ void st_step(double4_t (&acc)[FM][FN], double (&an)[FM][4],
-    double (&bn)[FN][4], st_cursor<FM, FN> &u, double (&ac)[FM][4], const double (&bc)[FN][4],
-    const double (&dc)[FM], uint32_t kc, int cc, const int (&bcol)[FN], int lg) {
-    switch(st_form(u.sp)) {
-    case ST_FORM_VA_VB:
-        load_form<FM, FN, ST_FORM_VA_VB>(an, bn, u.r, u.sp, u.c, bcol, lg);
-        mma_chunk_st<FM, FN>(acc, ac, bc, dc, kc, cc, lg);
-        break;
-    case ST_FORM_VA_ROW:
-        load_form<FM, FN, ST_FORM_VA_ROW>(an, bn, u.r, u.sp, u.c, bcol, lg);
-        mma_chunk_st<FM, FN>(acc, ac, bc, dc, kc, cc, lg);
-        break;
-    case ST_FORM_VA_AR:
-        load_form<FM, FN, ST_FORM_VA_AR>(an, bn, u.r, u.sp, u.c, bcol, lg);
-        mma_chunk_st<FM, FN>(acc, ac, bc, dc, kc, cc, lg);
-        break;
-    case ST_FORM_VA_VTAR:
-        load_form<FM, FN, ST_FORM_VA_VTAR>(an, bn, u.r, u.sp, u.c, bcol, lg);
-        mma_chunk_st<FM, FN>(acc, ac, bc, dc, kc, cc, lg);
-        break;
-    default:
-        load_form<FM, FN, ST_FORM_ANY>(an, bn, u.r, u.sp, u.c, bcol, lg);
-        mma_chunk_st<FM, FN>(acc, ac, bc, dc, kc, cc, lg);
-        break;
-    }
-}
-
-template<int FM, int FN, int W, int PIPE>
 __device__ __forceinline__ void stacked_body(const stack_desc *__restrict__ stacks,
     const stack_pair *__restrict__ spairs, const stack_arow *__restrict__ arow,
     const stack_crow *__restrict__ crow, const gemm_tile *__restrict__ tiles,
     uint32_t ntiles, double *red);
 
-//! PIPE 0: one chunk in registers at a time; 1: the next chunk's operands
-//! load during the current chunk's products; 2: also the descriptor and row
-//! sources of the chunk after that; 3: as 2, with one branch-free block of
-//! loads and products per operand form.
-template<int FM, int FN, int W, int PIPE>
+template<int FM, int FN, int W>
 __global__ void __launch_bounds__(64 * W)
 gemm_stacked_kernel(const stack_desc *__restrict__ stacks,
     const stack_pair *__restrict__ spairs, const stack_arow *__restrict__ arow,
     const stack_crow *__restrict__ crow, const gemm_tile *__restrict__ tiles,
     uint32_t ntiles) {
     __shared__ double red[(W > 1 ? W - 1 : 1) * FM * FN * 4 * 64];
-    stacked_body<FM, FN, W, PIPE>(stacks, spairs, arow, crow, tiles, ntiles, red);
+    stacked_body<FM, FN, W>(stacks, spairs, arow, crow, tiles, ntiles, red);
 }
 
 //! The same kernel compiled for OCC waves per SIMD (register budget
@@ -1023,11 +846,11 @@ gemm_stacked_occ_kernel(const stack_desc *__restrict__ stacks,
     const stack_crow *__restrict__ crow, const gemm_tile *__restrict__ tiles,
     uint32_t ntiles) {
     __shared__ double red[(W > 1 ? W - 1 : 1) * FM * FN * 4 * 64];
-    stacked_body<FM, FN, W, 2>(stacks, spairs, arow, crow, tiles, ntiles, red);
+    stacked_body<FM, FN, W>(stacks, spairs, arow, crow, tiles, ntiles, red);
 }
 
 //! One (16 FM) x (16 FN) tile of a stack at rows m0, columns n0.
-template<int FM, int FN, int W, int PIPE>
+template<int FM, int FN, int W>
 __device__ __forceinline__ void stacked_tile(const stack_desc &st,
     const stack_pair *__restrict__ spairs, const stack_arow *__restrict__ arow,
     const stack_crow *__restrict__ crow, int m0, int n0, double *red) {
@@ -1055,56 +878,7 @@ __device__ __forceinline__ void stacked_tile(const stack_desc &st,
     uint32_t px = pbeg;
     int cx = wave;
     seek_chunk_st(spairs, pend, px, cx);
-    if(PIPE == 0) {
-        // single buffer: fewer registers, latency hidden by other waves
-        double ax[FM][4], bx[FN][4];
-        st_rowsrc<FM, FN> rx;
-        uint32_t pr = 0xffffffffu;
-        stack_pair sx;
-        while(px < pend) {
-            if(px != pr) {
-                sx = spairs[px];
-                st_rows<FM, FN>(rx, arow, st.arow_begin + (px - pbeg) * st.rows, srow, sx, bcol);
-                pr = px;
-            }
-            load_chunk_st_any<FM, FN>(ax, bx, rx, sx, cx, bcol, lg);
-            mma_chunk_st<FM, FN>(acc, ax, bx, rx.d, sx.k, cx, lg);
-            cx += W;
-            seek_chunk_st(spairs, pend, px, cx);
-        }
-    } else if(PIPE == 1 && px < pend) {
-        double ax[FM][4], bx[FN][4], ay[FM][4], by[FN][4];
-        st_rowsrc<FM, FN> rx, ry;
-        stack_pair sx = spairs[px];
-        st_rows<FM, FN>(rx, arow, st.arow_begin + (px - pbeg) * st.rows, srow, sx, bcol);
-        load_chunk_st_any<FM, FN>(ax, bx, rx, sx, cx, bcol, lg);
-        while(true) {
-            uint32_t py = px;
-            int cy = cx + W;
-            seek_chunk_st(spairs, pend, py, cy);
-            const bool hy = py < pend;
-            if(!hy) { py = px; cy = cx; }       // dummy in-bounds load
-            const stack_pair sy = spairs[py];
-            if(py == px) ry = rx;
-            else st_rows<FM, FN>(ry, arow, st.arow_begin + (py - pbeg) * st.rows, srow, sy, bcol);
-            load_chunk_st_any<FM, FN>(ay, by, ry, sy, cy, bcol, lg);
-            mma_chunk_st<FM, FN>(acc, ax, bx, rx.d, sx.k, cx, lg);
-            if(!hy) break;
-            uint32_t pz = py;
-            int cz = cy + W;
-            seek_chunk_st(spairs, pend, pz, cz);
-            const bool hz = pz < pend;
-            if(!hz) { pz = py; cz = cy; }
-            sx = spairs[pz];
-            if(pz == py) rx = ry;
-            else st_rows<FM, FN>(rx, arow, st.arow_begin + (pz - pbeg) * st.rows, srow, sx, bcol);
-            load_chunk_st_any<FM, FN>(ax, bx, rx, sx, cz, bcol, lg);
-            mma_chunk_st<FM, FN>(acc, ay, by, ry.d, sy.k, cy, lg);
-            if(!hz) break;
-            px = pz;
-            cx = cz;
-        }
-    } else if(PIPE == 2 && px < pend) {
+    if(px < pend) {
         // three stages: operands of chunk i + 1 and the descriptor and row
         // sources of chunk i + 2 are in flight during the products of chunk i
         st_cursor<FM, FN> u;
@@ -1141,44 +915,6 @@ __device__ __forceinline__ void stacked_tile(const stack_desc &st,
             ccx = u.c;
             st_advance<FM, FN, W>(u, spairs, arow, st, srow, bcol);
             mma_chunk_st<FM, FN>(acc, ay, by, dy, ky, ccy, lg);
-            if(!vx) break;
-        }
-    } else if(PIPE == 3 && px < pend) {
-        // u1: the chunk loaded during the current products; u2: the chunk
-        // after it, whose descriptor and row sources load one step earlier
-        st_cursor<FM, FN> u1, u2;
-        u1.p = px;
-        u1.c = cx;
-        u1.valid = true;
-        u1.sp = spairs[px];
-        st_rows_a<FM, FN>(u1.r, arow, st.arow_begin + (px - pbeg) * st.rows, srow);
-        double ax[FM][4], bx[FN][4], ay[FM][4], by[FN][4];
-        double dx[FM], dy[FM];
-        load_form<FM, FN, ST_FORM_ANY>(ax, bx, u1.r, u1.sp, u1.c, bcol, lg);
-#pragma unroll
-        for(int i = 0; i < FM; i++) dx[i] = u1.r.d[i];
-        uint32_t kx = u1.sp.k, ky;
-        int ccx = u1.c, ccy;
-        u2 = u1;
-        st_advance_a<FM, FN, W>(u2, spairs, arow, st, srow);
-        while(true) {
-            u1 = u2;
-            st_advance_a<FM, FN, W>(u2, spairs, arow, st, srow);
-            const bool vy = u1.valid;           // else a dummy in-bounds load
-            st_step<FM, FN>(acc, ay, by, u1, ax, bx, dx, kx, ccx, bcol, lg);
-#pragma unroll
-            for(int i = 0; i < FM; i++) dy[i] = u1.r.d[i];
-            ky = u1.sp.k;
-            ccy = u1.c;
-            if(!vy) break;
-            u1 = u2;
-            st_advance_a<FM, FN, W>(u2, spairs, arow, st, srow);
-            const bool vx = u1.valid;
-            st_step<FM, FN>(acc, ax, bx, u1, ay, by, dy, ky, ccy, bcol, lg);
-#pragma unroll
-            for(int i = 0; i < FM; i++) dx[i] = u1.r.d[i];
-            kx = u1.sp.k;
-            ccx = u1.c;
             if(!vx) break;
         }
     }
@@ -1234,7 +970,7 @@ __device__ __forceinline__ void stacked_tile(const stack_desc &st,
     if(W > 1) __syncthreads();   // red is reused by the next tile
 }
 
-template<int FM, int FN, int W, int PIPE>
+template<int FM, int FN, int W>
 __device__ __forceinline__ void stacked_body(const stack_desc *__restrict__ stacks,
     const stack_pair *__restrict__ spairs, const stack_arow *__restrict__ arow,
     const stack_crow *__restrict__ crow, const gemm_tile *__restrict__ tiles,
@@ -1242,276 +978,35 @@ __device__ __forceinline__ void stacked_body(const stack_desc *__restrict__ stac
     for(uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         const gemm_tile tile = tiles[t];
         const stack_desc st = stacks[tile.cblock];
-        stacked_tile<FM, FN, W, PIPE>(st, spairs, arow, crow, int(tile.tm) * 16 * FM,
+        stacked_tile<FM, FN, W>(st, spairs, arow, crow, int(tile.tm) * 16 * FM,
             int(tile.tn) * 16 * FN, red);
     }
 }
 
-// LDS-staged stacked kernel.  A workgroup of four waves computes a
-// (16 FM) x (32 FN) tile: waves g = 0, 1 (k group) x h = 0, 1 (column half).
-// The chunks of the stack's pair list are dealt to the two k groups in turn
-// (as to the two waves of the two-wave split-K kernels); the two waves of a
-// group share the group's A chunk, staged in LDS once per chunk (each lane
-// loads 16 bytes of one row, scaled by the row coefficient and zeroed past
-// the extent), and load their own B columns into registers.  Group 1's
-// partial tile is added to group 0's in LDS at the end, so every C element
-// gets the same sums in the same order as in the two-wave split-K kernels.
-static const int kLdsRowStride = 18;    // doubles per staged A row (144 bytes)
-
-//! Staging of one A chunk: lane (row srw + 16 j, segment seg) holds k =
-//! 16 c + 2 seg and 2 seg + 1 of its rows.
-template<int FM, int FN>
-__device__ __forceinline__ void lds_stage_load(double2_t (&sa)[FM], const st_rowsrc<FM, FN> &r,
-    const stack_pair &sp, int c, int seg) {
-    const uint32_t K = sp.k;
-    const uint32_t k = 16 * c + 2 * seg;
-    if(sp.flags & kPairVecA) {
-        const uint32_t k0 = min(k, K - 2);
-#pragma unroll
-        for(int j = 0; j < FM; j++) sa[j] = *(gdouble2 *)((gdouble *)r.p[j] + k0);
-        return;
-    }
-    const uint32_t k0 = min(k, K - 1), k1 = min(k + 1, K - 1);
-    if(sp.flags & kPairAKMajor) {
-#pragma unroll
-        for(int j = 0; j < FM; j++) {
-            gdouble *pa = (gdouble *)r.p[j];
-            sa[j].x = pa[k0 * r.lda[j]];
-            sa[j].y = pa[k1 * r.lda[j]];
-        }
-    } else {
-#pragma unroll
-        for(int j = 0; j < FM; j++) {
-            gdouble *pa = (gdouble *)r.p[j];
-            sa[j].x = pa[k0];
-            sa[j].y = pa[k1];
-        }
-    }
-}
-
-template<int FM, int FN>
-__device__ __forceinline__ void lds_stage_store(double *buf, const double2_t (&sa)[FM],
-    const st_rowsrc<FM, FN> &r, uint32_t K, int c, int srw, int seg) {
-    const uint32_t k = 16 * c + 2 * seg;
-    const bool v0 = k < K, v1 = k + 1 < K;
-#pragma unroll
-    for(int j = 0; j < FM; j++) {
-        double2_t w;
-        w.x = sa[j].x * (v0 ? r.d[j] : 0.0);
-        w.y = sa[j].y * (v1 ? r.d[j] : 0.0);
-        *(double2_t *)(buf + (srw + 16 * j) * kLdsRowStride + 2 * seg) = w;
-    }
-}
-
-//! One step of the LDS-staged tile: stage chunk un (A through registers into
-//! wbuf, zeros when un is past the group's last chunk; B into bn) while the
-//! chunk staged in rbuf (with B in bc) is multiplied.  One basic block per
-//! B form.
-template<int FM, int FN, int FORM>
-__device__ __forceinline__ void lds_step(double4_t (&acc)[FM][FN], double (&bn)[FN][4],
-    const double (&bc)[FN][4], st_cursor<FM, FN> &un, const double *rbuf, double *wbuf,
-    const int (&bcol)[FN], int lr, int lg, int srw, int seg) {
-    double2_t sa[FM];
-    lds_stage_load<FM, FN>(sa, un.r, un.sp, un.c, seg);
-    load_b_form<FM, FN, FORM>(bn, un.r, un.sp, un.c, bcol, lg);
-    double af[FM][4];
-#pragma unroll
-    for(int i = 0; i < FM; i++) {
-        const double *rp = rbuf + (16 * i + lr) * kLdsRowStride + 4 * lg;
-        const double2_t v0 = *(const double2_t *)rp;
-        const double2_t v1 = *(const double2_t *)(rp + 2);
-        af[i][0] = v0.x; af[i][1] = v0.y; af[i][2] = v1.x; af[i][3] = v1.y;
-    }
-#pragma unroll
-    for(int q = 0; q < 4; q++)
-#pragma unroll
-        for(int i = 0; i < FM; i++)
-#pragma unroll
-            for(int j = 0; j < FN; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i][q], bc[j][q], acc[i][j],
-                    0, 0, 0);
-    lds_stage_store<FM, FN>(wbuf, sa, un.r, un.valid ? un.sp.k : 0u, un.c, srw, seg);
-}
-
-template<int FM, int FN>
-__device__ __forceinline__ void lds_step_any(double4_t (&acc)[FM][FN], double (&bn)[FN][4],
-    const double (&bc)[FN][4], st_cursor<FM, FN> &un, const double *rbuf, double *wbuf,
-    const int (&bcol)[FN], int lr, int lg, int srw, int seg) {
-    switch(st_bform(un.sp)) {
-    case ST_FORM_VA_VB:
-        lds_step<FM, FN, ST_FORM_VA_VB>(acc, bn, bc, un, rbuf, wbuf, bcol, lr, lg, srw, seg); break;
-    case ST_FORM_VA_ROW:
-        lds_step<FM, FN, ST_FORM_VA_ROW>(acc, bn, bc, un, rbuf, wbuf, bcol, lr, lg, srw, seg); break;
-    case ST_FORM_VA_AR:
-        lds_step<FM, FN, ST_FORM_VA_AR>(acc, bn, bc, un, rbuf, wbuf, bcol, lr, lg, srw, seg); break;
-    case ST_FORM_VA_VTAR:
-        lds_step<FM, FN, ST_FORM_VA_VTAR>(acc, bn, bc, un, rbuf, wbuf, bcol, lr, lg, srw, seg); break;
-    default:
-        lds_step<FM, FN, ST_FORM_ANY>(acc, bn, bc, un, rbuf, wbuf, bcol, lr, lg, srw, seg); break;
-    }
-}
-
-template<int FM, int FN>
-__device__ __forceinline__ void lds_tile(const stack_desc &st,
-    const stack_pair *__restrict__ spairs, const stack_arow *__restrict__ arow,
-    const stack_crow *__restrict__ crow, int m0, int n0, double *lds) {
-    constexpr int ABUF = 16 * FM * kLdsRowStride;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int g = wave & 1, h = wave >> 1;
-    const int lr = lane & 15, lg = lane >> 4;
-    const int lig = lane + 64 * h;
-    const int seg = lig & 7, srw = lig >> 3;
-    const int nw = n0 + 16 * FN * h;
-    const int mrem = int(st.rows) - m0, nrem = int(st.n) - nw;
-    double *abuf = lds + g * 2 * ABUF;
-
-    double4_t acc[FM][FN];
-#pragma unroll
-    for(int i = 0; i < FM; i++)
-#pragma unroll
-        for(int j = 0; j < FN; j++) acc[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
-
-    int srow[FM], bcol[FN];
-#pragma unroll
-    for(int j = 0; j < FM; j++) srow[j] = (srw + 16 * j) < mrem ? m0 + srw + 16 * j : m0;
-#pragma unroll
-    for(int f = 0; f < FN; f++) bcol[f] = (16 * f + lr) < nrem ? nw + 16 * f + lr : n0;
-
-    const int nchunk = int(st.nchunk);
-    if(nchunk > 0) {
-        const uint32_t pbeg = st.pair_begin, pend = st.pair_begin + st.npairs;
-        // the group's first chunk; a group without chunks keeps an in-bounds
-        // cursor on chunk 0, stages zeros and only joins the barriers
-        st_cursor<FM, FN> u, u2;
-        u.p = pbeg;
-        u.c = g;
-        seek_chunk_st(spairs, pend, u.p, u.c);
-        u.valid = u.p < pend;
-        if(!u.valid) { u.p = pbeg; u.c = 0; }
-        u.sp = spairs[u.p];
-        st_rows_a<FM, FN>(u.r, arow, st.arow_begin + (u.p - pbeg) * st.rows, srow);
-        st_cols<FM, FN>(u.r, u.sp, bcol);
-        double bx[FN][4], by[FN][4];
-        {
-            double2_t sa[FM];
-            lds_stage_load<FM, FN>(sa, u.r, u.sp, u.c, seg);
-            load_b_st<FM, FN>(bx, u.r, u.sp, u.c, bcol, lg);
-            lds_stage_store<FM, FN>(abuf, sa, u.r, u.valid ? u.sp.k : 0u, u.c, srw, seg);
-        }
-        u2 = u;
-        st_advance_a<FM, FN, 2>(u2, spairs, arow, st, srow);
-        __syncthreads();
-        // iteration it multiplies chunk it (LDS buffer it & 1, B in bx or by)
-        // and stages chunk it + 1 in the other buffer
-        const int niter = (nchunk + 1) >> 1;
-        for(int it = 0; it < niter; it += 2) {
-            st_cursor<FM, FN> un = u2;
-            st_advance_a<FM, FN, 2>(u2, spairs, arow, st, srow);
-            lds_step_any<FM, FN>(acc, by, bx, un, abuf, abuf + ABUF, bcol, lr, lg, srw, seg);
-            __syncthreads();
-            if(it + 1 >= niter) break;
-            un = u2;
-            st_advance_a<FM, FN, 2>(u2, spairs, arow, st, srow);
-            lds_step_any<FM, FN>(acc, bx, by, un, abuf + ABUF, abuf, bcol, lr, lg, srw, seg);
-            __syncthreads();
-        }
-    }
-
-    // group 1's partial tile onto group 0's, then the C rows
-    double *red = lds;
-    if(g == 1) {
-        double *r = red + h * (FM * FN * 4 * 64);
-#pragma unroll
-        for(int i = 0; i < FM; i++)
-#pragma unroll
-            for(int j = 0; j < FN; j++)
-#pragma unroll
-                for(int v = 0; v < 4; v++)
-                    r[((i * FN + j) * 4 + v) * 64 + lane] = acc[i][j][v];
-    }
-    __syncthreads();
-    if(g == 0) {
-        const double *r = red + h * (FM * FN * 4 * 64);
-#pragma unroll
-        for(int i = 0; i < FM; i++)
-#pragma unroll
-            for(int j = 0; j < FN; j++)
-#pragma unroll
-                for(int v = 0; v < 4; v++)
-                    acc[i][j][v] += r[((i * FN + j) * 4 + v) * 64 + lane];
-#pragma unroll
-        for(int i = 0; i < FM; i++) {
-#pragma unroll
-            for(int v = 0; v < 4; v++) {
-                const int row = 16 * i + lg + 4 * v;
-                if(row >= mrem) continue;
-                const stack_crow cr = crow[st.crow_begin + m0 + row];
-#pragma unroll
-                for(int j = 0; j < FN; j++) {
-                    const int col = 16 * j + lr;
-                    if(col < nrem) {
-                        double *cp = cr.c + (nw + col);
-                        double x = acc[i][j][v];
-                        if(!cr.zero) x += *cp;
-                        *cp = x;
-                    }
-                }
-            }
-        }
-    }
-    __syncthreads();   // LDS is reused by the next tile
-}
-
-template<int FM, int FN>
-__global__ void __launch_bounds__(256)
-gemm_stacked_lds_kernel(const stack_desc *__restrict__ stacks,
-    const stack_pair *__restrict__ spairs, const stack_arow *__restrict__ arow,
-    const stack_crow *__restrict__ crow, const gemm_tile *__restrict__ tiles,
-    uint32_t ntiles) {
-    constexpr int NA = 4 * 16 * FM * kLdsRowStride, NR = 2 * FM * FN * 4 * 64;
-    __shared__ double lds[NA > NR ? NA : NR];
-    for(uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-        const gemm_tile tile = tiles[t];
-        const stack_desc st = stacks[tile.cblock];
-        lds_tile<FM, FN>(st, spairs, arow, crow, int(tile.tm) * 16 * FM,
-            int(tile.tn) * 32 * FN, lds);
-    }
-}
-
 //! Stacked kernel over tiles of varying height and width (16 fm x 16 fn,
-//! fm <= 4, fn <= FNX): every stack is covered by full tiles and one
+//! fm <= 4, fn <= 2): every stack is covered by full tiles and one
 //! narrower tile per remainder, so rows and columns are padded to 16 only.
-template<int W, int FNX>
+template<int W>
 __global__ void __launch_bounds__(64 * W)
 gemm_stacked_var_kernel(const stack_desc *__restrict__ stacks,
     const stack_pair *__restrict__ spairs, const stack_arow *__restrict__ arow,
     const stack_crow *__restrict__ crow, const var_tile *__restrict__ tiles,
     uint32_t ntiles) {
-    __shared__ double red[(W > 1 ? W - 1 : 1) * 4 * FNX * 4 * 64];
+    __shared__ double red[(W > 1 ? W - 1 : 1) * 4 * 2 * 4 * 64];
     for(uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         const var_tile vt = tiles[t];
         const stack_desc st = stacks[vt.stack];
         const int m0 = 16 * int(vt.r16), n0 = 16 * int(vt.c16);
         switch(vt.fm * 4 + vt.fn) {
-        case 1 * 4 + 1: stacked_tile<1, 1, W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-        case 2 * 4 + 1: stacked_tile<2, 1, W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-        case 3 * 4 + 1: stacked_tile<3, 1, W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-        case 4 * 4 + 1: stacked_tile<4, 1, W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-        case 1 * 4 + 2: stacked_tile<1, 2, W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-        case 2 * 4 + 2: stacked_tile<2, 2, W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-        case 3 * 4 + 2: stacked_tile<3, 2, W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-        case 4 * 4 + 2: stacked_tile<4, 2, W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-        default:
-            if(FNX >= 3) {
-                switch(vt.fm) {
-                case 1: stacked_tile<1, (FNX >= 3 ? 3 : 1), W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-                case 2: stacked_tile<2, (FNX >= 3 ? 3 : 1), W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-                case 3: stacked_tile<3, (FNX >= 3 ? 3 : 1), W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-                default: stacked_tile<4, (FNX >= 3 ? 3 : 1), W, 2>(st, spairs, arow, crow, m0, n0, red); break;
-                }
-            }
-            break;
+        case 1 * 4 + 1: stacked_tile<1, 1, W>(st, spairs, arow, crow, m0, n0, red); break;
+        case 2 * 4 + 1: stacked_tile<2, 1, W>(st, spairs, arow, crow, m0, n0, red); break;
+        case 3 * 4 + 1: stacked_tile<3, 1, W>(st, spairs, arow, crow, m0, n0, red); break;
+        case 4 * 4 + 1: stacked_tile<4, 1, W>(st, spairs, arow, crow, m0, n0, red); break;
+        case 1 * 4 + 2: stacked_tile<1, 2, W>(st, spairs, arow, crow, m0, n0, red); break;
+        case 2 * 4 + 2: stacked_tile<2, 2, W>(st, spairs, arow, crow, m0, n0, red); break;
+        case 3 * 4 + 2: stacked_tile<3, 2, W>(st, spairs, arow, crow, m0, n0, red); break;
+        case 4 * 4 + 2: stacked_tile<4, 2, W>(st, spairs, arow, crow, m0, n0, red); break;
+        default: break;
         }
     }
 }
@@ -1520,14 +1015,9 @@ hipError_t launch_gemm_stacked_var(int cfg, const stack_desc *st, const stack_pa
     const stack_arow *ar, const stack_crow *cr, const var_tile *tiles, uint32_t ntiles,
     hipStream_t s) {
     if(ntiles == 0) return hipSuccess;
-    if(cfg == STACK_VAR_64x32_W4)
-        hipLaunchKernelGGL((gemm_stacked_var_kernel<4, 2>), dim3(ntiles), dim3(256), 0, s,
-            st, sp, ar, cr, tiles, ntiles);
-    else if(cfg == STACK_VAR_64x48_W4)
-        hipLaunchKernelGGL((gemm_stacked_var_kernel<4, 3>), dim3(ntiles), dim3(256), 0, s,
-            st, sp, ar, cr, tiles, ntiles);
-    else
-        return hipErrorInvalidValue;
+    if(cfg != STACK_VAR_64x32_W4) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((gemm_stacked_var_kernel<4>), dim3(ntiles), dim3(256), 0, s,
+        st, sp, ar, cr, tiles, ntiles);
     return hipGetLastError();
 }
 
@@ -1540,11 +1030,11 @@ static hipError_t launch_stacked_occ_t(const stack_desc *st, const stack_pair *s
     return hipGetLastError();
 }
 
-template<int FM, int FN, int W, int PIPE = 2>
+template<int FM, int FN, int W>
 static hipError_t launch_stacked_t(const stack_desc *st, const stack_pair *sp,
     const stack_arow *ar, const stack_crow *cr, const gemm_tile *tiles, uint32_t ntiles,
     hipStream_t s) {
-    hipLaunchKernelGGL((gemm_stacked_kernel<FM, FN, W, PIPE>), dim3(ntiles), dim3(64 * W), 0, s,
+    hipLaunchKernelGGL((gemm_stacked_kernel<FM, FN, W>), dim3(ntiles), dim3(64 * W), 0, s,
         st, sp, ar, cr, tiles, ntiles);
     return hipGetLastError();
 }
@@ -1556,18 +1046,7 @@ hipError_t launch_gemm_stacked(int cfg, const stack_desc *st, const stack_pair *
     switch(cfg) {
     case STACK_16x64_W4: return launch_stacked_t<1, 4, 4>(st, sp, ar, cr, tiles, ntiles, s);
     case STACK_32x32_W4: return launch_stacked_t<2, 2, 4>(st, sp, ar, cr, tiles, ntiles, s);
-    case STACK_32x64_W4: return launch_stacked_t<2, 4, 4>(st, sp, ar, cr, tiles, ntiles, s);
-    case STACK_64x32_W4: return launch_stacked_t<4, 2, 4, 3>(st, sp, ar, cr, tiles, ntiles, s);
-    case STACK_LDS_64x64:
-        hipLaunchKernelGGL((gemm_stacked_lds_kernel<4, 2>), dim3(ntiles), dim3(256), 0, s,
-            st, sp, ar, cr, tiles, ntiles);
-        return hipGetLastError();
-    case STACK_48x64_W4: return launch_stacked_t<3, 4, 4>(st, sp, ar, cr, tiles, ntiles, s);
-    case STACK_64x48_W4: return launch_stacked_t<4, 3, 4, 3>(st, sp, ar, cr, tiles, ntiles, s);
     case STACK_48x32_W4: return launch_stacked_t<3, 2, 4>(st, sp, ar, cr, tiles, ntiles, s);
-    case STACK_64x32_W4_P1: return launch_stacked_t<4, 2, 4, 1>(st, sp, ar, cr, tiles, ntiles, s);
-    case STACK_64x48_W2: return launch_stacked_t<4, 3, 2>(st, sp, ar, cr, tiles, ntiles, s);
-    case STACK_48x64_W2: return launch_stacked_t<3, 4, 2>(st, sp, ar, cr, tiles, ntiles, s);
     case STACK_48x32_W4_O2: return launch_stacked_occ_t<3, 2, 4, 2>(st, sp, ar, cr, tiles, ntiles, s);
     case STACK_32x32_W4_O3: return launch_stacked_occ_t<2, 2, 4, 3>(st, sp, ar, cr, tiles, ntiles, s);
     case STACK_16x64_W4_O3: return launch_stacked_occ_t<1, 4, 4, 3>(st, sp, ar, cr, tiles, ntiles, s);

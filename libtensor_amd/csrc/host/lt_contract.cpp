@@ -249,6 +249,10 @@ struct contract_plan {
     dev::stack_crow *d_crows;
     dev::gemm_tile *d_stiles;
     dev::var_tile *d_vtiles;
+    // the workgroup-tiled kernels' stacks: one per stack, then one per C
+    // block (per-block launches), each list ending with an empty one
+    std::vector<dev::tile_stack> tstacks;
+    dev::tile_stack *d_tstacks, *d_bstacks;
     // C blocks reading the same B operands (same order and layouts) share a
     // group; n_xcd: XCDs of the device
     std::vector<size_t> cb_group;
@@ -298,6 +302,7 @@ struct contract_plan {
         d_cb(0), d_pairs(0), d_tiles_sorted(0), d_tiles_block(0), scratch(0),
         scratch_elems(0), ctx(0), events(false), graph(0), gexec(0), graph_launches(0),
         d_stacks(0), d_spairs(0), d_arows(0), d_crows(0), d_stiles(0), d_vtiles(0),
+        d_tstacks(0), d_bstacks(0),
         n_groups(0), n_xcd(8),
         n_prep_st_chunks(0), d_prep_st(0), d_pst_cd(0), d_pst_co(0),
         oz_slices(0), oz_tile(0), oz_tile_set(-1), d_oz_split(0), d_oz_items(0), n_oz_items(0), d_oz_pairs(0),
@@ -324,6 +329,8 @@ hipError_t launch_grouped_list(const contract_plan &pl, int k, const void *d_lis
     if(dev::is_var(k))
         return dev::launch_gemm_stacked_var(k, pl.d_stacks, pl.d_spairs, pl.d_arows, pl.d_crows,
             (const dev::var_tile*)d_list, n, s);
+    if(dev::is_tile(k))
+        return dev::launch_gemm_tile(k, pl.d_tstacks, (const dev::gemm_tile*)d_list, n, s);
     if(dev::is_stacked(k))
         return dev::launch_gemm_stacked(k, pl.d_stacks, pl.d_spairs, pl.d_arows, pl.d_crows,
             (const dev::gemm_tile*)d_list, n, s);
@@ -335,6 +342,8 @@ hipError_t launch_grouped(const contract_plan &pl, int k, hipStream_t s) {
     if(dev::is_var(k))
         return dev::launch_gemm_stacked_var(k, pl.d_stacks, pl.d_spairs, pl.d_arows, pl.d_crows,
             pl.d_vtiles, (uint32_t)pl.vtiles.size(), s);
+    if(dev::is_tile(k))
+        return dev::launch_gemm_tile(k, pl.d_tstacks, pl.d_stiles, (uint32_t)pl.stiles.size(), s);
     if(dev::is_stacked(k))
         return dev::launch_gemm_stacked(k, pl.d_stacks, pl.d_spairs, pl.d_arows, pl.d_crows,
             pl.d_stiles, (uint32_t)pl.stiles.size(), s);
@@ -829,6 +838,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         std::copy(gs.begin(), gs.end(), pl.pairs.begin() + p0);
         std::copy(ts.begin(), ts.end(), pair_tab.begin() + p0);
     }
+    std::vector<std::vector<size_t> > stack_blocks;     // C blocks of a stack, in row order
     {
         std::map<std::pair<uint32_t, std::vector<bkey_t> >, std::vector<size_t> > groups;
         std::vector<std::pair<uint32_t, std::vector<bkey_t> > > order;
@@ -841,8 +851,40 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
             if(g.empty()) order.push_back(key);
             g.push_back(b);
         }
+        // The workgroup-tiled kernels address a pair's A rows by 32-bit byte
+        // offsets from its lowest one: a group whose A blocks of one pair lie
+        // farther apart is cut into several stacks.
+        std::vector<std::vector<size_t> > cut;
         for(size_t gi = 0; gi < order.size(); gi++) {
-            const std::vector<size_t> &bl = groups[order[gi]];
+            const std::vector<size_t> &all = groups[order[gi]];
+            std::vector<std::pair<uintptr_t, uintptr_t> > span;    // first and last byte per pair
+            for(size_t q = 0; q < all.size(); q++) {
+                const dev::gemm_cblock &cq = pl.cblocks[all[q]];
+                std::vector<std::pair<uintptr_t, uintptr_t> > with(span);
+                bool fits = q > 0;
+                if(!fits) with.assign(cq.pair_end - cq.pair_begin, std::make_pair(~uintptr_t(0), uintptr_t(0)));
+                for(size_t j = 0; j < with.size(); j++) {
+                    const dev::gemm_pair &g = pl.pairs[cq.pair_begin + j];
+                    const uintptr_t p0 = (uintptr_t)g.a, p1 = p0 + size_t(cq.m) * g.k * sizeof(double);
+                    with[j].first = std::min(with[j].first, p0);
+                    with[j].second = std::max(with[j].second, p1);
+                    if(with[j].second - with[j].first >= (uintptr_t(1) << 32)) fits = false;
+                }
+                if(!fits) {
+                    cut.push_back(std::vector<size_t>());
+                    with.assign(cq.pair_end - cq.pair_begin, std::make_pair(uintptr_t(0), uintptr_t(0)));
+                    for(size_t j = 0; j < with.size(); j++) {
+                        const dev::gemm_pair &g = pl.pairs[cq.pair_begin + j];
+                        with[j].first = (uintptr_t)g.a;
+                        with[j].second = (uintptr_t)g.a + size_t(cq.m) * g.k * sizeof(double);
+                    }
+                }
+                span.swap(with);
+                cut.back().push_back(all[q]);
+            }
+        }
+        for(size_t gi = 0; gi < cut.size(); gi++) {
+            const std::vector<size_t> &bl = cut[gi];
             const dev::gemm_cblock &c0 = pl.cblocks[bl[0]];
             dev::stack_desc sd;
             std::memset(&sd, 0, sizeof(sd));
@@ -863,6 +905,14 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
                 dev::stack_pair sp;
                 std::memset(&sp, 0, sizeof(sp));
                 sp.b = g.b; sp.k = g.k; sp.ldb = g.ldb; sp.flags = g.flags;
+                // element (k, n) at k ks1 + n ns1 unless read through tables
+                // (kd, nd beyond every index: the quotients are zero)
+                const bool nm = (g.flags & dev::kPairBNMajor) != 0;
+                sp.kd = sp.nd = dev::make_fastdiv(1u << 30);
+                sp.ks1 = nm ? 1 : (int32_t)g.ldb;
+                sp.ns1 = nm ? (int32_t)g.ldb : 1;
+                if(tb.koff < 0 ? !nm : sd.n < 2 || pl.otab[tb.noff + 1] == pl.otab[tb.noff] + 1)
+                    sp.flags |= dev::kPairBNFast;
                 double bscale = 1.0;
                 if(tb.koff >= 0) {
                     sp.b = tb.y;
@@ -896,6 +946,13 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
                         if(pairs_ok) sp.flags |= dev::kPairVecBT;
                     }
                 }
+                bool unit = true;
+                for(size_t q = 0; q < bl.size(); q++) {
+                    const dev::gemm_pair &gq = pl.pairs[pl.cblocks[bl[q]].pair_begin + j];
+                    if(q == 0 || (uintptr_t)gq.a < (uintptr_t)sp.a) sp.a = gq.a;
+                    unit = unit && gq.d * bscale == 1.0;
+                }
+                if(unit) sp.flags |= dev::kPairUnit;
                 pl.spairs.push_back(sp);
                 pl.spair_tab.push_back(std::make_pair(tb.koff, tb.noff));
                 ks += double(g.k);
@@ -909,6 +966,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
                         ar.p = (gq.flags & dev::kPairAKMajor) ? gq.a + r : gq.a + size_t(r) * gq.lda;
                         ar.d = gq.d * bscale;
                         ar.lda = gq.lda;
+                        ar.off = (uint32_t)((uintptr_t)ar.p - (uintptr_t)sp.a);
                         pl.arows.push_back(ar);
                     }
                 }
@@ -925,6 +983,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
             }
             pl.stacks.push_back(sd);
             pl.stack_ksum.push_back(ks);
+            stack_blocks.push_back(bl);
         }
         dev::stack_desc z;
         std::memset(&z, 0, sizeof(z));
@@ -1123,6 +1182,8 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     size_t o_ps = sz; sz = align256(sz + pl.prep_st.size() * sizeof(dev::perm_desc));
     size_t o_scd = sz; sz = align256(sz + scd.size() * 4);
     size_t o_sco = sz; sz = align256(sz + sco.size() * 4);
+    const size_t n_ts = pl.stacks.size(), n_bs = pl.cblocks.size();
+    size_t o_ts = sz; sz = align256(sz + (n_ts + n_bs) * sizeof(dev::tile_stack));
     std::vector<char> host(sz, 0);
     auto put = [&](size_t off, const void *src, size_t n) { if(n) std::memcpy(&host[off], src, n); };
     put(o_prep, pl.prep.data(), pl.prep.size() * sizeof(dev::perm_desc));
@@ -1151,6 +1212,34 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         }
         put(o_sp, pl.spairs.data(), pl.spairs.size() * sizeof(dev::stack_pair));
     }
+    {
+        const dev::stack_pair *sp = (const dev::stack_pair*)((char*)pl.lists.mem + o_sp);
+        const dev::stack_arow *ar = (const dev::stack_arow*)((char*)pl.lists.mem + o_ar);
+        const dev::stack_crow *cr = (const dev::stack_crow*)((char*)pl.lists.mem + o_cr);
+        dev::tile_stack z;
+        std::memset(&z, 0, sizeof(z));
+        pl.tstacks.assign(n_ts + n_bs, z);
+        for(size_t i = 0; i + 1 < n_ts; i++) {
+            const dev::stack_desc &sd = pl.stacks[i];
+            dev::tile_stack &t = pl.tstacks[i];
+            t.pairs = sp + sd.pair_begin;
+            t.arow = ar + sd.arow_begin;
+            t.crow = cr + sd.crow_begin;
+            t.rows = t.astride = sd.rows;
+            t.n = sd.n; t.npairs = sd.npairs; t.nchunk = sd.nchunk;
+            // a C block of the stack: its rows of the stack's lists
+            uint32_t r0 = 0;
+            for(size_t q = 0; q < stack_blocks[i].size(); q++) {
+                dev::tile_stack &b = pl.tstacks[n_ts + stack_blocks[i][q]];
+                b = t;
+                b.rows = pl.cblocks[stack_blocks[i][q]].m;
+                b.arow += r0;
+                b.crow += r0;
+                r0 += b.rows;
+            }
+        }
+        put(o_ts, pl.tstacks.data(), pl.tstacks.size() * sizeof(dev::tile_stack));
+    }
     ctx.upload_new(pl.lists.mem, host.data(), sz);
     char *base = (char*)pl.lists.mem;
     pl.d_prep = (dev::perm_desc*)(base + o_prep);
@@ -1165,6 +1254,8 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     pl.d_spairs = (dev::stack_pair*)(base + o_sp);
     pl.d_arows = (dev::stack_arow*)(base + o_ar);
     pl.d_crows = (dev::stack_crow*)(base + o_cr);
+    pl.d_tstacks = (dev::tile_stack*)(base + o_ts);
+    pl.d_bstacks = pl.d_tstacks + n_ts;
     pl.d_prep_st = (dev::perm_desc*)(base + o_ps);
     pl.d_pst_cd = (uint32_t*)(base + o_scd);
     pl.d_pst_co = (uint32_t*)(base + o_sco);
@@ -1191,7 +1282,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         if(dev::is_var(k)) {
             // full 64-row tiles and one tile per row / column remainder,
             // largest (k sum x area) first
-            const uint32_t fnx = (k == dev::STACK_VAR_64x48_W4) ? 3 : 2;
+            const uint32_t fnx = 2;
             std::vector<std::pair<double, dev::var_tile> > vt;
             for(size_t si = 0; si + 1 < pl.stacks.size(); si++) {
                 const dev::stack_desc &sd = pl.stacks[si];
@@ -1693,7 +1784,8 @@ void btod_contract2::build_ozaki(int slices) {
 
 void btod_contract2::enqueue(int mode, hipStream_t s, bool timed, size_t &launches) {
     contract_plan &pl = *m_plan;
-    if(mode == MODE_GROUPED && dev::is_stacked(pl.tile_cfg)) {
+    if((mode == MODE_GROUPED && dev::is_stacked(pl.tile_cfg)) ||
+        (mode == MODE_PER_BLOCK && dev::is_tile(pl.tile_cfg))) {
         if(pl.n_prep_st_chunks) {
             hip_check(dev::launch_permute(pl.d_prep_st, pl.d_pst_cd, pl.d_pst_co,
                 pl.n_prep_st_chunks, s), "permute (prepare)");
@@ -1735,8 +1827,11 @@ void btod_contract2::enqueue(int mode, hipStream_t s, bool timed, size_t &launch
         for(size_t b = 0; b + 1 < pl.block_tile_begin.size(); b++) {
             uint32_t t0 = pl.block_tile_begin[b], t1 = pl.block_tile_begin[b + 1];
             if(t1 == t0) continue;
-            hip_check(dev::launch_gemm(pl.tile_cfg, pl.d_cb, pl.d_pairs,
-                pl.d_tiles_block + t0, t1 - t0, t1 - t0, ctx.side(j++)), "gemm (per block)");
+            hip_check(dev::is_tile(pl.tile_cfg) ?
+                dev::launch_gemm_tile(pl.tile_cfg, pl.d_bstacks, pl.d_tiles_block + t0, t1 - t0,
+                    ctx.side(j++)) :
+                dev::launch_gemm(pl.tile_cfg, pl.d_cb, pl.d_pairs,
+                    pl.d_tiles_block + t0, t1 - t0, t1 - t0, ctx.side(j++)), "gemm (per block)");
             launches++;
         }
         ctx.side_join(s);
@@ -1894,15 +1989,10 @@ void btod_contract2::perform_sliced(btensor &c, bool add, double d, double slice
     const uint32_t per = (nt + nslices - 1) / nslices;
     for(uint32_t t0 = 0; t0 < nt; t0 += per) {
         const uint32_t n = std::min(per, nt - t0);
-        if(dev::is_var(k))
-            hip_check(dev::launch_gemm_stacked_var(k, pl.d_stacks, pl.d_spairs, pl.d_arows,
-                pl.d_crows, pl.d_vtiles + t0, n, s), "gemm (slice)");
-        else if(dev::is_stacked(k))
-            hip_check(dev::launch_gemm_stacked(k, pl.d_stacks, pl.d_spairs, pl.d_arows,
-                pl.d_crows, pl.d_stiles + t0, n, s), "gemm (slice)");
-        else
-            hip_check(dev::launch_gemm(k, pl.d_cb, pl.d_pairs, pl.d_tiles_sorted + t0, n, n, s),
-                "gemm (slice)");
+        const void *list = dev::is_var(k) ? (const void*)(pl.d_vtiles + t0) :
+            dev::is_stacked(k) ? (const void*)(pl.d_stiles + t0) :
+            (const void*)(pl.d_tiles_sorted + t0);
+        hip_check(launch_grouped_list(pl, k, list, n, s), "gemm (slice)");
         if(t0 + n < nt) {
             hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
             between();
@@ -1984,7 +2074,12 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
                     0.0, s), "fill");
             }
         }
-        if(!pl.empty && pl.n_prep_chunks)
+        if(pl.empty) continue;
+        if(dev::is_tile(pl.tile_cfg)) {
+            if(pl.n_prep_st_chunks)
+                hip_check(dev::launch_permute(pl.d_prep_st, pl.d_pst_cd, pl.d_pst_co,
+                    pl.n_prep_st_chunks, s), "permute (prepare)");
+        } else if(pl.n_prep_chunks)
             hip_check(dev::launch_permute(pl.d_prep, pl.d_prep_cd, pl.d_prep_co,
                 pl.n_prep_chunks, s), "permute (prepare)");
     }
@@ -1999,15 +2094,33 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
     }
     std::vector<dev::gemm_cblock> cbs;
     std::vector<dev::gemm_pair> prs;
+    std::vector<dev::tile_stack> tss;
     std::vector<std::pair<double, dev::gemm_tile> > tl;
     std::vector<char> host;
     size_t sz = 0;
     for(std::map<int, std::vector<size_t> >::iterator g = groups.begin(); g != groups.end(); ++g) {
-        cbs.clear(); prs.clear(); tl.clear();
+        cbs.clear(); prs.clear(); tl.clear(); tss.clear();
         uint32_t bm = 64, bn = 64;
         dev::tile_shape(g->first, bm, bn);
         for(size_t x = 0; x < g->second.size(); x++) {
             contract_plan &pl = *m_plans[g->second[x]];
+            if(dev::is_tile(g->first)) {
+                // stacks name their plan's lists by address
+                const uint32_t ts0 = (uint32_t)tss.size(), ns = (uint32_t)pl.stacks.size() - 1;
+                tss.insert(tss.end(), pl.tstacks.begin(), pl.tstacks.begin() + ns);
+                for(size_t t = 0; t < pl.stiles.size(); t++) {
+                    dev::gemm_tile y = pl.stiles[t];
+                    if(y.cblock >= ns) continue;                // padding tile
+                    const dev::stack_desc &sd = pl.stacks[y.cblock];
+                    const double rows = std::min<double>(bm, double(sd.rows) - double(y.tm) * bm);
+                    const double cols = std::min<double>(bn, double(sd.n) - double(y.tn) * bn);
+                    const double cost = 2.0 * rows * cols * pl.stack_ksum[y.cblock];
+                    y.cblock += ts0;
+                    tl.push_back(std::make_pair(cost, y));
+                    m_flops += cost;
+                }
+                continue;
+            }
             uint32_t cb0 = (uint32_t)cbs.size(), pr0 = (uint32_t)prs.size();
             for(size_t b = 0; b < pl.cblocks.size(); b++) {
                 dev::gemm_cblock cb = pl.cblocks[b];
@@ -2035,12 +2148,14 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
                 return x.first > y.first; });
         launch L;
         L.cfg = g->first;
-        L.ocb = sz; sz = align256(sz + cbs.size() * sizeof(dev::gemm_cblock));
+        L.ocb = sz;
+        sz = align256(sz + cbs.size() * sizeof(dev::gemm_cblock) + tss.size() * sizeof(dev::tile_stack));
         L.opr = sz; sz = align256(sz + prs.size() * sizeof(dev::gemm_pair));
         L.otl = sz; sz = align256(sz + tl.size() * sizeof(dev::gemm_tile));
         L.nt = (uint32_t)tl.size();
         host.resize(sz, 0);
         if(!cbs.empty()) std::memcpy(&host[L.ocb], cbs.data(), cbs.size() * sizeof(dev::gemm_cblock));
+        if(!tss.empty()) std::memcpy(&host[L.ocb], tss.data(), tss.size() * sizeof(dev::tile_stack));
         if(!prs.empty()) std::memcpy(&host[L.opr], prs.data(), prs.size() * sizeof(dev::gemm_pair));
         for(size_t t = 0; t < tl.size(); t++) {
             std::memcpy(&host[L.otl + t * sizeof(dev::gemm_tile)], &tl[t].second,
@@ -2076,9 +2191,11 @@ bool batch_run::step(double flop_budget) {
         double f = 0.0;
         do { f += L.tcost[t1]; t1++; } while(t1 < L.nt && f + L.tcost[t1] <= flop_budget);
         const uint32_t n = t1 - (uint32_t)m_tile;
-        hip_check(dev::launch_gemm(L.cfg, (dev::gemm_cblock*)(m_base + L.ocb),
-            (dev::gemm_pair*)(m_base + L.opr),
-            (dev::gemm_tile*)(m_base + L.otl) + m_tile, n, n, s), "gemm (batch)");
+        const dev::gemm_tile *list = (const dev::gemm_tile*)(m_base + L.otl) + m_tile;
+        hip_check(dev::is_tile(L.cfg) ?
+            dev::launch_gemm_tile(L.cfg, (const dev::tile_stack*)(m_base + L.ocb), list, n, s) :
+            dev::launch_gemm(L.cfg, (dev::gemm_cblock*)(m_base + L.ocb),
+                (dev::gemm_pair*)(m_base + L.opr), list, n, n, s), "gemm (batch)");
         m_tile = t1;
         return m_launch < m_launches.size() &&
             (m_tile < L.nt || m_launch + 1 < m_launches.size());
