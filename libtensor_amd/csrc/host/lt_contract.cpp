@@ -499,16 +499,21 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
 
     // aligned operand blocks needed by the pairs
     std::vector<size_t> usea, useb;
-    for(size_t t = 0; t < clsts.size(); t++) {
-        for(contr_list::const_iterator p = clsts[t].begin(); p != clsts[t].end(); ++p) {
-            usea.push_back(p->aia);
-            useb.push_back(p->aib);
+    auto collect_uses = [&]() {
+        usea.clear();
+        useb.clear();
+        for(size_t t = 0; t < clsts.size(); t++) {
+            for(contr_list::const_iterator p = clsts[t].begin(); p != clsts[t].end(); ++p) {
+                usea.push_back(p->aia);
+                useb.push_back(p->aib);
+            }
         }
-    }
-    std::sort(usea.begin(), usea.end());
-    usea.erase(std::unique(usea.begin(), usea.end()), usea.end());
-    std::sort(useb.begin(), useb.end());
-    useb.erase(std::unique(useb.begin(), useb.end()), useb.end());
+        std::sort(usea.begin(), usea.end());
+        usea.erase(std::unique(usea.begin(), usea.end()), usea.end());
+        std::sort(useb.begin(), useb.end());
+        useb.erase(std::unique(useb.begin(), useb.end()), useb.end());
+    };
+    collect_uses();
 
     // Where each aligned block comes from: stored canonical block Y and the
     // transformation (A orbit of Y -> idx) then perma then (syma2 orbit).
@@ -529,6 +534,83 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         s.tr.transform(tz);
         return s;
     };
+
+    std::unordered_map<size_t, src_t> srca, srcb;
+    for(size_t i = 0; i < usea.size(); i++)
+        srca[usea[i]] = source_of(m_a, syma2, perma, bida, bida2, usea[i]);
+    for(size_t i = 0; i < useb.size(); i++)
+        srcb[useb[i]] = source_of(m_b, symb2, permb, bidb, bidb2, useb[i]);
+
+    // Coefficient of a pair, as gen_bto_contract2_block::compute_block:
+    // inverse orbit transformation of the unfolded block, then the pair's
+    // transformation, then ka / kb / kc.
+    auto pair_coeff = [&](const contr_list::value_type &p) {
+        orbit_info oa = oca.get(p.aia), ob = ocb.get(p.aib);
+        scalar_tr sa(oa.tr.st); sa.invert(); sa.transform(p.tra.st);
+        scalar_tr sb(ob.tr.st); sb.invert(); sb.transform(p.trb.st);
+        scalar_tr ka(sa), kb(sb), kc(m_kc);
+        ka.transform(scalar_tr(m_ka));
+        kb.transform(scalar_tr(m_kb));
+        return ka.c * kb.c * kc.c;
+    };
+
+    // Pairs of a C block that are the same product of the same stored blocks
+    // up to a relabelling of the contracted indices (the coalescing above
+    // compares the blocks' transformations and misses these where an operand
+    // block is reached through an exchange of its index pairs: a quarter of
+    // the pp-ladder's products) run once, with the sum of their coefficients.
+    // FLOPs and pairs are counted before, as the schedule has them.
+    double flops = 0.0;
+    size_t nsched_pairs = 0;
+    std::vector<std::vector<double> > pair_mult(clsts.size());
+    for(size_t t = 0; t < clsts.size(); t++) {
+        typedef std::vector<size_t> key_t;
+        struct kept_t { size_t pos; double c; };
+        std::map<key_t, kept_t> kept;
+        contr_list &cl = clsts[t];
+        std::vector<double> &mult = pair_mult[t];
+        contr_list::iterator p = cl.begin();
+        while(p != cl.end()) {
+            const src_t &sa = srca[p->aia], &sb = srcb[p->aib];
+            const double c = pair_coeff(*p) * sa.tr.st.c * sb.tr.st.c;
+            if(c == 0.0) { mult.push_back(1.0); ++p; continue; }    // (skipped below)
+            gemm_form g = aligned_gemm_form(contr, bisa2.block_dims(get_index(p->aia, bida2)),
+                bisb2.block_dims(get_index(p->aib, bidb2)));
+            flops += 2.0 * double(g.m) * double(g.n) * double(g.k);
+            nsched_pairs++;
+            // stored blocks, the stored dimension of every outer index, and
+            // the contracted dimensions as pairs in a fixed order
+            key_t key;
+            key.push_back(sa.y);
+            key.push_back(sb.y);
+            std::vector<std::pair<size_t, size_t> > inner;
+            const size_t NC = contr.NC(), NA = contr.NA(), NB = contr.NB();
+            for(size_t i = 0; i < NA; i++) {
+                if(contr.conn[NC + i] < NC + NA) key.push_back(sa.tr.perm[i]);
+                else inner.push_back(std::make_pair(size_t(sa.tr.perm[i]),
+                    size_t(sb.tr.perm[contr.conn[NC + i] - NC - NA])));
+            }
+            for(size_t i = 0; i < NB; i++)
+                if(contr.conn[NC + NA + i] < NC) key.push_back(sb.tr.perm[i]);
+            std::sort(inner.begin(), inner.end());
+            for(size_t i = 0; i < inner.size(); i++) {
+                key.push_back(inner[i].first);
+                key.push_back(inner[i].second);
+            }
+            std::map<key_t, kept_t>::iterator k = kept.find(key);
+            // (coefficients that cancel keep their pairs: an infinity or a
+            // NaN in the operands must still reach C)
+            if(k != kept.end() && mult[k->second.pos] + c / k->second.c != 0.0) {
+                mult[k->second.pos] += c / k->second.c;
+                p = cl.erase(p);
+                continue;
+            }
+            if(k == kept.end()) kept[key] = kept_t{mult.size(), c};
+            mult.push_back(1.0);
+            ++p;
+        }
+    }
+    collect_uses();
 
     // Operand layouts of the aligned product (the same for every pair):
     // A stored m x k (or k x m when ta), B stored k x n (or n x k when tb).
@@ -645,7 +727,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     std::unordered_map<size_t, opref> refa, refb;
     std::vector<std::pair<size_t, src_t> > prepa, prepb;
     for(size_t i = 0; i < usea.size(); i++) {
-        src_t s = source_of(m_a, syma2, perma, bida, bida2, usea[i]);
+        const src_t &s = srca[usea[i]];
         lt_require(m_a.is_nonzero(s.y), LT_ERR_INTERNAL, "pair uses a zero block of A");
         dims_t dz = bisa2.block_dims(get_index(usea[i], bida2));
         opref r;
@@ -659,7 +741,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         refa[usea[i]] = r;
     }
     for(size_t i = 0; i < useb.size(); i++) {
-        src_t s = source_of(m_b, symb2, permb, bidb, bidb2, useb[i]);
+        const src_t &s = srcb[useb[i]];
         lt_require(m_b.is_nonzero(s.y), LT_ERR_INTERNAL, "pair uses a zero block of B");
         dims_t dz = bisb2.block_dims(get_index(useb[i], bidb2));
         opref r;
@@ -723,7 +805,6 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     pl.ta = tc ? !gf0.tb : gf0.ta;
     pl.tb = tc ? !gf0.ta : gf0.tb;
 
-    double flops = 0.0;
     std::vector<tabref> pair_tab;
     std::vector<std::pair<size_t, size_t> > mn(batchc.size());
     for(size_t t = 0; t < batchc.size(); t++) {
@@ -760,17 +841,9 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         cb.zero = (cdst[t].direct && add) ? 0 : 1;
         cb.pair_begin = (uint32_t)pl.pairs.size();
         double ksum = 0.0;
+        size_t pi = 0;
         for(contr_list::const_iterator p = cl.begin(); p != cl.end(); ++p) {
-            // scalars as gen_bto_contract2_block::compute_block:
-            // inverse orbit transformation of the unfolded block, then the
-            // pair's transformation, then ka/kb/kc
-            orbit_info oa = oca.get(p->aia), ob = ocb.get(p->aib);
-            scalar_tr sa(oa.tr.st); sa.invert(); sa.transform(p->tra.st);
-            scalar_tr sb(ob.tr.st); sb.invert(); sb.transform(p->trb.st);
-            scalar_tr ka(sa), kb(sb), kc(m_kc);
-            ka.transform(scalar_tr(m_ka));
-            kb.transform(scalar_tr(m_kb));
-            double d = ka.c * kb.c * kc.c;
+            double d = pair_coeff(*p) * pair_mult[t][pi++];
             if(add) d *= dscale;
             if(d == 0.0) continue;
             dims_t da = bisa2.block_dims(get_index(p->aia, bida2));
@@ -807,7 +880,6 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
                     pair_tab.push_back(z);
                 }
             }
-            flops += 2.0 * double(g.m) * double(g.n) * double(g.k);
             ksum += double(g.k);
         }
         cb.pair_end = (uint32_t)pl.pairs.size();
@@ -1460,7 +1532,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     }
 
     m_stats.n_cblocks = null_cb;
-    m_stats.n_pairs = pl.pairs.size();
+    m_stats.n_pairs = nsched_pairs;
     m_stats.n_tiles = pl.tiles_by_block.size();
     m_stats.n_unfold = pl.prep.size();
     m_stats.flops = flops;
