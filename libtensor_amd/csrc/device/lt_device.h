@@ -187,8 +187,21 @@ struct tile_stack {
     uint32_t rows, astride, n, npairs;
     uint32_t nchunk, pad;
 };
-hipError_t launch_gemm_tile(int cfg, const tile_stack *st, const gemm_tile *tiles,
-    uint32_t ntiles, hipStream_t s);
+//! Work item of a workgroup-tiled launch: tile (tm, tn) of a stack over
+//! `count` chunks of its pair list, from chunk c of pair p on.  part < 0:
+//! these are all its chunks; else the place of its partial sums (in tiles).
+struct tile_item {
+    uint32_t stack;
+    uint16_t tm, tn;
+    uint32_t p, c, count;
+    int32_t part;
+};
+hipError_t launch_gemm_tile(int cfg, const tile_stack *st, const tile_item *items,
+    uint32_t nitems, double *parts, hipStream_t s);
+//! C of the tiles that launch_gemm_tile ran in parts (item.part: the place of
+//! the first part, item.count: parts).
+hipError_t launch_tile_sum(int cfg, const tile_stack *st, const tile_item *items, uint32_t n,
+    const double *parts, hipStream_t s);
 hipError_t launch_gemm_stacked(int cfg, const stack_desc *st, const stack_pair *sp,
     const stack_arow *ar, const stack_crow *cr, const gemm_tile *tiles, uint32_t ntiles,
     hipStream_t s);

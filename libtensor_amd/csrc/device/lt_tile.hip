@@ -21,6 +21,12 @@
 // fragments straight from memory (o, v: one ring contraction): o = 29, v = 131
 // in one block 3.48 to 2.16 ms a call, o = 48, v = 240 in uneven blocks 85.6 to
 // 58.1 ms (53 TFLOP/s).
+//
+// Where the tiles of a launch are too few to keep 256 CUs evenly busy, their
+// chunk sequences are cut into parts and a second kernel adds the parts'
+// partial tiles in order: pp-ladder o = 40, v = 200 (335 tiles of 64 rows)
+// 201 to 160 us, the first product of the quadratic CCD term (72 tiles)
+// 63 to 20 us.
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include "lt_device.h"
@@ -65,27 +71,73 @@ struct row_src {
 };
 
 //! Position in a stack's chunk sequence (16 k each): chunk c of pair p, of
-//! extent k, whose tables are in ring slot `slot`.
+//! extent k, whose tables are in ring slot `slot`; `left` chunks of the
+//! tile's part of the sequence from here on.
 struct chunk_pos {
-    uint32_t p, c, k, slot;
+    uint32_t p, c, k, slot, left;
     bool valid;
 };
 
-//! Moves `by` chunks on; past the last chunk the position stays and valid
-//! becomes false, so that a load issued from it stays in bounds.
-__device__ __forceinline__ chunk_pos chunk_advance(cpair *pairs, uint32_t npairs,
-    const chunk_pos &u, uint32_t by) {
+//! Moves `by` chunks on; past the part's last chunk the position stays and
+//! valid becomes false, so that a load issued from it stays in bounds.
+__device__ __forceinline__ chunk_pos chunk_advance(cpair *pairs, const chunk_pos &u, uint32_t by) {
     chunk_pos r = u;
+    r.valid = u.valid && by < u.left;
+    if(!r.valid) return r;
+    r.left -= by;
     r.c += by;
-    while(u.valid && 16 * r.c >= r.k) {
+    while(16 * r.c >= r.k) {
         r.c -= (r.k + 15) >> 4;
-        if(++r.p >= npairs) { r = u; r.valid = false; return r; }
-        r.k = pairs[r.p].k;
+        r.k = pairs[++r.p].k;
     }
-    if(!u.valid) r = u;
     if(r.p != u.p) r.slot = u.slot ^ 1;
     return r;
 }
+
+//! Where a tile's rows come from and go to: the row tables of a stack, ...
+struct stack_rows {
+    cpair *pairs;
+    garow *arow;
+    gcrow *crow;
+    uint32_t astride;
+    __device__ __forceinline__ row_src row(uint32_t p, uint32_t r) const {
+        garow *e = arow + (size_t(p) * astride + r);
+        row_src s;
+        s.d = e->d; s.off = e->off; s.lda = e->lda;
+        return s;
+    }
+    __device__ __forceinline__ void write(uint32_t r, uint32_t col, double x) const {
+        gcrow *cr = crow + r;
+        gout *cp = (gout *)(uintptr_t)cr->c + col;
+        *cp = cr->zero ? x : x + *cp;
+    }
+};
+
+//! ... or a dense matrix product (one pair).
+struct dense_rows {
+    cpair *pairs;
+    double d;
+    gout *c;
+    uint32_t rstep, lda, ldc, zero;     //!< bytes from row to row of A, its row length, that of C
+    __device__ __forceinline__ row_src row(uint32_t, uint32_t r) const {
+        row_src s;
+        s.d = d; s.off = r * rstep; s.lda = lda;
+        return s;
+    }
+    __device__ __forceinline__ void write(uint32_t r, uint32_t col, double x) const {
+        gout *cp = c + (size_t(r) * ldc + col);
+        *cp = zero ? x : x + *cp;
+    }
+};
+
+//! A tile and its part of the chunk sequence: `count` chunks from chunk c of
+//! pair p on.  part: where the tile's partial sums go (fragment order), or
+//! null: they are all there is and go to C.
+struct tile_part {
+    uint32_t m0, n0, mrem, nrem;
+    uint32_t p, c, count;
+    gout *part;
+};
 
 } // unnamed namespace
 
@@ -105,9 +157,8 @@ struct tile_smem {
     uint32_t cn[KG][2][BN];
 };
 
-template<int FM, int KG>
-__device__ __forceinline__ void tile_body(cstack *st, uint32_t m0, uint32_t n0,
-    tile_smem<FM, KG> &sm) {
+template<int FM, int KG, class SRC>
+__device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, tile_smem<FM, KG> &sm) {
 
     typedef tile_smem<FM, KG> S;
     constexpr int BM = S::BM, BN = S::BN;
@@ -118,11 +169,8 @@ __device__ __forceinline__ void tile_body(cstack *st, uint32_t m0, uint32_t n0,
     const int hi = tid >> 4, lo = tid & 15;
     const int hr = ((hi & 1) << 3) | (hi >> 1);  // as a row: rows 8 apart side by side (their LDS banks differ)
 
-    const uint32_t mrem = st->rows - m0, nrem = st->n - n0;
-    cpair *pairs = (cpair *)(uintptr_t)st->pairs;
-    garow *arow = (garow *)(uintptr_t)st->arow;
-    gcrow *crow = (gcrow *)(uintptr_t)st->crow;
-    const uint32_t npairs = st->npairs, astride = st->astride, nchunk = st->nchunk;
+    const uint32_t m0 = tp.m0, n0 = tp.n0, mrem = tp.mrem, nrem = tp.nrem, nchunk = tp.count;
+    cpair *pairs = src.pairs;
 
     double4_t acc[FM];
 #pragma unroll
@@ -133,10 +181,7 @@ __device__ __forceinline__ void tile_body(cstack *st, uint32_t m0, uint32_t n0,
         const uint32_t trow = uint32_t(tid) < mrem ? m0 + tid : m0;
         const uint32_t tcol = uint32_t(tid & 63) < nrem ? n0 + (tid & 63) : n0;
         auto info_load = [&](uint32_t p, row_src &ar, uint32_t &cn) {
-            if(tid < BM) {
-                garow *e = arow + (size_t(p) * astride + trow);
-                ar.d = e->d; ar.off = e->off; ar.lda = e->lda;
-            }
+            if(tid < BM) ar = src.row(p, trow);
             if(tid >= 192) {
                 cpair *sp = pairs + p;
                 if(tabled(sp)) cn = 8u * uint32_t(((gint *)(uintptr_t)sp->noff)[tcol]);
@@ -157,11 +202,12 @@ __device__ __forceinline__ void tile_body(cstack *st, uint32_t m0, uint32_t n0,
 
         // The group's next chunks: n1 to be loaded, n2 whose pair's tables
         // come next.  A group without a chunk keeps an in-bounds position on
-        // chunk 0 and multiplies zeros.
+        // the first one and multiplies zeros.
         chunk_pos first;
-        first.p = 0; first.c = 0; first.k = pairs[0].k; first.slot = 0; first.valid = true;
-        chunk_pos n1 = chunk_advance(pairs, npairs, first, g);
-        chunk_pos n2 = chunk_advance(pairs, npairs, n1, KG);
+        first.p = tp.p; first.c = tp.c; first.k = pairs[tp.p].k; first.slot = 0;
+        first.left = nchunk; first.valid = true;
+        chunk_pos n1 = chunk_advance(pairs, first, g);
+        chunk_pos n2 = chunk_advance(pairs, n1, KG);
         {
             row_src ar; uint32_t cq = 0;
             info_load(n1.p, ar, cq);
@@ -328,7 +374,7 @@ __device__ __forceinline__ void tile_body(cstack *st, uint32_t m0, uint32_t n0,
             }
             if(info) info_store(n2.slot, ar, cq);
             n1 = n2;
-            n2 = chunk_advance(pairs, npairs, n2, KG);
+            n2 = chunk_advance(pairs, n2, KG);
             __syncthreads();
         };
         // the first chunk into buffer 0, then a step for every chunk; a wave
@@ -349,13 +395,8 @@ __device__ __forceinline__ void tile_body(cstack *st, uint32_t m0, uint32_t n0,
 #pragma unroll
             for(int v = 0; v < 4; v++) {
                 const uint32_t row = 16 * i + lg + 4 * v, col = 16 * wave + lr;
-                if(row < mrem && col < nrem) {
-                    gcrow *cr = crow + (m0 + row);
-                    gout *cp = (gout *)(uintptr_t)cr->c + (n0 + col);
-                    double x = acc[i][v];
-                    if(!cr->zero) x += *cp;
-                    *cp = x;
-                }
+                if(tp.part) tp.part[((i * 4 + v) * 4 + wave) * 64 + lane] = acc[i][v];
+                else if(row < mrem && col < nrem) src.write(m0 + row, n0 + col, acc[i][v]);
             }
         return;
     }
@@ -373,50 +414,91 @@ __device__ __forceinline__ void tile_body(cstack *st, uint32_t m0, uint32_t n0,
         for(int q = 1; q < KG; q++) x += red[q * BM * BN + e];
         const int l = e & 63, w = (e >> 6) & 3, v = (e >> 8) & 3, i = e >> 10;
         const uint32_t row = 16 * i + (l >> 4) + 4 * v, col = 16 * w + (l & 15);
-        if(row < mrem && col < nrem) {
-            gcrow *cr = crow + (m0 + row);
-            gout *cp = (gout *)(uintptr_t)cr->c + (n0 + col);
-            if(!cr->zero) x += *cp;
-            *cp = x;
-        }
+        if(tp.part) tp.part[e] = x;
+        else if(row < mrem && col < nrem) src.write(m0 + row, n0 + col, x);
     }
 }
 
 //! A tile of height up to 16 FM: the loop compiled for its number of 16-row
 //! fragments (a condition per fragment inside one loop would make the
 //! compiler copy the accumulators).
-template<int FM, int KG, int FA>
-__device__ __forceinline__ void tile_height(cstack *st, uint32_t m0, uint32_t n0, uint32_t fa,
-    char *smem) {
-    if(FA == 1 || fa >= FA) tile_body<FA, KG>(st, m0, n0, *(tile_smem<FA, KG> *)smem);
-    else tile_height<FM, KG, (FA > 1 ? FA - 1 : 1)>(st, m0, n0, fa, smem);
+template<int FM, int KG, int FA, class SRC>
+__device__ __forceinline__ void tile_height(const SRC &src, const tile_part &tp, char *smem) {
+    if(FA == 1 || tp.mrem > 16 * (FA - 1)) tile_body<FA, KG>(src, tp, *(tile_smem<FA, KG> *)smem);
+    else tile_height<FM, KG, (FA > 1 ? FA - 1 : 1)>(src, tp, smem);
 }
 
-template<int FM, int KG, int OCC>
-__global__ void __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(OCC)))
-gemm_tile_kernel(const tile_stack *__restrict__ stacks, const gemm_tile *__restrict__ tiles) {
-    __shared__ __attribute__((aligned(16))) char smem[sizeof(tile_smem<FM, KG>)];
-    const gemm_tile tile = tiles[blockIdx.x];
-    cstack *st = (cstack *)(uintptr_t)(stacks + tile.cblock);
-    const uint32_t rows = st->rows, m0 = uint32_t(tile.tm) * (16 * FM);
-    if(rows == 0) return;                        // padding tile (whole workgroup)
-    // Workgroups that share a CU get different priorities, the same on its
-    // four SIMDs: a workgroup's waves then pass their barriers together
-    // instead of each waiting for another workgroup (4 % on large products).
+//! Workgroups that share a CU get different priorities, the same on its four
+//! SIMDs: a workgroup's waves then pass their barriers together instead of
+//! each waiting for another workgroup (4 % on large products).
+__device__ __forceinline__ void rank_workgroup() {
     switch((blockIdx.x >> 8) & 3) {
     case 0: __builtin_amdgcn_s_setprio(3); break;
     case 1: __builtin_amdgcn_s_setprio(2); break;
     case 2: __builtin_amdgcn_s_setprio(1); break;
     default: __builtin_amdgcn_s_setprio(0); break;
     }
-    tile_height<FM, KG, FM>(st, m0, uint32_t(tile.tn) * 64, (rows - m0 + 15) >> 4, smem);
 }
 
-hipError_t launch_gemm_tile(int cfg, const tile_stack *st, const gemm_tile *tiles,
-    uint32_t ntiles, hipStream_t s) {
-    if(ntiles == 0) return hipSuccess;
+template<int FM, int KG, int OCC>
+__global__ void __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(OCC)))
+gemm_tile_kernel(const tile_stack *__restrict__ stacks, const tile_item *__restrict__ items,
+    double *__restrict__ parts) {
+    __shared__ __attribute__((aligned(16))) char smem[sizeof(tile_smem<FM, KG>)];
+    const tile_item it = items[blockIdx.x];
+    cstack *st = (cstack *)(uintptr_t)(stacks + it.stack);
+    if(st->rows == 0) return;                    // padding tile (whole workgroup)
+    rank_workgroup();
+    stack_rows src;
+    src.pairs = (cpair *)(uintptr_t)st->pairs;
+    src.arow = (garow *)(uintptr_t)st->arow;
+    src.crow = (gcrow *)(uintptr_t)st->crow;
+    src.astride = st->astride;
+    tile_part tp;
+    tp.m0 = uint32_t(it.tm) * (16 * FM);
+    tp.n0 = uint32_t(it.tn) * 64;
+    tp.mrem = st->rows - tp.m0;
+    tp.nrem = st->n - tp.n0;
+    tp.p = it.p; tp.c = it.c; tp.count = it.count;
+    tp.part = it.part < 0 ? (gout *)0 : (gout *)(uintptr_t)parts + size_t(it.part) * (1024 * FM);
+    tile_height<FM, KG, FM>(src, tp, smem);
+}
+
+//! C of the tiles whose chunks were cut into parts: their partial sums added
+//! in the order of the parts.
+__global__ void __launch_bounds__(256)
+tile_sum_kernel(const tile_stack *__restrict__ stacks, const tile_item *__restrict__ items,
+    const double *__restrict__ parts, uint32_t fm) {
+    const tile_item it = items[blockIdx.x];      // part: the first part's place, count: parts
+    cstack *st = (cstack *)(uintptr_t)(stacks + it.stack);
+    const uint32_t m0 = uint32_t(it.tm) * (16 * fm), n0 = uint32_t(it.tn) * 64;
+    const uint32_t mrem = st->rows - m0, nrem = st->n - n0;
+    stack_rows src;
+    src.crow = (gcrow *)(uintptr_t)st->crow;
+    const uint32_t e = blockIdx.y * 256 + threadIdx.x;
+    const uint32_t l = e & 63, w = (e >> 6) & 3, v = (e >> 8) & 3, i = e >> 10;
+    const uint32_t row = 16 * i + (l >> 4) + 4 * v, col = 16 * w + (l & 15);
+    if(row >= mrem || col >= nrem) return;
+    gdouble *p = (gdouble *)(uintptr_t)parts + size_t(it.part) * (1024 * fm) + e;
+    double x = p[0];
+    for(uint32_t q = 1; q < it.count; q++) x += p[size_t(q) * (1024 * fm)];
+    src.write(m0 + row, n0 + col, x);
+}
+
+hipError_t launch_tile_sum(int cfg, const tile_stack *st, const tile_item *items, uint32_t n,
+    const double *parts, hipStream_t s) {
+    if(n == 0) return hipSuccess;
+    uint32_t bm, bn;
+    tile_shape(cfg, bm, bn);
+    hipLaunchKernelGGL(tile_sum_kernel, dim3(n, bm / 4), dim3(256), 0, s, st, items, parts, bm / 16);
+    return hipGetLastError();
+}
+
+hipError_t launch_gemm_tile(int cfg, const tile_stack *st, const tile_item *items,
+    uint32_t nitems, double *parts, hipStream_t s) {
+    if(nitems == 0) return hipSuccess;
 #define LT_TILE(FM, KG, OCC) \
-    hipLaunchKernelGGL((gemm_tile_kernel<FM, KG, OCC>), dim3(ntiles), dim3(256 * KG), 0, s, st, tiles)
+    hipLaunchKernelGGL((gemm_tile_kernel<FM, KG, OCC>), dim3(nitems), dim3(256 * KG), 0, s, st, items, parts)
     switch(cfg) {
     case WG_16x64_G4: LT_TILE(1, 4, 4); break;
     case WG_32x64_G4: LT_TILE(2, 4, 4); break;

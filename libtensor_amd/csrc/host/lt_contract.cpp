@@ -115,6 +115,8 @@ struct dev_lists {
         mem = 0;
         bytes = 0;
     }
+    //! At least `n` bytes (contents not kept).
+    void *at_least(context &c, size_t n) { return mem && bytes >= n ? mem : reset(c, n); }
     //! Replaces the allocation with a new one of `n` bytes.
     void *reset(context &c, size_t n) {
         release();
@@ -253,6 +255,13 @@ struct contract_plan {
     // block (per-block launches), each list ending with an empty one
     std::vector<dev::tile_stack> tstacks;
     dev::tile_stack *d_tstacks, *d_bstacks;
+    // their work items and the tiles run in parts: of the grouped launch, and
+    // per C block (items of block b from block_item_begin[b] on)
+    std::vector<dev::tile_item> titems, tsums, bitems, bsums;
+    std::vector<uint32_t> block_item_begin, block_sum_begin;
+    dev::tile_item *d_titems, *d_tsums, *d_bitems, *d_bsums;
+    size_t n_parts;                   // places for partial sums of the grouped launch
+    dev_lists parts;                  // partial sums (tiles)
     // C blocks reading the same B operands (same order and layouts) share a
     // group; n_xcd: XCDs of the device
     std::vector<size_t> cb_group;
@@ -302,7 +311,7 @@ struct contract_plan {
         d_cb(0), d_pairs(0), d_tiles_sorted(0), d_tiles_block(0), scratch(0),
         scratch_elems(0), ctx(0), events(false), graph(0), gexec(0), graph_launches(0),
         d_stacks(0), d_spairs(0), d_arows(0), d_crows(0), d_stiles(0), d_vtiles(0),
-        d_tstacks(0), d_bstacks(0),
+        d_tstacks(0), d_bstacks(0), d_titems(0), d_tsums(0), d_bitems(0), d_bsums(0), n_parts(0),
         n_groups(0), n_xcd(8),
         n_prep_st_chunks(0), d_prep_st(0), d_pst_cd(0), d_pst_co(0),
         oz_slices(0), oz_tile(0), oz_tile_set(-1), d_oz_split(0), d_oz_items(0), n_oz_items(0), d_oz_pairs(0),
@@ -330,7 +339,8 @@ hipError_t launch_grouped_list(const contract_plan &pl, int k, const void *d_lis
         return dev::launch_gemm_stacked_var(k, pl.d_stacks, pl.d_spairs, pl.d_arows, pl.d_crows,
             (const dev::var_tile*)d_list, n, s);
     if(dev::is_tile(k))
-        return dev::launch_gemm_tile(k, pl.d_tstacks, (const dev::gemm_tile*)d_list, n, s);
+        return dev::launch_gemm_tile(k, pl.d_tstacks, (const dev::tile_item*)d_list, n,
+            (double*)pl.parts.mem, s);
     if(dev::is_stacked(k))
         return dev::launch_gemm_stacked(k, pl.d_stacks, pl.d_spairs, pl.d_arows, pl.d_crows,
             (const dev::gemm_tile*)d_list, n, s);
@@ -342,8 +352,12 @@ hipError_t launch_grouped(const contract_plan &pl, int k, hipStream_t s) {
     if(dev::is_var(k))
         return dev::launch_gemm_stacked_var(k, pl.d_stacks, pl.d_spairs, pl.d_arows, pl.d_crows,
             pl.d_vtiles, (uint32_t)pl.vtiles.size(), s);
-    if(dev::is_tile(k))
-        return dev::launch_gemm_tile(k, pl.d_tstacks, pl.d_stiles, (uint32_t)pl.stiles.size(), s);
+    if(dev::is_tile(k)) {
+        hipError_t e = dev::launch_gemm_tile(k, pl.d_tstacks, pl.d_titems,
+            (uint32_t)pl.titems.size(), (double*)pl.parts.mem, s);
+        return e != hipSuccess ? e : dev::launch_tile_sum(k, pl.d_tstacks, pl.d_tsums,
+            (uint32_t)pl.tsums.size(), (double*)pl.parts.mem, s);
+    }
     if(dev::is_stacked(k))
         return dev::launch_gemm_stacked(k, pl.d_stacks, pl.d_spairs, pl.d_arows, pl.d_crows,
             pl.d_stiles, (uint32_t)pl.stiles.size(), s);
@@ -911,6 +925,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         std::copy(ts.begin(), ts.end(), pair_tab.begin() + p0);
     }
     std::vector<std::vector<size_t> > stack_blocks;     // C blocks of a stack, in row order
+    std::vector<uint32_t> block_pair0(pl.cblocks.size() + 1, 0);    // first pair of a C block's stack
     {
         std::map<std::pair<uint32_t, std::vector<bkey_t> >, std::vector<size_t> > groups;
         std::vector<std::pair<uint32_t, std::vector<bkey_t> > > order;
@@ -1056,6 +1071,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
             pl.stacks.push_back(sd);
             pl.stack_ksum.push_back(ks);
             stack_blocks.push_back(bl);
+            for(size_t q = 0; q < bl.size(); q++) block_pair0[bl[q]] = sd.pair_begin;
         }
         dev::stack_desc z;
         std::memset(&z, 0, sizeof(z));
@@ -1211,7 +1227,13 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         // launches, and each candidate costs two timed launches
         for(size_t i = 0; i < est.size(); i++)
             if(cfg != -2 || dev::is_stacked(est[i].second)) candidates.push_back(est[i].second);
-        if(cfg == -1 || add || !measure) candidates.resize(1);
+        if(cfg == -1) candidates.resize(1);
+        // No timing (accumulating plans, planning beside other work): the
+        // measured line between the small tiles that start fastest and the
+        // tiles that move least data (14 and 22 us for 1.3e8 FLOPs, 47 and
+        // 35 us for 3.9e8).
+        else if(add || !measure)
+            candidates.assign(1, flops < 2e8 ? dev::STACK_32x32_W4_O3 : dev::WG_64x64_G1);
         // the configuration measured for these operands (same pairs, same
         // work list for any result tensor) is reused without measuring again
         if(cfg == -2 && m_tuned_cfg >= 0 && m_tuned_va == pl.va && m_tuned_vb == pl.vb)
@@ -1332,6 +1354,136 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     pl.d_pst_cd = (uint32_t*)(base + o_scd);
     pl.d_pst_co = (uint32_t*)(base + o_sco);
 
+    // Work items of a workgroup-tiled configuration.  Where the tiles of the
+    // whole list are fewer than keep the CUs evenly busy (kItems, four per
+    // CU), the chunk sequences are cut into parts of about equal length (at
+    // least kMinChunks, which pays for a part's sums going through memory);
+    // how a stack is cut depends on the plan only, so per-block launches and
+    // batches add the same sums in the same order.
+    auto make_items = [&](int k, int order) {
+        const uint32_t kItems = 1024, kMinChunks = 16;
+        uint32_t bm, bn;
+        dev::tile_shape(k, bm, bn);
+        const size_t ns = pl.stacks.size() - 1, nb = pl.cblocks.size();
+        auto tiles_of = [&](const dev::tile_stack &t, uint32_t &tm, uint32_t &tn) {
+            tm = (t.rows + bm - 1) / bm;
+            tn = (t.n + bn - 1) / bn;
+            lt_require(tm < 65536 && tn < 65536, LT_ERR_PARAM, "stack too large");
+        };
+        double chunks = 0.0, ntiles = 0.0;
+        for(size_t i = 0; i < ns; i++) {
+            uint32_t tm, tn;
+            tiles_of(pl.tstacks[i], tm, tn);
+            ntiles += double(tm) * tn;
+            chunks += double(tm) * tn * pl.tstacks[i].nchunk;
+        }
+        const double len = std::max(double(kMinChunks), chunks / kItems);
+        auto cut = [&](const dev::tile_stack &t) {
+            return ntiles >= kItems ? 1u : std::max(1u, uint32_t(double(t.nchunk) / len + 0.5));
+        };
+        typedef std::pair<double, dev::tile_item> unit;
+        auto add_tile = [&](size_t stack, const dev::tile_stack &t, uint32_t i, uint32_t j, uint32_t pair0,
+            std::vector<unit> &units, std::vector<dev::tile_item> &sums, size_t &nparts) {
+            const uint32_t np = cut(t), fa = (std::min(bm, t.rows - i * bm) + 15) / 16;
+            dev::tile_item it;
+            it.stack = (uint32_t)stack; it.tm = (uint16_t)i; it.tn = (uint16_t)j;
+            it.p = 0; it.c = 0; it.part = -1;
+            if(np > 1) {
+                dev::tile_item sm = it;
+                sm.part = (int32_t)nparts; sm.count = np;
+                sums.push_back(sm);
+            }
+            uint32_t at = 0;
+            for(uint32_t q = 0; q < np; q++) {
+                const uint32_t end = uint32_t(uint64_t(t.nchunk) * (q + 1) / np);
+                it.count = end - at;
+                if(np > 1) it.part = (int32_t)nparts++;
+                units.push_back(std::make_pair(double(it.count) * fa, it));
+                for(; at < end; ) {
+                    const uint32_t left = (pl.spairs[pair0 + it.p].k + 15) / 16 - it.c;
+                    if(end - at < left) { it.c += end - at; at = end; }
+                    else { at += left; it.p++; it.c = 0; }
+                }
+            }
+        };
+        auto longer = [](const unit &x, const unit &y) { return x.first > y.first; };
+        std::vector<unit> units;
+        std::vector<double> scost(ns, 0.0);
+        pl.tsums.clear();
+        pl.n_parts = 0;
+        for(size_t i = 0; i < ns; i++) {
+            uint32_t tm, tn;
+            tiles_of(pl.tstacks[i], tm, tn);
+            const size_t u0 = units.size();
+            for(uint32_t a = 0; a < tm; a++) for(uint32_t b = 0; b < tn; b++)
+                add_tile(i, pl.tstacks[i], a, b, pl.stacks[i].pair_begin, units, pl.tsums, pl.n_parts);
+            for(size_t u = u0; u < units.size(); u++) scost[i] += units[u].first;
+        }
+        std::stable_sort(units.begin(), units.end(), longer);
+        pl.titems.clear();
+        if(order == 0) {
+            for(size_t i = 0; i < units.size(); i++) pl.titems.push_back(units[i].second);
+        } else {
+            // XCD-aware: stacks to XCDs longest first onto the least loaded,
+            // each XCD's items longest first at positions x, x + nx, ...; the
+            // padding items name the empty stack
+            std::vector<size_t> so(ns);
+            std::iota(so.begin(), so.end(), size_t(0));
+            std::stable_sort(so.begin(), so.end(), [&](size_t x, size_t y) { return scost[x] > scost[y]; });
+            std::vector<double> load(nx, 0.0);
+            std::vector<int> sx(ns, 0);
+            for(size_t i = 0; i < ns; i++) {
+                const int x = int(std::min_element(load.begin(), load.end()) - load.begin());
+                sx[so[i]] = x;
+                load[x] += scost[so[i]];
+            }
+            std::vector<std::vector<dev::tile_item> > q(nx);
+            size_t qmax = 0;
+            for(size_t i = 0; i < units.size(); i++) {
+                std::vector<dev::tile_item> &qq = q[sx[units[i].second.stack]];
+                qq.push_back(units[i].second);
+                qmax = std::max(qmax, qq.size());
+            }
+            dev::tile_item empty;
+            std::memset(&empty, 0, sizeof(empty));
+            empty.stack = (uint32_t)ns;
+            empty.part = -1;
+            pl.titems.assign(qmax * nx, empty);
+            for(int x = 0; x < nx; x++)
+                for(size_t l = 0; l < q[x].size(); l++) pl.titems[l * nx + x] = q[x][l];
+        }
+        // per C block, in block order
+        pl.bitems.clear(); pl.bsums.clear();
+        pl.block_item_begin.clear(); pl.block_sum_begin.clear();
+        size_t bparts = 0;
+        for(size_t b = 0; b < nb; b++) {
+            pl.block_item_begin.push_back((uint32_t)pl.bitems.size());
+            pl.block_sum_begin.push_back((uint32_t)pl.bsums.size());
+            const dev::tile_stack &t = pl.tstacks[pl.stacks.size() + b];
+            uint32_t tm, tn;
+            tiles_of(t, tm, tn);
+            std::vector<unit> bu;
+            for(uint32_t i = 0; i < tm; i++) for(uint32_t j = 0; j < tn; j++)
+                add_tile(b, t, i, j, block_pair0[b], bu, pl.bsums, bparts);
+            for(size_t u = 0; u < bu.size(); u++) pl.bitems.push_back(bu[u].second);
+        }
+        pl.block_item_begin.push_back((uint32_t)pl.bitems.size());
+        pl.block_sum_begin.push_back((uint32_t)pl.bsums.size());
+        const std::vector<dev::tile_item> *lists[4] = { &pl.titems, &pl.tsums, &pl.bitems, &pl.bsums };
+        dev::tile_item **at[4] = { &pl.d_titems, &pl.d_tsums, &pl.d_bitems, &pl.d_bsums };
+        size_t off[5] = { 0 };
+        for(int i = 0; i < 4; i++) off[i + 1] = align256(off[i] + lists[i]->size() * sizeof(dev::tile_item));
+        std::vector<char> host(off[4] ? off[4] : 256, 0);
+        for(int i = 0; i < 4; i++)
+            if(!lists[i]->empty())
+                std::memcpy(&host[off[i]], lists[i]->data(), lists[i]->size() * sizeof(dev::tile_item));
+        pl.stk_tiles.at_least(ctx, host.size());
+        ctx.upload_new(pl.stk_tiles.mem, host.data(), host.size());
+        for(int i = 0; i < 4; i++) *at[i] = (dev::tile_item*)((char*)pl.stk_tiles.mem + off[i]);
+        const size_t bytes = std::max(pl.n_parts, bparts) * bm * bn * sizeof(double);
+        if(bytes) pl.parts.at_least(ctx, bytes);
+    };
+
     // tile lists live in their own allocation (replaced by the autotuner)
     auto upload_tiles = [&](int k, int order) {
         make_tiles(k, order, pl.tiles_by_block, pl.block_tile_begin, pl.tiles_sorted);
@@ -1340,7 +1492,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         size_t nt = pl.tiles_sorted.size() * sizeof(dev::gemm_tile);
         size_t nb = pl.tiles_by_block.size() * sizeof(dev::gemm_tile);
         size_t tsz = align256(nt) + align256(nb) + 256;
-        pl.tiles.reset(ctx, tsz);
+        pl.tiles.at_least(ctx, tsz);
         std::vector<char> th(tsz, 0);
         if(nt) std::memcpy(&th[0], pl.tiles_sorted.data(), nt);
         if(nb) std::memcpy(&th[align256(nt)], pl.tiles_by_block.data(), nb);
@@ -1351,7 +1503,9 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         pl.tile_order = order;
         pl.stiles.clear();
         pl.vtiles.clear();
-        if(dev::is_var(k)) {
+        if(dev::is_tile(k)) {
+            make_items(k, order);
+        } else if(dev::is_var(k)) {
             // full 64-row tiles and one tile per row / column remainder,
             // largest (k sum x area) first
             const uint32_t fnx = 2;
@@ -1376,7 +1530,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
                     return x.first > y.first; });
             for(size_t i = 0; i < vt.size(); i++) pl.vtiles.push_back(vt[i].second);
             size_t nb = pl.vtiles.size() * sizeof(dev::var_tile);
-            pl.stk_tiles.reset(ctx, nb ? nb : 256);
+            pl.stk_tiles.at_least(ctx, nb ? nb : 256);
             if(nb) ctx.upload_new(pl.stk_tiles.mem, pl.vtiles.data(), nb);
             pl.d_vtiles = (dev::var_tile*)pl.stk_tiles.mem;
         } else if(dev::is_stacked(k)) {
@@ -1430,7 +1584,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
                     for(size_t l = 0; l < q[x].size(); l++) pl.stiles[l * nx + x] = q[x][l];
             }
             size_t nb = pl.stiles.size() * sizeof(dev::gemm_tile);
-            pl.stk_tiles.reset(ctx, nb ? nb : 256);
+            pl.stk_tiles.at_least(ctx, nb ? nb : 256);
             if(nb) ctx.upload_new(pl.stk_tiles.mem, pl.stiles.data(), nb);
             pl.d_stiles = (dev::gemm_tile*)pl.stk_tiles.mem;
         }
@@ -1448,23 +1602,14 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     // the accumulating path).
     if(candidates.size() > 1) {
         hipStream_t s = ctx.stream();
-        if(pl.n_prep_chunks)
-            hip_check(dev::launch_permute(pl.d_prep, pl.d_prep_cd, pl.d_prep_co,
-                pl.n_prep_chunks, s), "permute (prepare)");
-        // each candidate is timed with the prepare permute it needs (the
-        // stacked kernels read B operands in place and prepare less)
-        auto prep_for = [&](int k) -> hipError_t {
-            if(dev::is_stacked(k))
-                return pl.n_prep_st_chunks ? dev::launch_permute(pl.d_prep_st, pl.d_pst_cd,
-                    pl.d_pst_co, pl.n_prep_st_chunks, s) : hipSuccess;
-            return pl.n_prep_chunks ? dev::launch_permute(pl.d_prep, pl.d_prep_cd,
-                pl.d_prep_co, pl.n_prep_chunks, s) : hipSuccess;
-        };
+        // (the candidates are stacked kernels: one prepare for all of them)
+        if(pl.n_prep_st_chunks)
+            hip_check(dev::launch_permute(pl.d_prep_st, pl.d_pst_cd, pl.d_pst_co,
+                pl.n_prep_st_chunks, s), "permute (prepare)");
         // A large plan is timed on a sample of each candidate's launch list:
         // every stride-th group of nx consecutive tiles (a group keeps its
-        // XCD placement), about kTuneFlops of work.  The prepare permute is
-        // timed whole, the sampled launch scaled by the list's cost over the
-        // sample's (cost of a tile: the k sum of its block or stack times its
+        // XCD placement), about kTuneFlops of work, its time scaled by the
+        // list's cost over the sample's (cost of a tile: the k sum of its block or stack times its
         // fragment count).
         const double kTuneFlops = 2e11;
         const size_t stride = flops > 2.0 * kTuneFlops ? size_t(flops / kTuneFlops) : 1;
@@ -1480,7 +1625,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
             }
             scale = part > 0.0 ? tot / part : 1.0;
             const size_t nb = sub.size() * sizeof(tile_t);
-            tune_list.reset(ctx, nb ? nb : 256);
+            tune_list.at_least(ctx, nb ? nb : 256);
             if(nb) ctx.upload_new(tune_list.mem, sub.data(), nb);
             return (uint32_t)sub.size();
         };
@@ -1490,39 +1635,46 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
             if(dev::is_var(k))
                 return take(pl.vtiles, [&](const dev::var_tile &t) {
                     return ksum_of(pl.stack_ksum, t.stack) * t.fm * t.fn; }, scale);
+            if(dev::is_tile(k))
+                return take(pl.titems, [&](const dev::tile_item &t) { return double(t.count); }, scale);
             if(dev::is_stacked(k))
                 return take(pl.stiles, [&](const dev::gemm_tile &t) {
                     return ksum_of(pl.stack_ksum, t.cblock); }, scale);
             return take(pl.tiles_sorted, [&](const dev::gemm_tile &t) {
                 return ksum_of(cb_ksum, t.cblock); }, scale);
         };
+        // Every candidate in longest-first order, then the best three in the
+        // XCD-aware order.  A candidate's launch follows an untimed one
+        // without a pause, so that all are timed at working clocks (timed
+        // after an idle gap, the choice for the ring o = 29, v = 131 was a
+        // third slower than the best in repeated performs).
         float best = 1e30f;
         int bestk = cfg, besto = 0;
-        for(size_t ci = 0; ci < 2 * candidates.size(); ci++) {
-            int k = candidates[ci / 2], o = int(ci % 2);
+        auto time_one = [&](int k, int o) {
             upload_tiles(k, o);
             double scale = 1.0;
             const uint32_t ntune = stride > 1 ? sample(k, scale) : 0;
-            // one timed launch; a short one (first-launch overheads are
-            // then not negligible) is timed again
-            float ms = 0.f;
-            for(int rep = 0; rep < 2; rep++) {
-                float mp = 0.f, mg = 0.f;
-                hip_check(hipEventRecord(pl.ev[0], s), "hipEventRecord");
-                hip_check(prep_for(k), "autotune (prepare)");
-                hip_check(hipEventRecord(pl.ev[1], s), "hipEventRecord");
+            auto go = [&]() {
                 hip_check(stride > 1 ? launch_grouped_list(pl, k, tune_list.mem, ntune, s) :
                     launch_grouped(pl, k, s), "autotune");
-                hip_check(hipEventRecord(pl.ev[2], s), "hipEventRecord");
-                hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
-                hip_check(hipEventElapsedTime(&mp, pl.ev[0], pl.ev[1]), "hipEventElapsedTime");
-                hip_check(hipEventElapsedTime(&mg, pl.ev[1], pl.ev[2]), "hipEventElapsedTime");
-                ms = mp + float(mg * scale);
-                if(mp + mg > 20.f) break;
-            }
-            if(o == 0 || ms < m_stats.tune_ms[k]) m_stats.tune_ms[k] = ms;
+            };
+            go();
+            hip_check(hipEventRecord(pl.ev[1], s), "hipEventRecord");
+            go();
+            hip_check(hipEventRecord(pl.ev[2], s), "hipEventRecord");
+            hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+            float mg = 0.f;
+            hip_check(hipEventElapsedTime(&mg, pl.ev[1], pl.ev[2]), "hipEventElapsedTime");
+            const float ms = float(mg * scale);
+            if(m_stats.tune_ms[k] <= 0.0 || ms < m_stats.tune_ms[k]) m_stats.tune_ms[k] = ms;
             if(ms < best) { best = ms; bestk = k; besto = o; }
-        }
+        };
+        for(int k = 0; k < dev::TILE_COUNT; k++) m_stats.tune_ms[k] = 0.0;
+        for(size_t ci = 0; ci < candidates.size(); ci++) time_one(candidates[ci], 0);
+        std::vector<int> rank(candidates);
+        std::sort(rank.begin(), rank.end(), [&](int x, int y) {
+            return m_stats.tune_ms[x] < m_stats.tune_ms[y]; });
+        for(size_t ci = 0; ci < rank.size() && ci < 3; ci++) time_one(rank[ci], 1);
         cfg = bestk;
         upload_tiles(cfg, besto);
         m_tuned_cfg = cfg;
@@ -1896,14 +2048,23 @@ void btod_contract2::enqueue(int mode, hipStream_t s, bool timed, size_t &launch
         std::lock_guard<std::mutex> lk(ctx.side_lock());
         ctx.side_fork(s);
         int j = 0;
-        for(size_t b = 0; b + 1 < pl.block_tile_begin.size(); b++) {
+        const bool wg = dev::is_tile(pl.tile_cfg);
+        for(size_t b = 0; wg && b + 1 < pl.block_item_begin.size(); b++) {
+            const uint32_t t0 = pl.block_item_begin[b], t1 = pl.block_item_begin[b + 1];
+            const uint32_t s0 = pl.block_sum_begin[b], s1 = pl.block_sum_begin[b + 1];
+            if(t1 == t0) continue;
+            hipStream_t sd = ctx.side(j++);
+            hip_check(dev::launch_gemm_tile(pl.tile_cfg, pl.d_bstacks, pl.d_bitems + t0, t1 - t0,
+                (double*)pl.parts.mem, sd), "gemm (per block)");
+            hip_check(dev::launch_tile_sum(pl.tile_cfg, pl.d_bstacks, pl.d_bsums + s0, s1 - s0,
+                (double*)pl.parts.mem, sd), "gemm (per block, sums)");
+            launches += s1 > s0 ? 2 : 1;
+        }
+        for(size_t b = 0; !wg && b + 1 < pl.block_tile_begin.size(); b++) {
             uint32_t t0 = pl.block_tile_begin[b], t1 = pl.block_tile_begin[b + 1];
             if(t1 == t0) continue;
-            hip_check(dev::is_tile(pl.tile_cfg) ?
-                dev::launch_gemm_tile(pl.tile_cfg, pl.d_bstacks, pl.d_tiles_block + t0, t1 - t0,
-                    ctx.side(j++)) :
-                dev::launch_gemm(pl.tile_cfg, pl.d_cb, pl.d_pairs,
-                    pl.d_tiles_block + t0, t1 - t0, t1 - t0, ctx.side(j++)), "gemm (per block)");
+            hip_check(dev::launch_gemm(pl.tile_cfg, pl.d_cb, pl.d_pairs,
+                pl.d_tiles_block + t0, t1 - t0, t1 - t0, ctx.side(j++)), "gemm (per block)");
             launches++;
         }
         ctx.side_join(s);
@@ -2055,14 +2216,14 @@ void btod_contract2::perform_sliced(btensor &c, bool add, double d, double slice
     }
     hip_check(hipEventRecord(pl.ev[1], s), "hipEventRecord");
     const uint32_t nt = dev::is_var(k) ? (uint32_t)pl.vtiles.size() :
-        dev::is_stacked(k) ? (uint32_t)pl.stiles.size() : (uint32_t)pl.tiles_sorted.size();
+        dev::is_tile(k) ? (uint32_t)pl.titems.size() : dev::is_stacked(k) ? (uint32_t)pl.stiles.size() : (uint32_t)pl.tiles_sorted.size();
     const uint32_t nslices = (uint32_t)std::max(1.0, std::min(double(nt),
         std::ceil(m_stats.flops / slice_flops)));
     const uint32_t per = (nt + nslices - 1) / nslices;
     for(uint32_t t0 = 0; t0 < nt; t0 += per) {
         const uint32_t n = std::min(per, nt - t0);
         const void *list = dev::is_var(k) ? (const void*)(pl.d_vtiles + t0) :
-            dev::is_stacked(k) ? (const void*)(pl.d_stiles + t0) :
+            dev::is_tile(k) ? (const void*)(pl.d_titems + t0) : dev::is_stacked(k) ? (const void*)(pl.d_stiles + t0) :
             (const void*)(pl.d_tiles_sorted + t0);
         hip_check(launch_grouped_list(pl, k, list, n, s), "gemm (slice)");
         if(t0 + n < nt) {
@@ -2070,6 +2231,9 @@ void btod_contract2::perform_sliced(btensor &c, bool add, double d, double slice
             between();
         }
     }
+    if(dev::is_tile(k))
+        hip_check(dev::launch_tile_sum(k, pl.d_tstacks, pl.d_tsums, (uint32_t)pl.tsums.size(),
+            (double*)pl.parts.mem, s), "gemm (sums)");
     hip_check(hipEventRecord(pl.ev[2], s), "hipEventRecord");
     if(pl.n_wb_chunks)
         hip_check(dev::launch_permute(pl.d_wback, pl.d_wb_cd, pl.d_wb_co, pl.n_wb_chunks, s),
@@ -2168,10 +2332,13 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
     std::vector<dev::gemm_pair> prs;
     std::vector<dev::tile_stack> tss;
     std::vector<std::pair<double, dev::gemm_tile> > tl;
+    std::vector<std::pair<double, dev::tile_item> > til;
+    std::vector<dev::tile_item> tsm;
     std::vector<char> host;
     size_t sz = 0;
     for(std::map<int, std::vector<size_t> >::iterator g = groups.begin(); g != groups.end(); ++g) {
-        cbs.clear(); prs.clear(); tl.clear(); tss.clear();
+        cbs.clear(); prs.clear(); tl.clear(); tss.clear(); til.clear(); tsm.clear();
+        size_t nparts = 0;
         uint32_t bm = 64, bn = 64;
         dev::tile_shape(g->first, bm, bn);
         for(size_t x = 0; x < g->second.size(); x++) {
@@ -2180,17 +2347,26 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
                 // stacks name their plan's lists by address
                 const uint32_t ts0 = (uint32_t)tss.size(), ns = (uint32_t)pl.stacks.size() - 1;
                 tss.insert(tss.end(), pl.tstacks.begin(), pl.tstacks.begin() + ns);
-                for(size_t t = 0; t < pl.stiles.size(); t++) {
-                    dev::gemm_tile y = pl.stiles[t];
-                    if(y.cblock >= ns) continue;                // padding tile
-                    const dev::stack_desc &sd = pl.stacks[y.cblock];
+                for(size_t t = 0; t < pl.titems.size(); t++) {
+                    dev::tile_item y = pl.titems[t];
+                    if(y.stack >= ns) continue;                 // padding item
+                    const dev::stack_desc &sd = pl.stacks[y.stack];
                     const double rows = std::min<double>(bm, double(sd.rows) - double(y.tm) * bm);
                     const double cols = std::min<double>(bn, double(sd.n) - double(y.tn) * bn);
-                    const double cost = 2.0 * rows * cols * pl.stack_ksum[y.cblock];
-                    y.cblock += ts0;
-                    tl.push_back(std::make_pair(cost, y));
+                    const double cost = 2.0 * rows * cols * pl.stack_ksum[y.stack] *
+                        (sd.nchunk ? double(y.count) / sd.nchunk : 0.0);
+                    y.stack += ts0;
+                    if(y.part >= 0) y.part += (int32_t)nparts;
+                    til.push_back(std::make_pair(cost, y));
                     m_flops += cost;
                 }
+                for(size_t t = 0; t < pl.tsums.size(); t++) {
+                    dev::tile_item y = pl.tsums[t];
+                    y.stack += ts0;
+                    y.part += (int32_t)nparts;
+                    tsm.push_back(y);
+                }
+                nparts += pl.n_parts;
                 continue;
             }
             uint32_t cb0 = (uint32_t)cbs.size(), pr0 = (uint32_t)prs.size();
@@ -2218,13 +2394,20 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
         std::stable_sort(tl.begin(), tl.end(),
             [](const std::pair<double, dev::gemm_tile> &x, const std::pair<double, dev::gemm_tile> &y) {
                 return x.first > y.first; });
+        std::stable_sort(til.begin(), til.end(),
+            [](const std::pair<double, dev::tile_item> &x, const std::pair<double, dev::tile_item> &y) {
+                return x.first > y.first; });
         launch L;
         L.cfg = g->first;
+        L.nsum = (uint32_t)tsm.size();
+        L.part_bytes = nparts * bm * bn * sizeof(double);
         L.ocb = sz;
         sz = align256(sz + cbs.size() * sizeof(dev::gemm_cblock) + tss.size() * sizeof(dev::tile_stack));
         L.opr = sz; sz = align256(sz + prs.size() * sizeof(dev::gemm_pair));
-        L.otl = sz; sz = align256(sz + tl.size() * sizeof(dev::gemm_tile));
-        L.nt = (uint32_t)tl.size();
+        L.otl = sz;
+        sz = align256(sz + tl.size() * sizeof(dev::gemm_tile) + til.size() * sizeof(dev::tile_item));
+        L.osum = sz; sz = align256(sz + tsm.size() * sizeof(dev::tile_item));
+        L.nt = (uint32_t)(tl.size() + til.size());
         host.resize(sz, 0);
         if(!cbs.empty()) std::memcpy(&host[L.ocb], cbs.data(), cbs.size() * sizeof(dev::gemm_cblock));
         if(!tss.empty()) std::memcpy(&host[L.ocb], tss.data(), tss.size() * sizeof(dev::tile_stack));
@@ -2234,14 +2417,26 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
                 sizeof(dev::gemm_tile));
             L.tcost.push_back(tl[t].first);
         }
+        for(size_t t = 0; t < til.size(); t++) {
+            std::memcpy(&host[L.otl + t * sizeof(dev::tile_item)], &til[t].second,
+                sizeof(dev::tile_item));
+            L.tcost.push_back(til[t].first);
+        }
+        if(!tsm.empty()) std::memcpy(&host[L.osum], tsm.data(), tsm.size() * sizeof(dev::tile_item));
         m_launches.push_back(L);
     }
+    // partial sums behind the lists
+    size_t total = sz;
+    for(size_t i = 0; i < m_launches.size(); i++) {
+        m_launches[i].opart = total;
+        total = align256(total + m_launches[i].part_bytes);
+    }
     if(sz) {
-        if(merged.bytes < sz) {
+        if(merged.bytes < total) {
             merged.release();
             merged.ctx = &ctx;
-            merged.mem = ctx.alloc(sz);
-            merged.bytes = sz;
+            merged.mem = ctx.alloc(total);
+            merged.bytes = total;
         }
         hip_check(hipMemcpyAsync(merged.mem, host.data(), sz, hipMemcpyHostToDevice, s),
             "hipMemcpy H2D");
@@ -2263,11 +2458,18 @@ bool batch_run::step(double flop_budget) {
         double f = 0.0;
         do { f += L.tcost[t1]; t1++; } while(t1 < L.nt && f + L.tcost[t1] <= flop_budget);
         const uint32_t n = t1 - (uint32_t)m_tile;
-        const dev::gemm_tile *list = (const dev::gemm_tile*)(m_base + L.otl) + m_tile;
-        hip_check(dev::is_tile(L.cfg) ?
-            dev::launch_gemm_tile(L.cfg, (const dev::tile_stack*)(m_base + L.ocb), list, n, s) :
-            dev::launch_gemm(L.cfg, (dev::gemm_cblock*)(m_base + L.ocb),
-                (dev::gemm_pair*)(m_base + L.opr), list, n, n, s), "gemm (batch)");
+        if(dev::is_tile(L.cfg)) {
+            const dev::tile_stack *st = (const dev::tile_stack*)(m_base + L.ocb);
+            double *parts = (double*)(m_base + L.opart);
+            hip_check(dev::launch_gemm_tile(L.cfg, st, (const dev::tile_item*)(m_base + L.otl) + m_tile,
+                n, parts, s), "gemm (batch)");
+            if(t1 == L.nt)
+                hip_check(dev::launch_tile_sum(L.cfg, st, (const dev::tile_item*)(m_base + L.osum),
+                    L.nsum, parts, s), "gemm (batch, sums)");
+        } else
+            hip_check(dev::launch_gemm(L.cfg, (dev::gemm_cblock*)(m_base + L.ocb),
+                (dev::gemm_pair*)(m_base + L.opr),
+                (const dev::gemm_tile*)(m_base + L.otl) + m_tile, n, n, s), "gemm (batch)");
         m_tile = t1;
         return m_launch < m_launches.size() &&
             (m_tile < L.nt || m_launch + 1 < m_launches.size());

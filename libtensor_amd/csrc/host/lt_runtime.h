@@ -365,7 +365,12 @@ public:
     size_t live() const { return m_live.size(); }
 
 private:
-    struct launch { int cfg; size_t ocb, opr, otl; uint32_t nt; std::vector<double> tcost; };
+    struct launch {
+        int cfg;
+        size_t ocb, opr, otl, osum, opart, part_bytes;
+        uint32_t nt, nsum;
+        std::vector<double> tcost;
+    };
     std::vector<batch_item> &m_items;
     std::vector<size_t> m_live;
     std::vector<contract_plan*> m_plans;
