@@ -20,8 +20,9 @@ struct fastdiv {
 };
 fastdiv make_fastdiv(uint32_t d);
 
-//! dst = alpha * P(src) (+ dst if accumulate).  dims are the destination
-//! dimensions after fusing; sstride[i] is the source stride of destination
+//! dst = alpha * P(src) + beta * add, add in the destination's layout (the
+//! destination itself to accumulate, another tensor for a sum of two terms in
+//! one pass, or null).  dims are the destination dimensions after fusing; sstride[i] is the source stride of destination
 //! dimension i; the destination is contiguous.
 struct perm_desc {
     const double *src;
@@ -31,17 +32,20 @@ struct perm_desc {
     fastdiv div[kPermMaxOrder];       //!< destination dimensions
     uint32_t sstride[kPermMaxOrder];  //!< source strides
     double alpha;
-    int32_t accumulate;
+    const double *add;
+    double beta;
     //! Transposing descriptors (the source's unit-stride dimension is
-    //! destination dimension tile_p < n - 1): 32 x 32 tiles over
+    //! destination dimension tile_p < n - 1): tiles of tile_s x tile_s over
     //! (tile_p, n - 1) staged in LDS, read and written contiguously.
     //! -1: element-wise gather.
     int32_t tile_p;
+    uint32_t tile_s;
     uint32_t tsq;                     //!< source stride of dimension n - 1
     fastdiv dps;                      //!< destination stride of tile_p
     fastdiv tdp, tdq;                 //!< extents of tile_p and n - 1
 };
-static const uint32_t kPermTile = 32;
+//! Tile side: 64 where both extents are beyond 32 (PERMFIG), else 32.
+static const uint32_t kPermTile = 32, kPermTileMax = 64;
 static const uint32_t kPermTileItem = 0x80000000u;
 
 //! One C block of a grouped GEMM: C(m x n, leading dimension ldc) is
@@ -213,6 +217,38 @@ hipError_t launch_gemm_stacked(int cfg, const stack_desc *st, const stack_pair *
 hipError_t launch_permute(const perm_desc *descs, const uint32_t *chunk_desc,
     const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s);
 static const uint32_t kPermChunk = 2048;
+//! One permutation, its descriptor passed with the launch and its work items
+//! numbered by the grid.
+hipError_t launch_permute_one(const perm_desc &d, hipStream_t s);
+
+// ---- dense contractions (lt_dense.hip) ----
+
+//! A composite index of a dense contraction: dimensions in falling order of
+//! significance; o0, o1 the element strides of each in the two tensors that
+//! have it.
+static const int kDenseMaxOrder = 8;
+struct dense_axis {
+    uint32_t n, ext;                  //!< dimensions, product of their extents
+    fastdiv div[kDenseMaxOrder];
+    uint32_t s0[kDenseMaxOrder], s1[kDenseMaxOrder];
+};
+//! C(m, n) = (zero ? 0 : C) + d sum_k A(m, k) B(k, n) with every operand at
+//! its own strides: axis m over A and C, n over B and C, k over A and B.
+struct dense_args {
+    const double *a, *b;
+    double *c;
+    double d;
+    dense_axis m, n, k;
+    int32_t zero;
+    uint32_t rows_fast;               //!< bit 0 (1): A (B) is contiguous along m (n), else along k
+};
+//! Tile configurations of the dense kernel.
+enum dense_cfg { DENSE_16x64_G4 = 0, DENSE_32x64_G4 = 1, DENSE_64x64_G1 = 2 };
+void dense_tile_shape(int cfg, uint32_t &bm, uint32_t &bn);
+//! nparts > 1: the k range in that many parts, whose partial sums go through
+//! `parts` (tiles x nparts x bm x bn doubles).
+hipError_t launch_gemm_dense(int cfg, const dense_args &a, uint32_t nparts, double *parts,
+    hipStream_t s);
 
 //! Grouped FP64 MFMA GEMM over a tile list (operand layouts per pair).
 //! nwg workgroups loop over the tiles (nwg == ntiles gives one workgroup
@@ -285,6 +321,9 @@ hipError_t launch_fill(double *p, size_t n, double v, hipStream_t s);
 //! Dot product of permuted operands: sum_i a[i] * b(P(i)) over descriptors
 //! whose `src` is b and `dst` is (const) a; partials[wg] receive one value
 //! per workgroup, then a final pass sums them in a fixed order into *out.
+//! Workgroups of a dot product (each with its range of the chunks), so at most
+//! this many partial sums.
+static const uint32_t kDotGroups = 2048;
 hipError_t launch_dot(const perm_desc *descs, const uint32_t *chunk_desc,
     const uint32_t *chunk_off, uint32_t nchunks, double *partials,
     double *out, hipStream_t s);
@@ -292,6 +331,8 @@ hipError_t launch_dot(const perm_desc *descs, const uint32_t *chunk_desc,
 //! Size of the fixed device scratch region of the no-allocation entry
 //! points (one per GPU, held until the process ends).
 static const size_t kNoallocScratchBytes = size_t(32) << 20;
+//! Behind it, room for the partial sums of a contraction cut along k.
+static const size_t kNoallocPartBytes = size_t(2) << 20;
 static const int kMaxDevices = 64;
 //! Device address of that region on `device`, which must be the current
 //! device on the first call for it (resolved once, then cached).

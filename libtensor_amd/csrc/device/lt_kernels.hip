@@ -74,64 +74,75 @@ __device__ __forceinline__ uint32_t src_offset(const perm_desc &d, uint32_t e) {
     return off;
 }
 
-__global__ void __launch_bounds__(256)
-permute_kernel(const perm_desc *__restrict__ descs,
-    const uint32_t *__restrict__ chunk_desc,
-    const uint32_t *__restrict__ chunk_off) {
+//! alpha v + beta w with one rounding of beta w and one of the sum.
+__device__ __forceinline__ double perm_sum(double alpha, double v, double beta, double w) {
+#pragma clang fp contract(off)
+    const double t = beta * w;
+    return __builtin_fma(alpha, v, t);
+}
 
-    __shared__ double tile[kPermTile][kPermTile + 1];
-    const uint32_t ch = blockIdx.x;
-    const uint32_t cd = chunk_desc[ch];
-    const perm_desc d = descs[cd & ~kPermTileItem];
-    const uint32_t base = chunk_off[ch];
-
-    if(cd & kPermTileItem) {
-        // 32 x 32 tile over destination dimensions (p, q = n - 1); the
-        // source is contiguous along p, the destination along q
-        // (extents and strides from dedicated fields: indexing the
-        // descriptor's arrays with a runtime dimension would put it in
-        // scratch memory)
-        const uint32_t dq = d.tdq.d, dp = d.tdp.d;
-        const uint32_t q0 = base - fdiv(base, d.tdq) * dq;
-        const uint32_t e1 = fdiv(base, d.dps);
-        const uint32_t p0 = e1 - fdiv(e1, d.tdp) * dp;
-        const uint32_t np = min(kPermTile, dp - p0), nq = min(kPermTile, dq - q0);
-        const uint32_t s0 = src_offset(d, base), sq = d.tsq, dps = d.dps.d;
-        const uint32_t ti = threadIdx.x & 31, tj = threadIdx.x >> 5;
+//! One tile of S x S over destination dimensions (p, q = n - 1): the source is
+//! contiguous along p, the destination along q (extents and strides from
+//! dedicated fields: indexing the descriptor's arrays with a runtime dimension
+//! would put it in scratch memory).
+template<int S>
+__device__ __forceinline__ void permute_tile(const perm_desc &d, uint32_t base, double *tile) {
+    constexpr int RW = 256 / S;          // rows at a time
+    const uint32_t dq = d.tdq.d, dp = d.tdp.d;
+    const uint32_t q0 = base - fdiv(base, d.tdq) * dq;
+    const uint32_t e1 = fdiv(base, d.dps);
+    const uint32_t p0 = e1 - fdiv(e1, d.tdp) * dp;
+    const uint32_t np = min(uint32_t(S), dp - p0), nq = min(uint32_t(S), dq - q0);
+    const uint32_t s0 = src_offset(d, base), sq = d.tsq, dps = d.dps.d;
+    const uint32_t ti = threadIdx.x % S, tj = threadIdx.x / S;
+    double w[S / RW];
 #pragma unroll
-        for(uint32_t r = 0; r < kPermTile; r += 8) {
-            const uint32_t iq = tj + r;
-            if(ti < np && iq < nq) tile[iq][ti] = d.src[s0 + ti + iq * sq];
-        }
-        __syncthreads();
-#pragma unroll
-        for(uint32_t r = 0; r < kPermTile; r += 8) {
-            const uint32_t ip = tj + r;
-            if(ti < nq && ip < np) {
-                double *o = d.dst + base + ip * dps + ti;
-                const double v = d.alpha * tile[ti][ip];
-                *o = d.accumulate ? v + *o : v;
-            }
-        }
-        return;
+    for(int r = 0; r < S / RW; r++) {
+        const uint32_t iq = tj + RW * r;
+        if(ti < np && iq < nq) w[r] = d.src[s0 + ti + iq * sq];
     }
+#pragma unroll
+    for(int r = 0; r < S / RW; r++) {
+        const uint32_t iq = tj + RW * r;
+        if(ti < np && iq < nq) tile[iq * (S + 1) + ti] = w[r];
+    }
+    if(d.add) {
+#pragma unroll
+        for(int r = 0; r < S / RW; r++) {
+            const uint32_t ip = tj + RW * r;
+            if(ti < nq && ip < np) w[r] = d.add[base + ip * dps + ti];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for(int r = 0; r < S / RW; r++) {
+        const uint32_t ip = tj + RW * r;
+        if(ti < nq && ip < np) {
+            const double v = tile[ti * (S + 1) + ip];
+            d.dst[base + ip * dps + ti] = d.add ? perm_sum(d.alpha, v, d.beta, w[r]) : d.alpha * v;
+        }
+    }
+}
 
-    // element-wise gather: each thread owns kPermChunk / 256 elements of the
-    // chunk; all source offsets are computed and all loads issued before the
-    // first store, so every thread has that many gathers in flight
+//! Element-wise gather of one chunk: each thread owns kPermChunk / 256
+//! elements; all source offsets are computed and all loads issued before the
+//! first store, so every thread has that many gathers in flight.
+__device__ __forceinline__ void permute_gather(const perm_desc &d, uint32_t base) {
     constexpr int E = kPermChunk / 256;
     const uint32_t end = min(base + kPermChunk, d.total);
-    double v[E];
+    double v[E], w[E];
 #pragma unroll
     for(int i = 0; i < E; i++) {
         const uint32_t e = min(base + threadIdx.x + 256u * i, end - 1);
         v[i] = d.src[src_offset(d, e)];
     }
-    if(d.accumulate) {
+    if(d.add) {
+#pragma unroll
+        for(int i = 0; i < E; i++) w[i] = d.add[min(base + threadIdx.x + 256u * i, end - 1)];
 #pragma unroll
         for(int i = 0; i < E; i++) {
             const uint32_t e = base + threadIdx.x + 256u * i;
-            if(e < end) d.dst[e] = d.alpha * v[i] + d.dst[e];
+            if(e < end) d.dst[e] = perm_sum(d.alpha, v[i], d.beta, w[i]);
         }
     } else {
 #pragma unroll
@@ -142,6 +153,21 @@ permute_kernel(const perm_desc *__restrict__ descs,
     }
 }
 
+__global__ void __launch_bounds__(256)
+permute_kernel(const perm_desc *__restrict__ descs,
+    const uint32_t *__restrict__ chunk_desc,
+    const uint32_t *__restrict__ chunk_off) {
+
+    __shared__ double tile[kPermTileMax * (kPermTileMax + 1)];
+    const uint32_t ch = blockIdx.x;
+    const uint32_t cd = chunk_desc[ch];
+    const perm_desc d = descs[cd & ~kPermTileItem];
+    const uint32_t base = chunk_off[ch];
+    if(!(cd & kPermTileItem)) permute_gather(d, base);
+    else if(d.tile_s == kPermTileMax) permute_tile<kPermTileMax>(d, base, tile);
+    else permute_tile<kPermTile>(d, base, tile);
+}
+
 hipError_t launch_permute(const perm_desc *descs, const uint32_t *chunk_desc,
     const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s) {
     if(nchunks == 0) return hipSuccess;
@@ -150,29 +176,141 @@ hipError_t launch_permute(const perm_desc *descs, const uint32_t *chunk_desc,
     return hipGetLastError();
 }
 
+//! Work items of one descriptor by number: per destination dimension the
+//! items along it and the destination elements from one to the next.
+struct perm_items {
+    fastdiv it[kPermMaxOrder];
+    uint32_t step[kPermMaxOrder];
+};
+
+template<int S>
+__global__ void __launch_bounds__(256) permute_tiles_kernel(perm_desc d, perm_items g) {
+    __shared__ double tile[S * (S + 1)];
+    uint32_t x = blockIdx.x, base = 0;
+#pragma unroll
+    for(int i = kPermMaxOrder - 1; i >= 0; i--) {
+        if(i < (int)d.n) {
+            const uint32_t q = fdiv(x, g.it[i]);
+            base += (x - q * g.it[i].d) * g.step[i];
+            x = q;
+        }
+    }
+    permute_tile<S>(d, base, tile);
+}
+
+__global__ void __launch_bounds__(256) permute_gather_kernel(perm_desc d) {
+    permute_gather(d, blockIdx.x * kPermChunk);
+}
+
+hipError_t launch_permute_one(const perm_desc &d, hipStream_t s) {
+    if(d.total == 0) return hipSuccess;
+    if(d.tile_p < 0) {
+        hipLaunchKernelGGL(permute_gather_kernel, dim3((d.total + kPermChunk - 1) / kPermChunk),
+            dim3(256), 0, s, d);
+        return hipGetLastError();
+    }
+    perm_items g;
+    uint64_t stride = 1, items = 1;
+    for(int i = int(d.n) - 1; i >= 0; i--) {
+        const bool tiled = i == d.tile_p || i == int(d.n) - 1;
+        const uint32_t ext = d.div[i].d, st = tiled ? d.tile_s : 1, cnt = (ext + st - 1) / st;
+        g.it[i] = make_fastdiv(cnt);
+        g.step[i] = uint32_t(stride * st);
+        stride *= ext;
+        items *= cnt;
+    }
+    for(int i = int(d.n); i < kPermMaxOrder; i++) { g.it[i] = make_fastdiv(1); g.step[i] = 0; }
+    if(d.tile_s == kPermTileMax)
+        hipLaunchKernelGGL(permute_tiles_kernel<kPermTileMax>, dim3((uint32_t)items), dim3(256), 0, s, d, g);
+    else
+        hipLaunchKernelGGL(permute_tiles_kernel<kPermTile>, dim3((uint32_t)items), dim3(256), 0, s, d, g);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // Dot product
+//
+// Bound by memory bandwidth.  A fixed number of workgroups, each over a range
+// of the chunks with all loads of a chunk issued before the first product, so
+// the sum of the partial results stays a few microseconds whatever the size
+// (one workgroup and one partial sum per chunk: 17 us of summing for 26 M
+// elements).  Transposed operands go through LDS tiles as in the permute.
+
+template<int S>
+__device__ __forceinline__ double dot_tile(const perm_desc &d, uint32_t base, double *tile) {
+    constexpr int RW = 256 / S;
+    const uint32_t dq = d.tdq.d, dp = d.tdp.d;
+    const uint32_t q0 = base - fdiv(base, d.tdq) * dq;
+    const uint32_t e1 = fdiv(base, d.dps);
+    const uint32_t p0 = e1 - fdiv(e1, d.tdp) * dp;
+    const uint32_t np = min(uint32_t(S), dp - p0), nq = min(uint32_t(S), dq - q0);
+    const uint32_t s0 = src_offset(d, base), sq = d.tsq, dps = d.dps.d;
+    const uint32_t ti = threadIdx.x % S, tj = threadIdx.x / S;
+    double v[S / RW], w[S / RW];
+#pragma unroll
+    for(int r = 0; r < S / RW; r++) {
+        const uint32_t i = tj + RW * r;
+        if(ti < np && i < nq) v[r] = d.src[s0 + ti + i * sq];
+        w[r] = ti < nq && i < np ? d.dst[base + i * dps + ti] : 0.0;
+    }
+    __syncthreads();                       // the tile of the item before is read
+#pragma unroll
+    for(int r = 0; r < S / RW; r++) {
+        const uint32_t i = tj + RW * r;
+        if(ti < np && i < nq) tile[i * (S + 1) + ti] = v[r];
+    }
+    __syncthreads();
+    double acc = 0.0;
+#pragma unroll
+    for(int r = 0; r < S / RW; r++) {
+        const uint32_t i = tj + RW * r;
+        if(ti < nq && i < np) acc += w[r] * tile[ti * (S + 1) + i];
+    }
+    return acc;
+}
 
 __global__ void __launch_bounds__(256)
 dot_kernel(const perm_desc *__restrict__ descs,
     const uint32_t *__restrict__ chunk_desc,
-    const uint32_t *__restrict__ chunk_off, double *__restrict__ partials) {
+    const uint32_t *__restrict__ chunk_off, uint32_t nchunks, double *__restrict__ partials) {
 
-    __shared__ double red[256];
-    const uint32_t ch = blockIdx.x;
-    const perm_desc d = descs[chunk_desc[ch]];
-    const uint32_t base = chunk_off[ch];
-    const uint32_t end = min(base + kPermChunk, d.total);
-    double acc = 0.0;
-    for(uint32_t e = base + threadIdx.x; e < end; e += blockDim.x)
-        acc += d.dst[e] * d.src[src_offset(d, e)];
-    red[threadIdx.x] = acc * d.alpha;
+    constexpr int E = kPermChunk / 256;
+    __shared__ double tile[kPermTileMax * (kPermTileMax + 1)];
+    const uint32_t c0 = uint32_t(uint64_t(nchunks) * blockIdx.x / gridDim.x);
+    const uint32_t c1 = uint32_t(uint64_t(nchunks) * (blockIdx.x + 1) / gridDim.x);
+    double sum = 0.0;
+    for(uint32_t ch = c0; ch < c1; ch++) {
+        const uint32_t cd = chunk_desc[ch];
+        const perm_desc &d = descs[cd & ~kPermTileItem];
+        const uint32_t base = chunk_off[ch];
+        double acc = 0.0;
+        if(cd & kPermTileItem) {
+            acc = d.tile_s == kPermTileMax ? dot_tile<kPermTileMax>(d, base, tile) :
+                dot_tile<kPermTile>(d, base, tile);
+        } else {
+            const uint32_t end = min(base + kPermChunk, d.total);
+            double v[E], w[E];
+#pragma unroll
+            for(int i = 0; i < E; i++) {
+                const uint32_t e = min(base + threadIdx.x + 256u * i, end - 1);
+                v[i] = d.src[src_offset(d, e)];
+                w[i] = d.dst[e];
+            }
+#pragma unroll
+            for(int i = 0; i < E; i++)
+                if(base + threadIdx.x + 256u * i < end) acc += w[i] * v[i];
+        }
+        sum += acc * d.alpha;
+    }
+    __syncthreads();
+    double *red = tile;
+    red[threadIdx.x] = sum;
     __syncthreads();
     for(uint32_t w = 128; w > 0; w >>= 1) {
         if(threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
         __syncthreads();
     }
-    if(threadIdx.x == 0) partials[ch] = red[0];
+    if(threadIdx.x == 0) partials[blockIdx.x] = red[0];
 }
 
 __global__ void __launch_bounds__(256)
@@ -192,11 +330,12 @@ sum_kernel(const double *__restrict__ partials, uint32_t n, double *__restrict__
 hipError_t launch_dot(const perm_desc *descs, const uint32_t *chunk_desc,
     const uint32_t *chunk_off, uint32_t nchunks, double *partials,
     double *out, hipStream_t s) {
-    if(nchunks > 0) {
-        hipLaunchKernelGGL(dot_kernel, dim3(nchunks), dim3(256), 0, s,
-            descs, chunk_desc, chunk_off, partials);
+    const uint32_t ng = nchunks < kDotGroups ? nchunks : kDotGroups;
+    if(ng > 0) {
+        hipLaunchKernelGGL(dot_kernel, dim3(ng), dim3(256), 0, s,
+            descs, chunk_desc, chunk_off, nchunks, partials);
     }
-    hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, s, partials, nchunks, out);
+    hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, s, partials, ng, out);
     return hipGetLastError();
 }
 

@@ -16,7 +16,7 @@
 
 namespace {
 
-static __device__ __align__(256) char scratch[lta::dev::kNoallocScratchBytes];
+static __device__ __align__(256) char scratch[lta::dev::kNoallocScratchBytes + lta::dev::kNoallocPartBytes];
 
 std::mutex g_mtx;
 void *g_ptr[lta::dev::kMaxDevices];

@@ -93,298 +93,7 @@ contraction2 make_contraction(size_t N, size_t M, size_t K, const size_t *permc,
     return c;
 }
 
-//! Device memory for the temporaries of one dense operation: taken from the
-//! context's allocator and released when the arena goes out of scope, or
-//! carved out of a fixed device region (the no-allocation entry point; no
-//! allocation at all, LT_ERR_PARAM when the region is too small).  Callers
-//! take every buffer before their first device operation, so a refusal
-//! leaves the device untouched.
-class scratch_arena {
-public:
-    explicit scratch_arena(context &ctx, char *region = 0, size_t cap = 0) :
-        m_ctx(ctx), m_region(region), m_cap(cap), m_off(0), m_measure(false) { }
-    //! A measuring arena: take() hands out placeholder addresses and only
-    //! adds up the bytes (used() after the takes of a layout).
-    struct measuring { };
-    scratch_arena(context &ctx, measuring) :
-        m_ctx(ctx), m_region(0), m_cap(0), m_off(0), m_measure(true) { }
-    ~scratch_arena() {
-        if(!m_region && !m_measure) for(size_t i = 0; i < m_taken.size(); i++) m_ctx.free(m_taken[i]);
-    }
-    scratch_arena(const scratch_arena&) = delete;
-    scratch_arena &operator=(const scratch_arena&) = delete;
-    size_t used() const { return m_off; }
-    //! A 256-byte aligned buffer of `bytes` bytes.
-    char *take(size_t bytes) {
-        bytes = (std::max<size_t>(bytes, 8) + 255) & ~size_t(255);
-        if(m_measure) {
-            char *p = (char*)(uintptr_t(256) + m_off);
-            m_off += bytes;
-            return p;
-        }
-        if(!m_region) {
-            char *p = (char*)m_ctx.alloc(bytes);
-            m_taken.push_back(p);
-            return p;
-        }
-        if(bytes > m_cap - m_off) {
-            throw lt_error(LT_ERR_PARAM, "temporaries exceed the fixed scratch region of " +
-                std::to_string(m_cap) + " bytes");
-        }
-        char *p = m_region + m_off;
-        m_off += bytes;
-        return p;
-    }
-private:
-    context &m_ctx;
-    char *m_region;
-    size_t m_cap, m_off;
-    bool m_measure;
-    std::vector<void*> m_taken;
-};
-
-//! One permute launch: descriptor and work-item lists laid out for one
-//! upload (descriptor at 0, chunk descriptors at ocd, offsets at oco).
-struct permute_job {
-    std::vector<char> host;
-    size_t ocd, oco, nchunks;
-    char *mem;
-    permute_job() : ocd(0), oco(0), nchunks(0), mem(0) { }
-    void prepare(const double *src, const dims_t &dsrc, const tensor_tr &tr, double *dst,
-        bool accumulate, scratch_arena &ar) {
-        dev::perm_desc d = make_perm_desc_public(src, dsrc, tr, dst, accumulate);
-        std::vector<uint32_t> cd, co;
-        make_chunks(std::vector<dev::perm_desc>(1, d), cd, co);
-        nchunks = cd.size();
-        if(!nchunks) return;
-        ocd = (sizeof(d) + 255) & ~size_t(255);
-        oco = ocd + ((4 * cd.size() + 255) & ~size_t(255));
-        host.assign(oco + 4 * co.size(), 0);
-        std::memcpy(&host[0], &d, sizeof(d));
-        std::memcpy(&host[ocd], cd.data(), 4 * cd.size());
-        std::memcpy(&host[oco], co.data(), 4 * co.size());
-        mem = ar.take(host.size());
-    }
-    void upload(context &ctx) { if(nchunks) ctx.upload(mem, host.data(), host.size()); }
-    void launch(context &ctx) const {
-        if(!nchunks) return;
-        hip_check(dev::launch_permute((dev::perm_desc*)mem, (uint32_t*)(mem + ocd),
-            (uint32_t*)(mem + oco), (uint32_t)nchunks, ctx.stream()), "permute");
-    }
-};
-
-void dense_permute_in(context &ctx, const double *src, const dims_t &dsrc,
-    const tensor_tr &tr, double *dst, bool accumulate, scratch_arena &ar) {
-    permute_job j;
-    j.prepare(src, dsrc, tr, dst, accumulate, ar);
-    if(!j.nchunks) return;
-    j.upload(ctx);
-    ctx.activate();
-    j.launch(ctx);
-    ctx.sync();
-}
-
-//! One tod_contract2 laid out on the host: its operand copies and aligned
-//! result taken from `tmp`, its descriptor and tile lists from `dsc` (host
-//! images kept for the upload), all before any device operation.
-struct contract_job {
-    bool skip;                  //!< d == 0, C kept
-    bool fill;                  //!< d == 0, C := 0
-    double *c;
-    size_t cn;
-    permute_job ja, jb, jc;
-    char *mem;                  //!< GEMM block, pair and tile lists
-    std::vector<char> host;
-    uint32_t ntiles;
-    contract_job() : skip(false), fill(false), c(0), cn(0), mem(0), ntiles(0) { }
-    //! The uploads of the descriptor lists (each ordered after the stream).
-    void upload(context &cx) {
-        ja.upload(cx);
-        jb.upload(cx);
-        jc.upload(cx);
-        if(ntiles) cx.upload(mem, host.data(), host.size());
-    }
-    //! Every blob of the descriptor lists into a host image of the region
-    //! at `base` (one upload for many jobs).
-    void stage(char *image, const char *base) const {
-        const permute_job *js[3] = { &ja, &jb, &jc };
-        for(int i = 0; i < 3; i++)
-            if(js[i]->nchunks)
-                std::memcpy(image + (js[i]->mem - base), js[i]->host.data(), js[i]->host.size());
-        if(ntiles) std::memcpy(image + (mem - base), host.data(), host.size());
-    }
-    //! The launches, in stream order (no synchronization).
-    void launch(context &cx) const {
-        if(skip) return;
-        if(fill) {
-            hip_check(dev::launch_fill(c, cn, 0.0, cx.stream()), "fill");
-            return;
-        }
-        ja.launch(cx);
-        jb.launch(cx);
-        hip_check(dev::launch_gemm(dev::TILE_64x64, (dev::gemm_cblock*)mem,
-            (dev::gemm_pair*)(mem + 512), (dev::gemm_tile*)(mem + 1024),
-            ntiles, ntiles, cx.stream()), "gemm");
-        jc.launch(cx);
-    }
-};
-
-void contract_prepare(const contraction2 &contr, const dims_t &da, const double *a,
-    const dims_t &db, const double *b, double d, bool zero, double *c,
-    scratch_arena &tmp, scratch_arena &dsc, contract_job &j) {
-    dims_t dc = contract2_dims(contr, da, db);
-    // the GEMM kernels address operands with 32-bit byte offsets
-    const size_t lim = size_t(1) << 29;
-    lt_require(da.size() < lim && db.size() < lim && dc.size() < lim, LT_ERR_PARAM,
-        "tod_contract2: a tensor of 2^29 or more elements (32-bit byte offsets in the "
-        "GEMM kernels)");
-    j.c = c;
-    j.cn = dc.size();
-    if(d == 0.0) {
-        j.fill = zero;
-        j.skip = !zero;
-        return;
-    }
-    // align as tod_contract2::perform (tod_contract2_impl.h:124-135),
-    // permute A / B into scratch if needed, one GEMM, permute C back
-    contraction2_align al(contr);
-    contraction2 ca(contr);
-    ca.permute_a(al.perma);
-    ca.permute_b(al.permb);
-    ca.permute_c(al.permc);
-    dims_t da2(da), db2(db), dc2(dc);
-    da2.permute(al.perma);
-    db2.permute(al.permb);
-    dc2.permute(al.permc);
-
-    const double *pa = a, *pb = b;
-    if(!al.perma.is_identity()) {
-        double *t = (double*)tmp.take(da.size() * 8);
-        j.ja.prepare(a, da, tensor_tr(al.perma, scalar_tr()), t, false, dsc);
-        pa = t;
-    }
-    if(!al.permb.is_identity()) {
-        double *t = (double*)tmp.take(db.size() * 8);
-        j.jb.prepare(b, db, tensor_tr(al.permb, scalar_tr()), t, false, dsc);
-        pb = t;
-    }
-    double *pc = c;
-    bool cperm = !al.permc.is_identity();
-    if(cperm) {
-        pc = (double*)tmp.take(dc.size() * 8);
-        j.jc.prepare(pc, dc2, tensor_tr(al.permc.inverse(), scalar_tr()), c, !zero, dsc);
-    }
-    gemm_form g = aligned_gemm_form(ca, da2, db2);
-    dev::gemm_cblock cb;
-    dev::gemm_pair gp;
-    std::memset(&cb, 0, sizeof(cb));
-    std::memset(&gp, 0, sizeof(gp));
-    size_t lda = g.ta ? g.m : g.k, ldb = g.tb ? g.k : g.n;
-    bool ta = g.ta, tb = g.tb;
-    if(!g.tc) {
-        cb.m = (uint32_t)g.m; cb.n = (uint32_t)g.n;
-        gp.a = pa; gp.b = pb; gp.lda = (uint32_t)lda; gp.ldb = (uint32_t)ldb;
-    } else {
-        cb.m = (uint32_t)g.n; cb.n = (uint32_t)g.m;
-        gp.a = pb; gp.b = pa; gp.lda = (uint32_t)ldb; gp.ldb = (uint32_t)lda;
-        ta = !g.tb; tb = !g.ta;
-    }
-    cb.ldc = cb.n;
-    cb.c = pc;
-    cb.zero = (cperm || zero) ? 1 : 0;
-    cb.pair_begin = 0;
-    cb.pair_end = 1;
-    gp.k = (uint32_t)g.k;
-    gp.d = d;
-    gp.flags = (ta ? dev::kPairAKMajor : 0) | (tb ? dev::kPairBNMajor : 0);
-    uint32_t bm = 64, bn = 64;
-    dev::tile_shape(dev::TILE_64x64, bm, bn);
-    std::vector<dev::gemm_tile> tiles;
-    for(uint32_t i = 0; i < (cb.m + bm - 1) / bm; i++)
-        for(uint32_t jj = 0; jj < (cb.n + bn - 1) / bn; jj++) {
-            dev::gemm_tile t; t.cblock = 0; t.tm = (uint16_t)i; t.tn = (uint16_t)jj;
-            tiles.push_back(t);
-        }
-    size_t bytes = 512 + 512 + tiles.size() * sizeof(dev::gemm_tile);
-    j.mem = dsc.take(bytes);
-    j.host.assign(bytes, 0);
-    std::memcpy(&j.host[0], &cb, sizeof(cb));
-    std::memcpy(&j.host[512], &gp, sizeof(gp));
-    std::memcpy(&j.host[1024], tiles.data(), tiles.size() * sizeof(dev::gemm_tile));
-    j.ntiles = (uint32_t)tiles.size();
-}
-
-//! tod_contract2 with every temporary (aligned operand copies, the aligned
-//! result, descriptors and tile list) taken from `ar` before the first
-//! device operation.
-void dense_contract2_in(context &cx, const contraction2 &contr, const dims_t &da,
-    const double *a, const dims_t &db, const double *b, double d, bool zero, double *c,
-    scratch_arena &ar) {
-    contract_job j;
-    contract_prepare(contr, da, a, db, b, d, zero, c, ar, ar, j);
-    if(j.skip) return;
-    // device side, in stream order
-    j.upload(cx);
-    cx.activate();
-    j.launch(cx);
-    cx.sync();
-}
-
 } // unnamed namespace
-
-namespace lta {
-
-void dense_permute(context &ctx, const double *src, const dims_t &dsrc,
-    const tensor_tr &tr, double *dst, bool accumulate) {
-    scratch_arena ar(ctx);
-    dense_permute_in(ctx, src, dsrc, tr, dst, accumulate, ar);
-}
-
-void dense_contract2(context &cx, const contraction2 &contr, const dims_t &da, const double *a,
-    const dims_t &db, const double *b, double d, bool zero, double *c) {
-    scratch_arena ar(cx);
-    dense_contract2_in(cx, contr, da, a, db, b, d, zero, c, ar);
-}
-
-void dense_contract2_many(context &cx, const std::vector<dense_contract_item> &items,
-    double *c) {
-    if(items.empty()) return;
-    // every temporary and descriptor of all items in one allocation: the
-    // layout is measured first (same takes, placeholder addresses), then
-    // made in the allocation; the descriptors go up in one upload, the
-    // launches follow in item order, one synchronization at the end
-    size_t tbytes = 0, dbytes = 0;
-    {
-        scratch_arena mt(cx, scratch_arena::measuring()), md(cx, scratch_arena::measuring());
-        for(size_t i = 0; i < items.size(); i++) {
-            contract_job j;
-            contract_prepare(items[i].contr, items[i].da, items[i].a, items[i].db, items[i].b,
-                items[i].d, items[i].zero, c, mt, md, j);
-        }
-        tbytes = mt.used();
-        dbytes = md.used();
-    }
-    char *region = (char*)cx.alloc(std::max<size_t>(tbytes + dbytes, 256));
-    try {
-        scratch_arena at(cx, region, tbytes), ad(cx, region + tbytes, dbytes);
-        std::vector<contract_job> jobs(items.size());
-        for(size_t i = 0; i < items.size(); i++)
-            contract_prepare(items[i].contr, items[i].da, items[i].a, items[i].db, items[i].b,
-                items[i].d, items[i].zero, c, at, ad, jobs[i]);
-        std::vector<char> image(dbytes, 0);
-        for(size_t i = 0; i < jobs.size(); i++) jobs[i].stage(image.data(), region + tbytes);
-        if(dbytes) cx.upload(region + tbytes, image.data(), dbytes);
-        cx.activate();
-        for(size_t i = 0; i < jobs.size(); i++) jobs[i].launch(cx);
-        cx.sync();
-    } catch(...) {
-        cx.sync();
-        cx.free(region);
-        throw;
-    }
-    cx.free(region);
-}
-}
 
 extern "C" {
 
@@ -515,10 +224,10 @@ int lt_tod_add(lt_ctx *ctx, size_t n, const size_t *dims, size_t nops,
             if(i == 0) d0 = di;
             lt_require(di == d0, LT_ERR_DIMS, "tod_add: operands of different dimensions");
         }
-        for(size_t i = 0; i < nops; i++) {
-            tensor_tr tr(perm_or_identity(n, perms ? perms + i * n : 0), scalar_tr(c[i]));
-            dense_permute(*ctx->c, a[i], da, tr, b, !(zero && i == 0));
-        }
+        std::vector<tensor_tr> trs;
+        for(size_t i = 0; i < nops; i++)
+            trs.push_back(tensor_tr(perm_or_identity(n, perms ? perms + i * n : 0), scalar_tr(c[i])));
+        dense_add(*ctx->c, a, da, trs, b, zero != 0);
     });
 }
 
@@ -559,12 +268,8 @@ int lt_tod_contract2_noalloc(lt_ctx *ctx, size_t N, size_t M, size_t K,
         context &cx = *ctx->c;
         cx.require_device("tod_contract2_noalloc");
         contraction2 contr = make_contraction(N, M, K, permc, ka, kb);
-        cx.activate();
-        void *region = 0;
-        hip_check(dev::noalloc_scratch(cx.device(), &region), "scratch region address");
-        scratch_arena ar(cx, (char*)region, dev::kNoallocScratchBytes);
-        dense_contract2_in(cx, contr, dims_t::from(N + K, dims_a), a,
-            dims_t::from(M + K, dims_b), b, d, zero != 0, c, ar);
+        dense_contract2_noalloc(cx, contr, dims_t::from(N + K, dims_a), a,
+            dims_t::from(M + K, dims_b), b, d, zero != 0, c);
     });
 }
 
@@ -587,35 +292,8 @@ int lt_tod_dotprod(lt_ctx *ctx, size_t n, const size_t *dims_a,
         q.permute(pa.inverse());
         dev::perm_desc d = make_perm_desc_public(b, db, tensor_tr(q, scalar_tr(c)),
             const_cast<double*>(a), false);
-        std::vector<uint32_t> cd, co;
-        for(uint32_t off = 0; off < d.total; off += dev::kPermChunk) {
-            cd.push_back(0);
-            co.push_back(off);
-        }
-        size_t nch = cd.size();
-        size_t o_cd = 256, o_co = o_cd + ((4 * nch + 255) & ~size_t(255));
-        size_t o_part = o_co + ((4 * nch + 255) & ~size_t(255));
-        size_t o_out = o_part + ((8 * nch + 255) & ~size_t(255));
-        size_t bytes = o_out + 256;
-        char *mem = (char*)cx.alloc(bytes);
-        try {
-            std::vector<char> host(bytes, 0);
-            std::memcpy(&host[0], &d, sizeof(d));
-            if(nch) {
-                std::memcpy(&host[o_cd], cd.data(), 4 * nch);
-                std::memcpy(&host[o_co], co.data(), 4 * nch);
-            }
-            cx.upload(mem, host.data(), bytes);
-            cx.activate();
-            hip_check(dev::launch_dot((dev::perm_desc*)mem, (uint32_t*)(mem + o_cd),
-                (uint32_t*)(mem + o_co), (uint32_t)nch, (double*)(mem + o_part),
-                (double*)(mem + o_out), cx.stream()), "dot");
-            cx.download(result, mem + o_out, 8);
-        } catch(...) {
-            cx.free(mem);
-            throw;
-        }
-        cx.free(mem);
+        *result = run_dot(cx, *upload_launches(cx,
+            std::vector<std::vector<dev::perm_desc> >(1, std::vector<dev::perm_desc>(1, d))));
     });
 }
 

@@ -78,10 +78,12 @@ dev::perm_desc make_perm_desc(const double *src, const dims_t &dsrc,
         d.sstride[i] = i < nf ? (uint32_t)fs[i] : 0;
     }
     d.alpha = tr.st.c;
-    d.accumulate = accumulate ? 1 : 0;
+    d.add = accumulate ? dst : 0;
+    d.beta = 1.0;
     // transposing: the source's unit-stride dimension is not the
     // destination's fastest one
     d.tile_p = -1;
+    d.tile_s = dev::kPermTile;
     d.tsq = 0;
     d.dps = d.tdp = d.tdq = dev::make_fastdiv(1);
     if(nf >= 2 && fs[nf - 1] != 1) {
@@ -94,6 +96,7 @@ dev::perm_desc make_perm_desc(const double *src, const dims_t &dsrc,
             d.dps = dev::make_fastdiv((uint32_t)st);
             d.tdp = dev::make_fastdiv((uint32_t)fd[i]);
             d.tdq = dev::make_fastdiv((uint32_t)fd[nf - 1]);
+            if(std::min(fd[i], fd[nf - 1]) > dev::kPermTile) d.tile_s = dev::kPermTileMax;
             break;
         }
     }
@@ -156,7 +159,7 @@ void btod_contract2::check_block_sizes() const {
 }
 
 //! Work items of a list of permute descriptors: chunks of kPermChunk
-//! destination elements, or the corners of 32 x 32 tiles for transposing
+//! destination elements, or the corners of tiles for transposing
 //! descriptors.
 void make_chunks(const std::vector<dev::perm_desc> &ds, std::vector<uint32_t> &cd,
     std::vector<uint32_t> &co) {
@@ -181,7 +184,7 @@ void make_chunks(const std::vector<dev::perm_desc> &ds, std::vector<uint32_t> &c
             dims[j] = d.div[j].d;
             str[j] = acc;
             acc *= dims[j];
-            step[j] = (uint32_t(j) == p || uint32_t(j) == q) ? dev::kPermTile : 1;
+            step[j] = (uint32_t(j) == p || uint32_t(j) == q) ? d.tile_s : 1;
             idx[j] = 0;
         }
         while(true) {
@@ -1693,7 +1696,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     double bytes = 0.0;
     for(size_t i = 0; i < pl.prep.size(); i++) bytes += 16.0 * pl.prep[i].total;
     for(size_t i = 0; i < pl.wback.size(); i++)
-        bytes += (pl.wback[i].accumulate ? 24.0 : 16.0) * pl.wback[i].total;
+        bytes += (pl.wback[i].add ? 24.0 : 16.0) * pl.wback[i].total;
     m_stats.bytes_perm = bytes;
     m_stats.t_plan_ms = now_ms() - t0;
 }

@@ -25,7 +25,15 @@ double btod_dotprod(btensor &a, const tensor_tr &tra0, btensor &b, const tensor_
     const dims_t bid2 = bisa2.block_index_dims(), bida = a.bidims(), bidb = b.bidims();
     const perm_t pai = tra0.perm.inverse(), pbi = trb0.perm.inverse();
 
-    std::vector<dev::perm_desc> descs;
+    const double scale = tra0.st.c * trb0.st.c;
+
+    // descriptors and work items, kept per structure versions of A and B
+    const std::string key = "dot" + key_tensor(a, true) + key_tensor(b, true) + "|" +
+        key_part(tra0) + "|" + key_part(trb0);
+    std::shared_ptr<context::cached_launch> l = ctx.find_launch(key);
+    if(l) return run_dot(ctx, *l) * scale;
+    std::vector<std::vector<dev::perm_desc> > lists(1);
+    std::vector<dev::perm_desc> &descs = lists[0];
     for(size_t x = 0; x < bid2.size(); x++) {
         index_t ix = get_index(x, bid2);
         index_t ia = ix, ib = ix;
@@ -49,41 +57,9 @@ double btod_dotprod(btensor &a, const tensor_tr &tra0, btensor &b, const tensor_
         d.alpha *= ta.st.c * ta.st.c;
         descs.push_back(d);
     }
-    double scale = tra0.st.c * trb0.st.c;
-    if(descs.empty()) return 0.0;
-
-    std::vector<uint32_t> cd, co;
-    for(size_t i = 0; i < descs.size(); i++)
-        for(uint32_t off = 0; off < descs[i].total; off += dev::kPermChunk) {
-            cd.push_back((uint32_t)i);
-            co.push_back(off);
-        }
-    const size_t nch = cd.size();
-    size_t o_d = 0;
-    size_t o_cd = (descs.size() * sizeof(dev::perm_desc) + 255) & ~size_t(255);
-    size_t o_co = o_cd + ((4 * nch + 255) & ~size_t(255));
-    size_t o_p = o_co + ((4 * nch + 255) & ~size_t(255));
-    size_t o_out = o_p + ((8 * nch + 255) & ~size_t(255));
-    size_t bytes = o_out + 256;
-    std::vector<char> host(bytes, 0);
-    std::memcpy(&host[o_d], descs.data(), descs.size() * sizeof(dev::perm_desc));
-    std::memcpy(&host[o_cd], cd.data(), 4 * nch);
-    std::memcpy(&host[o_co], co.data(), 4 * nch);
-    char *mem = (char*)ctx.alloc(bytes);
-    double r = 0.0;
-    try {
-        ctx.upload(mem, host.data(), bytes);
-        ctx.activate();
-        hip_check(dev::launch_dot((dev::perm_desc*)(mem + o_d), (uint32_t*)(mem + o_cd),
-            (uint32_t*)(mem + o_co), (uint32_t)nch, (double*)(mem + o_p),
-            (double*)(mem + o_out), ctx.stream()), "dot");
-        ctx.download(&r, mem + o_out, sizeof(double));
-    } catch(...) {
-        ctx.free(mem);
-        throw;
-    }
-    ctx.free(mem);
-    return r * scale;
+    l = upload_launches(ctx, lists);
+    ctx.keep_launch(key, l);
+    return run_dot(ctx, *l) * scale;
 }
 
 } // namespace lta

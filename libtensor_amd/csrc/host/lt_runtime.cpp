@@ -61,7 +61,7 @@ context::~context() {
     }
     hipSetDevice(m_device);
     if(m_stream) hipStreamSynchronize(m_stream);
-    m_launch_cache.clear();      // their memory goes with the loop below
+    m_launch_cache.clear();
     for(std::map<void*, size_t>::iterator i = m_sizes.begin(); i != m_sizes.end(); ++i)
         hipFree(i->first);
     if(m_xfer_ev) hipEventDestroy(m_xfer_ev);
@@ -109,18 +109,19 @@ std::shared_ptr<context::cached_launch> context::find_launch(const std::string &
 }
 
 void context::keep_launch(const std::string &key, std::shared_ptr<cached_launch> l) {
-    std::vector<std::shared_ptr<cached_launch> > drop;
+    std::vector<std::shared_ptr<cached_launch> > drop;    // let go outside the lock
     {
         std::lock_guard<std::mutex> lk(m_cache_mtx);
-        if(!m_launch_cache.count(key)) m_launch_order.push_back(key);
-        m_launch_cache[key] = l;
+        std::shared_ptr<cached_launch> &e = m_launch_cache[key];
+        if(e) drop.push_back(e);
+        else m_launch_order.push_back(key);
+        e = l;
         while(m_launch_order.size() > kLaunchCache) {
             drop.push_back(m_launch_cache[m_launch_order.front()]);
             m_launch_cache.erase(m_launch_order.front());
             m_launch_order.erase(m_launch_order.begin());
         }
     }
-    for(size_t i = 0; i < drop.size(); i++) if(drop[i] && drop[i]->mem) free(drop[i]->mem);
 }
 
 void *context::staging(size_t bytes) {

@@ -85,7 +85,12 @@ public:
         std::vector<size_t> touched;     //!< blocks the launches write
         symmetry sym;                    //!< symmetry the result takes
         double bytes;                    //!< bytes the launches move
-        cached_launch() : mem(0), bytes(0.0) { }
+        explicit cached_launch(context &c) : mem(0), bytes(0.0), m_ctx(c) { }
+        ~cached_launch() { if(mem) m_ctx.free(mem); }
+        cached_launch(const cached_launch&) = delete;
+        cached_launch &operator=(const cached_launch&) = delete;
+    private:
+        context &m_ctx;
     };
     std::shared_ptr<cached_launch> find_launch(const std::string &key);
     void keep_launch(const std::string &key, std::shared_ptr<cached_launch> l);
@@ -270,6 +275,16 @@ std::shared_ptr<context::cached_launch> upload_launches(context &ctx,
 //! Runs the launches of a cached entry in order and waits; ms (optional)
 //! accumulates their device time.
 void run_launches(context &ctx, const context::cached_launch &l, double *ms);
+//! `second` adds to what `first` writes (same destination, the terms'
+//! sources apart from it): where one of the two keeps its source's order both
+//! become one descriptor, in `second` (`first` without elements), and true is
+//! returned.
+bool fuse_terms(dev::perm_desc &first, dev::perm_desc &second);
+//! fuse_terms over launches in order, for each block's first two terms.
+void fuse_launches(std::vector<std::vector<dev::perm_desc> > &lists);
+//! Scalar product of the (single) list of a cached entry: sum over its
+//! descriptors of dst * alpha P(src).
+double run_dot(context &ctx, const context::cached_launch &l);
 //! Launch-cache key parts: a transformation; a tensor's identity and (with
 //! version) its structure version.
 std::string key_part(const tensor_tr &tr);
@@ -297,11 +312,19 @@ struct exec_stats {
 
 //! Dense helpers on a context's stream (both synchronous): dst = or +=
 //! tr(src) (tod_copy), and C = or += d contract(A, B) of device arrays
-//! (tod_contract2: align, permute into scratch, one GEMM, permute back).
+//! (tod_contract2: one kernel at the operands' own strides).
 void dense_permute(context &ctx, const double *src, const dims_t &dsrc,
     const tensor_tr &tr, double *dst, bool accumulate);
 void dense_contract2(context &cx, const contraction2 &contr, const dims_t &da, const double *a,
     const dims_t &db, const double *b, double d, bool zero, double *c);
+//! The same with its temporaries in the device's fixed scratch region;
+//! LT_ERR_PARAM before any device work if the aligned form of the call would
+//! not fit there.
+void dense_contract2_noalloc(context &cx, const contraction2 &contr, const dims_t &da,
+    const double *a, const dims_t &db, const double *b, double d, bool zero, double *c);
+//! b = (zero) or += sum_i trs[i](a[i]), every a[i] of dimensions da (tod_add).
+void dense_add(context &cx, const double *const *a, const dims_t &da,
+    const std::vector<tensor_tr> &trs, double *b, bool zero);
 //! One term of dense_contract2_many: C = (zero) or += d contract(A, B).
 struct dense_contract_item {
     contraction2 contr;
@@ -311,7 +334,7 @@ struct dense_contract_item {
     bool zero;
 };
 //! The terms into one C in order, as that many dense_contract2 calls, with
-//! one allocation, one upload and one synchronization for all of them.
+//! one synchronization for all of them.
 void dense_contract2_many(context &cx, const std::vector<dense_contract_item> &items,
     double *c);
 

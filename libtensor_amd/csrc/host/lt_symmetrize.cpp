@@ -136,11 +136,14 @@ double symmetrizer::run(btensor &b, bool add, double d, int mode) {
                 const bool acc = r > 0 || had;
                 rounds[r].push_back(make_perm_desc_public(x.block_ptr(rs[k].ai), dx, tr,
                     b.block_ptr(ib), acc));
-                bytes += 8.0 * dx.size() * (acc ? 3 : 2);
                 r++;
             }
             if(r) touched.push_back(ib);
         }
+        fuse_launches(rounds);
+        for(size_t r = 0; r < rounds.size(); r++)
+            for(size_t k = 0; k < rounds[r].size(); k++)
+                bytes += 8.0 * rounds[r][k].total * (rounds[r][k].add ? 3 : 2);
         l = upload_launches(cx, rounds);
         l->touched = touched;
         l->bytes = bytes;
