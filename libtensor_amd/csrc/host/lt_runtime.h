@@ -84,8 +84,9 @@ public:
         std::vector<segment> segs;       //!< launched in order
         std::vector<size_t> touched;     //!< blocks the launches write
         symmetry sym;                    //!< symmetry the result takes
+        uint64_t uid;                    //!< its tag
         double bytes;                    //!< bytes the launches move
-        explicit cached_launch(context &c) : mem(0), bytes(0.0), m_ctx(c) { }
+        explicit cached_launch(context &c) : mem(0), uid(0), bytes(0.0), m_ctx(c) { }
         ~cached_launch() { if(mem) m_ctx.free(mem); }
         cached_launch(const cached_launch&) = delete;
         cached_launch &operator=(const cached_launch&) = delete;
