@@ -315,7 +315,7 @@ int lt_btod_contract2_ozaki_bounds(lt_btod_contract2 *op, size_t *aidx, double *
     double *cmax, size_t cap, size_t *count);
 /* C tile shape of the split-precision product kernel: -1 (default) = each
  * shape timed once on the plan's work list, the fastest kept; 0 = 16x32,
- * 1 = 16x64, 2 = 32x32 (rows x columns).  No counterpart in the reference. */
+ * 1 = 16x64, 2 = 48x64 (rows x columns).  No counterpart in the reference. */
 int lt_btod_contract2_set_ozaki_tile(lt_btod_contract2 *op, int tile);
 
 /* ---- btod_dotprod (libtensor/block_tensor/btod_dotprod.h:35-66:

@@ -442,7 +442,7 @@ class btod_contract2(object):
 
     def set_ozaki_tile(self, tile):
         """Split-precision tile shape: -1 measured (default), 0 16x32,
-        1 16x64, 2 32x32."""
+        1 16x64, 2 48x64."""
         call("lt_btod_contract2_set_ozaki_tile", self._h, int(tile))
 
 

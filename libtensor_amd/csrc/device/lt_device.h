@@ -288,8 +288,9 @@ struct oz_pair {
     uint32_t ia, ib;                  //!< split descriptors of the two operands
 };
 
-//! C tile shapes of the split-precision product kernel (rows x columns).
-enum oz_tile_cfg { OZ_TILE_16x32 = 0, OZ_TILE_16x64 = 1, OZ_TILE_32x32 = 2, OZ_TILE_COUNT = 3 };
+//! C tile shapes of the split-precision product (rows x columns): a tile per
+//! wave, or (48 x 64) per workgroup of four waves.
+enum oz_tile_cfg { OZ_TILE_16x32 = 0, OZ_TILE_16x64 = 1, OZ_TILE_48x64 = 2, OZ_TILE_COUNT = 3 };
 void oz_tile_shape(int tile, uint32_t &bm, uint32_t &bn);
 
 //! items: nitems pairs (descriptor, row).

@@ -30,7 +30,7 @@ void oz_tile_shape(int tile, uint32_t &bm, uint32_t &bn) {
     switch(tile) {
     case OZ_TILE_16x32: bm = 16; bn = 32; break;
     case OZ_TILE_16x64: bm = 16; bn = 64; break;
-    default: bm = 32; bn = 32; break;
+    default: bm = 48; bn = 64; break;
     }
 }
 
@@ -95,6 +95,18 @@ hipError_t launch_oz_split(const oz_split_desc *descs, const uint32_t *items,
     return hipGetLastError();
 }
 
+// c plus d times a pair's product of one element: its weights w[l] 2^-7 l
+// (exact) added by fused multiplications from the largest on, scaled by the
+// exponents of its row and column, and added to c with one more.
+template<int S>
+__device__ __forceinline__ double oz_add(double c, double d, const int (&w)[S], int ea, int eb) {
+    double x = 0.0;
+#pragma unroll
+    for(int l = 0; l < S; l++) x = __builtin_fma(double(w[l]), 1.0 / double(1ull << (7 * l)), x);
+    const bool nf = ea == kOzNonFinite || eb == kOzNonFinite;
+    return __builtin_fma(d, nf ? __builtin_nan("") : ldexp(x, ea + eb - 14), c);
+}
+
 // One wave per 16 FM x 16 FN C tile, four waves (tiles) per workgroup.
 // v_mfma_i32_16x16x64_i8 takes 16 bytes of A and of B per lane and returns
 // D[4 (l / 16) + v][l % 16], v = 0..3.  Lane l supplies row (A) / column (B)
@@ -105,9 +117,9 @@ hipError_t launch_oz_split(const oz_split_desc *descs, const uint32_t *items,
 // fragment-major panel chunk (a wave's load covers 8 whole cache lines).  Per
 // chunk the S slices of A are loaded once, each slice of B is loaded and
 // used at once: every product t + u = L <= S + 1 runs from registers into
-// the int32 accumulator of its weight L; at the end of a pair each weight is
-// scaled by 2^(e_i + f_j - 7 L) and added in FP64 in the order
-// L = 2, 3, ..., S + 1.
+// the int32 accumulator of its weight L; at the end of a pair the weights are
+// scaled by their powers of two and added in FP64 in the order L = 2, 3, ...,
+// S + 1 (oz_add).
 template<int S, int FM, int FN>
 __global__ void __launch_bounds__(256)
 oz_gemm_kernel(const gemm_cblock *__restrict__ cbs,
@@ -195,15 +207,14 @@ oz_gemm_kernel(const gemm_cblock *__restrict__ cbs,
 #pragma unroll
             for(int v = 0; v < 4; v++) ea[v] = pr.ea[orow[i][v]];
 #pragma unroll
-            for(int l = 0; l < S; l++)               // weight L = l + 2
+            for(int f = 0; f < FN; f++)
 #pragma unroll
-                for(int f = 0; f < FN; f++)
+                for(int v = 0; v < 4; v++) {
+                    int w[S];
 #pragma unroll
-                    for(int v = 0; v < 4; v++) {
-                        const bool nf = ea[v] == kOzNonFinite || eb[f] == kOzNonFinite;
-                        cacc[i][f][v] += nf ? __builtin_nan("") : pr.d * ldexp(
-                            double(acc[l][i][f][v]), ea[v] + eb[f] - 7 * (l + 2));
-                    }
+                    for(int l = 0; l < S; l++) w[l] = acc[l][i][f][v];
+                    cacc[i][f][v] = oz_add<S>(cacc[i][f][v], pr.d, w, ea[v], eb[f]);
+                }
         }
     }
 
@@ -223,6 +234,143 @@ oz_gemm_kernel(const gemm_cblock *__restrict__ cbs,
                 }
             }
         }
+}
+
+// The same product with a workgroup per tile of up to three row panels and four
+// column panels, for C blocks that fill it: per chunk the A slices of the tile
+// are staged in LDS (two buffers) and read by all four waves, each of which
+// multiplies them with its own column panel, held in registers.  Per 64-k
+// chunk a 48 x 64 tile so reads 7 S KB for 12 tiles of 16 x 16, where a wave
+// by itself reads 3 S KB for two of them, which the L2 caches bound (pp-ladder
+// o = 40, v = 200, 7 slices: 0.376 to 0.281 ms a call).  The next chunk's loads run
+// behind the products: A's into registers and from there into the other
+// buffer, a B slice's into its registers after its last use.  Element by
+// element the sums are those of the wave tiles.
+template<int S, int FA>
+__device__ __forceinline__ void oz_tile_body(const gemm_cblock &cb, const oz_pair *__restrict__ pairs,
+    const gemm_tile &tile, int4_t *buf) {
+
+    constexpr int U = S * FA, NU = (U + 3) / 4;     // 1 KB panel chunks of A, of one wave
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int lr = lane & 15, lg = lane >> 4;
+    const uint32_t ap = uint32_t(tile.tm) * 3, npan = (cb.n + 15) / 16;
+    const bool active = uint32_t(tile.tn) * 4 + wave < npan;
+    const uint32_t bp = min(uint32_t(tile.tn) * 4 + wave, npan - 1);
+    const uint32_t m0 = 16 * ap, col = 16 * bp + lr;
+    const bool in = active && col < cb.n;
+
+    double cacc[FA][4];
+    int4_t acc[S][FA], st[NU], bv[S];
+#pragma unroll
+    for(int i = 0; i < FA; i++)
+#pragma unroll
+        for(int v = 0; v < 4; v++) cacc[i][v] = 0.0;
+#pragma unroll
+    for(int l = 0; l < S; l++)
+#pragma unroll
+        for(int i = 0; i < FA; i++) acc[l][i] = int4_t{0, 0, 0, 0};
+
+    auto load_a = [&](const oz_pair &pr, uint32_t kc) {
+#pragma unroll
+        for(int q = 0; q < NU; q++) {
+            const uint32_t u = wave + 4 * q;
+            if(u < uint32_t(U)) st[q] = *(const int4_t *)(pr.a + size_t(u / FA) * pr.astride +
+                (size_t(ap + u % FA) * (pr.kp / 64) + kc) * 1024 + lane * 16);
+        }
+    };
+    auto store_a = [&](int b) {
+#pragma unroll
+        for(int q = 0; q < NU; q++) {
+            const uint32_t u = wave + 4 * q;
+            if(u < uint32_t(U)) buf[(b * U + u) * 64 + lane] = st[q];
+        }
+    };
+    auto load_b = [&](const oz_pair &pr, uint32_t kc, int us) {
+        bv[us] = *(const int4_t *)(pr.b + size_t(us) * pr.bstride + (size_t(bp) * (pr.kp / 64) + kc) * 1024 + lane * 16);
+    };
+    uint32_t p = cb.pair_begin, kc = 0;
+    while(p < cb.pair_end && pairs[p].kp == 0) p++;
+    if(p < cb.pair_end) {
+        oz_pair pr = pairs[p];
+        load_a(pr, 0);
+#pragma unroll
+        for(int us = 0; us < S; us++) load_b(pr, 0, us);
+        store_a(0);
+        __syncthreads();
+        int b = 0;
+        while(true) {
+            // the chunk after this one (past the last one: this one again)
+            uint32_t np = p, nkc = kc + 1;
+            oz_pair nx = pr;
+            bool last = false;
+            if(64 * nkc >= pr.kp) {
+                do np++; while(np < cb.pair_end && pairs[np].kp == 0);
+                last = np == cb.pair_end;
+                nkc = last ? kc : 0;
+                if(!last) nx = pairs[np];
+            }
+            load_a(nx, nkc);
+#pragma unroll
+            for(int ts = 0; ts < S; ts++) {
+                int4_t av[FA];
+#pragma unroll
+                for(int i = 0; i < FA; i++) av[i] = buf[(b * U + ts * FA + i) * 64 + lane];
+#pragma unroll
+                for(int us = S - 1 - ts; us >= 0; us--)  // t + u <= S + 1 (1-based)
+#pragma unroll
+                    for(int i = 0; i < FA; i++)
+                        acc[ts + us][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i], bv[us], acc[ts + us][i], 0, 0, 0);
+                load_b(nx, nkc, S - 1 - ts);
+            }
+            store_a(b ^ 1);
+            if(np != p) {                                // the pair's sums
+                const int eb = pr.eb[in ? col : 0];
+#pragma unroll
+                for(int i = 0; i < FA; i++)
+#pragma unroll
+                    for(int v = 0; v < 4; v++) {
+                        const uint32_t row = m0 + 16 * i + 4 * lg + v;
+                        const int ea = pr.ea[row < cb.m ? row : m0];
+                        int w[S];
+#pragma unroll
+                        for(int l = 0; l < S; l++) {
+                            w[l] = acc[l][i][v];
+                            acc[l][i][v] = 0;
+                        }
+                        cacc[i][v] = oz_add<S>(cacc[i][v], pr.d, w, ea, eb);
+                    }
+            }
+            if(last) break;
+            __syncthreads();
+            b ^= 1;
+            p = np;
+            kc = nkc;
+            pr = nx;
+        }
+    }
+#pragma unroll
+    for(int i = 0; i < FA; i++)
+#pragma unroll
+        for(int v = 0; v < 4; v++) {
+            const uint32_t row = m0 + 16 * i + 4 * lg + v;
+            if(in && row < cb.m) {
+                double *cp = cb.c + size_t(row) * cb.ldc + col;
+                *cp = cb.zero ? cacc[i][v] : cacc[i][v] + *cp;
+            }
+        }
+}
+
+template<int S>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(S > 7 ? 1 : 2)))
+oz_tile_kernel(const gemm_cblock *__restrict__ cbs, const oz_pair *__restrict__ pairs,
+    const gemm_tile *__restrict__ tiles) {
+    __shared__ int4_t buf[2 * S * 3 * 64];
+    const gemm_tile tile = tiles[blockIdx.x];
+    const gemm_cblock cb = cbs[tile.cblock];
+    const uint32_t rows = cb.m - 48 * uint32_t(tile.tm);
+    if(rows > 32) oz_tile_body<S, 3>(cb, pairs, tile, buf);
+    else if(rows > 16) oz_tile_body<S, 2>(cb, pairs, tile, buf);
+    else oz_tile_body<S, 1>(cb, pairs, tile, buf);
 }
 
 // Largest exponent of every split operand: one wave per operand, its rows'
@@ -348,7 +496,7 @@ static void launch_oz_s(const gemm_cblock *cb, const oz_pair *pairs,
         hipLaunchKernelGGL((oz_gemm_kernel<S, 1, 4>), grid, block, 0, s, cb, pairs, tiles, ntiles);
         break;
     default:
-        hipLaunchKernelGGL((oz_gemm_kernel<S, 2, 2>), grid, block, 0, s, cb, pairs, tiles, ntiles);
+        hipLaunchKernelGGL(oz_tile_kernel<S>, dim3(ntiles), block, 0, s, cb, pairs, tiles);
         break;
     }
 }

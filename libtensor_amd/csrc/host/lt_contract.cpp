@@ -1822,9 +1822,9 @@ void btod_contract2::build_ozaki(int slices) {
     // XCD with its own L2.  The C blocks of a group (same B operands) go to
     // one XCD, groups longest first onto the least loaded XCD; a group's
     // tiles run column tile by column tile, so the row tiles that read the
-    // same B slice panels run together.  Workgroup w takes four tiles of XCD
-    // w % nx's queue, or of the longest remaining queue once its own is
-    // empty.  The order changes no result: each tile is one wave's sums.
+    // same B slice panels run together.  Workgroup w takes its four tiles
+    // (one of 48 x 64) of XCD w % nx's queue, or of the longest remaining queue once its own is
+    // empty.  The order changes no result: each tile's sums are its own.
     std::vector<dev::gemm_tile> tl[dev::OZ_TILE_COUNT];
     {
         const size_t nb = pl.cblocks.size();
@@ -1885,13 +1885,14 @@ void btod_contract2::build_ozaki(int slices) {
             std::vector<size_t> qp(nx, 0);
             tl[k].reserve(total);
             for(size_t w = 0; tl[k].size() < total; w++) {
-                for(int j = 0; j < 4 && tl[k].size() < total; j++) {
+                for(int j = 0; j < per_wg && tl[k].size() < total; j++) {
                     size_t x = w % nx;
                     if(qp[x] >= q[x].size()) {
                         size_t left = 0;
                         for(size_t y = 0; y < nx; y++)
                             if(q[y].size() - qp[y] > left) { left = q[y].size() - qp[y]; x = y; }
                     }
+            const int per_wg = k == dev::OZ_TILE_48x64 ? 1 : 4;
                     tl[k].push_back(q[x][qp[x]++]);
                 }
             }
