@@ -6,7 +6,9 @@
 // threads one chunk ahead, so the loop adds two offsets per element.
 // What bounds it at the sizes such calls have (k of some hundreds to
 // thousands): the chunk loop's latency and the launch; k ranges are cut into
-// parts where the tiles leave CUs idle.  FIGURES
+// parts where the tiles leave CUs idle.  o = 15, v = 45 ring (675 x 675 x
+// 675, all three tensors permuted): 27 us, 40 a call, where three copies, a
+// product of 64 x 64 tiles and the lists and temporaries of all took 0.43 ms.
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include "lt_device.h"

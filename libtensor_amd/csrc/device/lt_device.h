@@ -44,7 +44,8 @@ struct perm_desc {
     fastdiv dps;                      //!< destination stride of tile_p
     fastdiv tdp, tdq;                 //!< extents of tile_p and n - 1
 };
-//! Tile side: 64 where both extents are beyond 32 (PERMFIG), else 32.
+//! Tile side: 64 where both extents are beyond 32 (rows of 512 bytes:
+//! 37 x 61 x 83 x 91 to 83 x 37 x 91 x 61 in 63 instead of 71 us), else 32.
 static const uint32_t kPermTile = 32, kPermTileMax = 64;
 static const uint32_t kPermTileItem = 0x80000000u;
 
@@ -98,8 +99,8 @@ struct gemm_tile {
 //! operands, rows concatenated; _On: compiled for n waves per SIMD); used by
 //! grouped launches, per-block launches run the SPLITK configuration of the
 //! same shape.  WG_*_Gn: workgroup tiles over stacks with both operands
-//! staged in LDS, the k chunks dealt to n groups of four waves (grouped and
-//! per-block launches).
+//! staged in LDS, the k chunks dealt to n groups of waves, one per 16 columns
+//! (grouped and per-block launches).
 enum { TILE_64x64 = 0, TILE_32x64 = 1, TILE_64x32 = 2, TILE_32x32 = 3,
        SPLITK_16x64_W4 = 4, SPLITK_32x32_W4 = 5, SPLITK_32x64_W4 = 6,
        SPLITK_64x32_W4 = 7, SPLITK_16x64_W2 = 8, SPLITK_32x32_W2 = 9,
@@ -108,7 +109,7 @@ enum { TILE_64x64 = 0, TILE_32x64 = 1, TILE_64x32 = 2, TILE_32x32 = 3,
        WG_80x64_G2 = 15, WG_48x64_G4 = 16, WG_64x64_G4 = 17,
        STACK_48x32_W4 = 18, WG_64x64_G1 = 19, WG_96x64_G1 = 20,
        WG_112x64_G1 = 21, STACK_48x32_W4_O2 = 22, STACK_32x32_W4_O3 = 23,
-       STACK_16x64_W4_O3 = 24, STACK_VAR_64x32_W4 = 25, WG_32x64_G2 = 26,
+       STACK_16x64_W4_O3 = 24, STACK_VAR_64x32_W4 = 25, WG_96x128_G1 = 26,
        WG_16x64_G4 = 27, TILE_COUNT = 28 };
 void tile_shape(int cfg, uint32_t &bm, uint32_t &bn);
 inline bool is_stacked(int cfg) { return cfg >= STACK_16x64_W4 && cfg < TILE_COUNT; }
@@ -116,7 +117,7 @@ inline bool is_stacked(int cfg) { return cfg >= STACK_16x64_W4 && cfg < TILE_COU
 inline bool is_tile(int cfg) {
     switch(cfg) {
     case WG_32x64_G4: case WG_80x64_G2: case WG_48x64_G4: case WG_64x64_G4: case WG_64x64_G1:
-    case WG_96x64_G1: case WG_112x64_G1: case WG_32x64_G2: case WG_16x64_G4: return true;
+    case WG_96x64_G1: case WG_112x64_G1: case WG_96x128_G1: case WG_16x64_G4: return true;
     default: return false;
     }
 }

@@ -44,9 +44,10 @@ void tile_shape(int cfg, uint32_t &bm, uint32_t &bn) {
     case WG_16x64_G4: bm = 16; bn = 64; break;
     case SPLITK_32x32_W4: case SPLITK_32x32_W2: case STACK_32x32_W4: case STACK_32x32_W4_O3:
         bm = 32; bn = 32; break;
-    case SPLITK_32x64_W4: case WG_32x64_G4: case WG_32x64_G2: bm = 32; bn = 64; break;
+    case SPLITK_32x64_W4: case WG_32x64_G4: bm = 32; bn = 64; break;
     case SPLITK_64x32_W4: bm = 64; bn = 32; break;
     case WG_48x64_G4: bm = 48; bn = 64; break;
+    case WG_96x128_G1: bm = 96; bn = 128; break;
     case WG_80x64_G2: bm = 80; bn = 64; break;
     case WG_96x64_G1: bm = 96; bn = 64; break;
     case WG_112x64_G1: bm = 112; bn = 64; break;

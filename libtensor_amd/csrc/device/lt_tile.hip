@@ -1,8 +1,8 @@
 // Workgroup-tiled FP64 MFMA GEMM over stacks (C blocks that share their B
 // operands, rows concatenated; lt_device.h: tile_stack).
 //
-// A workgroup computes a tile of up to 16 FM rows x 64 columns: KG groups of
-// four waves take the 16-k chunks of the stack's pair list in turn, each wave
+// A workgroup computes a tile of up to 16 FM rows x 16 NW columns: KG groups of
+// NW waves take the 16-k chunks of the stack's pair list in turn, each wave
 // multiplies one 16-column strip against all rows of the tile, and the groups'
 // partial tiles are added in LDS in group order (fixed summation order, one
 // writer per C element).  A group stages its chunk in two LDS buffers, rows of
@@ -15,12 +15,18 @@
 // them as it can: addresses move on in scalar registers, the accumulators stay
 // in place (in architectural registers: kernels whose accumulators the compiler
 // copied to and from the accumulation registers in every step reached 48), and
-// loads and LDS writes are spread between the products.  The 4 x 64 rows and
-// columns a chunk brings in are loaded once per workgroup in whole 128-byte
-// lines, in either operand layout.  Measured against the kernels that load
+// loads and LDS writes are spread between the products.  The rows and columns
+// a chunk brings in are loaded once per workgroup in runs of 128 bytes, in
+// either operand layout.  Measured against the kernels that load
 // fragments straight from memory (o, v: one ring contraction): o = 29, v = 131
 // in one block 3.48 to 2.16 ms a call, o = 48, v = 240 in uneven blocks 85.6 to
 // 58.1 ms (53 TFLOP/s).
+//
+// What is left is loading: a wave's load of 64 x 8 bytes takes 17 to 19 cycles
+// of its CU, and rows that are not whole cache lines come twice from the L2
+// cache.  Eight waves over 128 columns share the rows of A (7 loads a thread
+// and chunk for 24 products instead of 10): 96 x 128 instead of 96 x 64 tiles,
+// the same rings 2.13 to 1.98 and 58.9 to 56.7 ms.
 //
 // Where the tiles of a launch are too few to keep 256 CUs evenly busy, their
 // chunk sequences are cut into parts and a second kernel adds the parts'
@@ -94,7 +100,7 @@ __device__ __forceinline__ chunk_pos chunk_advance(cpair *pairs, const chunk_pos
     return r;
 }
 
-//! Where a tile's rows come from and go to: the row tables of a stack, ...
+//! Where a tile's rows come from and go to: the row tables of a stack.
 struct stack_rows {
     cpair *pairs;
     garow *arow;
@@ -113,23 +119,6 @@ struct stack_rows {
     }
 };
 
-//! ... or a dense matrix product (one pair).
-struct dense_rows {
-    cpair *pairs;
-    double d;
-    gout *c;
-    uint32_t rstep, lda, ldc, zero;     //!< bytes from row to row of A, its row length, that of C
-    __device__ __forceinline__ row_src row(uint32_t, uint32_t r) const {
-        row_src s;
-        s.d = d; s.off = r * rstep; s.lda = lda;
-        return s;
-    }
-    __device__ __forceinline__ void write(uint32_t r, uint32_t col, double x) const {
-        gout *cp = c + (size_t(r) * ldc + col);
-        *cp = zero ? x : x + *cp;
-    }
-};
-
 //! A tile and its part of the chunk sequence: `count` chunks from chunk c of
 //! pair p on.  part: where the tile's partial sums go (fragment order), or
 //! null: they are all there is and go to C.
@@ -143,31 +132,35 @@ struct tile_part {
 
 static const int kTileRow = 18;     // doubles per staged row of 16 k (144 bytes: b128 reads of 16 rows use every bank once)
 
-template<int FM, int KG>
+//! NW: waves to a group, 16 columns each.  16 NW / 4 rows are staged at a time:
+//! PA passes over the rows of A (the last one may go past them), four over B's.
+template<int FM, int KG, int NW>
 struct tile_smem {
-    static constexpr int BM = 16 * FM, BN = 64;
-    static constexpr int CH = (BM + BN) * kTileRow;      // one staged chunk: A rows, then B columns
+    static constexpr int BM = 16 * FM, BN = 16 * NW, RP = 4 * NW;
+    static constexpr int PA = (BM + RP - 1) / RP, RA = PA * RP;
+    static constexpr int CH = (RA + BN) * kTileRow;      // one staged chunk: A rows, then B columns
     static constexpr int NST = KG * 2 * CH, NRED = KG == 1 ? 0 : KG * BM * BN;
     alignas(16) double ch[NST > NRED ? NST : NRED];
     // tables of two pairs per group: scales, offsets and strides of
     // the rows of A, offsets of the columns of B
-    double rd[KG][2][BM];
-    uint32_t ro[KG][2][BM];
-    uint32_t rl[KG][2][BM];
+    double rd[KG][2][RA];
+    uint32_t ro[KG][2][RA];
+    uint32_t rl[KG][2][RA];
     uint32_t cn[KG][2][BN];
 };
 
-template<int FM, int KG, class SRC>
-__device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, tile_smem<FM, KG> &sm) {
+template<int FM, int KG, int NW>
+__device__ __forceinline__ void tile_body(const stack_rows &src, const tile_part &tp, tile_smem<FM, KG, NW> &sm) {
 
-    typedef tile_smem<FM, KG> S;
-    constexpr int BM = S::BM, BN = S::BN;
-    const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
-    const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
-    const int tid = threadIdx.x & 255, lane = tid & 63;
+    typedef tile_smem<FM, KG, NW> S;
+    constexpr int BM = S::BM, BN = S::BN, RP = S::RP, PA = S::PA, GT = 64 * NW;
+    const int g = __builtin_amdgcn_readfirstlane(threadIdx.x / GT);
+    const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) % NW);
+    const int tid = threadIdx.x % GT, lane = tid & 63;
     const int lr = lane & 15, lg = lane >> 4;
-    const int hi = tid >> 4, lo = tid & 15;
-    const int hr = ((hi & 1) << 3) | (hi >> 1);  // as a row: rows 8 apart side by side (their LDS banks differ)
+    const int hi = (tid >> 4) & 15, lo = tid & 15, up = (tid >> 4) & 16;
+    const int hr = (((hi & 1) << 3) | (hi >> 1)) + up;  // as a row: rows 8 apart side by side (their LDS banks differ)
+    const int lw = lo + up;                             // row of the threads along rows
 
     const uint32_t m0 = tp.m0, n0 = tp.n0, mrem = tp.mrem, nrem = tp.nrem, nchunk = tp.count;
     cpair *pairs = src.pairs;
@@ -179,10 +172,10 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
     if(nchunk > 0) {
         // rows / column of the pair tables this thread stages (past the extent: the first one)
         const uint32_t trow = uint32_t(tid) < mrem ? m0 + tid : m0;
-        const uint32_t tcol = uint32_t(tid & 63) < nrem ? n0 + (tid & 63) : n0;
+        const uint32_t tc = uint32_t(tid) % BN, tcol = tc < nrem ? n0 + tc : n0;
         auto info_load = [&](uint32_t p, row_src &ar, uint32_t &cn) {
-            if(tid < BM) ar = src.row(p, trow);
-            if(tid >= 192) {
+            if(tid < S::RA) ar = src.row(p, trow);
+            if(tid >= GT - BN) {
                 cpair *sp = pairs + p;
                 if(tabled(sp)) cn = 8u * uint32_t(((gint *)(uintptr_t)sp->noff)[tcol]);
                 else {
@@ -192,12 +185,12 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
             }
         };
         auto info_store = [&](int slot, const row_src &ar, uint32_t cn) {
-            if(tid < BM) {
+            if(tid < S::RA) {
                 sm.rd[g][slot][tid] = ar.d;
                 sm.ro[g][slot][tid] = ar.off;
                 sm.rl[g][slot][tid] = ar.lda;
             }
-            if(tid >= 192) sm.cn[g][slot][tid - 192] = cn;
+            if(tid >= GT - BN) sm.cn[g][slot][tc] = cn;
         };
 
         // The group's next chunks: n1 to be loaded, n2 whose pair's tables
@@ -218,26 +211,26 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
         // Addresses of this thread's elements of the last chunk loaded: byte
         // offsets of rows (A) and columns (B) from uniform bases, which move
         // on from chunk to chunk.
-        uint32_t ao[FM], bo[4], kr = 0;
+        uint32_t ao[PA], bo[4], kr = 0;
         uint32_t abase = 0, bbase = 0;     // bytes from the pair's A and B
-        double v[FM + 4];                  // the chunk on its way
+        double v[PA + 4];                  // the chunk on its way
         uint32_t cur = 0xffffffffu;        // pair of the addresses
         uint32_t fl = 0, bstep = 0;        // its flags (kTab: B through offset tables), step of B from chunk to chunk
         const gchar *pa = 0, *pb = 0, *qa = 0, *qb = 0;
         const uint32_t kTab = 0x80000000u;
         // places of the thread's elements in an LDS buffer, by mapping: rows
         // (columns) adjacent in memory run along 16 threads, else k does
-        const int a0 = hr * kTileRow + lo, a1 = lo * kTileRow + hi;
+        const int a0 = hr * kTileRow + lo, a1 = lw * kTileRow + hi;
 
         // Addresses from the pair tables, k past the extent on its last element.
         auto locate = [&](cpair *sp, const chunk_pos &n) {
             const uint32_t K = n.k;
             const bool akm = (fl & kPairAKMajor) != 0, bnf = (fl & kPairBNFast) != 0;
-            const int ra = akm ? lo : hr, rb = bnf ? lo : hr;
+            const int ra = akm ? lw : hr, rb = bnf ? lw : hr;
             const uint32_t kac = min(16 * n.c + (akm ? hi : lo), K - 1), kbc = min(16 * n.c + (bnf ? hi : lo), K - 1);
 #pragma unroll
-            for(int j = 0; j < FM; j++)
-                ao[j] = sm.ro[g][n.slot][ra + 16 * j] + 8u * (akm ? kac * sm.rl[g][n.slot][ra + 16 * j] : kac);
+            for(int j = 0; j < PA; j++)
+                ao[j] = sm.ro[g][n.slot][ra + RP * j] + 8u * (akm ? kac * sm.rl[g][n.slot][ra + RP * j] : kac);
             uint32_t ko;
             if(fl & kTab) ko = 8u * uint32_t(((gint *)(uintptr_t)sp->koff)[kbc]);
             else {
@@ -246,7 +239,7 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
                 ko = 8u * (q * uint32_t(sp->ks0) + kr * uint32_t(sp->ks1));
             }
 #pragma unroll
-            for(int j = 0; j < 4; j++) bo[j] = ko + sm.cn[g][n.slot][rb + 16 * j];
+            for(int j = 0; j < 4; j++) bo[j] = ko + sm.cn[g][n.slot][rb + RP * j];
             abase = bbase = 0;
         };
         // Addresses of chunk n.  Within a pair only the uniform bases move on
@@ -266,7 +259,7 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
             } else if(n.valid) {
                 if(fl & kPairAKMajor) {
 #pragma unroll
-                    for(int j = 0; j < FM; j++) ao[j] += 128u * KG * sm.rl[g][n.slot][lo + 16 * j];
+                    for(int j = 0; j < PA; j++) ao[j] += 128u * KG * sm.rl[g][n.slot][lw + RP * j];
                 }
                 abase += (fl & kPairAKMajor) ? 0u : 128u * KG;
                 bbase += (fl & kPairOffArith) ? 0u : bstep;
@@ -287,15 +280,15 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
         };
         // Element e of the thread (rows of A, then columns of B): its load,
         // and its way into an LDS buffer (A scaled).
-        constexpr int E = FM + 4;
-        double sc[FM];
+        constexpr int E = PA + 4;
+        double sc[PA];
         auto load = [&](int e) {
-            if(e < FM) v[e] = *(gdouble *)(qa + ao[e < FM ? e : 0]);
-            else v[e] = *(gdouble *)(qb + bo[e < FM ? 0 : e - FM]);
+            if(e < PA) v[e] = *(gdouble *)(qa + ao[e < PA ? e : 0]);
+            else v[e] = *(gdouble *)(qb + bo[e < PA ? 0 : e - PA]);
         };
         auto put = [&](int e, double *wa, double *wb) {
-            if(e < FM) wa[16 * e * kTileRow] = v[e] * sc[e < FM ? e : 0];
-            else wb[16 * e * kTileRow] = v[e];
+            if(e < PA) wa[RP * e * kTileRow] = v[e] * sc[e < PA ? e : 0];
+            else wb[RP * (e - PA) * kTileRow] = v[e];
         };
         // Past a pair's extent both operands are zero, and everywhere in a
         // chunk past the group's last one.
@@ -303,7 +296,7 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
             const bool la = n.valid && 16 * n.c + ((fl & kPairAKMajor) ? hi : lo) < n.k;
             const bool lb = n.valid && 16 * n.c + ((fl & kPairBNFast) ? hi : lo) < n.k;
 #pragma unroll
-            for(int e = 0; e < E; e++) v[e] = (e < FM ? la : lb) ? v[e] : 0.0;
+            for(int e = 0; e < E; e++) v[e] = (e < PA ? la : lb) ? v[e] : 0.0;
         };
 
         // One step: products of the staged chunk; between them, the loads of
@@ -318,10 +311,10 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
             row_src ar; uint32_t cq = 0;
             seek(n1);
             const bool akm = (fl & kPairAKMajor) != 0, bnf = (fl & kPairBNFast) != 0;
-            const double *rd = &sm.rd[g][n1.slot][akm ? lo : hr];
-            double *wa = base + wtog + (akm ? a1 : a0), *wb = base + wtog + (bnf ? a1 : a0);
+            const double *rd = &sm.rd[g][n1.slot][akm ? lw : hr];
+            double *wa = base + wtog + (akm ? a1 : a0), *wb = base + wtog + S::RA * kTileRow + (bnf ? a1 : a0);
             double2_t b0, b1, x0, x1, y0, y1;
-            const double *bp = base + rtog + (BM + 16 * wave + lr) * kTileRow + 4 * lg;
+            const double *bp = base + rtog + (S::RA + 16 * wave + lr) * kTileRow + 4 * lg;
             const double *ap = base + rtog + lr * kTileRow + 4 * lg;
             if constexpr(mult) {
                 b0 = *(const double2_t *)bp; b1 = *(const double2_t *)(bp + 2);
@@ -352,7 +345,7 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
                 }
             }
 #pragma unroll
-            for(int e = 0; e < FM; e++) sc[e] = rd[16 * e];
+            for(int e = 0; e < PA; e++) sc[e] = rd[RP * e];
             if(edge) clip(n1);
 #pragma unroll
             for(int h = H; h < 2 * FM; h++) {
@@ -395,7 +388,7 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
 #pragma unroll
             for(int v = 0; v < 4; v++) {
                 const uint32_t row = 16 * i + lg + 4 * v, col = 16 * wave + lr;
-                if(tp.part) tp.part[((i * 4 + v) * 4 + wave) * 64 + lane] = acc[i][v];
+                if(tp.part) tp.part[((i * 4 + v) * NW + wave) * 64 + lane] = acc[i][v];
                 else if(row < mrem && col < nrem) src.write(m0 + row, n0 + col, acc[i][v]);
             }
         return;
@@ -406,13 +399,13 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
     for(int i = 0; i < FM; i++)
 #pragma unroll
         for(int v = 0; v < 4; v++)
-            red[g * BM * BN + ((i * 4 + v) * 4 + wave) * 64 + lane] = acc[i][v];
+            red[g * BM * BN + ((i * 4 + v) * NW + wave) * 64 + lane] = acc[i][v];
     __syncthreads();
-    for(int e = threadIdx.x; e < BM * BN; e += 256 * KG) {
+    for(int e = threadIdx.x; e < BM * BN; e += GT * KG) {
         double x = red[e];
 #pragma unroll
         for(int q = 1; q < KG; q++) x += red[q * BM * BN + e];
-        const int l = e & 63, w = (e >> 6) & 3, v = (e >> 8) & 3, i = e >> 10;
+        const int l = e & 63, w = (e >> 6) % NW, v = (e / GT) & 3, i = e / (4 * GT);
         const uint32_t row = 16 * i + (l >> 4) + 4 * v, col = 16 * w + (l & 15);
         if(tp.part) tp.part[e] = x;
         else if(row < mrem && col < nrem) src.write(m0 + row, n0 + col, x);
@@ -422,10 +415,10 @@ __device__ __forceinline__ void tile_body(const SRC &src, const tile_part &tp, t
 //! A tile of height up to 16 FM: the loop compiled for its number of 16-row
 //! fragments (a condition per fragment inside one loop would make the
 //! compiler copy the accumulators).
-template<int FM, int KG, int FA, class SRC>
-__device__ __forceinline__ void tile_height(const SRC &src, const tile_part &tp, char *smem) {
-    if(FA == 1 || tp.mrem > 16 * (FA - 1)) tile_body<FA, KG>(src, tp, *(tile_smem<FA, KG> *)smem);
-    else tile_height<FM, KG, (FA > 1 ? FA - 1 : 1)>(src, tp, smem);
+template<int FM, int KG, int NW, int FA>
+__device__ __forceinline__ void tile_height(const stack_rows &src, const tile_part &tp, char *smem) {
+    if(FA == 1 || tp.mrem > 16 * (FA - 1)) tile_body<FA, KG, NW>(src, tp, *(tile_smem<FA, KG, NW> *)smem);
+    else tile_height<FM, KG, NW, (FA > 1 ? FA - 1 : 1)>(src, tp, smem);
 }
 
 //! Workgroups that share a CU get different priorities, the same on its four
@@ -440,11 +433,11 @@ __device__ __forceinline__ void rank_workgroup() {
     }
 }
 
-template<int FM, int KG, int OCC>
-__global__ void __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(OCC)))
+template<int FM, int KG, int OCC, int NW>
+__global__ void __launch_bounds__(64 * NW * KG) __attribute__((amdgpu_waves_per_eu(OCC)))
 gemm_tile_kernel(const tile_stack *__restrict__ stacks, const tile_item *__restrict__ items,
     double *__restrict__ parts) {
-    __shared__ __attribute__((aligned(16))) char smem[sizeof(tile_smem<FM, KG>)];
+    __shared__ __attribute__((aligned(16))) char smem[sizeof(tile_smem<FM, KG, NW>)];
     const tile_item it = items[blockIdx.x];
     cstack *st = (cstack *)(uintptr_t)(stacks + it.stack);
     if(st->rows == 0) return;                    // padding tile (whole workgroup)
@@ -456,32 +449,32 @@ gemm_tile_kernel(const tile_stack *__restrict__ stacks, const tile_item *__restr
     src.astride = st->astride;
     tile_part tp;
     tp.m0 = uint32_t(it.tm) * (16 * FM);
-    tp.n0 = uint32_t(it.tn) * 64;
+    tp.n0 = uint32_t(it.tn) * (16 * NW);
     tp.mrem = st->rows - tp.m0;
     tp.nrem = st->n - tp.n0;
     tp.p = it.p; tp.c = it.c; tp.count = it.count;
-    tp.part = it.part < 0 ? (gout *)0 : (gout *)(uintptr_t)parts + size_t(it.part) * (1024 * FM);
-    tile_height<FM, KG, FM>(src, tp, smem);
+    tp.part = it.part < 0 ? (gout *)0 : (gout *)(uintptr_t)parts + size_t(it.part) * (256 * NW * FM);
+    tile_height<FM, KG, NW, FM>(src, tp, smem);
 }
 
 //! C of the tiles whose chunks were cut into parts: their partial sums added
 //! in the order of the parts.
 __global__ void __launch_bounds__(256)
 tile_sum_kernel(const tile_stack *__restrict__ stacks, const tile_item *__restrict__ items,
-    const double *__restrict__ parts, uint32_t fm) {
+    const double *__restrict__ parts, uint32_t fm, uint32_t lnw) {
     const tile_item it = items[blockIdx.x];      // part: the first part's place, count: parts
     cstack *st = (cstack *)(uintptr_t)(stacks + it.stack);
-    const uint32_t m0 = uint32_t(it.tm) * (16 * fm), n0 = uint32_t(it.tn) * 64;
+    const uint32_t m0 = uint32_t(it.tm) * (16 * fm), n0 = uint32_t(it.tn) * (16u << lnw);
     const uint32_t mrem = st->rows - m0, nrem = st->n - n0;
     stack_rows src;
     src.crow = (gcrow *)(uintptr_t)st->crow;
     const uint32_t e = blockIdx.y * 256 + threadIdx.x;
-    const uint32_t l = e & 63, w = (e >> 6) & 3, v = (e >> 8) & 3, i = e >> 10;
+    const uint32_t l = e & 63, w = (e >> 6) & ((1u << lnw) - 1), v = (e >> (6 + lnw)) & 3, i = e >> (8 + lnw);
     const uint32_t row = 16 * i + (l >> 4) + 4 * v, col = 16 * w + (l & 15);
     if(row >= mrem || col >= nrem) return;
-    gdouble *p = (gdouble *)(uintptr_t)parts + size_t(it.part) * (1024 * fm) + e;
+    gdouble *p = (gdouble *)(uintptr_t)parts + size_t(it.part) * (256u * fm << lnw) + e;
     double x = p[0];
-    for(uint32_t q = 1; q < it.count; q++) x += p[size_t(q) * (1024 * fm)];
+    for(uint32_t q = 1; q < it.count; q++) x += p[size_t(q) * (256u * fm << lnw)];
     src.write(m0 + row, n0 + col, x);
 }
 
@@ -490,25 +483,26 @@ hipError_t launch_tile_sum(int cfg, const tile_stack *st, const tile_item *items
     if(n == 0) return hipSuccess;
     uint32_t bm, bn;
     tile_shape(cfg, bm, bn);
-    hipLaunchKernelGGL(tile_sum_kernel, dim3(n, bm / 4), dim3(256), 0, s, st, items, parts, bm / 16);
+    hipLaunchKernelGGL(tile_sum_kernel, dim3(n, bm * bn / 256), dim3(256), 0, s, st, items, parts, bm / 16,
+        bn == 128 ? 3u : 2u);
     return hipGetLastError();
 }
 
 hipError_t launch_gemm_tile(int cfg, const tile_stack *st, const tile_item *items,
     uint32_t nitems, double *parts, hipStream_t s) {
     if(nitems == 0) return hipSuccess;
-#define LT_TILE(FM, KG, OCC) \
-    hipLaunchKernelGGL((gemm_tile_kernel<FM, KG, OCC>), dim3(nitems), dim3(256 * KG), 0, s, st, items, parts)
+#define LT_TILE(FM, KG, OCC, NW) \
+    hipLaunchKernelGGL((gemm_tile_kernel<FM, KG, OCC, NW>), dim3(nitems), dim3(64 * NW * KG), 0, s, st, items, parts)
     switch(cfg) {
-    case WG_16x64_G4: LT_TILE(1, 4, 4); break;
-    case WG_32x64_G4: LT_TILE(2, 4, 4); break;
-    case WG_32x64_G2: LT_TILE(2, 2, 4); break;
-    case WG_48x64_G4: LT_TILE(3, 4, 4); break;
-    case WG_64x64_G4: LT_TILE(4, 4, 4); break;
-    case WG_64x64_G1: LT_TILE(4, 1, 4); break;
-    case WG_80x64_G2: LT_TILE(5, 2, 2); break;
-    case WG_96x64_G1: LT_TILE(6, 1, 3); break;
-    case WG_112x64_G1: LT_TILE(7, 1, 2); break;
+    case WG_16x64_G4: LT_TILE(1, 4, 4, 4); break;
+    case WG_32x64_G4: LT_TILE(2, 4, 4, 4); break;
+    case WG_96x128_G1: LT_TILE(6, 1, 4, 8); break;
+    case WG_48x64_G4: LT_TILE(3, 4, 4, 4); break;
+    case WG_64x64_G4: LT_TILE(4, 4, 4, 4); break;
+    case WG_64x64_G1: LT_TILE(4, 1, 4, 4); break;
+    case WG_80x64_G2: LT_TILE(5, 2, 2, 4); break;
+    case WG_96x64_G1: LT_TILE(6, 1, 3, 4); break;
+    case WG_112x64_G1: LT_TILE(7, 1, 2, 4); break;
     default: return hipErrorInvalidValue;
     }
 #undef LT_TILE

@@ -1385,6 +1385,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
             return ntiles >= kItems ? 1u : std::max(1u, uint32_t(double(t.nchunk) / len + 0.5));
         };
         typedef std::pair<double, dev::tile_item> unit;
+        std::vector<uint32_t> part_of;            // of each unit: its place along k
         auto add_tile = [&](size_t stack, const dev::tile_stack &t, uint32_t i, uint32_t j, uint32_t pair0,
             std::vector<unit> &units, std::vector<dev::tile_item> &sums, size_t &nparts) {
             const uint32_t np = cut(t), fa = (std::min(bm, t.rows - i * bm) + 15) / 16;
@@ -1402,6 +1403,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
                 it.count = end - at;
                 if(np > 1) it.part = (int32_t)nparts++;
                 units.push_back(std::make_pair(double(it.count) * fa, it));
+                part_of.push_back(q);
                 for(; at < end; ) {
                     const uint32_t left = (pl.spairs[pair0 + it.p].k + 15) / 16 - it.c;
                     if(end - at < left) { it.c += end - at; at = end; }
@@ -1411,49 +1413,55 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         };
         auto longer = [](const unit &x, const unit &y) { return x.first > y.first; };
         std::vector<unit> units;
-        std::vector<double> scost(ns, 0.0);
         pl.tsums.clear();
         pl.n_parts = 0;
         for(size_t i = 0; i < ns; i++) {
             uint32_t tm, tn;
             tiles_of(pl.tstacks[i], tm, tn);
-            const size_t u0 = units.size();
             for(uint32_t a = 0; a < tm; a++) for(uint32_t b = 0; b < tn; b++)
                 add_tile(i, pl.tstacks[i], a, b, pl.stacks[i].pair_begin, units, pl.tsums, pl.n_parts);
-            for(size_t u = u0; u < units.size(); u++) scost[i] += units[u].first;
         }
-        std::stable_sort(units.begin(), units.end(), longer);
         pl.titems.clear();
         if(order == 0) {
+            std::stable_sort(units.begin(), units.end(), longer);
             for(size_t i = 0; i < units.size(); i++) pl.titems.push_back(units[i].second);
         } else {
-            // XCD-aware: stacks to XCDs longest first onto the least loaded,
-            // each XCD's items longest first at positions x, x + nx, ...; the
+            // XCD-aware: the items part by part, in strips of kStrip columns of
+            // tiles, cut into one piece of equal work per XCD, so that the
+            // items an XCD's L2 serves at a time share rows of A and columns
+            // of B (o = 29, v = 131: 25 instead of 45 M lines from beyond the
+            // L2 caches; o = 48, v = 240 in uneven blocks 61.4 to 59.0 ms);
+            // each piece longest first at positions x, x + nx, ...; the
             // padding items name the empty stack
-            std::vector<size_t> so(ns);
-            std::iota(so.begin(), so.end(), size_t(0));
-            std::stable_sort(so.begin(), so.end(), [&](size_t x, size_t y) { return scost[x] > scost[y]; });
-            std::vector<double> load(nx, 0.0);
-            std::vector<int> sx(ns, 0);
-            for(size_t i = 0; i < ns; i++) {
-                const int x = int(std::min_element(load.begin(), load.end()) - load.begin());
-                sx[so[i]] = x;
-                load[x] += scost[so[i]];
-            }
-            std::vector<std::vector<dev::tile_item> > q(nx);
-            size_t qmax = 0;
+            const uint32_t kStrip = 8;
+            std::vector<std::pair<std::array<uint32_t, 5>, size_t> > seq(units.size());
+            double total = 0.0;
             for(size_t i = 0; i < units.size(); i++) {
-                std::vector<dev::tile_item> &qq = q[sx[units[i].second.stack]];
-                qq.push_back(units[i].second);
-                qmax = std::max(qmax, qq.size());
+                const dev::tile_item &t = units[i].second;
+                seq[i].first = {{ part_of[i], t.stack, t.tn / kStrip, t.tm, t.tn }};
+                seq[i].second = i;
+                total += units[i].first;
             }
+            std::sort(seq.begin(), seq.end());
+            std::vector<std::vector<unit> > q(nx);
+            double sum = 0.0;
+            for(size_t i = 0; i < seq.size(); i++) {
+                const unit &u = units[seq[i].second];
+                const int x = total > 0.0 ? std::min(nx - 1, int((sum + 0.5 * u.first) * nx / total)) : 0;
+                q[x].push_back(u);
+                sum += u.first;
+            }
+            size_t qmax = 0;
+            for(int x = 0; x < nx; x++) qmax = std::max(qmax, q[x].size());
             dev::tile_item empty;
             std::memset(&empty, 0, sizeof(empty));
             empty.stack = (uint32_t)ns;
             empty.part = -1;
             pl.titems.assign(qmax * nx, empty);
-            for(int x = 0; x < nx; x++)
-                for(size_t l = 0; l < q[x].size(); l++) pl.titems[l * nx + x] = q[x][l];
+            for(int x = 0; x < nx; x++) {
+                std::stable_sort(q[x].begin(), q[x].end(), longer);
+                for(size_t l = 0; l < q[x].size(); l++) pl.titems[l * nx + x] = q[x][l].second;
+            }
         }
         // per C block, in block order
         pl.bitems.clear(); pl.bsums.clear();
@@ -1884,6 +1892,7 @@ void btod_contract2::build_ozaki(int slices) {
             }
             std::vector<size_t> qp(nx, 0);
             tl[k].reserve(total);
+            const int per_wg = k == dev::OZ_TILE_48x64 ? 1 : 4;
             for(size_t w = 0; tl[k].size() < total; w++) {
                 for(int j = 0; j < per_wg && tl[k].size() < total; j++) {
                     size_t x = w % nx;
@@ -1892,7 +1901,6 @@ void btod_contract2::build_ozaki(int slices) {
                         for(size_t y = 0; y < nx; y++)
                             if(q[y].size() - qp[y] > left) { left = q[y].size() - qp[y]; x = y; }
                     }
-            const int per_wg = k == dev::OZ_TILE_48x64 ? 1 : 4;
                     tl[k].push_back(q[x][qp[x]++]);
                 }
             }
