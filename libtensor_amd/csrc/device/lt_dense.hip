@@ -257,6 +257,8 @@ hipError_t launch_gemm_dense(int cfg, const dense_args &a, uint32_t nparts, doub
         hipLaunchKernelGGL((gemm_dense_kernel<2, 4, 4>), grid, dim3(1024), 0, s, a, ntn, parts); break;
     case DENSE_64x64_G1:
         hipLaunchKernelGGL((gemm_dense_kernel<4, 1, 4>), grid, dim3(256), 0, s, a, ntn, parts); break;
+    case DENSE_64x64_G2:
+        hipLaunchKernelGGL((gemm_dense_kernel<4, 2, 4>), grid, dim3(512), 0, s, a, ntn, parts); break;
     default: return hipErrorInvalidValue;
     }
     hipError_t e = hipGetLastError();

@@ -244,7 +244,7 @@ struct dense_args {
     uint32_t rows_fast;               //!< bit 0 (1): A (B) is contiguous along m (n), else along k
 };
 //! Tile configurations of the dense kernel.
-enum dense_cfg { DENSE_16x64_G4 = 0, DENSE_32x64_G4 = 1, DENSE_64x64_G1 = 2 };
+enum dense_cfg { DENSE_16x64_G4 = 0, DENSE_32x64_G4 = 1, DENSE_64x64_G1 = 2, DENSE_64x64_G2 = 3 };
 void dense_tile_shape(int cfg, uint32_t &bm, uint32_t &bn);
 //! nparts > 1: the k range in that many parts, whose partial sums go through
 //! `parts` (tiles x nparts x bm x bn doubles).
@@ -334,7 +334,7 @@ hipError_t launch_dot(const perm_desc *descs, const uint32_t *chunk_desc,
 //! points (one per GPU, held until the process ends).
 static const size_t kNoallocScratchBytes = size_t(32) << 20;
 //! Behind it, room for the partial sums of a contraction cut along k.
-static const size_t kNoallocPartBytes = size_t(2) << 20;
+static const size_t kNoallocPartBytes = size_t(4) << 20;
 static const int kMaxDevices = 64;
 //! Device address of that region on `device`, which must be the current
 //! device on the first call for it (resolved once, then cached).

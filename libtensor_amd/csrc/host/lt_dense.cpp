@@ -26,7 +26,7 @@ const size_t kScatterBytes = size_t(32) << 20;
 //! Workgroups a contraction is cut into (tiles, or parts of tiles) at most
 //! when its tiles alone leave CUs idle.
 const size_t kSplitGroups = 256;
-static_assert(kSplitGroups * 1024 * sizeof(double) <= dev::kNoallocPartBytes,
+static_assert(kSplitGroups * 2048 * sizeof(double) <= dev::kNoallocPartBytes,
     "partial sums of a split contraction in the scratch region");
 
 //! One dimension of an axis: its positions in the two tensors it belongs to.
@@ -276,22 +276,25 @@ void prepare(const contraction2 &contr, dims_t da, const double *a, dims_t db, c
     j.g.zero = zero ? 1 : 0;
     j.g.rows_fast = (arf ? 1 : 0) | (brf ? 2 : 0);
 
-    // Tiles: 64 x 64 where they fill the CUs, 32 x 64 with the k range in
-    // four groups of waves where those come to half the CUs, else 16 x 64
-    // tiles cut along k, 16 chunks of k and more to a part.
+    // Tiles: 64 x 64 where they keep the CUs busy, the k range in two groups
+    // of waves below 1.5 to a CU; 32 x 64 in four groups from half the CUs on,
+    // else 16 x 64 in four, both cut along k into parts (of 16 chunks of k and
+    // more) that come to a workgroup per CU.  us a call, with each shape in
+    // this order: 2000 x 1500 x 600 86, 91, 130, 184; 1000 x 1000 x 500 47,
+    // 43, 52, 65; 675 x 675 x 675 54, 49, 40, 48; 500 x 500 x 2000 115, 98, 50
+    // (68 uncut), 56; 300 x 300 x 300 34, 33, 27, 23; 128 x 128 x 4000 28 with
+    // the last cut, 79 uncut.
     const size_t mm = j.g.m.ext, nn = j.g.n.ext, nch = (size_t(j.g.k.ext) + 15) / 16;
     const size_t tn = (nn + 63) / 64;
     j.nparts = 1;
-    if((mm + 63) / 64 * tn >= 384) j.cfg = dev::DENSE_64x64_G1;
-    else if((mm + 31) / 32 * tn >= 128) j.cfg = dev::DENSE_32x64_G4;
-    else {
-        j.cfg = dev::DENSE_16x64_G4;
-        const size_t t = (mm + 15) / 16 * tn;
-        if(t < kSplitGroups)
-            j.nparts = (uint32_t)std::max<size_t>(1, std::min(kSplitGroups / t, nch / 16));
-    }
+    const size_t t64 = (mm + 63) / 64 * tn;
+    j.cfg = t64 >= 384 ? dev::DENSE_64x64_G1 : t64 >= 200 ? dev::DENSE_64x64_G2 :
+        (mm + 31) / 32 * tn >= 128 ? dev::DENSE_32x64_G4 : dev::DENSE_16x64_G4;
     uint32_t bm = 0, bn = 0;
     dev::dense_tile_shape(j.cfg, bm, bn);
+    const size_t t = (mm + bm - 1) / bm * tn;
+    if(bm < 64 && t < kSplitGroups)
+        j.nparts = (uint32_t)std::max<size_t>(1, std::min(kSplitGroups / t, nch / 16));
     j.part_bytes = j.nparts == 1 ? 0 : (mm + bm - 1) / bm * tn * j.nparts * bm * bn * sizeof(double);
 }
 
