@@ -45,9 +45,14 @@ struct perm_desc {
     fastdiv tdp, tdq;                 //!< extents of tile_p and n - 1
 };
 //! Tile side: 64 where both extents are beyond 32 (rows of 512 bytes:
-//! 37 x 61 x 83 x 91 to 83 x 37 x 91 x 61 in 63 instead of 71 us), else 32.
-static const uint32_t kPermTile = 32, kPermTileMax = 64;
+//! 37 x 61 x 83 x 91 to 83 x 37 x 91 x 61 in 63 instead of 71 us), else 32;
+//! also 32 below kPermTileMin elements, where a launch has too few tiles.
+static const uint32_t kPermTile = 32, kPermTileMax = 64, kPermTileMin = 1u << 18;
 static const uint32_t kPermTileItem = 0x80000000u;
+//! Launches that write this many elements (32 MiB, what the L2 caches hold) and
+//! more write past the caches (`stream`: 37 x 61 x 83 x 91 transposed 62 to
+//! 53 us, 5.1 TB/s).
+static const uint32_t kPermStream = 1u << 22;
 
 //! One C block of a grouped GEMM: C(m x n, leading dimension ldc) is
 //! overwritten (zero != 0) or accumulated with the sum over its pairs.
@@ -216,7 +221,7 @@ hipError_t launch_gemm_stacked(int cfg, const stack_desc *st, const stack_pair *
 //! elements, or (chunk_desc[j] | kPermTileItem) and the destination index
 //! of a tile's corner for transposing descriptors.
 hipError_t launch_permute(const perm_desc *descs, const uint32_t *chunk_desc,
-    const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s);
+    const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s, bool stream = false);
 static const uint32_t kPermChunk = 2048;
 //! One permutation, its descriptor passed with the launch and its work items
 //! numbered by the grid.
@@ -326,8 +331,9 @@ hipError_t launch_fill(double *p, size_t n, double v, hipStream_t s);
 //! Workgroups of a dot product (each with its range of the chunks), so at most
 //! this many partial sums.
 static const uint32_t kDotGroups = 2048;
+//! tiles: some work items are tiles of transposing descriptors.
 hipError_t launch_dot(const perm_desc *descs, const uint32_t *chunk_desc,
-    const uint32_t *chunk_off, uint32_t nchunks, double *partials,
+    const uint32_t *chunk_off, uint32_t nchunks, bool tiles, double *partials,
     double *out, hipStream_t s);
 
 //! Size of the fixed device scratch region of the no-allocation entry

@@ -18,6 +18,7 @@ namespace lta {
 namespace dev {
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
+typedef double double2_t __attribute__((ext_vector_type(2)));
 
 fastdiv make_fastdiv(uint32_t d) {
     fastdiv f;
@@ -75,6 +76,15 @@ __device__ __forceinline__ uint32_t src_offset(const perm_desc &d, uint32_t e) {
     return off;
 }
 
+//! Work item of workgroup b of n: workgroups go to the 8 XCDs in turn, and each
+//! XCD takes a contiguous piece of the items, so that the cache lines that
+//! neighbouring items share meet in one L2 cache (two-term sum and scalar
+//! product of 26 M elements: 297 to 293 us).
+__device__ __forceinline__ uint32_t xcd_item(uint32_t b, uint32_t n) {
+    const uint32_t x = b & 7, q = n >> 3, r = n & 7;
+    return x * q + min(x, r) + (b >> 3);
+}
+
 //! alpha v + beta w with one rounding of beta w and one of the sum.
 __device__ __forceinline__ double perm_sum(double alpha, double v, double beta, double w) {
 #pragma clang fp contract(off)
@@ -82,11 +92,18 @@ __device__ __forceinline__ double perm_sum(double alpha, double v, double beta, 
     return __builtin_fma(alpha, v, t);
 }
 
+//! Element e of the destination (NT: past the caches, perm_desc::stream).
+template<bool NT>
+__device__ __forceinline__ void perm_store(const perm_desc &d, uint32_t e, double x) {
+    if constexpr(NT) __builtin_nontemporal_store(x, d.dst + e);
+    else d.dst[e] = x;
+}
+
 //! One tile of S x S over destination dimensions (p, q = n - 1): the source is
 //! contiguous along p, the destination along q (extents and strides from
 //! dedicated fields: indexing the descriptor's arrays with a runtime dimension
 //! would put it in scratch memory).
-template<int S>
+template<int S, bool NT>
 __device__ __forceinline__ void permute_tile(const perm_desc &d, uint32_t base, double *tile) {
     constexpr int RW = 256 / S;          // rows at a time
     const uint32_t dq = d.tdq.d, dp = d.tdp.d;
@@ -96,31 +113,41 @@ __device__ __forceinline__ void permute_tile(const perm_desc &d, uint32_t base, 
     const uint32_t np = min(uint32_t(S), dp - p0), nq = min(uint32_t(S), dq - q0);
     const uint32_t s0 = src_offset(d, base), sq = d.tsq, dps = d.dps.d;
     const uint32_t ti = threadIdx.x % S, tj = threadIdx.x / S;
-    double w[S / RW];
+    constexpr int R = S / RW;
+    double w[R];
+    // a tile whose rows adjoin in memory is moved as one run (no idle lanes at
+    // short rows: 158 to 147 us for a two-term sum of 26 M elements)
+    const uint32_t nn = np * nq;
+    const bool ls = sq == np, ld = dps == nq;
 #pragma unroll
-    for(int r = 0; r < S / RW; r++) {
-        const uint32_t iq = tj + RW * r;
-        if(ti < np && iq < nq) w[r] = d.src[s0 + ti + iq * sq];
+    for(int r = 0; r < R; r++) {
+        const uint32_t e = threadIdx.x + 256 * r, iq = tj + RW * r;
+        if(ls ? e < nn : ti < np && iq < nq) w[r] = d.src[s0 + (ls ? e : ti + iq * sq)];
     }
 #pragma unroll
-    for(int r = 0; r < S / RW; r++) {
-        const uint32_t iq = tj + RW * r;
-        if(ti < np && iq < nq) tile[iq * (S + 1) + ti] = w[r];
+    for(int r = 0; r < R; r++) {
+        const uint32_t e = threadIdx.x + 256 * r;
+        uint32_t iq = tj + RW * r, ip = ti;
+        if(ls) { iq = fdiv(e, d.tdp); ip = e - iq * dp; }
+        if(ls ? e < nn : ti < np && iq < nq) tile[iq * (S + 1) + ip] = w[r];
     }
     if(d.add) {
 #pragma unroll
-        for(int r = 0; r < S / RW; r++) {
-            const uint32_t ip = tj + RW * r;
-            if(ti < nq && ip < np) w[r] = d.add[base + ip * dps + ti];
+        for(int r = 0; r < R; r++) {
+            const uint32_t e = threadIdx.x + 256 * r, ip = tj + RW * r;
+            if(ld ? e < nn : ti < nq && ip < np) w[r] = d.add[base + (ld ? e : ip * dps + ti)];
         }
     }
     __syncthreads();
 #pragma unroll
-    for(int r = 0; r < S / RW; r++) {
-        const uint32_t ip = tj + RW * r;
-        if(ti < nq && ip < np) {
-            const double v = tile[ti * (S + 1) + ip];
-            d.dst[base + ip * dps + ti] = d.add ? perm_sum(d.alpha, v, d.beta, w[r]) : d.alpha * v;
+    for(int r = 0; r < R; r++) {
+        const uint32_t e = threadIdx.x + 256 * r;
+        uint32_t ip = tj + RW * r, iq = ti;
+        if(ld) { ip = fdiv(e, d.tdq); iq = e - ip * dq; }
+        if(ld ? e < nn : ti < nq && ip < np) {
+            const double v = tile[iq * (S + 1) + ip];
+            perm_store<NT>(d, base + (ld ? e : ip * dps + ti),
+                d.add ? perm_sum(d.alpha, v, d.beta, w[r]) : d.alpha * v);
         }
     }
 }
@@ -128,6 +155,7 @@ __device__ __forceinline__ void permute_tile(const perm_desc &d, uint32_t base, 
 //! Element-wise gather of one chunk: each thread owns kPermChunk / 256
 //! elements; all source offsets are computed and all loads issued before the
 //! first store, so every thread has that many gathers in flight.
+template<bool NT>
 __device__ __forceinline__ void permute_gather(const perm_desc &d, uint32_t base) {
     constexpr int E = kPermChunk / 256;
     const uint32_t end = min(base + kPermChunk, d.total);
@@ -143,36 +171,37 @@ __device__ __forceinline__ void permute_gather(const perm_desc &d, uint32_t base
 #pragma unroll
         for(int i = 0; i < E; i++) {
             const uint32_t e = base + threadIdx.x + 256u * i;
-            if(e < end) d.dst[e] = perm_sum(d.alpha, v[i], d.beta, w[i]);
+            if(e < end) perm_store<NT>(d, e, perm_sum(d.alpha, v[i], d.beta, w[i]));
         }
     } else {
 #pragma unroll
         for(int i = 0; i < E; i++) {
             const uint32_t e = base + threadIdx.x + 256u * i;
-            if(e < end) d.dst[e] = d.alpha * v[i];
+            if(e < end) perm_store<NT>(d, e, d.alpha * v[i]);
         }
     }
 }
 
+template<bool NT>
 __global__ void __launch_bounds__(256)
 permute_kernel(const perm_desc *__restrict__ descs,
     const uint32_t *__restrict__ chunk_desc,
     const uint32_t *__restrict__ chunk_off) {
 
     __shared__ double tile[kPermTileMax * (kPermTileMax + 1)];
-    const uint32_t ch = blockIdx.x;
+    const uint32_t ch = xcd_item(blockIdx.x, gridDim.x);
     const uint32_t cd = chunk_desc[ch];
     const perm_desc d = descs[cd & ~kPermTileItem];
     const uint32_t base = chunk_off[ch];
-    if(!(cd & kPermTileItem)) permute_gather(d, base);
-    else if(d.tile_s == kPermTileMax) permute_tile<kPermTileMax>(d, base, tile);
-    else permute_tile<kPermTile>(d, base, tile);
+    if(!(cd & kPermTileItem)) permute_gather<NT>(d, base);
+    else if(d.tile_s == kPermTileMax) permute_tile<kPermTileMax, NT>(d, base, tile);
+    else permute_tile<kPermTile, NT>(d, base, tile);
 }
 
 hipError_t launch_permute(const perm_desc *descs, const uint32_t *chunk_desc,
-    const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s) {
+    const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s, bool stream) {
     if(nchunks == 0) return hipSuccess;
-    hipLaunchKernelGGL(permute_kernel, dim3(nchunks), dim3(256), 0, s,
+    hipLaunchKernelGGL(stream ? permute_kernel<true> : permute_kernel<false>, dim3(nchunks), dim3(256), 0, s,
         descs, chunk_desc, chunk_off);
     return hipGetLastError();
 }
@@ -184,10 +213,10 @@ struct perm_items {
     uint32_t step[kPermMaxOrder];
 };
 
-template<int S>
+template<int S, bool NT>
 __global__ void __launch_bounds__(256) permute_tiles_kernel(perm_desc d, perm_items g) {
     __shared__ double tile[S * (S + 1)];
-    uint32_t x = blockIdx.x, base = 0;
+    uint32_t x = xcd_item(blockIdx.x, gridDim.x), base = 0;
 #pragma unroll
     for(int i = kPermMaxOrder - 1; i >= 0; i--) {
         if(i < (int)d.n) {
@@ -196,17 +225,19 @@ __global__ void __launch_bounds__(256) permute_tiles_kernel(perm_desc d, perm_it
             x = q;
         }
     }
-    permute_tile<S>(d, base, tile);
+    permute_tile<S, NT>(d, base, tile);
 }
 
+template<bool NT>
 __global__ void __launch_bounds__(256) permute_gather_kernel(perm_desc d) {
-    permute_gather(d, blockIdx.x * kPermChunk);
+    permute_gather<NT>(d, xcd_item(blockIdx.x, gridDim.x) * kPermChunk);
 }
 
 hipError_t launch_permute_one(const perm_desc &d, hipStream_t s) {
     if(d.total == 0) return hipSuccess;
+    const bool stream = d.total >= kPermStream;
     if(d.tile_p < 0) {
-        hipLaunchKernelGGL(permute_gather_kernel, dim3((d.total + kPermChunk - 1) / kPermChunk),
+        hipLaunchKernelGGL(stream ? permute_gather_kernel<true> : permute_gather_kernel<false>, dim3((d.total + kPermChunk - 1) / kPermChunk),
             dim3(256), 0, s, d);
         return hipGetLastError();
     }
@@ -221,10 +252,10 @@ hipError_t launch_permute_one(const perm_desc &d, hipStream_t s) {
         items *= cnt;
     }
     for(int i = int(d.n); i < kPermMaxOrder; i++) { g.it[i] = make_fastdiv(1); g.step[i] = 0; }
-    if(d.tile_s == kPermTileMax)
-        hipLaunchKernelGGL(permute_tiles_kernel<kPermTileMax>, dim3((uint32_t)items), dim3(256), 0, s, d, g);
-    else
-        hipLaunchKernelGGL(permute_tiles_kernel<kPermTile>, dim3((uint32_t)items), dim3(256), 0, s, d, g);
+    auto k = d.tile_s == kPermTileMax ?
+        (stream ? permute_tiles_kernel<kPermTileMax, true> : permute_tiles_kernel<kPermTileMax, false>) :
+        (stream ? permute_tiles_kernel<kPermTile, true> : permute_tiles_kernel<kPermTile, false>);
+    hipLaunchKernelGGL(k, dim3((uint32_t)items), dim3(256), 0, s, d, g);
     return hipGetLastError();
 }
 
@@ -235,7 +266,9 @@ hipError_t launch_permute_one(const perm_desc &d, hipStream_t s) {
 // of the chunks with all loads of a chunk issued before the first product, so
 // the sum of the partial results stays a few microseconds whatever the size
 // (one workgroup and one partial sum per chunk: 17 us of summing for 26 M
-// elements).  Transposed operands go through LDS tiles as in the permute.
+// elements).  Transposed operands go through LDS tiles as in the permute, in a
+// kernel of their own: the LDS of a tile halves the workgroups of a CU (26 M
+// elements in order: 89 us with it, 76 without, 5.5 TB/s).
 
 template<int S>
 __device__ __forceinline__ double dot_tile(const perm_desc &d, uint32_t base, double *tile) {
@@ -270,36 +303,51 @@ __device__ __forceinline__ double dot_tile(const perm_desc &d, uint32_t base, do
     return acc;
 }
 
+template<bool TILES>
 __global__ void __launch_bounds__(256)
 dot_kernel(const perm_desc *__restrict__ descs,
     const uint32_t *__restrict__ chunk_desc,
     const uint32_t *__restrict__ chunk_off, uint32_t nchunks, double *__restrict__ partials) {
 
     constexpr int E = kPermChunk / 256;
-    __shared__ double tile[kPermTileMax * (kPermTileMax + 1)];
-    const uint32_t c0 = uint32_t(uint64_t(nchunks) * blockIdx.x / gridDim.x);
-    const uint32_t c1 = uint32_t(uint64_t(nchunks) * (blockIdx.x + 1) / gridDim.x);
+    __shared__ double tile[TILES ? kPermTileMax * (kPermTileMax + 1) : 256];
+    const uint32_t wg = xcd_item(blockIdx.x, gridDim.x);
+    const uint32_t c0 = uint32_t(uint64_t(nchunks) * wg / gridDim.x);
+    const uint32_t c1 = uint32_t(uint64_t(nchunks) * (wg + 1) / gridDim.x);
     double sum = 0.0;
     for(uint32_t ch = c0; ch < c1; ch++) {
         const uint32_t cd = chunk_desc[ch];
         const perm_desc &d = descs[cd & ~kPermTileItem];
         const uint32_t base = chunk_off[ch];
         double acc = 0.0;
-        if(cd & kPermTileItem) {
+        if(TILES && (cd & kPermTileItem)) {
             acc = d.tile_s == kPermTileMax ? dot_tile<kPermTileMax>(d, base, tile) :
                 dot_tile<kPermTile>(d, base, tile);
         } else {
             const uint32_t end = min(base + kPermChunk, d.total);
             double v[E], w[E];
+            if(d.n == 1 && d.sstride[0] == 1 && end - base == kPermChunk &&
+                ((uintptr_t(d.src) | uintptr_t(d.dst)) & 15) == 0) {
+                const double2_t *x = (const double2_t *)(d.src + base), *y = (const double2_t *)(d.dst + base);
 #pragma unroll
-            for(int i = 0; i < E; i++) {
-                const uint32_t e = min(base + threadIdx.x + 256u * i, end - 1);
-                v[i] = d.src[src_offset(d, e)];
-                w[i] = d.dst[e];
+                for(int i = 0; i < E; i += 2) {
+                    const double2_t p = x[threadIdx.x + 128 * i], q = y[threadIdx.x + 128 * i];
+                    v[i] = p.x; v[i + 1] = p.y;
+                    w[i] = q.x; w[i + 1] = q.y;
+                }
+#pragma unroll
+                for(int i = 0; i < E; i++) acc += w[i] * v[i];
+            } else {
+#pragma unroll
+                for(int i = 0; i < E; i++) {
+                    const uint32_t e = min(base + threadIdx.x + 256u * i, end - 1);
+                    v[i] = d.src[src_offset(d, e)];
+                    w[i] = d.dst[e];
+                }
+#pragma unroll
+                for(int i = 0; i < E; i++)
+                    if(base + threadIdx.x + 256u * i < end) acc += w[i] * v[i];
             }
-#pragma unroll
-            for(int i = 0; i < E; i++)
-                if(base + threadIdx.x + 256u * i < end) acc += w[i] * v[i];
         }
         sum += acc * d.alpha;
     }
@@ -329,11 +377,11 @@ sum_kernel(const double *__restrict__ partials, uint32_t n, double *__restrict__
 }
 
 hipError_t launch_dot(const perm_desc *descs, const uint32_t *chunk_desc,
-    const uint32_t *chunk_off, uint32_t nchunks, double *partials,
+    const uint32_t *chunk_off, uint32_t nchunks, bool tiles, double *partials,
     double *out, hipStream_t s) {
     const uint32_t ng = nchunks < kDotGroups ? nchunks : kDotGroups;
     if(ng > 0) {
-        hipLaunchKernelGGL(dot_kernel, dim3(ng), dim3(256), 0, s,
+        hipLaunchKernelGGL(tiles ? dot_kernel<true> : dot_kernel<false>, dim3(ng), dim3(256), 0, s,
             descs, chunk_desc, chunk_off, nchunks, partials);
     }
     hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, s, partials, ng, out);
@@ -756,7 +804,6 @@ __device__ __forceinline__ int32_t koff_at(const stack_pair &sp, uint32_t k) {
     return 0;
 }
 
-typedef double double2_t __attribute__((ext_vector_type(2)));
 typedef const double2_t __attribute__((address_space(1))) gdouble2;
 
 // Operand loads of one chunk (16 k) of a stacked tile.  Lane (lr, lg) holds

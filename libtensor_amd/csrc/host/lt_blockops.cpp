@@ -20,7 +20,7 @@
 // overwrites, later ones accumulate), so no two descriptors of a launch
 // share a destination; a block's first two terms are one descriptor where
 // one of them needs no permutation: 24 instead of 40 bytes an element
-// (26 M elements, one term transposed: 240 to 158 us).
+// (26 M elements, one term transposed: 240 to 147 us).
 #include "lt_runtime.h"
 
 #include <algorithm>
@@ -165,6 +165,12 @@ std::shared_ptr<context::cached_launch> upload_launches(context &ctx,
     size_t sz = 0;
     for(size_t i = 0; i < lists.size(); i++) {
         if(lists[i].empty()) continue;
+        size_t total = 0;
+        bool tiles = false;
+        for(size_t k = 0; k < lists[i].size(); k++) {
+            total += lists[i][k].total;
+            tiles = tiles || lists[i][k].tile_p >= 0;
+        }
         std::vector<uint32_t> cd, co;
         make_chunks(lists[i], cd, co);
         if(cd.empty()) continue;
@@ -173,6 +179,8 @@ std::shared_ptr<context::cached_launch> upload_launches(context &ctx,
         g.o_cd = sz; sz = (sz + 4 * cd.size() + 255) & ~size_t(255);
         g.o_co = sz; sz = (sz + 4 * co.size() + 255) & ~size_t(255);
         g.nchunks = cd.size();
+        g.stream = total >= dev::kPermStream;
+        g.tiles = tiles;
         host.resize(sz, 0);
         std::memcpy(&host[g.o_d], lists[i].data(), lists[i].size() * sizeof(dev::perm_desc));
         std::memcpy(&host[g.o_cd], cd.data(), 4 * cd.size());
@@ -204,7 +212,7 @@ void run_launches(context &ctx, const context::cached_launch &l, double *ms) {
             const context::cached_launch::segment &g = l.segs[i];
             hip_check(dev::launch_permute((dev::perm_desc*)(base + g.o_d),
                 (uint32_t*)(base + g.o_cd), (uint32_t*)(base + g.o_co),
-                (uint32_t)g.nchunks, s), "permute");
+                (uint32_t)g.nchunks, s, g.stream), "permute");
         }
         if(ms) hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
         ctx.sync();
@@ -265,7 +273,7 @@ double run_dot(context &ctx, const context::cached_launch &l) {
     double r = 0.0;
     ctx.activate();
     hip_check(dev::launch_dot((dev::perm_desc*)(base + g.o_d), (uint32_t*)(base + g.o_cd),
-        (uint32_t*)(base + g.o_co), (uint32_t)g.nchunks, part, part + dev::kDotGroups,
+        (uint32_t*)(base + g.o_co), (uint32_t)g.nchunks, g.tiles, part, part + dev::kDotGroups,
         ctx.stream()), "dot");
     ctx.download(&r, part + dev::kDotGroups, sizeof(double));
     return r;

@@ -96,7 +96,8 @@ dev::perm_desc make_perm_desc(const double *src, const dims_t &dsrc,
             d.dps = dev::make_fastdiv((uint32_t)st);
             d.tdp = dev::make_fastdiv((uint32_t)fd[i]);
             d.tdq = dev::make_fastdiv((uint32_t)fd[nf - 1]);
-            if(std::min(fd[i], fd[nf - 1]) > dev::kPermTile) d.tile_s = dev::kPermTileMax;
+            if(std::min(fd[i], fd[nf - 1]) > dev::kPermTile && total >= dev::kPermTileMin)
+                d.tile_s = dev::kPermTileMax;
             break;
         }
     }

@@ -79,7 +79,7 @@ public:
     //! kLaunchCache entries, the oldest dropped first.
     struct cached_launch {
         //! one permute launch: descriptors at o_d, work items at o_cd / o_co
-        struct segment { size_t o_d, o_cd, o_co, nchunks; };
+        struct segment { size_t o_d, o_cd, o_co, nchunks; bool stream, tiles; };
         void *mem;
         std::vector<segment> segs;       //!< launched in order
         std::vector<size_t> touched;     //!< blocks the launches write
