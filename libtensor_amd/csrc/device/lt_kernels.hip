@@ -5,8 +5,8 @@
 //     C blocks: LDS-staged workgroup tiles (gemm_kernel), split-K tiles with
 //     operands loaded straight into MFMA fragments per C block
 //     (gemm_direct_kernel) or over stacks of C blocks that share their B
-//     operands (gemm_stacked_kernel, its varying-shape and LDS-staged
-//     variants).  Every workgroup owns one C tile and runs the whole list of
+//     operands (gemm_stacked_kernel and its varying-shape variant; the
+//     workgroup tiles over stacks are in lt_tile.hip).  Every workgroup owns one C tile and runs the whole list of
 //     that tile, the waves' partial tiles are added in LDS in wave order: each
 //     C element is written once with a fixed summation order (no atomics),
 //   * permuted dot product with a fixed-order two-pass reduction,
