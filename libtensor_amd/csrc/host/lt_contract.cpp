@@ -209,6 +209,16 @@ dev::perm_desc make_perm_desc_public(const double *src, const dims_t &dsrc,
     return make_perm_desc(src, dsrc, tr, dst, accumulate);
 }
 
+//! Work items of a workgroup-tiled launch and the tiles among them that run in
+//! parts of about part_len chunks (0: every tile runs whole); places: for
+//! their partial sums.
+struct tile_lists {
+    std::vector<dev::tile_item> items, sums;
+    double part_len;
+    size_t places;
+    tile_lists() : part_len(0.0), places(0) { }
+};
+
 //! Execution plan cached by the operation (valid while the structure of A,
 //! B and C does not change).
 struct contract_plan {
@@ -259,13 +269,16 @@ struct contract_plan {
     // block (per-block launches), each list ending with an empty one
     std::vector<dev::tile_stack> tstacks;
     dev::tile_stack *d_tstacks, *d_bstacks;
+    std::vector<uint32_t> block_pair0;        // first pair of a C block's stack
     // their work items and the tiles run in parts: of the grouped launch, and
-    // per C block (items of block b from block_item_begin[b] on)
-    std::vector<dev::tile_item> titems, tsums, bitems, bsums;
+    // per C block (items of block b from block_item_begin[b] on, made by the
+    // first per-block perform)
+    tile_lists tl;
     std::vector<uint32_t> block_item_begin, block_sum_begin;
     dev::tile_item *d_titems, *d_tsums, *d_bitems, *d_bsums;
-    size_t n_parts;                   // places for partial sums of the grouped launch
-    dev_lists parts;                  // partial sums (tiles)
+    dev_lists parts;                  // partial sums (tiles), from the first launch on
+    dev_lists blk_items, blk_parts;   // the same of the per-block launches
+    std::vector<double*> blk_base;    // per side stream used: its places
     // C blocks reading the same B operands (same order and layouts) share a
     // group; n_xcd: XCDs of the device
     std::vector<size_t> cb_group;
@@ -315,7 +328,7 @@ struct contract_plan {
         d_cb(0), d_pairs(0), d_tiles_sorted(0), d_tiles_block(0), scratch(0),
         scratch_elems(0), ctx(0), events(false), graph(0), gexec(0), graph_launches(0),
         d_stacks(0), d_spairs(0), d_arows(0), d_crows(0), d_stiles(0), d_vtiles(0),
-        d_tstacks(0), d_bstacks(0), d_titems(0), d_tsums(0), d_bitems(0), d_bsums(0), n_parts(0),
+        d_tstacks(0), d_bstacks(0), d_titems(0), d_tsums(0), d_bitems(0), d_bsums(0),
         n_groups(0), n_xcd(8),
         n_prep_st_chunks(0), d_prep_st(0), d_pst_cd(0), d_pst_co(0),
         oz_slices(0), oz_tile(0), oz_tile_set(-1), d_oz_split(0), d_oz_items(0), n_oz_items(0), d_oz_pairs(0),
@@ -334,6 +347,219 @@ struct contract_plan {
         if(events) for(int i = 0; i < 4; i++) hipEventDestroy(ev[i]);
     }
 };
+
+//! A work item and its cost (chunks times 16-row fragments).
+typedef std::pair<double, dev::tile_item> tile_unit;
+
+static bool longer(const tile_unit &x, const tile_unit &y) { return x.first > y.first; }
+
+static void tiles_of(const dev::tile_stack &t, uint32_t bm, uint32_t bn, uint32_t &tm, uint32_t &tn) {
+    tm = (t.rows + bm - 1) / bm;
+    tn = (t.n + bn - 1) / bn;
+    lt_require(tm < 65536 && tn < 65536, LT_ERR_PARAM, "stack too large");
+}
+
+//! Parts that a stack's tiles are cut into: by the plan's part length only, so
+//! that per-block launches and batches add the same sums in the same order.
+static uint32_t parts_of(const dev::tile_stack &t, double part_len) {
+    return part_len == 0.0 ? 1u : std::max(1u, uint32_t(double(t.nchunk) / part_len + 0.5));
+}
+
+//! The items of tile (i, j) of a stack (pairs from pair0 on), a part each;
+//! place: of each item, its part along k.  A tile in parts also goes to sums,
+//! its partial sums to the places from nparts on.
+static void add_tile(const contract_plan &pl, double part_len, size_t stack, const dev::tile_stack &t,
+    uint32_t bm, uint32_t i, uint32_t j, uint32_t pair0, std::vector<tile_unit> &units,
+    std::vector<uint32_t> &place, std::vector<dev::tile_item> &sums, size_t &nparts) {
+
+    const uint32_t np = parts_of(t, part_len), fa = (std::min(bm, t.rows - i * bm) + 15) / 16;
+    dev::tile_item it;
+    it.stack = (uint32_t)stack; it.tm = (uint16_t)i; it.tn = (uint16_t)j;
+    it.p = 0; it.c = 0; it.part = -1;
+    if(np > 1) {
+        dev::tile_item sm = it;
+        sm.part = (int32_t)nparts; sm.count = np;
+        sums.push_back(sm);
+    }
+    uint32_t at = 0;
+    for(uint32_t q = 0; q < np; q++) {
+        const uint32_t end = uint32_t(uint64_t(t.nchunk) * (q + 1) / np);
+        it.count = end - at;
+        if(np > 1) it.part = (int32_t)nparts++;
+        units.push_back(std::make_pair(double(it.count) * fa, it));
+        place.push_back(q);
+        for(; at < end; ) {
+            const uint32_t left = (pl.spairs[pair0 + it.p].k + 15) / 16 - it.c;
+            if(end - at < left) { it.c += end - at; at = end; }
+            else { at += left; it.p++; it.c = 0; }
+        }
+    }
+}
+
+//! Work items of a workgroup-tiled configuration's grouped launch.  Where the
+//! tiles of the whole list are fewer than keep the CUs evenly busy (kItems,
+//! four per CU), the chunk sequences are cut into parts of about equal length
+//! (at least kMinChunks, which pays for a part's sums going through memory):
+//! kItems + tiles / 2 parts at most.  cut false: no tile is cut.
+static void list_items(const contract_plan &pl, int k, int order, bool cut, tile_lists &tl) {
+    const uint32_t kItems = 1024, kMinChunks = 16;
+    uint32_t bm, bn;
+    dev::tile_shape(k, bm, bn);
+    const size_t ns = pl.stacks.size() - 1;
+    double chunks = 0.0, ntiles = 0.0;
+    for(size_t i = 0; i < ns; i++) {
+        uint32_t tm, tn;
+        tiles_of(pl.tstacks[i], bm, bn, tm, tn);
+        ntiles += double(tm) * tn;
+        chunks += double(tm) * tn * pl.tstacks[i].nchunk;
+    }
+    tl.part_len = cut && ntiles < kItems ? std::max(double(kMinChunks), chunks / kItems) : 0.0;
+    std::vector<tile_unit> units;
+    std::vector<uint32_t> place;
+    tl.sums.clear();
+    tl.places = 0;
+    for(size_t i = 0; i < ns; i++) {
+        uint32_t tm, tn;
+        tiles_of(pl.tstacks[i], bm, bn, tm, tn);
+        for(uint32_t a = 0; a < tm; a++) for(uint32_t b = 0; b < tn; b++)
+            add_tile(pl, tl.part_len, i, pl.tstacks[i], bm, a, b, pl.stacks[i].pair_begin, units, place,
+                tl.sums, tl.places);
+    }
+    tl.items.clear();
+    if(order == 0) {
+        std::stable_sort(units.begin(), units.end(), longer);
+        for(size_t i = 0; i < units.size(); i++) tl.items.push_back(units[i].second);
+    } else {
+        // XCD-aware: the items part by part, in strips of kStrip columns of
+        // tiles, cut into one piece of equal work per XCD, so that the
+        // items an XCD's L2 serves at a time share rows of A and columns
+        // of B (o = 29, v = 131: 25 instead of 45 M lines from beyond the
+        // L2 caches; o = 48, v = 240 in uneven blocks 61.4 to 59.0 ms);
+        // each piece longest first at positions x, x + nx, ...; the
+        // padding items name the empty stack
+        const uint32_t kStrip = 8;
+        const int nx = pl.n_xcd;
+        std::vector<std::pair<std::array<uint32_t, 5>, size_t> > seq(units.size());
+        double total = 0.0;
+        for(size_t i = 0; i < units.size(); i++) {
+            const dev::tile_item &t = units[i].second;
+            seq[i].first = {{ place[i], t.stack, t.tn / kStrip, t.tm, t.tn }};
+            seq[i].second = i;
+            total += units[i].first;
+        }
+        std::sort(seq.begin(), seq.end());
+        std::vector<std::vector<tile_unit> > q(nx);
+        double sum = 0.0;
+        for(size_t i = 0; i < seq.size(); i++) {
+            const tile_unit &u = units[seq[i].second];
+            const int x = total > 0.0 ? std::min(nx - 1, int((sum + 0.5 * u.first) * nx / total)) : 0;
+            q[x].push_back(u);
+            sum += u.first;
+        }
+        size_t qmax = 0;
+        for(int x = 0; x < nx; x++) qmax = std::max(qmax, q[x].size());
+        dev::tile_item empty;
+        std::memset(&empty, 0, sizeof(empty));
+        empty.stack = (uint32_t)ns;
+        empty.part = -1;
+        tl.items.assign(qmax * nx, empty);
+        for(int x = 0; x < nx; x++) {
+            std::stable_sort(q[x].begin(), q[x].end(), longer);
+            for(size_t l = 0; l < q[x].size(); l++) tl.items[l * nx + x] = q[x][l].second;
+        }
+    }
+}
+
+//! The lists of a plan's grouped launch, on the device.
+static void make_items(contract_plan &pl, int k, int order, bool cut = true) {
+    list_items(pl, k, order, cut, pl.tl);
+    const size_t ni = pl.tl.items.size() * sizeof(dev::tile_item), ns = pl.tl.sums.size() * sizeof(dev::tile_item);
+    const size_t o_sums = align256(ni);
+    std::vector<char> host(std::max<size_t>(256, o_sums + align256(ns)), 0);
+    if(ni) std::memcpy(&host[0], pl.tl.items.data(), ni);
+    if(ns) std::memcpy(&host[o_sums], pl.tl.sums.data(), ns);
+    pl.stk_tiles.at_least(*pl.ctx, host.size());
+    pl.ctx->upload_new(pl.stk_tiles.mem, host.data(), host.size());
+    pl.d_titems = (dev::tile_item*)pl.stk_tiles.mem;
+    pl.d_tsums = (dev::tile_item*)((char*)pl.stk_tiles.mem + o_sums);
+}
+
+//! Memory for the partial sums of the grouped launch, before its first one.
+//! Partial sums are no part of what a plan must fit: where there is no room
+//! for them, the tiles run whole.
+static void ensure_parts(contract_plan &pl) {
+    if(!dev::is_tile(pl.tile_cfg) || pl.tl.places == 0) return;
+    uint32_t bm, bn;
+    dev::tile_shape(pl.tile_cfg, bm, bn);
+    try {
+        pl.parts.at_least(*pl.ctx, pl.tl.places * bm * bn * sizeof(double));
+    } catch(const lt_error &e) {
+        if(e.code != LT_ERR_NOMEM) throw;
+        make_items(pl, pl.tile_cfg, 0, false);
+        pl.block_item_begin.clear();
+    }
+}
+
+//! Work items of the per-block launches, in block order, before the first of
+//! them.  The blocks that a side stream runs use the same places for their
+//! partial sums one after the other: a padded tile per part of every block at
+//! once would be many times the grouped launch's places where C blocks have
+//! few rows.  Without room for that, one stream runs all blocks in the grouped
+//! launch's places (a block has no more parts than its stack).
+static void ensure_block_items(contract_plan &pl) {
+    if(!dev::is_tile(pl.tile_cfg) || !pl.block_item_begin.empty()) return;
+    uint32_t bm, bn;
+    dev::tile_shape(pl.tile_cfg, bm, bn);
+    std::vector<tile_unit> items;
+    std::vector<dev::tile_item> sums;
+    std::vector<uint32_t> place, begin, sum_begin;
+    std::vector<size_t> need(context::kSideStreams, 0);
+    auto lists = [&]() {
+        items.clear(); sums.clear(); begin.clear(); sum_begin.clear();
+        need.assign(need.size(), 0);
+        for(size_t b = 0; b < pl.cblocks.size(); b++) {       // (the last one is empty)
+            begin.push_back((uint32_t)items.size());
+            sum_begin.push_back((uint32_t)sums.size());
+            const dev::tile_stack &t = pl.tstacks[pl.stacks.size() + b];
+            uint32_t tm, tn;
+            tiles_of(t, bm, bn, tm, tn);
+            size_t n = 0;
+            for(uint32_t i = 0; i < tm; i++) for(uint32_t j = 0; j < tn; j++)
+                add_tile(pl, pl.tl.part_len, b, t, bm, i, j, pl.block_pair0[b], items, place, sums, n);
+            size_t &x = need[b % need.size()];
+            x = std::max(x, n);
+        }
+        begin.push_back((uint32_t)items.size());
+        sum_begin.push_back((uint32_t)sums.size());
+    };
+    lists();
+    size_t places = 0;
+    for(size_t i = 0; i < need.size(); i++) places += need[i];
+    std::vector<double*> base(need.size(), (double*)0);
+    if(places) {
+        try {
+            double *p = (double*)pl.blk_parts.at_least(*pl.ctx, places * bm * bn * sizeof(double));
+            for(size_t i = 0; i < need.size(); p += need[i] * bm * bn, i++) base[i] = p;
+        } catch(const lt_error &e) {
+            if(e.code != LT_ERR_NOMEM) throw;
+            ensure_parts(pl);
+            lists();
+            base.assign(1, (double*)pl.parts.mem);
+        }
+    }
+    const size_t o_sums = align256(items.size() * sizeof(dev::tile_item));
+    std::vector<char> host(std::max<size_t>(256, o_sums + align256(sums.size() * sizeof(dev::tile_item))), 0);
+    for(size_t i = 0; i < items.size(); i++)
+        std::memcpy(&host[i * sizeof(dev::tile_item)], &items[i].second, sizeof(dev::tile_item));
+    if(!sums.empty()) std::memcpy(&host[o_sums], sums.data(), sums.size() * sizeof(dev::tile_item));
+    pl.blk_items.at_least(*pl.ctx, host.size());
+    pl.ctx->upload(pl.blk_items.mem, host.data(), host.size());
+    pl.d_bitems = (dev::tile_item*)pl.blk_items.mem;
+    pl.d_bsums = (dev::tile_item*)((char*)pl.blk_items.mem + o_sums);
+    pl.blk_base = base;
+    pl.block_sum_begin = sum_begin;
+    pl.block_item_begin = begin;
+}
 
 //! The grouped GEMM launch of configuration k over a tile list of its own
 //! (n tiles at d_list: the autotuner's sample of a large plan).
@@ -358,9 +584,9 @@ hipError_t launch_grouped(const contract_plan &pl, int k, hipStream_t s) {
             pl.d_vtiles, (uint32_t)pl.vtiles.size(), s);
     if(dev::is_tile(k)) {
         hipError_t e = dev::launch_gemm_tile(k, pl.d_tstacks, pl.d_titems,
-            (uint32_t)pl.titems.size(), (double*)pl.parts.mem, s);
+            (uint32_t)pl.tl.items.size(), (double*)pl.parts.mem, s);
         return e != hipSuccess ? e : dev::launch_tile_sum(k, pl.d_tstacks, pl.d_tsums,
-            (uint32_t)pl.tsums.size(), (double*)pl.parts.mem, s);
+            (uint32_t)pl.tl.sums.size(), (double*)pl.parts.mem, s);
     }
     if(dev::is_stacked(k))
         return dev::launch_gemm_stacked(k, pl.d_stacks, pl.d_spairs, pl.d_arows, pl.d_crows,
@@ -929,7 +1155,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         std::copy(ts.begin(), ts.end(), pair_tab.begin() + p0);
     }
     std::vector<std::vector<size_t> > stack_blocks;     // C blocks of a stack, in row order
-    std::vector<uint32_t> block_pair0(pl.cblocks.size() + 1, 0);    // first pair of a C block's stack
+    pl.block_pair0.assign(pl.cblocks.size() + 1, 0);
     {
         std::map<std::pair<uint32_t, std::vector<bkey_t> >, std::vector<size_t> > groups;
         std::vector<std::pair<uint32_t, std::vector<bkey_t> > > order;
@@ -1075,7 +1301,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
             pl.stacks.push_back(sd);
             pl.stack_ksum.push_back(ks);
             stack_blocks.push_back(bl);
-            for(size_t q = 0; q < bl.size(); q++) block_pair0[bl[q]] = sd.pair_begin;
+            for(size_t q = 0; q < bl.size(); q++) pl.block_pair0[bl[q]] = sd.pair_begin;
         }
         dev::stack_desc z;
         std::memset(&z, 0, sizeof(z));
@@ -1358,144 +1584,6 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     pl.d_pst_cd = (uint32_t*)(base + o_scd);
     pl.d_pst_co = (uint32_t*)(base + o_sco);
 
-    // Work items of a workgroup-tiled configuration.  Where the tiles of the
-    // whole list are fewer than keep the CUs evenly busy (kItems, four per
-    // CU), the chunk sequences are cut into parts of about equal length (at
-    // least kMinChunks, which pays for a part's sums going through memory);
-    // how a stack is cut depends on the plan only, so per-block launches and
-    // batches add the same sums in the same order.
-    auto make_items = [&](int k, int order) {
-        const uint32_t kItems = 1024, kMinChunks = 16;
-        uint32_t bm, bn;
-        dev::tile_shape(k, bm, bn);
-        const size_t ns = pl.stacks.size() - 1, nb = pl.cblocks.size();
-        auto tiles_of = [&](const dev::tile_stack &t, uint32_t &tm, uint32_t &tn) {
-            tm = (t.rows + bm - 1) / bm;
-            tn = (t.n + bn - 1) / bn;
-            lt_require(tm < 65536 && tn < 65536, LT_ERR_PARAM, "stack too large");
-        };
-        double chunks = 0.0, ntiles = 0.0;
-        for(size_t i = 0; i < ns; i++) {
-            uint32_t tm, tn;
-            tiles_of(pl.tstacks[i], tm, tn);
-            ntiles += double(tm) * tn;
-            chunks += double(tm) * tn * pl.tstacks[i].nchunk;
-        }
-        const double len = std::max(double(kMinChunks), chunks / kItems);
-        auto cut = [&](const dev::tile_stack &t) {
-            return ntiles >= kItems ? 1u : std::max(1u, uint32_t(double(t.nchunk) / len + 0.5));
-        };
-        typedef std::pair<double, dev::tile_item> unit;
-        std::vector<uint32_t> part_of;            // of each unit: its place along k
-        auto add_tile = [&](size_t stack, const dev::tile_stack &t, uint32_t i, uint32_t j, uint32_t pair0,
-            std::vector<unit> &units, std::vector<dev::tile_item> &sums, size_t &nparts) {
-            const uint32_t np = cut(t), fa = (std::min(bm, t.rows - i * bm) + 15) / 16;
-            dev::tile_item it;
-            it.stack = (uint32_t)stack; it.tm = (uint16_t)i; it.tn = (uint16_t)j;
-            it.p = 0; it.c = 0; it.part = -1;
-            if(np > 1) {
-                dev::tile_item sm = it;
-                sm.part = (int32_t)nparts; sm.count = np;
-                sums.push_back(sm);
-            }
-            uint32_t at = 0;
-            for(uint32_t q = 0; q < np; q++) {
-                const uint32_t end = uint32_t(uint64_t(t.nchunk) * (q + 1) / np);
-                it.count = end - at;
-                if(np > 1) it.part = (int32_t)nparts++;
-                units.push_back(std::make_pair(double(it.count) * fa, it));
-                part_of.push_back(q);
-                for(; at < end; ) {
-                    const uint32_t left = (pl.spairs[pair0 + it.p].k + 15) / 16 - it.c;
-                    if(end - at < left) { it.c += end - at; at = end; }
-                    else { at += left; it.p++; it.c = 0; }
-                }
-            }
-        };
-        auto longer = [](const unit &x, const unit &y) { return x.first > y.first; };
-        std::vector<unit> units;
-        pl.tsums.clear();
-        pl.n_parts = 0;
-        for(size_t i = 0; i < ns; i++) {
-            uint32_t tm, tn;
-            tiles_of(pl.tstacks[i], tm, tn);
-            for(uint32_t a = 0; a < tm; a++) for(uint32_t b = 0; b < tn; b++)
-                add_tile(i, pl.tstacks[i], a, b, pl.stacks[i].pair_begin, units, pl.tsums, pl.n_parts);
-        }
-        pl.titems.clear();
-        if(order == 0) {
-            std::stable_sort(units.begin(), units.end(), longer);
-            for(size_t i = 0; i < units.size(); i++) pl.titems.push_back(units[i].second);
-        } else {
-            // XCD-aware: the items part by part, in strips of kStrip columns of
-            // tiles, cut into one piece of equal work per XCD, so that the
-            // items an XCD's L2 serves at a time share rows of A and columns
-            // of B (o = 29, v = 131: 25 instead of 45 M lines from beyond the
-            // L2 caches; o = 48, v = 240 in uneven blocks 61.4 to 59.0 ms);
-            // each piece longest first at positions x, x + nx, ...; the
-            // padding items name the empty stack
-            const uint32_t kStrip = 8;
-            std::vector<std::pair<std::array<uint32_t, 5>, size_t> > seq(units.size());
-            double total = 0.0;
-            for(size_t i = 0; i < units.size(); i++) {
-                const dev::tile_item &t = units[i].second;
-                seq[i].first = {{ part_of[i], t.stack, t.tn / kStrip, t.tm, t.tn }};
-                seq[i].second = i;
-                total += units[i].first;
-            }
-            std::sort(seq.begin(), seq.end());
-            std::vector<std::vector<unit> > q(nx);
-            double sum = 0.0;
-            for(size_t i = 0; i < seq.size(); i++) {
-                const unit &u = units[seq[i].second];
-                const int x = total > 0.0 ? std::min(nx - 1, int((sum + 0.5 * u.first) * nx / total)) : 0;
-                q[x].push_back(u);
-                sum += u.first;
-            }
-            size_t qmax = 0;
-            for(int x = 0; x < nx; x++) qmax = std::max(qmax, q[x].size());
-            dev::tile_item empty;
-            std::memset(&empty, 0, sizeof(empty));
-            empty.stack = (uint32_t)ns;
-            empty.part = -1;
-            pl.titems.assign(qmax * nx, empty);
-            for(int x = 0; x < nx; x++) {
-                std::stable_sort(q[x].begin(), q[x].end(), longer);
-                for(size_t l = 0; l < q[x].size(); l++) pl.titems[l * nx + x] = q[x][l].second;
-            }
-        }
-        // per C block, in block order
-        pl.bitems.clear(); pl.bsums.clear();
-        pl.block_item_begin.clear(); pl.block_sum_begin.clear();
-        size_t bparts = 0;
-        for(size_t b = 0; b < nb; b++) {
-            pl.block_item_begin.push_back((uint32_t)pl.bitems.size());
-            pl.block_sum_begin.push_back((uint32_t)pl.bsums.size());
-            const dev::tile_stack &t = pl.tstacks[pl.stacks.size() + b];
-            uint32_t tm, tn;
-            tiles_of(t, tm, tn);
-            std::vector<unit> bu;
-            for(uint32_t i = 0; i < tm; i++) for(uint32_t j = 0; j < tn; j++)
-                add_tile(b, t, i, j, block_pair0[b], bu, pl.bsums, bparts);
-            for(size_t u = 0; u < bu.size(); u++) pl.bitems.push_back(bu[u].second);
-        }
-        pl.block_item_begin.push_back((uint32_t)pl.bitems.size());
-        pl.block_sum_begin.push_back((uint32_t)pl.bsums.size());
-        const std::vector<dev::tile_item> *lists[4] = { &pl.titems, &pl.tsums, &pl.bitems, &pl.bsums };
-        dev::tile_item **at[4] = { &pl.d_titems, &pl.d_tsums, &pl.d_bitems, &pl.d_bsums };
-        size_t off[5] = { 0 };
-        for(int i = 0; i < 4; i++) off[i + 1] = align256(off[i] + lists[i]->size() * sizeof(dev::tile_item));
-        std::vector<char> host(off[4] ? off[4] : 256, 0);
-        for(int i = 0; i < 4; i++)
-            if(!lists[i]->empty())
-                std::memcpy(&host[off[i]], lists[i]->data(), lists[i]->size() * sizeof(dev::tile_item));
-        pl.stk_tiles.at_least(ctx, host.size());
-        ctx.upload_new(pl.stk_tiles.mem, host.data(), host.size());
-        for(int i = 0; i < 4; i++) *at[i] = (dev::tile_item*)((char*)pl.stk_tiles.mem + off[i]);
-        const size_t bytes = std::max(pl.n_parts, bparts) * bm * bn * sizeof(double);
-        if(bytes) pl.parts.at_least(ctx, bytes);
-    };
-
     // tile lists live in their own allocation (replaced by the autotuner)
     auto upload_tiles = [&](int k, int order) {
         make_tiles(k, order, pl.tiles_by_block, pl.block_tile_begin, pl.tiles_sorted);
@@ -1515,8 +1603,9 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         pl.tile_order = order;
         pl.stiles.clear();
         pl.vtiles.clear();
+        pl.tl = tile_lists();
         if(dev::is_tile(k)) {
-            make_items(k, order);
+            make_items(pl, k, order);
         } else if(dev::is_var(k)) {
             // full 64-row tiles and one tile per row / column remainder,
             // largest (k sum x area) first
@@ -1648,7 +1737,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
                 return take(pl.vtiles, [&](const dev::var_tile &t) {
                     return ksum_of(pl.stack_ksum, t.stack) * t.fm * t.fn; }, scale);
             if(dev::is_tile(k))
-                return take(pl.titems, [&](const dev::tile_item &t) { return double(t.count); }, scale);
+                return take(pl.tl.items, [&](const dev::tile_item &t) { return double(t.count); }, scale);
             if(dev::is_stacked(k))
                 return take(pl.stiles, [&](const dev::gemm_tile &t) {
                     return ksum_of(pl.stack_ksum, t.cblock); }, scale);
@@ -1664,6 +1753,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         int bestk = cfg, besto = 0;
         auto time_one = [&](int k, int o) {
             upload_tiles(k, o);
+            ensure_parts(pl);
             double scale = 1.0;
             const uint32_t ntune = stride > 1 ? sample(k, scale) : 0;
             auto go = [&]() {
@@ -1688,6 +1778,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
             return m_stats.tune_ms[x] < m_stats.tune_ms[y]; });
         for(size_t ci = 0; ci < rank.size() && ci < 3; ci++) time_one(rank[ci], 1);
         cfg = bestk;
+        pl.parts.release();           // of another candidate's size
         upload_tiles(cfg, besto);
         m_tuned_cfg = cfg;
         m_tuned_order = besto;
@@ -2066,11 +2157,12 @@ void btod_contract2::enqueue(int mode, hipStream_t s, bool timed, size_t &launch
             const uint32_t t0 = pl.block_item_begin[b], t1 = pl.block_item_begin[b + 1];
             const uint32_t s0 = pl.block_sum_begin[b], s1 = pl.block_sum_begin[b + 1];
             if(t1 == t0) continue;
-            hipStream_t sd = ctx.side(j++);
+            const size_t i = b % pl.blk_base.size();
+            hipStream_t sd = ctx.side(int(i));
             hip_check(dev::launch_gemm_tile(pl.tile_cfg, pl.d_bstacks, pl.d_bitems + t0, t1 - t0,
-                (double*)pl.parts.mem, sd), "gemm (per block)");
+                pl.blk_base[i], sd), "gemm (per block)");
             hip_check(dev::launch_tile_sum(pl.tile_cfg, pl.d_bstacks, pl.d_bsums + s0, s1 - s0,
-                (double*)pl.parts.mem, sd), "gemm (per block, sums)");
+                pl.blk_base[i], sd), "gemm (per block, sums)");
             launches += s1 > s0 ? 2 : 1;
         }
         for(size_t b = 0; !wg && b + 1 < pl.block_tile_begin.size(); b++) {
@@ -2118,6 +2210,8 @@ void btod_contract2::run(btensor &c, int mode) {
         ensure_ozaki();
         m_stats.ozaki_slices = pl.oz_slices;
     }
+    if(mode == MODE_GROUPED) ensure_parts(pl);
+    if(mode == MODE_PER_BLOCK) ensure_block_items(pl);
     // The grouped perform runs as a HIP graph (prepare permute, grouped
     // GEMM, write-back permute: kernel nodes only), captured once per plan.
     const bool graph = m_use_graph && mode == MODE_GROUPED;
@@ -2210,6 +2304,7 @@ void btod_contract2::perform_sliced(btensor &c, bool add, double d, double slice
         }
     }
     if(pl.empty) return;
+    ensure_parts(pl);
     hip_check(hipEventRecord(pl.ev[0], s), "hipEventRecord");
     if(pl.add) {
         for(size_t i = 0; i < pl.c_out.size(); i++) {
@@ -2229,7 +2324,7 @@ void btod_contract2::perform_sliced(btensor &c, bool add, double d, double slice
     }
     hip_check(hipEventRecord(pl.ev[1], s), "hipEventRecord");
     const uint32_t nt = dev::is_var(k) ? (uint32_t)pl.vtiles.size() :
-        dev::is_tile(k) ? (uint32_t)pl.titems.size() : dev::is_stacked(k) ? (uint32_t)pl.stiles.size() : (uint32_t)pl.tiles_sorted.size();
+        dev::is_tile(k) ? (uint32_t)pl.tl.items.size() : dev::is_stacked(k) ? (uint32_t)pl.stiles.size() : (uint32_t)pl.tiles_sorted.size();
     const uint32_t nslices = (uint32_t)std::max(1.0, std::min(double(nt),
         std::ceil(m_stats.flops / slice_flops)));
     const uint32_t per = (nt + nslices - 1) / nslices;
@@ -2245,7 +2340,7 @@ void btod_contract2::perform_sliced(btensor &c, bool add, double d, double slice
         }
     }
     if(dev::is_tile(k))
-        hip_check(dev::launch_tile_sum(k, pl.d_tstacks, pl.d_tsums, (uint32_t)pl.tsums.size(),
+        hip_check(dev::launch_tile_sum(k, pl.d_tstacks, pl.d_tsums, (uint32_t)pl.tl.sums.size(),
             (double*)pl.parts.mem, s), "gemm (sums)");
     hip_check(hipEventRecord(pl.ev[2], s), "hipEventRecord");
     if(pl.n_wb_chunks)
@@ -2349,19 +2444,22 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
     std::vector<dev::tile_item> tsm;
     std::vector<char> host;
     size_t sz = 0;
-    for(std::map<int, std::vector<size_t> >::iterator g = groups.begin(); g != groups.end(); ++g) {
+    // one launch over the plans x0 .. x1 - 1 of a group, their tiles from `lists`
+    auto add_launch = [&](int cfg, const std::vector<size_t> &group, size_t x0, size_t x1,
+        const std::vector<const tile_lists*> &lists) {
         cbs.clear(); prs.clear(); tl.clear(); tss.clear(); til.clear(); tsm.clear();
         size_t nparts = 0;
         uint32_t bm = 64, bn = 64;
-        dev::tile_shape(g->first, bm, bn);
-        for(size_t x = 0; x < g->second.size(); x++) {
-            contract_plan &pl = *m_plans[g->second[x]];
-            if(dev::is_tile(g->first)) {
+        dev::tile_shape(cfg, bm, bn);
+        for(size_t x = x0; x < x1; x++) {
+            contract_plan &pl = *m_plans[group[x]];
+            if(dev::is_tile(cfg)) {
+                const tile_lists &pt = *lists[x];
                 // stacks name their plan's lists by address
                 const uint32_t ts0 = (uint32_t)tss.size(), ns = (uint32_t)pl.stacks.size() - 1;
                 tss.insert(tss.end(), pl.tstacks.begin(), pl.tstacks.begin() + ns);
-                for(size_t t = 0; t < pl.titems.size(); t++) {
-                    dev::tile_item y = pl.titems[t];
+                for(size_t t = 0; t < pt.items.size(); t++) {
+                    dev::tile_item y = pt.items[t];
                     if(y.stack >= ns) continue;                 // padding item
                     const dev::stack_desc &sd = pl.stacks[y.stack];
                     const double rows = std::min<double>(bm, double(sd.rows) - double(y.tm) * bm);
@@ -2373,13 +2471,13 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
                     til.push_back(std::make_pair(cost, y));
                     m_flops += cost;
                 }
-                for(size_t t = 0; t < pl.tsums.size(); t++) {
-                    dev::tile_item y = pl.tsums[t];
+                for(size_t t = 0; t < pt.sums.size(); t++) {
+                    dev::tile_item y = pt.sums[t];
                     y.stack += ts0;
                     y.part += (int32_t)nparts;
                     tsm.push_back(y);
                 }
-                nparts += pl.n_parts;
+                nparts += pt.places;
                 continue;
             }
             uint32_t cb0 = (uint32_t)cbs.size(), pr0 = (uint32_t)prs.size();
@@ -2411,9 +2509,8 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
             [](const std::pair<double, dev::tile_item> &x, const std::pair<double, dev::tile_item> &y) {
                 return x.first > y.first; });
         launch L;
-        L.cfg = g->first;
+        L.cfg = cfg;
         L.nsum = (uint32_t)tsm.size();
-        L.part_bytes = nparts * bm * bn * sizeof(double);
         L.ocb = sz;
         sz = align256(sz + cbs.size() * sizeof(dev::gemm_cblock) + tss.size() * sizeof(dev::tile_stack));
         L.opr = sz; sz = align256(sz + prs.size() * sizeof(dev::gemm_pair));
@@ -2437,20 +2534,59 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
         }
         if(!tsm.empty()) std::memcpy(&host[L.osum], tsm.data(), tsm.size() * sizeof(dev::tile_item));
         m_launches.push_back(L);
-    }
-    // partial sums behind the lists
-    size_t total = sz;
-    for(size_t i = 0; i < m_launches.size(); i++) {
-        m_launches[i].opart = total;
-        total = align256(total + m_launches[i].part_bytes);
-    }
-    if(sz) {
-        if(merged.bytes < total) {
-            merged.release();
-            merged.ctx = &ctx;
-            merged.mem = ctx.alloc(total);
-            merged.bytes = total;
+    };
+    // The launches of a group of workgroup tiles use the same memory for their
+    // partial sums one after the other: kBatchParts, or what the largest plan
+    // needs; a batch that needs more takes several launches.  Without room for
+    // them the tiles run whole.
+    const size_t kBatchParts = size_t(256) << 20;
+    size_t total = 0;
+    for(int cut = 1; ; cut = 0) {
+        m_launches.clear();
+        host.clear();
+        sz = 0;
+        m_flops = 0.0;
+        size_t parts = 0;
+        for(std::map<int, std::vector<size_t> >::iterator g = groups.begin(); g != groups.end(); ++g) {
+            const std::vector<size_t> &q = g->second;
+            std::vector<tile_lists> whole(cut ? 0 : q.size());
+            std::vector<const tile_lists*> lists(q.size());
+            for(size_t x = 0; x < q.size(); x++) {
+                lists[x] = &m_plans[q[x]]->tl;
+                if(cut || !dev::is_tile(g->first) || lists[x]->places == 0) continue;
+                list_items(*m_plans[q[x]], g->first, 0, false, whole[x]);
+                lists[x] = &whole[x];
+            }
+            uint32_t bm = 64, bn = 64;
+            dev::tile_shape(g->first, bm, bn);
+            size_t x0 = 0, places = 0;
+            for(size_t x = 0; x < q.size(); x++) {
+                const size_t n = lists[x]->places;
+                if(x > x0 && (places + n) * bm * bn * sizeof(double) > kBatchParts) {
+                    add_launch(g->first, q, x0, x, lists);
+                    x0 = x;
+                    places = 0;
+                }
+                places += n;
+                parts = std::max(parts, places * bm * bn * sizeof(double));
+            }
+            add_launch(g->first, q, x0, q.size(), lists);
         }
+        total = sz + parts;
+        if(merged.bytes >= total || !sz) break;
+        merged.release();
+        merged.ctx = &ctx;
+        try {
+            merged.mem = ctx.alloc(total);
+        } catch(const lt_error &e) {
+            if(e.code != LT_ERR_NOMEM || !parts) throw;
+            continue;
+        }
+        merged.bytes = total;
+        break;
+    }
+    for(size_t i = 0; i < m_launches.size(); i++) m_launches[i].opart = sz;   // behind the lists
+    if(sz) {
         hip_check(hipMemcpyAsync(merged.mem, host.data(), sz, hipMemcpyHostToDevice, s),
             "hipMemcpy H2D");
         // the host buffer goes out of scope: the copy must have read it
@@ -2555,6 +2691,7 @@ bool btod_contract2::try_plan(btensor &c, bool add, double d, bool measure, int 
     try {
         if(!plan_valid(c, add, d, mode)) build_plan(c, add, d, measure);
         if(mode == MODE_OZAKI) ensure_ozaki();
+        if(mode == MODE_PER_BLOCK) ensure_block_items(*m_plan);
         return true;
     } catch(const lt_error &e) {
         if(e.code != LT_ERR_NOMEM) throw;

@@ -391,7 +391,7 @@ public:
 private:
     struct launch {
         int cfg;
-        size_t ocb, opr, otl, osum, opart, part_bytes;
+        size_t ocb, opr, otl, osum, opart;
         uint32_t nt, nsum;
         std::vector<double> tcost;
     };
