@@ -352,7 +352,13 @@ void run_jobs(context &cx, std::vector<dense_job> &jobs) {
     double *pp = 0;
     if(parts) {
         lk.lock();
-        pp = (double*)cx.staging(parts);
+        try {
+            pp = (double*)cx.staging(parts);
+        } catch(const lt_error &e) {
+            // no room for partial sums: every k range whole
+            if(e.code != LT_ERR_NOMEM) throw;
+            for(size_t i = 0; i < jobs.size(); i++) jobs[i].nparts = 1;
+        }
     }
     cx.activate();
     try {

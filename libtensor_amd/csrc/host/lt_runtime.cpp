@@ -129,9 +129,15 @@ void *context::staging(size_t bytes) {
         if(m_stage) free(m_stage);
         m_stage = 0;
         m_stage_bytes = 0;
-        size_t n = std::max<size_t>(bytes, 65536);
-        m_stage = alloc(n);
-        m_stage_bytes = n;
+        const size_t n = std::max<size_t>(bytes, 65536);
+        try {
+            m_stage = alloc(n);
+            m_stage_bytes = n;
+        } catch(const lt_error &e) {
+            if(e.code != LT_ERR_NOMEM || n == bytes) throw;
+            m_stage = alloc(bytes);
+            m_stage_bytes = bytes;
+        }
     }
     return m_stage;
 }
