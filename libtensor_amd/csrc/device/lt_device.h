@@ -220,8 +220,12 @@ hipError_t launch_gemm_stacked(int cfg, const stack_desc *st, const stack_pair *
 //! descriptor and the first destination element of a chunk of kPermChunk
 //! elements, or (chunk_desc[j] | kPermTileItem) and the destination index
 //! of a tile's corner for transposing descriptors.
+//! What a list of descriptors needs of the kernel: stores past the caches
+//! (kPermStream), tiles (the largest tile_s of them, 0: no item is a tile),
+//! sums (`add` of some descriptor).
+struct perm_kind { bool stream, add; uint32_t tile; };
 hipError_t launch_permute(const perm_desc *descs, const uint32_t *chunk_desc,
-    const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s, bool stream = false);
+    const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s, perm_kind kind);
 static const uint32_t kPermChunk = 2048;
 //! One permutation, its descriptor passed with the launch and its work items
 //! numbered by the grid.

@@ -103,7 +103,7 @@ __device__ __forceinline__ void perm_store(const perm_desc &d, uint32_t e, doubl
 //! contiguous along p, the destination along q (extents and strides from
 //! dedicated fields: indexing the descriptor's arrays with a runtime dimension
 //! would put it in scratch memory).
-template<int S, bool NT>
+template<int S, bool NT, bool ADD>
 __device__ __forceinline__ void permute_tile(const perm_desc &d, uint32_t base, double *tile) {
     constexpr int RW = 256 / S;          // rows at a time
     const uint32_t dq = d.tdq.d, dp = d.tdp.d;
@@ -131,7 +131,7 @@ __device__ __forceinline__ void permute_tile(const perm_desc &d, uint32_t base, 
         if(ls) { iq = fdiv(e, d.tdp); ip = e - iq * dp; }
         if(ls ? e < nn : ti < np && iq < nq) tile[iq * (S + 1) + ip] = w[r];
     }
-    if(d.add) {
+    if(ADD && d.add) {
 #pragma unroll
         for(int r = 0; r < R; r++) {
             const uint32_t e = threadIdx.x + 256 * r, ip = tj + RW * r;
@@ -147,7 +147,7 @@ __device__ __forceinline__ void permute_tile(const perm_desc &d, uint32_t base, 
         if(ld ? e < nn : ti < nq && ip < np) {
             const double v = tile[iq * (S + 1) + ip];
             perm_store<NT>(d, base + (ld ? e : ip * dps + ti),
-                d.add ? perm_sum(d.alpha, v, d.beta, w[r]) : d.alpha * v);
+                ADD && d.add ? perm_sum(d.alpha, v, d.beta, w[r]) : d.alpha * v);
         }
     }
 }
@@ -155,7 +155,7 @@ __device__ __forceinline__ void permute_tile(const perm_desc &d, uint32_t base, 
 //! Element-wise gather of one chunk: each thread owns kPermChunk / 256
 //! elements; all source offsets are computed and all loads issued before the
 //! first store, so every thread has that many gathers in flight.
-template<bool NT>
+template<bool NT, bool ADD>
 __device__ __forceinline__ void permute_gather(const perm_desc &d, uint32_t base) {
     constexpr int E = kPermChunk / 256;
     const uint32_t end = min(base + kPermChunk, d.total);
@@ -165,7 +165,7 @@ __device__ __forceinline__ void permute_gather(const perm_desc &d, uint32_t base
         const uint32_t e = min(base + threadIdx.x + 256u * i, end - 1);
         v[i] = d.src[src_offset(d, e)];
     }
-    if(d.add) {
+    if(ADD && d.add) {
 #pragma unroll
         for(int i = 0; i < E; i++) w[i] = d.add[min(base + threadIdx.x + 256u * i, end - 1)];
 #pragma unroll
@@ -182,28 +182,47 @@ __device__ __forceinline__ void permute_gather(const perm_desc &d, uint32_t base
     }
 }
 
-template<bool NT>
+//! TILE: the largest tile side of the list's items (0: none is a tile), ADD:
+//! some descriptors are sums.  A kernel per kind: the 33 KB of LDS of 64-wide
+//! tiles let four workgroups onto a CU instead of eight, and in short launches
+//! the first instructions' way to the CU shows.
+template<bool NT, int TILE, bool ADD>
 __global__ void __launch_bounds__(256)
 permute_kernel(const perm_desc *__restrict__ descs,
     const uint32_t *__restrict__ chunk_desc,
     const uint32_t *__restrict__ chunk_off) {
 
-    __shared__ double tile[kPermTileMax * (kPermTileMax + 1)];
+    __shared__ double tile[TILE ? TILE * (TILE + 1) : 1];
     const uint32_t ch = xcd_item(blockIdx.x, gridDim.x);
     const uint32_t cd = chunk_desc[ch];
     const perm_desc d = descs[cd & ~kPermTileItem];
     const uint32_t base = chunk_off[ch];
-    if(!(cd & kPermTileItem)) permute_gather<NT>(d, base);
-    else if(d.tile_s == kPermTileMax) permute_tile<kPermTileMax, NT>(d, base, tile);
-    else permute_tile<kPermTile, NT>(d, base, tile);
+    if constexpr(TILE == 0) {
+        permute_gather<NT, ADD>(d, base);
+    } else {
+        if(!(cd & kPermTileItem)) permute_gather<NT, ADD>(d, base);
+        else if(TILE == kPermTileMax && d.tile_s == kPermTileMax) permute_tile<TILE, NT, ADD>(d, base, tile);
+        else permute_tile<kPermTile, NT, ADD>(d, base, tile);
+    }
+}
+
+template<bool NT, bool ADD>
+static hipError_t launch_permute_t(const perm_desc *descs, const uint32_t *chunk_desc,
+    const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s, uint32_t tile) {
+    auto k = tile == 0 ? permute_kernel<NT, 0, ADD> : tile == kPermTile ? permute_kernel<NT, kPermTile, ADD> :
+        permute_kernel<NT, kPermTileMax, ADD>;
+    hipLaunchKernelGGL(k, dim3(nchunks), dim3(256), 0, s, descs, chunk_desc, chunk_off);
+    return hipGetLastError();
 }
 
 hipError_t launch_permute(const perm_desc *descs, const uint32_t *chunk_desc,
-    const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s, bool stream) {
+    const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s, perm_kind kind) {
     if(nchunks == 0) return hipSuccess;
-    hipLaunchKernelGGL(stream ? permute_kernel<true> : permute_kernel<false>, dim3(nchunks), dim3(256), 0, s,
-        descs, chunk_desc, chunk_off);
-    return hipGetLastError();
+    if(kind.stream)
+        return kind.add ? launch_permute_t<true, true>(descs, chunk_desc, chunk_off, nchunks, s, kind.tile) :
+            launch_permute_t<true, false>(descs, chunk_desc, chunk_off, nchunks, s, kind.tile);
+    return kind.add ? launch_permute_t<false, true>(descs, chunk_desc, chunk_off, nchunks, s, kind.tile) :
+        launch_permute_t<false, false>(descs, chunk_desc, chunk_off, nchunks, s, kind.tile);
 }
 
 //! Work items of one descriptor by number: per destination dimension the
@@ -225,12 +244,12 @@ __global__ void __launch_bounds__(256) permute_tiles_kernel(perm_desc d, perm_it
             x = q;
         }
     }
-    permute_tile<S, NT>(d, base, tile);
+    permute_tile<S, NT, true>(d, base, tile);
 }
 
 template<bool NT>
 __global__ void __launch_bounds__(256) permute_gather_kernel(perm_desc d) {
-    permute_gather<NT>(d, xcd_item(blockIdx.x, gridDim.x) * kPermChunk);
+    permute_gather<NT, true>(d, xcd_item(blockIdx.x, gridDim.x) * kPermChunk);
 }
 
 hipError_t launch_permute_one(const perm_desc &d, hipStream_t s) {

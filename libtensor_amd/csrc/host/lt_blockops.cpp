@@ -64,7 +64,7 @@ void run_permutes(context &ctx, const std::vector<dev::perm_desc> &descs, double
             hip_check(hipEventRecord(ev[0], ctx.stream()), "hipEventRecord");
         }
         hip_check(dev::launch_permute((dev::perm_desc*)mem, (uint32_t*)(mem + o_cd),
-            (uint32_t*)(mem + o_co), (uint32_t)cd.size(), ctx.stream()), "permute");
+            (uint32_t*)(mem + o_co), (uint32_t)cd.size(), ctx.stream(), list_kind(descs)), "permute");
         if(ms) hip_check(hipEventRecord(ev[1], ctx.stream()), "hipEventRecord");
         ctx.sync();
         if(ms) {
@@ -179,7 +179,8 @@ std::shared_ptr<context::cached_launch> upload_launches(context &ctx,
         g.o_cd = sz; sz = (sz + 4 * cd.size() + 255) & ~size_t(255);
         g.o_co = sz; sz = (sz + 4 * co.size() + 255) & ~size_t(255);
         g.nchunks = cd.size();
-        g.stream = total >= dev::kPermStream;
+        g.kind = list_kind(lists[i]);
+        g.kind.stream = total >= dev::kPermStream;
         g.tiles = tiles;
         host.resize(sz, 0);
         std::memcpy(&host[g.o_d], lists[i].data(), lists[i].size() * sizeof(dev::perm_desc));
@@ -212,7 +213,7 @@ void run_launches(context &ctx, const context::cached_launch &l, double *ms) {
             const context::cached_launch::segment &g = l.segs[i];
             hip_check(dev::launch_permute((dev::perm_desc*)(base + g.o_d),
                 (uint32_t*)(base + g.o_cd), (uint32_t*)(base + g.o_co),
-                (uint32_t)g.nchunks, s, g.stream), "permute");
+                (uint32_t)g.nchunks, s, g.kind), "permute");
         }
         if(ms) hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
         ctx.sync();

@@ -204,6 +204,15 @@ void make_chunks(const std::vector<dev::perm_desc> &ds, std::vector<uint32_t> &c
     }
 }
 
+dev::perm_kind list_kind(const std::vector<dev::perm_desc> &ds) {
+    dev::perm_kind k = { false, false, 0 };
+    for(size_t i = 0; i < ds.size(); i++) {
+        k.add = k.add || ds[i].add;
+        if(ds[i].tile_p >= 0) k.tile = std::max(k.tile, ds[i].tile_s);
+    }
+    return k;
+}
+
 dev::perm_desc make_perm_desc_public(const double *src, const dims_t &dsrc,
     const tensor_tr &tr, double *dst, bool accumulate) {
     return make_perm_desc(src, dsrc, tr, dst, accumulate);
@@ -287,6 +296,7 @@ struct contract_plan {
     dev::perm_desc *d_prep, *d_wback;
     uint32_t *d_prep_cd, *d_prep_co, *d_wb_cd, *d_wb_co;
     uint32_t n_prep_chunks, n_wb_chunks;
+    dev::perm_kind prep_kind, wb_kind, prep_st_kind, oz_prep_kind;    // of the four permute lists
     dev::gemm_cblock *d_cb;
     dev::gemm_pair *d_pairs;
     dev::gemm_tile *d_tiles_sorted, *d_tiles_block;
@@ -325,6 +335,7 @@ struct contract_plan {
     contract_plan() : batch(false), va(0), vb(0), cuid(0), c(0), add(false), d(1.0), empty(false),
         ta(false), tb(false), tile_cfg(0), tile_order(0), d_prep(0), d_wback(0), d_prep_cd(0),
         d_prep_co(0), d_wb_cd(0), d_wb_co(0), n_prep_chunks(0), n_wb_chunks(0),
+        prep_kind(), wb_kind(), prep_st_kind(), oz_prep_kind(),
         d_cb(0), d_pairs(0), d_tiles_sorted(0), d_tiles_block(0), scratch(0),
         scratch_elems(0), ctx(0), events(false), graph(0), gexec(0), graph_launches(0),
         d_stacks(0), d_spairs(0), d_arows(0), d_crows(0), d_stiles(0), d_vtiles(0),
@@ -1489,6 +1500,9 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     pl.n_prep_chunks = (uint32_t)pcd.size();
     pl.n_wb_chunks = (uint32_t)wcd.size();
     pl.n_prep_st_chunks = (uint32_t)scd.size();
+    pl.prep_kind = list_kind(pl.prep);
+    pl.wb_kind = list_kind(pl.wback);
+    pl.prep_st_kind = list_kind(pl.prep_st);
     size_t sz = 0;
     size_t o_prep = sz; sz = align256(sz + pl.prep.size() * sizeof(dev::perm_desc));
     size_t o_wb = sz; sz = align256(sz + pl.wback.size() * sizeof(dev::perm_desc));
@@ -1706,7 +1720,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         // (the candidates are stacked kernels: one prepare for all of them)
         if(pl.n_prep_st_chunks)
             hip_check(dev::launch_permute(pl.d_prep_st, pl.d_pst_cd, pl.d_pst_co,
-                pl.n_prep_st_chunks, s), "permute (prepare)");
+                pl.n_prep_st_chunks, s, pl.prep_st_kind), "permute (prepare)");
         // A large plan is timed on a sample of each candidate's launch list:
         // every stride-th group of nx consecutive tiles (a group keeps its
         // XCD placement), about kTuneFlops of work, its time scaled by the
@@ -2046,6 +2060,7 @@ void btod_contract2::build_ozaki(int slices) {
     pl.d_oz_prep_cd = (uint32_t*)(base + o_pmcd);
     pl.d_oz_prep_co = (uint32_t*)(base + o_pmco);
     pl.n_oz_prep_chunks = (uint32_t)pm_cd.size();
+    pl.oz_prep_kind = list_kind(prep_mut);
     pl.oz_prep_own = true;
     if(pl.n_oz_items > n_mut) {
         // operands of immutable tensors (in place or invariant copies,
@@ -2054,7 +2069,7 @@ void btod_contract2::build_ozaki(int slices) {
         if(!pi_cd.empty())
             hip_check(dev::launch_permute((const dev::perm_desc*)(base + o_pi),
                 (const uint32_t*)(base + o_picd), (const uint32_t*)(base + o_pico),
-                (uint32_t)pi_cd.size(), ctx.stream()), "permute (prepare, immutable operands)");
+                (uint32_t)pi_cd.size(), ctx.stream(), list_kind(prep_inv)), "permute (prepare, immutable operands)");
         hip_check(dev::launch_oz_split(pl.d_oz_split, pl.d_oz_items + 2 * n_mut,
             pl.n_oz_items - n_mut, ctx.stream()), "split (ozaki, immutable operands)");
     }
@@ -2075,7 +2090,7 @@ void btod_contract2::build_ozaki(int slices) {
         ctx.activate();
         if(pl.n_prep_chunks)
             hip_check(dev::launch_permute(pl.d_prep, pl.d_prep_cd, pl.d_prep_co,
-                pl.n_prep_chunks, s), "permute (prepare)");
+                pl.n_prep_chunks, s, pl.prep_kind), "permute (prepare)");
         hip_check(dev::launch_oz_split(pl.d_oz_split, pl.d_oz_items, pl.n_oz_items_mut, s),
             "split (ozaki)");
         float bestms = 1e30f;
@@ -2116,18 +2131,18 @@ void btod_contract2::enqueue(int mode, hipStream_t s, bool timed, size_t &launch
         (mode == MODE_PER_BLOCK && dev::is_tile(pl.tile_cfg))) {
         if(pl.n_prep_st_chunks) {
             hip_check(dev::launch_permute(pl.d_prep_st, pl.d_pst_cd, pl.d_pst_co,
-                pl.n_prep_st_chunks, s), "permute (prepare)");
+                pl.n_prep_st_chunks, s, pl.prep_st_kind), "permute (prepare)");
             launches++;
         }
     } else if(mode == MODE_OZAKI && pl.oz_prep_own) {
         if(pl.n_oz_prep_chunks) {
             hip_check(dev::launch_permute(pl.d_oz_prep, pl.d_oz_prep_cd, pl.d_oz_prep_co,
-                pl.n_oz_prep_chunks, s), "permute (prepare)");
+                pl.n_oz_prep_chunks, s, pl.oz_prep_kind), "permute (prepare)");
             launches++;
         }
     } else if(pl.n_prep_chunks) {
         hip_check(dev::launch_permute(pl.d_prep, pl.d_prep_cd, pl.d_prep_co,
-            pl.n_prep_chunks, s), "permute (prepare)");
+            pl.n_prep_chunks, s, pl.prep_kind), "permute (prepare)");
         launches++;
     }
     if(timed) hip_check(hipEventRecord(pl.ev[1], s), "hipEventRecord");
@@ -2180,7 +2195,7 @@ void btod_contract2::enqueue(int mode, hipStream_t s, bool timed, size_t &launch
     if(timed && mode != MODE_OZAKI) hip_check(hipEventRecord(pl.ev[2], s), "hipEventRecord");
     if(pl.n_wb_chunks) {
         hip_check(dev::launch_permute(pl.d_wback, pl.d_wb_cd, pl.d_wb_co,
-            pl.n_wb_chunks, s), "permute (write back)");
+            pl.n_wb_chunks, s, pl.wb_kind), "permute (write back)");
         launches++;
     }
 }
@@ -2317,10 +2332,10 @@ void btod_contract2::perform_sliced(btensor &c, bool add, double d, double slice
     if(dev::is_stacked(k)) {
         if(pl.n_prep_st_chunks)
             hip_check(dev::launch_permute(pl.d_prep_st, pl.d_pst_cd, pl.d_pst_co,
-                pl.n_prep_st_chunks, s), "permute (prepare)");
+                pl.n_prep_st_chunks, s, pl.prep_st_kind), "permute (prepare)");
     } else if(pl.n_prep_chunks) {
         hip_check(dev::launch_permute(pl.d_prep, pl.d_prep_cd, pl.d_prep_co,
-            pl.n_prep_chunks, s), "permute (prepare)");
+            pl.n_prep_chunks, s, pl.prep_kind), "permute (prepare)");
     }
     hip_check(hipEventRecord(pl.ev[1], s), "hipEventRecord");
     const uint32_t nt = dev::is_var(k) ? (uint32_t)pl.vtiles.size() :
@@ -2344,7 +2359,7 @@ void btod_contract2::perform_sliced(btensor &c, bool add, double d, double slice
             (double*)pl.parts.mem, s), "gemm (sums)");
     hip_check(hipEventRecord(pl.ev[2], s), "hipEventRecord");
     if(pl.n_wb_chunks)
-        hip_check(dev::launch_permute(pl.d_wback, pl.d_wb_cd, pl.d_wb_co, pl.n_wb_chunks, s),
+        hip_check(dev::launch_permute(pl.d_wback, pl.d_wb_cd, pl.d_wb_co, pl.n_wb_chunks, s, pl.wb_kind),
             "permute (write back)");
     hip_check(hipEventRecord(pl.ev[3], s), "hipEventRecord");
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
@@ -2422,10 +2437,10 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
         if(dev::is_tile(pl.tile_cfg)) {
             if(pl.n_prep_st_chunks)
                 hip_check(dev::launch_permute(pl.d_prep_st, pl.d_pst_cd, pl.d_pst_co,
-                    pl.n_prep_st_chunks, s), "permute (prepare)");
+                    pl.n_prep_st_chunks, s, pl.prep_st_kind), "permute (prepare)");
         } else if(pl.n_prep_chunks)
             hip_check(dev::launch_permute(pl.d_prep, pl.d_prep_cd, pl.d_prep_co,
-                pl.n_prep_chunks, s), "permute (prepare)");
+                pl.n_prep_chunks, s, pl.prep_kind), "permute (prepare)");
     }
 
     // one grouped GEMM per kernel configuration: the work lists of the
@@ -2635,7 +2650,7 @@ void batch_run::finish() {
         contract_plan &pl = *m_plans[q];
         if(!pl.empty && pl.n_wb_chunks)
             hip_check(dev::launch_permute(pl.d_wback, pl.d_wb_cd, pl.d_wb_co,
-                pl.n_wb_chunks, s), "permute (write back)");
+                pl.n_wb_chunks, s, pl.wb_kind), "permute (write back)");
     }
     hip_check(hipEventRecord(m_plans[0]->ev[3], s), "hipEventRecord");
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");

@@ -79,7 +79,7 @@ public:
     //! kLaunchCache entries, the oldest dropped first.
     struct cached_launch {
         //! one permute launch: descriptors at o_d, work items at o_cd / o_co
-        struct segment { size_t o_d, o_cd, o_co, nchunks; bool stream, tiles; };
+        struct segment { size_t o_d, o_cd, o_co, nchunks; dev::perm_kind kind; bool tiles; };
         void *mem;
         std::vector<segment> segs;       //!< launched in order
         std::vector<size_t> touched;     //!< blocks the launches write
@@ -228,6 +228,10 @@ void host_transform(const double *src, const dims_t &dsrc, const tensor_tr &tr,
 //! descriptors for dev::launch_permute.
 void make_chunks(const std::vector<dev::perm_desc> &ds, std::vector<uint32_t> &cd,
     std::vector<uint32_t> &co);
+
+//! The kernel that a list of permute descriptors needs (stores through the
+//! caches).
+dev::perm_kind list_kind(const std::vector<dev::perm_desc> &ds);
 
 //! Device permute descriptor for dst = c * P(src) (dimensions fused).
 dev::perm_desc make_perm_desc_public(const double *src, const dims_t &dsrc,
