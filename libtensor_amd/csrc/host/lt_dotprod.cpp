@@ -30,7 +30,7 @@ double btod_dotprod(btensor &a, const tensor_tr &tra0, btensor &b, const tensor_
     // descriptors and work items, kept per structure versions of A and B
     const std::string key = "dot" + key_tensor(a, true) + key_tensor(b, true) + "|" +
         key_part(tra0) + "|" + key_part(trb0);
-    std::shared_ptr<context::cached_launch> l = ctx.find_launch(key);
+    std::shared_ptr<context::cached_launch> l = ctx.find_launch(key, context::DOT_PRODUCTS);
     if(l) return run_dot(ctx, *l) * scale;
     std::vector<std::vector<dev::perm_desc> > lists(1);
     std::vector<dev::perm_desc> &descs = lists[0];
@@ -58,7 +58,7 @@ double btod_dotprod(btensor &a, const tensor_tr &tra0, btensor &b, const tensor_
         descs.push_back(d);
     }
     l = upload_launches(ctx, lists);
-    ctx.keep_launch(key, l);
+    ctx.keep_launch(key, l, context::DOT_PRODUCTS);
     return run_dot(ctx, *l) * scale;
 }
 

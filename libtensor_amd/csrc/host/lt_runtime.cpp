@@ -61,7 +61,7 @@ context::~context() {
     }
     hipSetDevice(m_device);
     if(m_stream) hipStreamSynchronize(m_stream);
-    m_launch_cache.clear();
+    drop_launches();
     for(std::map<void*, size_t>::iterator i = m_sizes.begin(); i != m_sizes.end(); ++i)
         hipFree(i->first);
     if(m_xfer_ev) hipEventDestroy(m_xfer_ev);
@@ -102,26 +102,44 @@ void context::activate() const {
     hip_check(hipSetDevice(m_device), "hipSetDevice");
 }
 
-std::shared_ptr<context::cached_launch> context::find_launch(const std::string &key) {
+std::shared_ptr<context::cached_launch> context::find_launch(const std::string &key, launch_set set) {
     std::lock_guard<std::mutex> lk(m_cache_mtx);
-    std::map<std::string, std::shared_ptr<cached_launch> >::iterator i = m_launch_cache.find(key);
-    return i == m_launch_cache.end() ? std::shared_ptr<cached_launch>() : i->second;
+    launch_cache &c = m_launches[set];
+    std::map<std::string, std::shared_ptr<cached_launch> >::iterator i = c.lists.find(key);
+    if(i == c.lists.end()) return std::shared_ptr<cached_launch>();
+    c.used(key);
+    return i->second;
 }
 
-void context::keep_launch(const std::string &key, std::shared_ptr<cached_launch> l) {
+void context::keep_launch(const std::string &key, std::shared_ptr<cached_launch> l, launch_set set) {
     std::vector<std::shared_ptr<cached_launch> > drop;    // let go outside the lock
     {
         std::lock_guard<std::mutex> lk(m_cache_mtx);
-        std::shared_ptr<cached_launch> &e = m_launch_cache[key];
+        launch_cache &c = m_launches[set];
+        std::shared_ptr<cached_launch> &e = c.lists[key];
         if(e) drop.push_back(e);
-        else m_launch_order.push_back(key);
         e = l;
-        while(m_launch_order.size() > kLaunchCache) {
-            drop.push_back(m_launch_cache[m_launch_order.front()]);
-            m_launch_cache.erase(m_launch_order.front());
-            m_launch_order.erase(m_launch_order.begin());
+        c.used(key);
+        while(c.order.size() > c.max) {
+            drop.push_back(c.lists[c.order.front()]);
+            c.lists.erase(c.order.front());
+            c.order.erase(c.order.begin());
         }
     }
+}
+
+//! Lets go of every kept list (one in use goes with its last user); false if
+//! there was none.
+bool context::drop_launches() {
+    std::map<std::string, std::shared_ptr<cached_launch> > drop[2];
+    {
+        std::lock_guard<std::mutex> lk(m_cache_mtx);
+        for(int i = 0; i < 2; i++) {
+            drop[i].swap(m_launches[i].lists);
+            m_launches[i].order.clear();
+        }
+    }
+    return !drop[0].empty() || !drop[1].empty();
 }
 
 void *context::staging(size_t bytes) {
@@ -144,24 +162,35 @@ void *context::staging(size_t bytes) {
 
 void *context::alloc(size_t bytes) {
     if(bytes == 0) bytes = 8;
+    std::string why;
+    void *p = try_alloc(bytes, why);
+    if(!p && drop_launches()) p = try_alloc(bytes, why);
+    if(!p) throw lt_error(LT_ERR_NOMEM, why);
+    return p;
+}
+
+void *context::try_alloc(size_t bytes, std::string &why) {
     std::lock_guard<std::mutex> lk(m_mtx);
     if(m_used + bytes > m_cap) {
-        throw lt_error(LT_ERR_NOMEM, "device memory budget exceeded");
+        why = "device memory budget exceeded";
+        return 0;
     }
     void *p = 0;
     if(m_device < 0) {
         p = std::aligned_alloc(256, (bytes + 255) & ~size_t(255));
-        lt_require(p != 0, LT_ERR_NOMEM, "host allocation failed");
+        if(!p) {
+            why = "host allocation failed";
+            return 0;
+        }
         std::memset(p, 0, bytes);
-        m_sizes[p] = bytes;
-        m_used += bytes;
-        return p;
-    }
-    activate();
-    hipError_t e = hipMalloc(&p, bytes);
-    if(e != hipSuccess) {
-        hipGetLastError();
-        throw lt_error(LT_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    } else {
+        activate();
+        hipError_t e = hipMalloc(&p, bytes);
+        if(e != hipSuccess) {
+            hipGetLastError();
+            why = std::string("hipMalloc: ") + hipGetErrorString(e);
+            return 0;
+        }
     }
     m_sizes[p] = bytes;
     m_used += bytes;

@@ -3,6 +3,7 @@
 // tensors, and the btod_contract2 operation with its cached execution plan.
 #pragma once
 
+#include <algorithm>
 #include <atomic>
 #include <functional>
 #include <map>
@@ -75,8 +76,10 @@ public:
 
     //! Uploaded descriptor lists of block operations, kept per key (the
     //! operation, its operands' identities and structure versions, its
-    //! scalars): a repeated call launches without rebuilding them.  At most
-    //! kLaunchCache entries, the oldest dropped first.
+    //! scalars): a repeated call launches without rebuilding them.  Scalar
+    //! products have a cache of their own (an iteration has many of them, which
+    //! would push out the lists of its sums and copies).  The entry unused for
+    //! longest is dropped first, all where device memory runs short.
     struct cached_launch {
         //! one permute launch: descriptors at o_d, work items at o_cd / o_co
         struct segment { size_t o_d, o_cd, o_co, nchunks; dev::perm_kind kind; bool tiles; };
@@ -93,9 +96,9 @@ public:
     private:
         context &m_ctx;
     };
-    std::shared_ptr<cached_launch> find_launch(const std::string &key);
-    void keep_launch(const std::string &key, std::shared_ptr<cached_launch> l);
-    static const size_t kLaunchCache = 32;
+    enum launch_set { BLOCK_OPS = 0, DOT_PRODUCTS = 1 };
+    std::shared_ptr<cached_launch> find_launch(const std::string &key, launch_set set = BLOCK_OPS);
+    void keep_launch(const std::string &key, std::shared_ptr<cached_launch> l, launch_set set = BLOCK_OPS);
 
     //! Side streams (default priority, created on first use) for independent
     //! launches: side_fork makes them wait for the work enqueued on s so
@@ -114,8 +117,19 @@ private:
     hipEvent_t m_xfer_ev; //!< orders ordered uploads after the compute stream
     std::mutex m_xfer_mtx;
     std::mutex m_cache_mtx;
-    std::map<std::string, std::shared_ptr<cached_launch> > m_launch_cache;
-    std::vector<std::string> m_launch_order;
+    struct launch_cache {
+        size_t max;
+        std::map<std::string, std::shared_ptr<cached_launch> > lists;
+        std::vector<std::string> order;      // least recently used first
+        void used(const std::string &key) {
+            std::vector<std::string>::iterator i = std::find(order.begin(), order.end(), key);
+            if(i != order.end()) order.erase(i);
+            order.push_back(key);
+        }
+    };
+    launch_cache m_launches[2] = { { 32, {}, {} }, { 64, {}, {} } };
+    bool drop_launches();
+    void *try_alloc(size_t bytes, std::string &why);
     size_t m_cap;
     std::atomic<size_t> m_used;
     std::mutex m_mtx;
