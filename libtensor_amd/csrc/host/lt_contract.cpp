@@ -1469,12 +1469,23 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         for(size_t i = 0; i < est.size(); i++)
             if(cfg != -2 || dev::is_stacked(est[i].second)) candidates.push_back(est[i].second);
         if(cfg == -1) candidates.resize(1);
-        // No timing (accumulating plans, planning beside other work): the
-        // measured line between the small tiles that start fastest and the
-        // tiles that move least data (14 and 22 us for 1.3e8 FLOPs, 47 and
-        // 35 us for 3.9e8).
-        else if(add || !measure)
+        // No timing, a launch by itself (accumulating plans, memory-bounded
+        // batches): the measured line between the small tiles that start
+        // fastest and the tiles that move least data (14 and 22 us for 1.3e8
+        // FLOPs, 47 and 35 us for 3.9e8).
+        else if(pl.batch || (add && measure))
             candidates.assign(1, flops < 2e8 ? dev::STACK_32x32_W4_O3 : dev::WG_64x64_G1);
+        // No timing, a launch merged with others' (the request loop): tiles
+        // over stacks in either case, small ones until a request by itself
+        // fills the CUs.  us to run batches of 1, 4 and 16 with 32 x 64 tiles,
+        // 64 x 64 and the split-K tiles that stacked fragment kernels leave to
+        // merged launches: ladders of 8.5e6 FLOPs 56, 60, 97; 62, 67, 88; 61,
+        // 103, 292; of 3.8e7 54, 65, 133; 70, 83, 112; 59, 113, 333; rings of
+        // 6.8e6 52, 89, 214; 61, 96, 221; 56, 89, 208; of 1.3e8 59, 129, 386;
+        // 64, 110, 299; 68, 126, 338; ladders of 3.9e8 102, 274, 995; 87, 194,
+        // 700; 168, 459, 1637.
+        else if(!measure)
+            candidates.assign(1, flops < 5e7 ? dev::WG_32x64_G4 : dev::WG_64x64_G1);
         // the configuration measured for these operands (same pairs, same
         // work list for any result tensor) is reused without measuring again
         if(cfg == -2 && m_tuned_cfg >= 0 && m_tuned_va == pl.va && m_tuned_vb == pl.vb)
@@ -2465,7 +2476,7 @@ batch_run::batch_run(std::vector<batch_item> &items, dev_buffer &merged) :
         cbs.clear(); prs.clear(); tl.clear(); tss.clear(); til.clear(); tsm.clear();
         size_t nparts = 0;
         uint32_t bm = 64, bn = 64;
-        dev::tile_shape(cfg, bm, bn);
+        dev::tile_shape(dev::unstacked(cfg), bm, bn);     // (of the kernel that runs the tiles)
         for(size_t x = x0; x < x1; x++) {
             contract_plan &pl = *m_plans[group[x]];
             if(dev::is_tile(cfg)) {

@@ -466,7 +466,7 @@ public:
         const std::function<void()> &between);
     //! Builds the execution plan for C unless it is cached (device memory
     //! for work lists and operand scratch, kernel autotuning).  measure
-    //! false: the kernel configuration is chosen by the padding estimate
+    //! false: the kernel configuration is chosen by the FLOPs
     //! instead of timed launches (callers whose stream is shared with other
     //! work, where timings would include that work).
     void prepare(btensor &c, bool add, double d, bool measure = true);
