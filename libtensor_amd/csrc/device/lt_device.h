@@ -87,8 +87,6 @@ static const uint32_t kPairVecBT = 16;
 static const uint32_t kPairOffArith = 32;
 //! B whose consecutive columns are adjacent in memory.
 static const uint32_t kPairBNFast = 64;
-//! Every A row of the pair has coefficient 1.
-static const uint32_t kPairUnit = 128;
 
 //! Work item of a grouped GEMM launch: one output tile of one C block.
 struct gemm_tile {

@@ -243,6 +243,7 @@ struct contract_plan {
     std::vector<dev::gemm_pair> pairs;
     std::vector<dev::gemm_tile> tiles_sorted, tiles_by_block;
     std::vector<uint32_t> block_tile_begin;
+    size_t n_tiles;                                   // tiles of all C blocks
     std::vector<double> cb_ksum;                      // sum of k over a C block's pairs
     std::vector<size_t> c_out;                        // canonical C blocks written
     bool batch;                                       // built for a batch of the schedule
@@ -336,7 +337,7 @@ struct contract_plan {
         ta(false), tb(false), tile_cfg(0), tile_order(0), d_prep(0), d_wback(0), d_prep_cd(0),
         d_prep_co(0), d_wb_cd(0), d_wb_co(0), n_prep_chunks(0), n_wb_chunks(0),
         prep_kind(), wb_kind(), prep_st_kind(), oz_prep_kind(),
-        d_cb(0), d_pairs(0), d_tiles_sorted(0), d_tiles_block(0), scratch(0),
+        d_cb(0), d_pairs(0), d_tiles_sorted(0), d_tiles_block(0), n_tiles(0), scratch(0),
         scratch_elems(0), ctx(0), events(false), graph(0), gexec(0), graph_launches(0),
         d_stacks(0), d_spairs(0), d_arows(0), d_crows(0), d_stiles(0), d_vtiles(0),
         d_tstacks(0), d_bstacks(0), d_titems(0), d_tsums(0), d_bitems(0), d_bsums(0),
@@ -1274,13 +1275,10 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
                         if(pairs_ok) sp.flags |= dev::kPairVecBT;
                     }
                 }
-                bool unit = true;
                 for(size_t q = 0; q < bl.size(); q++) {
                     const dev::gemm_pair &gq = pl.pairs[pl.cblocks[bl[q]].pair_begin + j];
                     if(q == 0 || (uintptr_t)gq.a < (uintptr_t)sp.a) sp.a = gq.a;
-                    unit = unit && gq.d * bscale == 1.0;
                 }
-                if(unit) sp.flags |= dev::kPairUnit;
                 pl.spairs.push_back(sp);
                 pl.spair_tab.push_back(std::make_pair(tb.koff, tb.noff));
                 ks += double(g.k);
@@ -1611,19 +1609,28 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
 
     // tile lists live in their own allocation (replaced by the autotuner)
     auto upload_tiles = [&](int k, int order) {
-        make_tiles(k, order, pl.tiles_by_block, pl.block_tile_begin, pl.tiles_sorted);
-        // the sorted list can be longer than the per-block list (padding
-        // tiles of the XCD-aware order)
-        size_t nt = pl.tiles_sorted.size() * sizeof(dev::gemm_tile);
-        size_t nb = pl.tiles_by_block.size() * sizeof(dev::gemm_tile);
-        size_t tsz = align256(nt) + align256(nb) + 256;
-        pl.tiles.at_least(ctx, tsz);
-        std::vector<char> th(tsz, 0);
-        if(nt) std::memcpy(&th[0], pl.tiles_sorted.data(), nt);
-        if(nb) std::memcpy(&th[align256(nt)], pl.tiles_by_block.data(), nb);
-        ctx.upload_new(pl.tiles.mem, th.data(), tsz);
-        pl.d_tiles_sorted = (dev::gemm_tile*)pl.tiles.mem;
-        pl.d_tiles_block = (dev::gemm_tile*)((char*)pl.tiles.mem + align256(nt));
+        if(!dev::is_tile(k)) {
+            make_tiles(k, order, pl.tiles_by_block, pl.block_tile_begin, pl.tiles_sorted);
+            // the sorted list can be longer than the per-block list (padding
+            // tiles of the XCD-aware order)
+            size_t nt = pl.tiles_sorted.size() * sizeof(dev::gemm_tile);
+            size_t nb = pl.tiles_by_block.size() * sizeof(dev::gemm_tile);
+            size_t tsz = align256(nt) + align256(nb) + 256;
+            pl.tiles.at_least(ctx, tsz);
+            std::vector<char> th(tsz, 0);
+            if(nt) std::memcpy(&th[0], pl.tiles_sorted.data(), nt);
+            if(nb) std::memcpy(&th[align256(nt)], pl.tiles_by_block.data(), nb);
+            ctx.upload_new(pl.tiles.mem, th.data(), tsz);
+            pl.d_tiles_sorted = (dev::gemm_tile*)pl.tiles.mem;
+            pl.d_tiles_block = (dev::gemm_tile*)((char*)pl.tiles.mem + align256(nt));
+            pl.n_tiles = pl.tiles_by_block.size();
+        } else {                     // (its items come from the stacks alone)
+            uint32_t bm, bn;
+            dev::tile_shape(k, bm, bn);
+            pl.n_tiles = 0;
+            for(size_t b = 0; b < null_cb; b++)
+                pl.n_tiles += size_t((pl.cblocks[b].m + bm - 1) / bm) * ((pl.cblocks[b].n + bn - 1) / bn);
+        }
         pl.tile_cfg = k;
         pl.tile_order = order;
         pl.stiles.clear();
@@ -1813,7 +1820,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
 
     m_stats.n_cblocks = null_cb;
     m_stats.n_pairs = nsched_pairs;
-    m_stats.n_tiles = pl.tiles_by_block.size();
+    m_stats.n_tiles = pl.n_tiles;
     m_stats.n_unfold = pl.prep.size();
     m_stats.flops = flops;
     m_stats.tile_cfg = cfg;
