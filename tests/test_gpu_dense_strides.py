@@ -69,7 +69,22 @@ def test_contract2_into_operand(gpu_ctx):
     assert np.all(abs(da.download() - a @ b) <= 2 * 72 * EPS * (abs(a) @ abs(b)))
 
 
-@pytest.mark.parametrize("dims", [(31, 3, 33), (32, 32), (33, 2, 33), (63, 65), (64, 3, 64), (130, 2, 67), (1, 200), (9, 1, 7, 40)], ids=str)
+# C beyond 32 MiB whose contiguous dimension leads neither index well: its
+# product goes through a contiguous copy, operands with short runs too
+STAGED = [(("iakc", "kcjb", "bija"), (59, 5, 239, 61, 2, 3)), (("ikac", "ckbj", "ajbi"), (5, 61, 59, 239, 1, 7)),
+          (("kica", "kcjb", "bija"), (59, 5, 239, 61, 2, 3)), (("kica", "kjcb", "bija"), (401, 5, 431, 5, 2, 3))]
+
+
+@pytest.mark.parametrize("zero", [True, False])
+@pytest.mark.parametrize("orders,shape", STAGED, ids=str)
+def test_contract2_into_short_runs(gpu_ctx, orders, shape, zero):
+    test_contract2(gpu_ctx, orders, shape, zero)
+
+
+# (from 2^18 elements on tiles are 64 wide where both extents are beyond 32,
+# from 2^22 on they are stored past the caches)
+@pytest.mark.parametrize("dims", [(31, 3, 33), (32, 32), (33, 2, 33), (63, 65), (64, 3, 64), (130, 2, 67), (1, 200), (9, 1, 7, 40),
+                                  (65, 63, 65), (33, 300, 33), (64, 65, 64), (130, 40, 67), (163, 161, 163), (1100, 31, 130)], ids=str)
 def test_permutes_sums_products(gpu_ctx, dims):
     print("permute", dims, flush=True)
     rng = np.random.default_rng(len(dims))
@@ -93,3 +108,14 @@ def test_permutes_sums_products(gpu_ctx, dims):
     y = rng.standard_normal(xt.shape)
     r = lt.tod_dotprod(dx, _dev(gpu_ctx, y), perm, None)
     assert abs(r - np.vdot(xt, y)) <= 2 * x.size * EPS * np.vdot(abs(xt), abs(y))
+
+
+def test_long_runs_past_the_caches(gpu_ctx):
+    x = np.random.default_rng(5).standard_normal((70, 61, 1009))
+    dx, out = _dev(gpu_ctx, x), lt.device_array(gpu_ctx, (61, 70, 1009))
+    lt.tod_copy(dx, out, (1, 0, 2), 3.0)
+    assert np.array_equal(out.download(), 3.0 * x.transpose(1, 0, 2))
+    lt.tod_copy(dx, out, (1, 0, 2), -1.0, zero=False)
+    # 3 x is rounded, and 3 x - x: at most (3 + 2) u |x|
+    ref = x.transpose(1, 0, 2)
+    assert np.all(abs(out.download() - 2.0 * ref) <= 5 * EPS * abs(ref) * (1 + EPS))

@@ -51,3 +51,28 @@ def test_zero_coefficient(gpu_ctx):
     c = P.make_result_tensor(gpu_ctx, prob)
     zero.perform(c)
     assert not np.any(c.to_dense())
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("where", [0, 1])
+@pytest.mark.parametrize("name", ["ladder_full", "ladder_perm", "self_ladder", "randsym_222"])
+def test_non_finite_elements_reach_the_result(gpu_ctx, name, where, value):
+    """An infinity or a NaN in a stored block: the same elements of C are
+    infinite and NaN as in the full list's sums (pairs whose coefficients
+    cancel are not left out)."""
+    prob, dense, meta, result = G.load(name)
+    a, b, op = P.build(gpu_ctx, prob, dense)
+    t = b if where else a
+    x = t.req_nonzero_blocks()[0]
+    blk = t.get_block(x)
+    blk.flat[blk.size // 2] = value
+    t.set_block(x, blk)
+    c = P.make_result_tensor(gpu_ctx, prob)
+    op.perform(c)
+    seen = 0
+    for x in op.get_schedule():
+        got, ref = c.get_block(x), op.compute_block_host(x, c.block_dims(x))
+        assert np.array_equal(np.isnan(got), np.isnan(ref)), x
+        assert np.array_equal(np.isinf(got), np.isinf(ref)), x
+        seen += np.count_nonzero(~np.isfinite(ref))
+    assert seen

@@ -12,8 +12,9 @@ pytestmark = pytest.mark.gpu
 CASES = [((31, 12, 33), ([7], [], [16])),
          ((72, 74, 70), ([5], [9], [])),
          ((66, 65, 64), ([], [], [])),
-         ((131, 33, 97), ([33], [1], [64]))]
-PERMS = [(2, 1, 0), (1, 2, 0), (0, 2, 1)]
+         ((131, 33, 97), ([33], [1], [64])),
+         ((170, 160, 165), ([40], [], [100]))]          # 2^22 elements: stores past the caches
+PERMS = [(2, 1, 0), (1, 2, 0), (0, 2, 1), (1, 0, 2)]
 
 
 def _tensor(ctx, dims, splits, data=None):

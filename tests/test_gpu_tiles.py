@@ -75,3 +75,29 @@ def test_non_finite_values_stay_in_their_rows_and_columns(gpu_ctx, cfg):
         ref = 0.5 * (a @ b)
     assert np.array_equal(np.isfinite(got), np.isfinite(ref))
     assert np.array_equal(np.isnan(got), np.isnan(ref))
+
+
+# 24 chunks of k and more: the tiles are cut into parts, inside pairs and at
+# their ends, and a second kernel adds the parts' sums
+CUT = [(33, 70, 400), (16, 64, 3000), (97, 129, 1033), (113, 66, 777)]
+
+
+@pytest.mark.parametrize("cfg", WG)
+@pytest.mark.parametrize("layout", [(False, False), (True, False), (False, True), (True, True)])
+def test_tiles_cut_along_k(gpu_ctx, cfg, layout):
+    ta, tb = layout
+    for m, n, k in CUT:
+        for sk in ([], [k // 2], [k // 3, k // 3 + 1, k - 17], [16 * (k // 32)]):
+            print("cut tiles", cfg, layout, m, n, k, sk, flush=True)
+            a, b, op, c = _product(gpu_ctx, m, n, k, ta, tb, [m // 3, m // 3 + 1], [n // 2], sk, m * 7919 + n * 31 + k)
+            op.set_tile(cfg)
+            ref, bound = 0.5 * (a @ b), (k + 2) * 2.0 ** -53 * (np.abs(a) @ np.abs(b)) * 2
+            op.perform(c, lt.LT_MODE_GROUPED)
+            got = c.to_dense()
+            assert np.all(np.abs(got - ref) <= bound), (m, n, k, sk)
+            op.perform(c, lt.LT_MODE_PER_BLOCK)
+            assert np.array_equal(c.to_dense(), got), (m, n, k, sk)
+            op.perform_add(c, -3.0, lt.LT_MODE_GROUPED)
+            assert np.all(np.abs(c.to_dense() + 2 * ref) <= 5 * bound), (m, n, k, sk)
+            op.perform_add(c, 3.0, lt.LT_MODE_PER_BLOCK)
+            assert np.all(np.abs(c.to_dense() - ref) <= 9 * bound), (m, n, k, sk)
