@@ -103,7 +103,7 @@ __device__ __forceinline__ void perm_store(const perm_desc &d, uint32_t e, doubl
 //! contiguous along p, the destination along q (extents and strides from
 //! dedicated fields: indexing the descriptor's arrays with a runtime dimension
 //! would put it in scratch memory).
-template<int S, bool NT, bool ADD>
+template<int S, bool NT, bool ADD, bool RUNS>
 __device__ __forceinline__ void permute_tile(const perm_desc &d, uint32_t base, double *tile) {
     constexpr int RW = 256 / S;          // rows at a time
     const uint32_t dq = d.tdq.d, dp = d.tdp.d;
@@ -115,10 +115,10 @@ __device__ __forceinline__ void permute_tile(const perm_desc &d, uint32_t base, 
     const uint32_t ti = threadIdx.x % S, tj = threadIdx.x / S;
     constexpr int R = S / RW;
     double w[R];
-    // a tile whose rows adjoin in memory is moved as one run (no idle lanes at
-    // short rows: 158 to 147 us for a two-term sum of 26 M elements)
+    // RUNS: a tile whose rows adjoin in memory is moved as one run (no idle
+    // lanes at short rows)
     const uint32_t nn = np * nq;
-    const bool ls = sq == np, ld = dps == nq;
+    const bool ls = RUNS && sq == np, ld = RUNS && dps == nq;
 #pragma unroll
     for(int r = 0; r < R; r++) {
         const uint32_t e = threadIdx.x + 256 * r, iq = tj + RW * r;
@@ -183,10 +183,10 @@ __device__ __forceinline__ void permute_gather(const perm_desc &d, uint32_t base
 }
 
 //! TILE: the largest tile side of the list's items (0: none is a tile), ADD:
-//! some descriptors are sums.  A kernel per kind: the 33 KB of LDS of 64-wide
-//! tiles let four workgroups onto a CU instead of eight, and in short launches
-//! the first instructions' way to the CU shows.
-template<bool NT, int TILE, bool ADD>
+//! some descriptors are sums, RUNS: tiles of short rows as runs.  A kernel per
+//! kind: the 33 KB of LDS of 64-wide tiles let four workgroups onto a CU instead
+//! of eight, and in short launches every instruction shows (perm_runs).
+template<bool NT, int TILE, bool ADD, bool RUNS>
 __global__ void __launch_bounds__(256)
 permute_kernel(const perm_desc *__restrict__ descs,
     const uint32_t *__restrict__ chunk_desc,
@@ -201,28 +201,27 @@ permute_kernel(const perm_desc *__restrict__ descs,
         permute_gather<NT, ADD>(d, base);
     } else {
         if(!(cd & kPermTileItem)) permute_gather<NT, ADD>(d, base);
-        else if(TILE == kPermTileMax && d.tile_s == kPermTileMax) permute_tile<TILE, NT, ADD>(d, base, tile);
-        else permute_tile<kPermTile, NT, ADD>(d, base, tile);
+        else if(TILE == kPermTileMax && d.tile_s == kPermTileMax) permute_tile<TILE, NT, ADD, RUNS>(d, base, tile);
+        else permute_tile<kPermTile, NT, ADD, RUNS>(d, base, tile);
     }
 }
 
-template<bool NT, bool ADD>
-static hipError_t launch_permute_t(const perm_desc *descs, const uint32_t *chunk_desc,
-    const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s, uint32_t tile) {
-    auto k = tile == 0 ? permute_kernel<NT, 0, ADD> : tile == kPermTile ? permute_kernel<NT, kPermTile, ADD> :
-        permute_kernel<NT, kPermTileMax, ADD>;
-    hipLaunchKernelGGL(k, dim3(nchunks), dim3(256), 0, s, descs, chunk_desc, chunk_off);
-    return hipGetLastError();
+template<bool NT, bool ADD, bool RUNS>
+static auto permute_kernel_of(uint32_t tile) {
+    return tile == 0 ? permute_kernel<NT, 0, ADD, false> : tile == kPermTile ? permute_kernel<NT, kPermTile, ADD, RUNS> :
+        permute_kernel<NT, kPermTileMax, ADD, RUNS>;
 }
 
 hipError_t launch_permute(const perm_desc *descs, const uint32_t *chunk_desc,
     const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s, perm_kind kind) {
     if(nchunks == 0) return hipSuccess;
-    if(kind.stream)
-        return kind.add ? launch_permute_t<true, true>(descs, chunk_desc, chunk_off, nchunks, s, kind.tile) :
-            launch_permute_t<true, false>(descs, chunk_desc, chunk_off, nchunks, s, kind.tile);
-    return kind.add ? launch_permute_t<false, true>(descs, chunk_desc, chunk_off, nchunks, s, kind.tile) :
-        launch_permute_t<false, false>(descs, chunk_desc, chunk_off, nchunks, s, kind.tile);
+    auto k = !kind.stream ? (kind.add ? permute_kernel_of<false, true, false>(kind.tile) :
+            permute_kernel_of<false, false, false>(kind.tile)) :
+        !kind.runs ? (kind.add ? permute_kernel_of<true, true, false>(kind.tile) :
+            permute_kernel_of<true, false, false>(kind.tile)) :
+        kind.add ? permute_kernel_of<true, true, true>(kind.tile) : permute_kernel_of<true, false, true>(kind.tile);
+    hipLaunchKernelGGL(k, dim3(nchunks), dim3(256), 0, s, descs, chunk_desc, chunk_off);
+    return hipGetLastError();
 }
 
 //! Work items of one descriptor by number: per destination dimension the
@@ -232,7 +231,7 @@ struct perm_items {
     uint32_t step[kPermMaxOrder];
 };
 
-template<int S, bool NT>
+template<int S, bool NT, bool RUNS>
 __global__ void __launch_bounds__(256) permute_tiles_kernel(perm_desc d, perm_items g) {
     __shared__ double tile[S * (S + 1)];
     uint32_t x = xcd_item(blockIdx.x, gridDim.x), base = 0;
@@ -244,7 +243,7 @@ __global__ void __launch_bounds__(256) permute_tiles_kernel(perm_desc d, perm_it
             x = q;
         }
     }
-    permute_tile<S, NT, true>(d, base, tile);
+    permute_tile<S, NT, true, RUNS>(d, base, tile);
 }
 
 template<bool NT>
@@ -271,9 +270,10 @@ hipError_t launch_permute_one(const perm_desc &d, hipStream_t s) {
         items *= cnt;
     }
     for(int i = int(d.n); i < kPermMaxOrder; i++) { g.it[i] = make_fastdiv(1); g.step[i] = 0; }
-    auto k = d.tile_s == kPermTileMax ?
-        (stream ? permute_tiles_kernel<kPermTileMax, true> : permute_tiles_kernel<kPermTileMax, false>) :
-        (stream ? permute_tiles_kernel<kPermTile, true> : permute_tiles_kernel<kPermTile, false>);
+    auto k = d.tile_s == kPermTileMax ? (!stream ? permute_tiles_kernel<kPermTileMax, false, false> :
+            perm_runs(d) ? permute_tiles_kernel<kPermTileMax, true, true> : permute_tiles_kernel<kPermTileMax, true, false>) :
+        !stream ? permute_tiles_kernel<kPermTile, false, false> :
+            perm_runs(d) ? permute_tiles_kernel<kPermTile, true, true> : permute_tiles_kernel<kPermTile, true, false>;
     hipLaunchKernelGGL(k, dim3((uint32_t)items), dim3(256), 0, s, d, g);
     return hipGetLastError();
 }

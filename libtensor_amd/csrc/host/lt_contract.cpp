@@ -205,9 +205,10 @@ void make_chunks(const std::vector<dev::perm_desc> &ds, std::vector<uint32_t> &c
 }
 
 dev::perm_kind list_kind(const std::vector<dev::perm_desc> &ds) {
-    dev::perm_kind k = { false, false, 0 };
+    dev::perm_kind k = { false, false, false, 0 };
     for(size_t i = 0; i < ds.size(); i++) {
         k.add = k.add || ds[i].add;
+        k.runs = k.runs || dev::perm_runs(ds[i]);
         if(ds[i].tile_p >= 0) k.tile = std::max(k.tile, ds[i].tile_s);
     }
     return k;

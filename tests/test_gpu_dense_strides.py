@@ -81,10 +81,12 @@ def test_contract2_into_short_runs(gpu_ctx, orders, shape, zero):
     test_contract2(gpu_ctx, orders, shape, zero)
 
 
-# (from 2^18 elements on tiles are 64 wide where both extents are beyond 32,
-# from 2^22 on they are stored past the caches)
+# (from 2^20 elements on tiles are 64 wide where the shorter side has 33 to 63
+# elements, and in scalar products where both are beyond 32; from 2^22 on they
+# are stored past the caches, short rows that adjoin as one run)
 @pytest.mark.parametrize("dims", [(31, 3, 33), (32, 32), (33, 2, 33), (63, 65), (64, 3, 64), (130, 2, 67), (1, 200), (9, 1, 7, 40),
-                                  (65, 63, 65), (33, 300, 33), (64, 65, 64), (130, 40, 67), (163, 161, 163), (1100, 31, 130)], ids=str)
+                                  (65, 63, 65), (33, 300, 33), (64, 65, 64), (130, 40, 67), (163, 161, 163), (1100, 31, 130),
+                                  (33, 970, 33), (63, 270, 63), (40, 660, 41), (41, 2600, 41), (9, 52000, 9)], ids=str)
 def test_permutes_sums_products(gpu_ctx, dims):
     print("permute", dims, flush=True)
     rng = np.random.default_rng(len(dims))
@@ -110,12 +112,13 @@ def test_permutes_sums_products(gpu_ctx, dims):
     assert abs(r - np.vdot(xt, y)) <= 2 * x.size * EPS * np.vdot(abs(xt), abs(y))
 
 
-def test_long_runs_past_the_caches(gpu_ctx):
-    x = np.random.default_rng(5).standard_normal((70, 61, 1009))
-    dx, out = _dev(gpu_ctx, x), lt.device_array(gpu_ctx, (61, 70, 1009))
-    lt.tod_copy(dx, out, (1, 0, 2), 3.0)
-    assert np.array_equal(out.download(), 3.0 * x.transpose(1, 0, 2))
-    lt.tod_copy(dx, out, (1, 0, 2), -1.0, zero=False)
+@pytest.mark.parametrize("dims,perm", [((70, 61, 1009), (1, 0, 2)), ((50000, 9, 11), (0, 2, 1)), ((3000, 33, 45), (0, 2, 1))], ids=str)
+def test_past_the_caches(gpu_ctx, dims, perm):
+    x = np.random.default_rng(5).standard_normal(dims)
+    ref = x.transpose(perm)
+    dx, out = _dev(gpu_ctx, x), lt.device_array(gpu_ctx, ref.shape)
+    lt.tod_copy(dx, out, perm, 3.0)
+    assert np.array_equal(out.download(), 3.0 * ref)
+    lt.tod_copy(dx, out, perm, -1.0, zero=False)
     # 3 x is rounded, and 3 x - x: at most (3 + 2) u |x|
-    ref = x.transpose(1, 0, 2)
     assert np.all(abs(out.download() - 2.0 * ref) <= 5 * EPS * abs(ref) * (1 + EPS))

@@ -8,12 +8,15 @@ import libtensor_amd as lt
 
 pytestmark = pytest.mark.gpu
 
-# extents, split points: blocks below and (both swapped extents beyond 32, 2^18 elements and more) above the line
+# extents, split points: blocks whose tiles are 32 or 64 wide (shorter side 33 to
+# 63, blocks from 2^18 elements on in lists from 2^20 on)
 CASES = [((31, 12, 33), ([7], [], [16])),
          ((72, 74, 70), ([5], [9], [])),
          ((66, 65, 64), ([], [], [])),
          ((131, 33, 97), ([33], [1], [64])),
-         ((170, 160, 165), ([40], [], [100]))]          # 2^22 elements: stores past the caches
+         ((45, 560, 42), ([], [20], [])),
+         # from 2^22 elements on: stores past the caches, short rows as runs
+         ((170, 160, 165), ([40], [], [100])), ((5000, 90, 11), ([100], [40], [])), ((62, 1100, 63), ([], [30], []))]
 PERMS = [(2, 1, 0), (1, 2, 0), (0, 2, 1), (1, 0, 2)]
 
 
