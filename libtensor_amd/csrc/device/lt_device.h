@@ -44,10 +44,8 @@ struct perm_desc {
     fastdiv dps;                      //!< destination stride of tile_p
     fastdiv tdp, tdq;                 //!< extents of tile_p and n - 1
 };
-//! Tile side: 64 where both extents are beyond 32 (rows of 512 bytes:
-//! 37 x 61 x 83 x 91 to 83 x 37 x 91 x 61 in 63 instead of 71 us), else 32;
-//! also 32 below kPermTileMin elements, where a launch has too few tiles.
-static const uint32_t kPermTile = 32, kPermTileMax = 64, kPermTileMin = 1u << 18;
+//! Tile sides; kPermWideList, kPermWide: see widen_tiles.
+static const uint32_t kPermTile = 32, kPermTileMax = 64, kPermWideList = 1u << 20, kPermWide = 1u << 18;
 static const uint32_t kPermTileItem = 0x80000000u;
 //! Launches that write this many elements (32 MiB, what the L2 caches hold) and
 //! more write past the caches (`stream`: 37 x 61 x 83 x 91 transposed 62 to

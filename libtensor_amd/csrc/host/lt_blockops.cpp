@@ -159,12 +159,13 @@ void add_descs(btensor &b, btensor &s, const tensor_tr &tr, double d,
 
 //! Uploads descriptor lists (one launch each) into one device buffer.
 std::shared_ptr<context::cached_launch> upload_launches(context &ctx,
-    const std::vector<std::vector<dev::perm_desc> > &lists) {
+    std::vector<std::vector<dev::perm_desc> > lists) {
     std::shared_ptr<context::cached_launch> l(new context::cached_launch(ctx));
     std::vector<char> host;
     size_t sz = 0;
     for(size_t i = 0; i < lists.size(); i++) {
         if(lists[i].empty()) continue;
+        widen_tiles(lists[i].data(), lists[i].size());
         size_t total = 0;
         bool tiles = false;
         for(size_t k = 0; k < lists[i].size(); k++) {

@@ -96,8 +96,6 @@ dev::perm_desc make_perm_desc(const double *src, const dims_t &dsrc,
             d.dps = dev::make_fastdiv((uint32_t)st);
             d.tdp = dev::make_fastdiv((uint32_t)fd[i]);
             d.tdq = dev::make_fastdiv((uint32_t)fd[nf - 1]);
-            if(std::min(fd[i], fd[nf - 1]) > dev::kPermTile && total >= dev::kPermTileMin)
-                d.tile_s = dev::kPermTileMax;
             break;
         }
     }
@@ -201,6 +199,19 @@ void make_chunks(const std::vector<dev::perm_desc> &ds, std::vector<uint32_t> &c
             }
             if(j < 0) break;
         }
+    }
+}
+
+void widen_tiles(dev::perm_desc *ds, size_t n) {
+    size_t total = 0;
+    for(size_t i = 0; i < n; i++) total += ds[i].total;
+    if(total < dev::kPermWideList) return;
+    for(size_t i = 0; i < n; i++) {
+        dev::perm_desc &d = ds[i];
+        if(d.tile_p < 0 || d.total < dev::kPermWide) continue;
+        const uint64_t p = d.tdp.d, q = d.tdq.d, m = std::min(p, q);
+        const uint64_t wide = ((p + 63) / 64) * ((q + 63) / 64) * 4096, narrow = ((p + 31) / 32) * ((q + 31) / 32) * 1024;
+        if(m > 32 && m < 64 && m % 16 && 3 * wide <= 4 * narrow) d.tile_s = dev::kPermTileMax;
     }
 }
 
@@ -1504,6 +1515,9 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
 
     // upload all lists in one allocation
     std::vector<uint32_t> pcd, pco, wcd, wco, scd, sco;
+    widen_tiles(pl.prep.data(), pl.prep.size());
+    widen_tiles(pl.wback.data(), pl.wback.size());
+    widen_tiles(pl.prep_st.data(), pl.prep_st.size());
     make_chunks(pl.prep, pcd, pco);
     make_chunks(pl.wback, wcd, wco);
     make_chunks(pl.prep_st, scd, sco);
@@ -2043,6 +2057,8 @@ void btod_contract2::build_ozaki(int slices) {
         sz = align256(sz + tl[k].size() * sizeof(dev::gemm_tile));
     }
     std::vector<uint32_t> pm_cd, pm_co, pi_cd, pi_co;
+    widen_tiles(prep_mut.data(), prep_mut.size());
+    widen_tiles(prep_inv.data(), prep_inv.size());
     make_chunks(prep_mut, pm_cd, pm_co);
     make_chunks(prep_inv, pi_cd, pi_co);
     size_t o_pm = sz; sz = align256(sz + prep_mut.size() * sizeof(dev::perm_desc));

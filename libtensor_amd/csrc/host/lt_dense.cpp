@@ -307,16 +307,19 @@ void launch(context &cx, dense_job &j, char *mem, double *parts) {
         return;
     }
     if(j.copy_a) {
+        widen_tiles(&j.pa, 1);
         j.g.a = j.pa.dst = (double*)mem;
         mem += round256(8 * j.na);
         hip_check(dev::launch_permute_one(j.pa, cx.stream()), "permute");
     }
     if(j.copy_b) {
+        widen_tiles(&j.pb, 1);
         j.g.b = j.pb.dst = (double*)mem;
         mem += round256(8 * j.nb);
         hip_check(dev::launch_permute_one(j.pb, cx.stream()), "permute");
     }
     if(j.copy_c) {
+        widen_tiles(&j.pc, 1);
         j.pc.src = j.g.c = (double*)mem;
         j.g.zero = 1;
     }
@@ -374,7 +377,8 @@ void run_jobs(context &cx, std::vector<dense_job> &jobs) {
 
 void dense_permute(context &cx, const double *src, const dims_t &dsrc,
     const tensor_tr &tr, double *dst, bool accumulate) {
-    const dev::perm_desc d = make_perm_desc_public(src, dsrc, tr, dst, accumulate);
+    dev::perm_desc d = make_perm_desc_public(src, dsrc, tr, dst, accumulate);
+    widen_tiles(&d, 1);
     if(!d.total) return;
     cx.activate();
     hip_check(dev::launch_permute_one(d, cx.stream()), "permute");
@@ -391,6 +395,7 @@ void dense_add(context &cx, const double *const *a, const dims_t &da,
     if(zero && ds.size() > 1 && !overlap(a[0], da.size(), b, da.size()) &&
         !overlap(a[1], da.size(), b, da.size())) fuse_terms(ds[0], ds[1]);
     cx.activate();
+    for(size_t i = 0; i < ds.size(); i++) widen_tiles(&ds[i], 1);
     for(size_t i = 0; i < ds.size(); i++)
         if(ds[i].total) hip_check(dev::launch_permute_one(ds[i], cx.stream()), "permute");
     cx.sync();

@@ -243,6 +243,16 @@ void host_transform(const double *src, const dims_t &dsrc, const tensor_tr &tr,
 void make_chunks(const std::vector<dev::perm_desc> &ds, std::vector<uint32_t> &cd,
     std::vector<uint32_t> &co);
 
+//! Gives the descriptors of one launch tiles of 64 instead of 32 where those
+//! hold a whole short side (33 to 63 elements, not in whole cache lines) and
+//! leave hardly more lanes idle, in launches of kPermWideList elements and more
+//! (below, too few tiles), blocks of kPermWide and more.  us with tiles of 32
+//! and 64: 40^4 reversed 14.7, 12.1; 35 x 3000 x 35 21.5, 16.1; 37 x 61 x 83 x 91
+//! to 83 x 37 x 91 x 61 out of memory 88, 77 a call; two-term sum of blocks of 41
+//! to 63 (26 M elements) 270, 265.  Not so for sides of 48 (+=: 25.1, 26.5), 64
+//! (9.7, 10.6), 70 x 80 (117, 141) or in short launches (512 x 513: 4.3, 6.8).
+void widen_tiles(dev::perm_desc *ds, size_t n);
+
 //! The kernel that a list of permute descriptors needs (stores through the
 //! caches).
 dev::perm_kind list_kind(const std::vector<dev::perm_desc> &ds);
@@ -290,7 +300,7 @@ void run_permutes(context &ctx, const std::vector<dev::perm_desc> &descs, double
 //! Descriptor lists (one launch each, in order) uploaded into one device
 //! buffer, for the context's launch cache.
 std::shared_ptr<context::cached_launch> upload_launches(context &ctx,
-    const std::vector<std::vector<dev::perm_desc> > &lists);
+    std::vector<std::vector<dev::perm_desc> > lists);
 //! Runs the launches of a cached entry in order and waits; ms (optional)
 //! accumulates their device time.
 void run_launches(context &ctx, const context::cached_launch &l, double *ms);
