@@ -326,17 +326,18 @@ template<bool TILES>
 __global__ void __launch_bounds__(256)
 dot_kernel(const perm_desc *__restrict__ descs,
     const uint32_t *__restrict__ chunk_desc,
-    const uint32_t *__restrict__ chunk_off, uint32_t nchunks, double *__restrict__ partials) {
+    const uint32_t *__restrict__ chunk_off, uint32_t nchunks, uint32_t per, uint32_t rest,
+    double *__restrict__ partials) {
 
     constexpr int E = kPermChunk / 256;
     __shared__ double tile[TILES ? kPermTileMax * (kPermTileMax + 1) : 256];
-    const uint32_t wg = xcd_item(blockIdx.x, gridDim.x);
-    const uint32_t c0 = uint32_t(uint64_t(nchunks) * wg / gridDim.x);
-    const uint32_t c1 = uint32_t(uint64_t(nchunks) * (wg + 1) / gridDim.x);
+    // per chunks a workgroup, one more in `rest` of all kDotGroups (none in fewer)
+    const uint32_t wg = TILES || nchunks > gridDim.x ? xcd_item(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t c0 = wg * per + wg * rest / kDotGroups, c1 = (wg + 1) * per + (wg + 1) * rest / kDotGroups;
     double sum = 0.0;
     for(uint32_t ch = c0; ch < c1; ch++) {
         const uint32_t cd = chunk_desc[ch];
-        const perm_desc &d = descs[cd & ~kPermTileItem];
+        const perm_desc d = descs[cd & ~kPermTileItem];
         const uint32_t base = chunk_off[ch];
         double acc = 0.0;
         if(TILES && (cd & kPermTileItem)) {
@@ -401,7 +402,7 @@ hipError_t launch_dot(const perm_desc *descs, const uint32_t *chunk_desc,
     const uint32_t ng = nchunks < kDotGroups ? nchunks : kDotGroups;
     if(ng > 0) {
         hipLaunchKernelGGL(tiles ? dot_kernel<true> : dot_kernel<false>, dim3(ng), dim3(256), 0, s,
-            descs, chunk_desc, chunk_off, nchunks, partials);
+            descs, chunk_desc, chunk_off, nchunks, nchunks / ng, nchunks % ng, partials);
     }
     hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, s, partials, ng, out);
     return hipGetLastError();

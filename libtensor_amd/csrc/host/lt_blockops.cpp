@@ -266,22 +266,6 @@ void fuse_launches(std::vector<std::vector<dev::perm_desc> > &lists) {
             [](const dev::perm_desc &d) { return d.total == 0; }), lists[i].end());
 }
 
-double run_dot(context &ctx, const context::cached_launch &l) {
-    if(l.segs.empty()) return 0.0;
-    const context::cached_launch::segment &g = l.segs[0];
-    std::lock_guard<std::mutex> lk(ctx.staging_lock());
-    const size_t np = std::min<size_t>(g.nchunks, dev::kDotGroups);
-    double *part = (double*)ctx.staging((np + 1) * sizeof(double));
-    char *base = (char*)l.mem;
-    double r = 0.0;
-    ctx.activate();
-    hip_check(dev::launch_dot((dev::perm_desc*)(base + g.o_d), (uint32_t*)(base + g.o_cd),
-        (uint32_t*)(base + g.o_co), (uint32_t)g.nchunks, g.tiles, part, part + np,
-        ctx.stream()), "dot");
-    ctx.download(&r, part + np, sizeof(double));
-    return r;
-}
-
 namespace {
 
 std::vector<size_t> distinct(std::vector<size_t> v) {

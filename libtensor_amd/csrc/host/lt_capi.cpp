@@ -292,8 +292,7 @@ int lt_tod_dotprod(lt_ctx *ctx, size_t n, const size_t *dims_a,
         q.permute(pa.inverse());
         dev::perm_desc d = make_perm_desc_public(b, db, tensor_tr(q, scalar_tr(c)),
             const_cast<double*>(a), false);
-        *result = run_dot(cx, *upload_launches(cx,
-            std::vector<std::vector<dev::perm_desc> >(1, std::vector<dev::perm_desc>(1, d))));
+        *result = dense_dotprod(cx, d);
     });
 }
 

@@ -12,7 +12,81 @@
 // partial sums are added in a fixed order.
 #include "lt_runtime.h"
 
+#include <algorithm>
+#include <cstring>
+
 namespace lta {
+
+namespace {
+
+//! A transposing descriptor is read by tiles only where a tile is well filled
+//! and reading element by element, in the destination's order, would not find
+//! its source lines in the caches (0.4 M elements: 5 to 6 us by elements in every
+//! order, 5 to 10 by tiles).  4 M elements, us by elements and by tiles
+//! (p: extent contiguous in the source, q: in the destination): p = q = 4, 8,
+//! 12, 16 and 32 at the ends of a three-dimensional tensor 27, 44, 61, 76, 77;
+//! 303, 83, 42, 28, 15.  Matrices with p = 5, 8, 12 and 16: 30, 43, 61, 80; 40,
+//! 28, 22, 18; with q = 5, 8, 16 and 24: 15, 15, 15, 14; 42, 28, 18, 16.  Last
+//! two dimensions swapped, p = q = 16, 32, 40, 48 and 64: 17, 16, 16, 16, 18; 27,
+//! 16, 18, 15, 15.  fill: elements that a tile must hold on the average, 144
+//! where the list is kept, 512 where it is made for one product (7 ns an item).
+void choose_tiles(dev::perm_desc &d, uint64_t fill) {
+    if(d.tile_p < 0) return;
+    const uint64_t p = d.tdp.d, q = d.tdq.d;
+    const uint64_t s = d.tile_s = std::min(p, q) > dev::kPermTile ? dev::kPermTileMax : dev::kPermTile;
+    const uint64_t tiles = ((p + s - 1) / s) * ((q + s - 1) / s);
+    if(d.total < (1u << 19) || std::min(p, q) < 8 || p * q < fill * tiles || (q <= 24 && d.dps.d == q) ||
+        8 * d.tsq * q <= 16384) d.tile_p = -1;
+}
+
+//! Partial sums of n work items, and the product behind them.
+size_t dot_bytes(size_t n) { return (std::min<size_t>(n, dev::kDotGroups) + 1) * sizeof(double); }
+
+//! The product of lists in device memory, partial sums at `part`.
+double run_dot(context &ctx, const char *base, const context::cached_launch::segment &g, double *part) {
+    double *out = part + std::min<size_t>(g.nchunks, dev::kDotGroups);
+    double r = 0.0;
+    hip_check(dev::launch_dot((dev::perm_desc*)(base + g.o_d), (uint32_t*)(base + g.o_cd),
+        (uint32_t*)(base + g.o_co), (uint32_t)g.nchunks, g.tiles, part, out, ctx.stream()), "dot");
+    ctx.download(&r, out, sizeof(double));
+    return r;
+}
+
+//! Scalar product of the (single) list of a cached entry: sum over its
+//! descriptors of dst * alpha P(src).
+double run_dot(context &ctx, const context::cached_launch &l) {
+    if(l.segs.empty()) return 0.0;
+    std::lock_guard<std::mutex> lk(ctx.staging_lock());
+    double *part = (double*)ctx.staging(dot_bytes(l.segs[0].nchunks));
+    ctx.activate();
+    return run_dot(ctx, (const char*)l.mem, l.segs[0], part);
+}
+
+} // unnamed namespace
+
+double dense_dotprod(context &ctx, dev::perm_desc d) {
+    choose_tiles(d, 512);
+    std::vector<uint32_t> cd, co;
+    make_chunks(std::vector<dev::perm_desc>(1, d), cd, co);
+    if(cd.empty()) return 0.0;
+    // descriptor and work items in the staging area, partial sums behind them
+    context::cached_launch::segment g;
+    g.o_d = 0;
+    g.o_cd = (sizeof(d) + 255) & ~size_t(255);
+    g.o_co = g.o_cd + ((4 * cd.size() + 255) & ~size_t(255));
+    g.nchunks = cd.size();
+    g.tiles = d.tile_p >= 0;
+    const size_t bytes = g.o_co + ((4 * co.size() + 255) & ~size_t(255));
+    std::vector<char> host(bytes, 0);
+    std::memcpy(&host[0], &d, sizeof(d));
+    std::memcpy(&host[g.o_cd], cd.data(), 4 * cd.size());
+    std::memcpy(&host[g.o_co], co.data(), 4 * co.size());
+    std::lock_guard<std::mutex> lk(ctx.staging_lock());
+    char *mem = (char*)ctx.staging(bytes + dot_bytes(g.nchunks));
+    ctx.upload(mem, host.data(), bytes);
+    ctx.activate();
+    return run_dot(ctx, mem, g, (double*)(mem + bytes));
+}
 
 double btod_dotprod(btensor &a, const tensor_tr &tra0, btensor &b, const tensor_tr &trb0) {
     context &ctx = a.ctx();
@@ -55,6 +129,7 @@ double btod_dotprod(btensor &a, const tensor_tr &tra0, btensor &b, const tensor_
         dev::perm_desc d = make_perm_desc_public(b.block_ptr(sb.acidx), dyb, t,
             a.block_ptr(sa.acidx), false);
         d.alpha *= ta.st.c * ta.st.c;
+        choose_tiles(d, 144);
         descs.push_back(d);
     }
     l = upload_launches(ctx, lists);

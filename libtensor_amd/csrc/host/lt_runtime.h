@@ -276,6 +276,9 @@ void add_into(btensor &b, btensor &s, const tensor_tr &tr, double d, double *ms 
 //! btod_dotprod(A, tra, B, trb).calculate() on resident block tensors.
 double btod_dotprod(btensor &a, const tensor_tr &tra, btensor &b, const tensor_tr &trb);
 
+//! Sum of dst * alpha P(src) over a descriptor's elements (tod_dotprod).
+double dense_dotprod(context &ctx, dev::perm_desc d);
+
 //! btod_copy(a, tra).perform(b) (add false: B := tra(A), B takes the permuted
 //! symmetry of A) or perform(b, d) (add: B += d tra(A), B with that symmetry).
 void btod_copy(btensor &a, const tensor_tr &tra, btensor &b, bool add, double d);
@@ -311,9 +314,6 @@ void run_launches(context &ctx, const context::cached_launch &l, double *ms);
 bool fuse_terms(dev::perm_desc &first, dev::perm_desc &second);
 //! fuse_terms over launches in order, for each block's first two terms.
 void fuse_launches(std::vector<std::vector<dev::perm_desc> > &lists);
-//! Scalar product of the (single) list of a cached entry: sum over its
-//! descriptors of dst * alpha P(src).
-double run_dot(context &ctx, const context::cached_launch &l);
 //! Launch-cache key parts: a transformation; a tensor's identity and (with
 //! version) its structure version.
 std::string key_part(const tensor_tr &tr);
