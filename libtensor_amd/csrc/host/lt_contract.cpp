@@ -117,6 +117,11 @@ struct dev_lists {
         mem = 0;
         bytes = 0;
     }
+    void swap(dev_lists &o) {
+        std::swap(ctx, o.ctx);
+        std::swap(mem, o.mem);
+        std::swap(bytes, o.bytes);
+    }
     //! At least `n` bytes (contents not kept).
     void *at_least(context &c, size_t n) { return mem && bytes >= n ? mem : reset(c, n); }
     //! Replaces the allocation with a new one of `n` bytes.
@@ -698,8 +703,11 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     double t0 = now_ms();
     m_stats.n_plans++;
     context &ctx = m_a.ctx();
+    std::unique_ptr<contract_plan> last(std::move(m_plan));
     m_plan.reset(new contract_plan());
     contract_plan &pl = *m_plan;
+    if(last) pl.parts.swap(last->parts);      // (its work on the stream comes first)
+    last.reset();
     pl.va = m_a.version();
     pl.vb = m_b.version();
     pl.c = &c;
@@ -714,6 +722,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     std::vector<size_t> nza = m_a.nonzero_blocks(), nzb = m_b.nonzero_blocks();
     if(nza.empty() || nzb.empty() || sched.empty()) {
         pl.empty = true;
+        pl.parts.release();
         return;
     }
 
@@ -1833,6 +1842,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         m_tuned_vb = pl.vb;
     }
 
+    if(!dev::is_tile(cfg)) pl.parts.release();
     m_stats.n_cblocks = null_cb;
     m_stats.n_pairs = nsched_pairs;
     m_stats.n_tiles = pl.n_tiles;
