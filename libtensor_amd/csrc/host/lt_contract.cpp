@@ -29,6 +29,7 @@
 #include <chrono>
 #include <cmath>
 #include <numeric>
+#include <string>
 #include <unordered_map>
 
 namespace lta {
@@ -839,51 +840,57 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     // FLOPs and pairs are counted before, as the schedule has them.
     double flops = 0.0;
     size_t nsched_pairs = 0;
-    std::vector<std::vector<double> > pair_mult(clsts.size());
+    std::vector<std::vector<double> > pair_d(clsts.size());   // coefficient of every kept pair
+    struct kept_t { size_t pos; double c, d, mult; };
+    std::unordered_map<std::string, kept_t> kept;
+    std::string key;
+    std::vector<std::pair<size_t, size_t> > inner;
     for(size_t t = 0; t < clsts.size(); t++) {
-        typedef std::vector<size_t> key_t;
-        struct kept_t { size_t pos; double c; };
-        std::map<key_t, kept_t> kept;
+        kept.clear();
         contr_list &cl = clsts[t];
-        std::vector<double> &mult = pair_mult[t];
+        std::vector<double> &pd = pair_d[t];
         contr_list::iterator p = cl.begin();
         while(p != cl.end()) {
             const src_t &sa = srca[p->aia], &sb = srcb[p->aib];
-            const double c = pair_coeff(*p) * sa.tr.st.c * sb.tr.st.c;
-            if(c == 0.0) { mult.push_back(1.0); ++p; continue; }    // (skipped below)
+            const double d = pair_coeff(*p), c = d * sa.tr.st.c * sb.tr.st.c;
+            if(c == 0.0) { pd.push_back(d); ++p; continue; }        // (skipped below)
             gemm_form g = aligned_gemm_form(contr, bisa2.block_dims(get_index(p->aia, bida2)),
                 bisb2.block_dims(get_index(p->aib, bidb2)));
             flops += 2.0 * double(g.m) * double(g.n) * double(g.k);
             nsched_pairs++;
             // stored blocks, the stored dimension of every outer index, and
             // the contracted dimensions as pairs in a fixed order
-            key_t key;
-            key.push_back(sa.y);
-            key.push_back(sb.y);
-            std::vector<std::pair<size_t, size_t> > inner;
+            key.assign((const char*)&sa.y, sizeof(sa.y));
+            key.append((const char*)&sb.y, sizeof(sb.y));
+            inner.clear();
             const size_t NC = contr.NC(), NA = contr.NA(), NB = contr.NB();
             for(size_t i = 0; i < NA; i++) {
-                if(contr.conn[NC + i] < NC + NA) key.push_back(sa.tr.perm[i]);
+                if(contr.conn[NC + i] < NC + NA) key.push_back(char(sa.tr.perm[i]));
                 else inner.push_back(std::make_pair(size_t(sa.tr.perm[i]),
                     size_t(sb.tr.perm[contr.conn[NC + i] - NC - NA])));
             }
             for(size_t i = 0; i < NB; i++)
-                if(contr.conn[NC + NA + i] < NC) key.push_back(sb.tr.perm[i]);
+                if(contr.conn[NC + NA + i] < NC) key.push_back(char(sb.tr.perm[i]));
             std::sort(inner.begin(), inner.end());
             for(size_t i = 0; i < inner.size(); i++) {
-                key.push_back(inner[i].first);
-                key.push_back(inner[i].second);
+                key.push_back(char(inner[i].first));
+                key.push_back(char(inner[i].second));
             }
-            std::map<key_t, kept_t>::iterator k = kept.find(key);
-            // (coefficients that cancel keep their pairs: an infinity or a
-            // NaN in the operands must still reach C)
-            if(k != kept.end() && mult[k->second.pos] + c / k->second.c != 0.0) {
-                mult[k->second.pos] += c / k->second.c;
-                p = cl.erase(p);
-                continue;
+            const std::pair<std::unordered_map<std::string, kept_t>::iterator, bool> k =
+                kept.insert(std::make_pair(key, kept_t{pd.size(), c, d, 1.0}));
+            if(!k.second) {
+                // (coefficients that cancel keep their pairs: an infinity or a
+                // NaN in the operands must still reach C)
+                kept_t &f = k.first->second;
+                const double mult = f.mult + c / f.c;
+                if(mult != 0.0 && std::isfinite(mult * f.c)) {
+                    f.mult = mult;
+                    pd[f.pos] = f.d * mult;
+                    p = cl.erase(p);
+                    continue;
+                }
             }
-            if(k == kept.end()) kept[key] = kept_t{mult.size(), c};
-            mult.push_back(1.0);
+            pd.push_back(d);
             ++p;
         }
     }
@@ -1120,7 +1127,7 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         double ksum = 0.0;
         size_t pi = 0;
         for(contr_list::const_iterator p = cl.begin(); p != cl.end(); ++p) {
-            double d = pair_coeff(*p) * pair_mult[t][pi++];
+            double d = pair_d[t][pi++];
             if(add) d *= dscale;
             if(d == 0.0) continue;
             dims_t da = bisa2.block_dims(get_index(p->aia, bida2));
@@ -1205,8 +1212,19 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
         // offsets from its lowest one: a group whose A blocks of one pair lie
         // farther apart is cut into several stacks.
         std::vector<std::vector<size_t> > cut;
+        uintptr_t first = ~uintptr_t(0), last = 0;             // of all A blocks
+        for(size_t b = 0; b < pl.cblocks.size(); b++)
+            for(uint32_t p = pl.cblocks[b].pair_begin; p < pl.cblocks[b].pair_end; p++) {
+                const uintptr_t a = (uintptr_t)pl.pairs[p].a;
+                first = std::min(first, a);
+                last = std::max(last, a + size_t(pl.cblocks[b].m) * pl.pairs[p].k * sizeof(double));
+            }
         for(size_t gi = 0; gi < order.size(); gi++) {
             const std::vector<size_t> &all = groups[order[gi]];
+            if(first < last && last - first < (uintptr_t(1) << 32)) {
+                cut.push_back(all);
+                continue;
+            }
             std::vector<std::pair<uintptr_t, uintptr_t> > span;    // first and last byte per pair
             for(size_t q = 0; q < all.size(); q++) {
                 const dev::gemm_cblock &cq = pl.cblocks[all[q]];
