@@ -281,6 +281,10 @@ int lt_btod_contract2_compute_block_host(lt_btod_contract2 *op, size_t aidx_c,
 int lt_btod_contract2_compute_block(lt_btod_contract2 *op, int zero, size_t aidx_c,
     const size_t *perm, double coeff, double *blk);
 int lt_btod_contract2_stats(lt_btod_contract2 *op, lt_stats *out);
+/* FLOPs that the products of the last plan run: lt_stats.flops counts the
+ * schedule's pairs, of which those that are the same product run once.  No
+ * counterpart in the reference. */
+int lt_btod_contract2_executed_flops(lt_btod_contract2 *op, double *flops);
 /* Kernel configuration of the contraction GEMM: 0..27 fixed, -1 chosen by a
  * padding estimate, -2 (default) measured on the plan's own work list when
  * it is built (autotuner). */

@@ -426,6 +426,13 @@ class btod_contract2(object):
         out["tune_ms"] = list(out["tune_ms"])
         return out
 
+    def executed_flops(self):
+        """FLOPs of the products that the last plan runs (pairs that are the
+        same product run once)."""
+        v = ctypes.c_double()
+        call("lt_btod_contract2_executed_flops", self._h, ctypes.byref(v))
+        return v.value
+
     def set_tile(self, cfg):
         call("lt_btod_contract2_set_tile", self._h, int(cfg))
 

@@ -139,6 +139,7 @@ _SIGS = {
     "lt_btod_contract2_compute_block": [vp, ctypes.c_int, ctypes.c_size_t, c_size_p,
                                         ctypes.c_double, vp],
     "lt_btod_contract2_stats": [vp, ctypes.POINTER(LtStats)],
+    "lt_btod_contract2_executed_flops": [vp, ctypes.POINTER(ctypes.c_double)],
     "lt_btod_contract2_set_tile": [vp, ctypes.c_int],
     "lt_btod_contract2_set_graph": [vp, ctypes.c_int],
 "lt_btod_contract2_set_async": [vp, ctypes.c_int],

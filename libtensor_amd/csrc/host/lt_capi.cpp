@@ -1099,6 +1099,13 @@ int lt_btod_contract2_stats(lt_btod_contract2 *op, lt_stats *out) {
     });
 }
 
+int lt_btod_contract2_executed_flops(lt_btod_contract2 *op, double *flops) {
+    return guard([&]() {
+        need(op, "op"); need(flops, "flops");
+        *flops = op->op->executed_flops();
+    });
+}
+
 int lt_btod_contract2_set_tile(lt_btod_contract2 *op, int cfg) {
     return guard([&]() {
         need(op, "op");

@@ -1861,6 +1861,9 @@ void btod_contract2::build_plan(btensor &c, bool add, double dscale, bool measur
     }
 
     if(!dev::is_tile(cfg)) pl.parts.release();
+    m_executed_flops = 0.0;
+    for(size_t b = 0; b < null_cb; b++)
+        m_executed_flops += 2.0 * double(pl.cblocks[b].m) * double(pl.cblocks[b].n) * cb_ksum[b];
     m_stats.n_cblocks = null_cb;
     m_stats.n_pairs = nsched_pairs;
     m_stats.n_tiles = pl.n_tiles;

@@ -506,6 +506,8 @@ public:
     //! split-precision tile shape (dev::oz_tile_cfg), -1 = measured per plan
     void set_ozaki_tile(int tile) { m_oz_tile = tile; }
     double flops() const { return m_stats.flops; }
+    //! FLOPs that the products of the last plan run (equal pairs once).
+    double executed_flops() const { return m_executed_flops; }
 
 private:
     contraction2 m_contr;
@@ -515,6 +517,7 @@ private:
     symmetry m_symc;
     std::vector<size_t> m_sched;
     exec_stats m_stats;
+    double m_executed_flops = 0.0;
     int m_tile_cfg;         //!< >= 0 fixed, -1 estimate, -2 autotune
     int m_tuned_cfg;        //!< configuration found by the autotuner
     int m_tuned_order;      //!< and its grouped-launch tile order

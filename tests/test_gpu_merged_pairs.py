@@ -43,6 +43,15 @@ def test_statistics_count_the_schedule(gpu_ctx):
     assert st["n_pairs"] == pairs and st["flops"] == flops
 
 
+@pytest.mark.parametrize("name,fewer", [("ladder_nosym", False), ("ring_small", False), ("ladder_full", True), ("ladder_perm", True)])
+def test_executed_flops(gpu_ctx, name, fewer):
+    prob, dense, meta, result = G.load(name)
+    a, b, op = P.build(gpu_ctx, prob, dense)
+    op.perform(P.make_result_tensor(gpu_ctx, prob))
+    run, listed = op.executed_flops(), op.stats()["flops"]
+    assert 0.5 * listed <= run < listed if fewer else run == listed
+
+
 def test_zero_coefficient(gpu_ctx):
     """A contraction scaled by zero writes zeros."""
     prob, dense, meta, result = G.load("ladder_full")
