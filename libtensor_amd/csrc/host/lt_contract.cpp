@@ -2256,7 +2256,7 @@ void btod_contract2::enqueue(int mode, hipStream_t s, bool timed, size_t &launch
         ctx.side_join(s);
     } else {
         hip_check(launch_grouped(pl, pl.tile_cfg, s), "gemm (grouped)");
-        launches++;
+        launches += dev::is_tile(pl.tile_cfg) && !pl.tl.sums.empty() ? 2 : 1;
     }
     if(timed && mode != MODE_OZAKI) hip_check(hipEventRecord(pl.ev[2], s), "hipEventRecord");
     if(pl.n_wb_chunks) {

@@ -36,7 +36,7 @@ void choose_tiles(dev::perm_desc &d, uint64_t fill) {
     const uint64_t s = d.tile_s = std::min(p, q) > dev::kPermTile ? dev::kPermTileMax : dev::kPermTile;
     const uint64_t tiles = ((p + s - 1) / s) * ((q + s - 1) / s);
     if(d.total < (1u << 19) || std::min(p, q) < 8 || p * q < fill * tiles || (q <= 24 && d.dps.d == q) ||
-        8 * d.tsq * q <= 16384) d.tile_p = -1;
+        8 * uint64_t(d.tsq) * q <= 16384) d.tile_p = -1;
 }
 
 //! Partial sums of n work items, and the product behind them.

@@ -484,7 +484,8 @@ public:
         return plan_valid(c, add, d, MODE_GROUPED);
     }
     //! Device memory a plan may take: four orientations of every stored A
-    //! and B block plus the scheduled C blocks (admission estimate).
+    //! and B block plus the scheduled C blocks (admission estimate; partial
+    //! sums take memory only where there is room).
     size_t footprint_estimate();
 
     //! Statistics of the last perform (device times wait for an
