@@ -222,9 +222,11 @@ hipError_t launch_gemm_stacked(int cfg, const stack_desc *st, const stack_pair *
 //! with stream only).
 struct perm_kind { bool stream, add, runs; uint32_t tile; };
 //! Tiles with rows shorter than the tile that adjoin in memory.  Launches past
-//! the caches move them as one run (two-term sum of 26 M elements 158 to
-//! 147 us); in shorter ones the divisions cost more than the idle lanes (blocks
-//! of 25 to 49 x 400 to 961 elements, 1.3 M in all: 8.2 us with runs, 6.7 without).
+//! the caches move them as one run where they add (two-term sum of 26 M elements
+//! 174 to 164 us a call, += of blocks of 37 to 55 248 to 216) or consist of one
+//! permutation (37 x 61 x 83 x 91 transposed 79.8 to 77.5 us); in copies of many
+//! blocks and in shorter launches the divisions cost more than the idle lanes
+//! (29 M elements 101 us without runs, 112 with; 1.3 M elements 6.7, 8.2).
 inline bool perm_runs(const perm_desc &d) {
     return d.tile_p >= 0 && ((d.tdp.d < d.tile_s && d.tsq == d.tdp.d) || (d.tdq.d < d.tile_s && d.dps.d == d.tdq.d));
 }

@@ -217,7 +217,7 @@ void widen_tiles(dev::perm_desc *ds, size_t n) {
         if(d.tile_p < 0 || d.total < dev::kPermWide) continue;
         const uint64_t p = d.tdp.d, q = d.tdq.d, m = std::min(p, q);
         const uint64_t wide = ((p + 63) / 64) * ((q + 63) / 64) * 4096, narrow = ((p + 31) / 32) * ((q + 31) / 32) * 1024;
-        if(m > 32 && m < 64 && m % 16 && 3 * wide <= 4 * narrow) d.tile_s = dev::kPermTileMax;
+        if(d.add != d.dst && m > 32 && m < 64 && m % 16 && 3 * wide <= 4 * narrow) d.tile_s = dev::kPermTileMax;
     }
 }
 
@@ -225,7 +225,7 @@ dev::perm_kind list_kind(const std::vector<dev::perm_desc> &ds) {
     dev::perm_kind k = { false, false, false, 0 };
     for(size_t i = 0; i < ds.size(); i++) {
         k.add = k.add || ds[i].add;
-        k.runs = k.runs || dev::perm_runs(ds[i]);
+        k.runs = k.runs || (ds[i].add && dev::perm_runs(ds[i]));
         if(ds[i].tile_p >= 0) k.tile = std::max(k.tile, ds[i].tile_s);
     }
     return k;

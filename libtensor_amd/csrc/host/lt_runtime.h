@@ -250,7 +250,9 @@ void make_chunks(const std::vector<dev::perm_desc> &ds, std::vector<uint32_t> &c
 //! and 64: 40^4 reversed 14.7, 12.1; 35 x 3000 x 35 21.5, 16.1; 37 x 61 x 83 x 91
 //! to 83 x 37 x 91 x 61 out of memory 88, 77 a call; two-term sum of blocks of 41
 //! to 63 (26 M elements) 270, 265.  Not so for sides of 48 (+=: 25.1, 26.5), 64
-//! (9.7, 10.6), 70 x 80 (117, 141) or in short launches (512 x 513: 4.3, 6.8).
+//! (9.7, 10.6), 70 x 80 (117, 141), in short launches (512 x 513: 4.3, 6.8) or
+//! where the destination is added to (blocks of 63 to 100, 108 M elements: 536,
+//! 804).
 void widen_tiles(dev::perm_desc *ds, size_t n);
 
 //! The kernel that a list of permute descriptors needs (stores through the
