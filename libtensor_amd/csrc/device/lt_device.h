@@ -345,6 +345,8 @@ static const uint32_t kDotGroups = 2048;
 hipError_t launch_dot(const perm_desc *descs, const uint32_t *chunk_desc,
     const uint32_t *chunk_off, uint32_t nchunks, bool tiles, double *partials,
     double *out, hipStream_t s);
+//! One descriptor element by element, without lists in memory.
+hipError_t launch_dot_one(const perm_desc &d, double *partials, double *out, hipStream_t s);
 
 //! Size of the fixed device scratch region of the no-allocation entry
 //! points (one per GPU, held until the process ends).

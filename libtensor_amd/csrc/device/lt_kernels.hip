@@ -324,6 +324,49 @@ __device__ __forceinline__ double dot_tile(const perm_desc &d, uint32_t base, do
     return acc;
 }
 
+//! One chunk element by element.
+__device__ __forceinline__ double dot_gather(const perm_desc &d, uint32_t base) {
+    constexpr int E = kPermChunk / 256;
+    double acc = 0.0;
+    const uint32_t end = min(base + kPermChunk, d.total);
+    double v[E], w[E];
+    if(d.n == 1 && d.sstride[0] == 1 && end - base == kPermChunk &&
+        ((uintptr_t(d.src) | uintptr_t(d.dst)) & 15) == 0) {
+        const double2_t *x = (const double2_t *)(d.src + base), *y = (const double2_t *)(d.dst + base);
+#pragma unroll
+        for(int i = 0; i < E; i += 2) {
+            const double2_t p = x[threadIdx.x + 128 * i], q = y[threadIdx.x + 128 * i];
+            v[i] = p.x; v[i + 1] = p.y;
+            w[i] = q.x; w[i + 1] = q.y;
+        }
+#pragma unroll
+        for(int i = 0; i < E; i++) acc += w[i] * v[i];
+    } else {
+#pragma unroll
+        for(int i = 0; i < E; i++) {
+            const uint32_t e = min(base + threadIdx.x + 256u * i, end - 1);
+            v[i] = d.src[src_offset(d, e)];
+            w[i] = d.dst[e];
+        }
+#pragma unroll
+        for(int i = 0; i < E; i++)
+            if(base + threadIdx.x + 256u * i < end) acc += w[i] * v[i];
+    }
+    return acc;
+}
+
+//! The workgroup's sum.
+__device__ __forceinline__ void dot_reduce(double sum, double *red, double *__restrict__ partials) {
+    __syncthreads();
+    red[threadIdx.x] = sum;
+    __syncthreads();
+    for(uint32_t w = 128; w > 0; w >>= 1) {
+        if(threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+        __syncthreads();
+    }
+    if(threadIdx.x == 0) partials[blockIdx.x] = red[0];
+}
+
 template<bool TILES>
 __global__ void __launch_bounds__(256)
 dot_kernel(const perm_desc *__restrict__ descs,
@@ -331,7 +374,6 @@ dot_kernel(const perm_desc *__restrict__ descs,
     const uint32_t *__restrict__ chunk_off, uint32_t nchunks, uint32_t per, uint32_t rest,
     double *__restrict__ partials) {
 
-    constexpr int E = kPermChunk / 256;
     __shared__ double tile[TILES ? kPermTileMax * (kPermTileMax + 1) : 256];
     // per chunks a workgroup, one more in `rest` of all kDotGroups (none in fewer)
     const uint32_t wg = TILES || nchunks > gridDim.x ? xcd_item(blockIdx.x, gridDim.x) : blockIdx.x;
@@ -346,42 +388,22 @@ dot_kernel(const perm_desc *__restrict__ descs,
             acc = d.tile_s == kPermTileMax ? dot_tile<kPermTileMax>(d, base, tile) :
                 dot_tile<kPermTile>(d, base, tile);
         } else {
-            const uint32_t end = min(base + kPermChunk, d.total);
-            double v[E], w[E];
-            if(d.n == 1 && d.sstride[0] == 1 && end - base == kPermChunk &&
-                ((uintptr_t(d.src) | uintptr_t(d.dst)) & 15) == 0) {
-                const double2_t *x = (const double2_t *)(d.src + base), *y = (const double2_t *)(d.dst + base);
-#pragma unroll
-                for(int i = 0; i < E; i += 2) {
-                    const double2_t p = x[threadIdx.x + 128 * i], q = y[threadIdx.x + 128 * i];
-                    v[i] = p.x; v[i + 1] = p.y;
-                    w[i] = q.x; w[i + 1] = q.y;
-                }
-#pragma unroll
-                for(int i = 0; i < E; i++) acc += w[i] * v[i];
-            } else {
-#pragma unroll
-                for(int i = 0; i < E; i++) {
-                    const uint32_t e = min(base + threadIdx.x + 256u * i, end - 1);
-                    v[i] = d.src[src_offset(d, e)];
-                    w[i] = d.dst[e];
-                }
-#pragma unroll
-                for(int i = 0; i < E; i++)
-                    if(base + threadIdx.x + 256u * i < end) acc += w[i] * v[i];
-            }
+            acc = dot_gather(d, base);
         }
         sum += acc * d.alpha;
     }
-    __syncthreads();
-    double *red = tile;
-    red[threadIdx.x] = sum;
-    __syncthreads();
-    for(uint32_t w = 128; w > 0; w >>= 1) {
-        if(threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if(threadIdx.x == 0) partials[blockIdx.x] = red[0];
+    dot_reduce(sum, tile, partials);
+}
+
+//! One descriptor, passed with the launch, element by element.
+__global__ void __launch_bounds__(256)
+dot_one_kernel(perm_desc d, uint32_t nchunks, uint32_t per, uint32_t rest, double *__restrict__ partials) {
+    __shared__ double red[256];
+    const uint32_t wg = nchunks > gridDim.x ? xcd_item(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t c0 = wg * per + wg * rest / kDotGroups, c1 = (wg + 1) * per + (wg + 1) * rest / kDotGroups;
+    double sum = 0.0;
+    for(uint32_t ch = c0; ch < c1; ch++) sum += dot_gather(d, ch * kPermChunk) * d.alpha;
+    dot_reduce(sum, red, partials);
 }
 
 __global__ void __launch_bounds__(256)
@@ -405,6 +427,16 @@ hipError_t launch_dot(const perm_desc *descs, const uint32_t *chunk_desc,
     if(ng > 0) {
         hipLaunchKernelGGL(tiles ? dot_kernel<true> : dot_kernel<false>, dim3(ng), dim3(256), 0, s,
             descs, chunk_desc, chunk_off, nchunks, nchunks / ng, nchunks % ng, partials);
+    }
+    hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, s, partials, ng, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_dot_one(const perm_desc &d, double *partials, double *out, hipStream_t s) {
+    const uint32_t nchunks = (d.total + kPermChunk - 1) / kPermChunk;
+    const uint32_t ng = nchunks < kDotGroups ? nchunks : kDotGroups;
+    if(ng > 0) {
+        hipLaunchKernelGGL(dot_one_kernel, dim3(ng), dim3(256), 0, s, d, nchunks, nchunks / ng, nchunks % ng, partials);
     }
     hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, s, partials, ng, out);
     return hipGetLastError();

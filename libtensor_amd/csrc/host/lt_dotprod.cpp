@@ -28,14 +28,16 @@ namespace {
 //! 303, 83, 42, 28, 15.  Matrices with p = 5, 8, 12 and 16: 30, 43, 61, 80; 40,
 //! 28, 22, 18; with q = 5, 8, 16 and 24: 15, 15, 15, 14; 42, 28, 18, 16.  Last
 //! two dimensions swapped, p = q = 16, 32, 40, 48 and 64: 17, 16, 16, 16, 18; 27,
-//! 16, 18, 15, 15.  fill: elements that a tile must hold on the average, 144
-//! where the list is kept, 512 where it is made for one product (7 ns an item).
-void choose_tiles(dev::perm_desc &d, uint64_t fill) {
+//! 16, 18, 15, 15.  fill: elements that a tile must hold on the average, least: in
+//! all; 144 and 2^19 where the list is kept, 512 and 2^22 where it is made and
+//! uploaded for one product (7 ns an item and about 35 us, where a product by
+//! elements passes its descriptor with the launch).
+void choose_tiles(dev::perm_desc &d, uint64_t fill, uint32_t least) {
     if(d.tile_p < 0) return;
     const uint64_t p = d.tdp.d, q = d.tdq.d;
     const uint64_t s = d.tile_s = std::min(p, q) > dev::kPermTile ? dev::kPermTileMax : dev::kPermTile;
     const uint64_t tiles = ((p + s - 1) / s) * ((q + s - 1) / s);
-    if(d.total < (1u << 19) || std::min(p, q) < 8 || p * q < fill * tiles || (q <= 24 && d.dps.d == q) ||
+    if(d.total < least || std::min(p, q) < 8 || p * q < fill * tiles || (q <= 24 && d.dps.d == q) ||
         8 * uint64_t(d.tsq) * q <= 16384) d.tile_p = -1;
 }
 
@@ -65,17 +67,28 @@ double run_dot(context &ctx, const context::cached_launch &l) {
 } // unnamed namespace
 
 double dense_dotprod(context &ctx, dev::perm_desc d) {
-    choose_tiles(d, 512);
+    if(!d.total) return 0.0;
+    choose_tiles(d, 512, 1u << 22);
+    if(d.tile_p < 0) {
+        const size_t n = (d.total + dev::kPermChunk - 1) / dev::kPermChunk;
+        double *out, r = 0.0;
+        std::lock_guard<std::mutex> lk(ctx.staging_lock());
+        double *part = (double*)ctx.staging(dot_bytes(n));
+        out = part + std::min<size_t>(n, dev::kDotGroups);
+        ctx.activate();
+        hip_check(dev::launch_dot_one(d, part, out, ctx.stream()), "dot");
+        ctx.download(&r, out, sizeof(double));
+        return r;
+    }
     std::vector<uint32_t> cd, co;
     make_chunks(std::vector<dev::perm_desc>(1, d), cd, co);
-    if(cd.empty()) return 0.0;
     // descriptor and work items in the staging area, partial sums behind them
     context::cached_launch::segment g;
     g.o_d = 0;
     g.o_cd = (sizeof(d) + 255) & ~size_t(255);
     g.o_co = g.o_cd + ((4 * cd.size() + 255) & ~size_t(255));
     g.nchunks = cd.size();
-    g.tiles = d.tile_p >= 0;
+    g.tiles = true;
     const size_t bytes = g.o_co + ((4 * co.size() + 255) & ~size_t(255));
     std::vector<char> host(bytes, 0);
     std::memcpy(&host[0], &d, sizeof(d));
@@ -129,7 +142,7 @@ double btod_dotprod(btensor &a, const tensor_tr &tra0, btensor &b, const tensor_
         dev::perm_desc d = make_perm_desc_public(b.block_ptr(sb.acidx), dyb, t,
             a.block_ptr(sa.acidx), false);
         d.alpha *= ta.st.c * ta.st.c;
-        choose_tiles(d, 144);
+        choose_tiles(d, 144, 1u << 19);
         descs.push_back(d);
     }
     l = upload_launches(ctx, lists);

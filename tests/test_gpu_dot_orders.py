@@ -12,7 +12,8 @@ CASES = [((n, 2 ** 19 // n ** 2 + 9, n), (2, 1, 0)) for n in (7, 8, 11, 12, 31, 
 CASES += [((n, 80000), (1, 0)) for n in (7, 8, 24, 25)] + [((80000, n), (1, 0)) for n in (7, 8, 24, 25)]
 CASES += [((2 ** 19 // n ** 2 + 1, n, n), (0, 2, 1)) for n in (44, 45, 46, 65)]
 CASES += [((725, 724), (1, 0)), ((724, 724), (1, 0)), ((725, 5, 145), (2, 0, 1)), ((3, 5, 2, 7, 4), (4, 2, 0, 3, 1)),
-          ((2100, 2000), (0, 1)), ((4100, 1025), (0, 1)), ((129, 257, 129), (1, 0, 2))]
+          ((2100, 2000), (0, 1)), ((4100, 1025), (0, 1)), ((129, 257, 129), (1, 0, 2)),
+          ((25, 6800, 25), (2, 1, 0)), ((22, 8700, 22), (2, 1, 0)), ((2050, 2050), (1, 0)), ((33, 3860, 33), (2, 1, 0))]
 
 
 @pytest.mark.parametrize("dims,perm", CASES, ids=str)
