@@ -342,11 +342,12 @@ __device__ __forceinline__ double dot_gather(const perm_desc &d, uint32_t base) 
 #pragma unroll
         for(int i = 0; i < E; i++) acc += w[i] * v[i];
     } else {
+        const perm_desc g = d;               // (all of it at once, where all is read)
 #pragma unroll
         for(int i = 0; i < E; i++) {
             const uint32_t e = min(base + threadIdx.x + 256u * i, end - 1);
-            v[i] = d.src[src_offset(d, e)];
-            w[i] = d.dst[e];
+            v[i] = g.src[src_offset(g, e)];
+            w[i] = g.dst[e];
         }
 #pragma unroll
         for(int i = 0; i < E; i++)
@@ -381,7 +382,7 @@ dot_kernel(const perm_desc *__restrict__ descs,
     double sum = 0.0;
     for(uint32_t ch = c0; ch < c1; ch++) {
         const uint32_t cd = chunk_desc[ch];
-        const perm_desc d = descs[cd & ~kPermTileItem];
+        const perm_desc &d = descs[cd & ~kPermTileItem];
         const uint32_t base = chunk_off[ch];
         double acc = 0.0;
         if(TILES && (cd & kPermTileItem)) {

@@ -105,25 +105,27 @@ void context::activate() const {
 std::shared_ptr<context::cached_launch> context::find_launch(const std::string &key, launch_set set) {
     std::lock_guard<std::mutex> lk(m_cache_mtx);
     launch_cache &c = m_launches[set];
-    std::map<std::string, std::shared_ptr<cached_launch> >::iterator i = c.lists.find(key);
+    std::map<std::string, launch_cache::entry>::iterator i = c.lists.find(key);
     if(i == c.lists.end()) return std::shared_ptr<cached_launch>();
-    c.used(key);
-    return i->second;
+    i->second.used = ++c.clock;
+    return i->second.l;
 }
 
 void context::keep_launch(const std::string &key, std::shared_ptr<cached_launch> l, launch_set set) {
-    std::vector<std::shared_ptr<cached_launch> > drop;    // let go outside the lock
+    std::shared_ptr<cached_launch> drop[2];               // let go outside the lock
     {
         std::lock_guard<std::mutex> lk(m_cache_mtx);
         launch_cache &c = m_launches[set];
-        std::shared_ptr<cached_launch> &e = c.lists[key];
-        if(e) drop.push_back(e);
-        e = l;
-        c.used(key);
-        while(c.order.size() > c.max) {
-            drop.push_back(c.lists[c.order.front()]);
-            c.lists.erase(c.order.front());
-            c.order.erase(c.order.begin());
+        launch_cache::entry &e = c.lists[key];
+        drop[0].swap(e.l);
+        e.l = l;
+        e.used = ++c.clock;
+        if(c.lists.size() > c.max) {
+            std::map<std::string, launch_cache::entry>::iterator old = c.lists.begin();
+            for(std::map<std::string, launch_cache::entry>::iterator i = c.lists.begin(); i != c.lists.end(); ++i)
+                if(i->second.used < old->second.used) old = i;
+            drop[1].swap(old->second.l);
+            c.lists.erase(old);
         }
     }
 }
@@ -131,13 +133,10 @@ void context::keep_launch(const std::string &key, std::shared_ptr<cached_launch>
 //! Lets go of every kept list (one in use goes with its last user); false if
 //! there was none.
 bool context::drop_launches() {
-    std::map<std::string, std::shared_ptr<cached_launch> > drop[2];
+    std::map<std::string, launch_cache::entry> drop[2];
     {
         std::lock_guard<std::mutex> lk(m_cache_mtx);
-        for(int i = 0; i < 2; i++) {
-            drop[i].swap(m_launches[i].lists);
-            m_launches[i].order.clear();
-        }
+        for(int i = 0; i < 2; i++) drop[i].swap(m_launches[i].lists);
     }
     return !drop[0].empty() || !drop[1].empty();
 }

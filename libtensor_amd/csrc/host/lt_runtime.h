@@ -3,7 +3,6 @@
 // tensors, and the btod_contract2 operation with its cached execution plan.
 #pragma once
 
-#include <algorithm>
 #include <atomic>
 #include <functional>
 #include <map>
@@ -118,16 +117,12 @@ private:
     std::mutex m_xfer_mtx;
     std::mutex m_cache_mtx;
     struct launch_cache {
+        struct entry { std::shared_ptr<cached_launch> l; uint64_t used; };
         size_t max;
-        std::map<std::string, std::shared_ptr<cached_launch> > lists;
-        std::vector<std::string> order;      // least recently used first
-        void used(const std::string &key) {
-            std::vector<std::string>::iterator i = std::find(order.begin(), order.end(), key);
-            if(i != order.end()) order.erase(i);
-            order.push_back(key);
-        }
+        uint64_t clock;                      // of uses
+        std::map<std::string, entry> lists;
     };
-    launch_cache m_launches[2] = { { 32, {}, {} }, { 64, {}, {} } };
+    launch_cache m_launches[2] = { { 32, 0, {} }, { 64, 0, {} } };
     bool drop_launches();
     void *try_alloc(size_t bytes, std::string &why);
     size_t m_cap;
