@@ -212,13 +212,9 @@ hipError_t launch_gemm_stacked(int cfg, const stack_desc *st, const stack_pair *
     const stack_arow *ar, const stack_crow *cr, const gemm_tile *tiles, uint32_t ntiles,
     hipStream_t s);
 
-//! Batched permutation: work item j is chunk_desc[j] / chunk_off[j]: a
-//! descriptor and the first destination element of a chunk of kPermChunk
-//! elements, or (chunk_desc[j] | kPermTileItem) and the destination index
-//! of a tile's corner for transposing descriptors.
 //! What a list of descriptors needs of the kernel: stores past the caches
 //! (kPermStream), tiles (the largest tile_s of them, 0: no item is a tile),
-//! sums (`add` of some descriptor), tiles as runs (perm_runs of some, read
+//! sums (`add` of some descriptor), tiles as runs (perm_runs of some sum, read
 //! with stream only).
 struct perm_kind { bool stream, add, runs; uint32_t tile; };
 //! Tiles with rows shorter than the tile that adjoin in memory.  Launches past
@@ -230,6 +226,10 @@ struct perm_kind { bool stream, add, runs; uint32_t tile; };
 inline bool perm_runs(const perm_desc &d) {
     return d.tile_p >= 0 && ((d.tdp.d < d.tile_s && d.tsq == d.tdp.d) || (d.tdq.d < d.tile_s && d.dps.d == d.tdq.d));
 }
+//! Batched permutation: work item j is chunk_desc[j] / chunk_off[j]: a
+//! descriptor and the first destination element of a chunk of kPermChunk
+//! elements, or (chunk_desc[j] | kPermTileItem) and the destination index
+//! of a tile's corner for transposing descriptors.
 hipError_t launch_permute(const perm_desc *descs, const uint32_t *chunk_desc,
     const uint32_t *chunk_off, uint32_t nchunks, hipStream_t s, perm_kind kind);
 static const uint32_t kPermChunk = 2048;
